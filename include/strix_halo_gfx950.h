@@ -90,6 +90,15 @@ extern "C" {
  * workgroup, which limits int4 per-channel calls to K <= 523776.  Results
  * are identical either way. */
 #define SHK_OPERANDS_STREAM 2
+/* FP6_EDGE entries (int4; block_m 16 or 64, block_n 64) run the fp6 tiles on
+ * shapes that are no multiple of them: the operands are converted with their
+ * rows padded to 32 and K to 128, and the output stops at M and N.  They take
+ * a workspace as FP6 entries do, of 3/4 byte per padded value, and K up to
+ * 262144; the conversion is part of the launch.  Launched without a workspace
+ * (or, by the no-allocation entry point, with one that does not fit its
+ * scratch), the call runs on the best entry of the same family that needs
+ * none; the results are the same. */
+#define SHK_OPERANDS_FP6_EDGE 3
 
 /* Tile schedules of a dense entry (reference metadata.KernelSchedule,
  * metadata.py:51-53).  STANDARD launches one workgroup per output tile;

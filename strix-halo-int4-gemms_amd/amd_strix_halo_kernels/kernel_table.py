@@ -49,6 +49,10 @@ OPERANDS_FP6 = 1
 # workgroups when given a zero-filled workspace (every launch leaves what it
 # used zero, counters and partials): sk_split_count / sk_workspace_bytes.
 OPERANDS_STREAM = 2
+# FP6_EDGE entries run the fp6 tiles on shapes that are no multiple of them:
+# the operands are converted with rows padded to 32 and K to 128, and the
+# output stops at M and N.
+OPERANDS_FP6_EDGE = 3
 FP6_MAX_K = 262144
 # Largest K of the fp6 entries (32-bit buffer offsets of a tile's panels);
 # per-channel calls with K > FP6_MAX_K run in exact K slices of FP6_MAX_K
@@ -102,7 +106,7 @@ class KernelDesc:
 
     @property
     def needs_workspace(self) -> bool:
-        return self.operand_format == OPERANDS_FP6
+        return self.operand_format in (OPERANDS_FP6, OPERANDS_FP6_EDGE)
 
     @property
     def is_stream(self) -> bool:
@@ -120,6 +124,9 @@ class KernelDesc:
         if not self.needs_workspace:
             return 0
         b_cols = 2 * n if self.epilogue_kind == EPI_KIND_SWIGLU else n
+        if self.operand_format == OPERANDS_FP6_EDGE:
+            kw = -(-k // 128) * 128
+            return ((-(-m // 32) + -(-b_cols // 32)) * 32 * kw * 3) // 4
         nbytes = (m * k * 3) // 4 + (b_cols * k * 3) // 4
         if self.scale_mode == SCALE_PER_CHANNEL and k > FP6_MAX_K:
             nbytes += 4 * m * b_cols
@@ -133,6 +140,8 @@ class KernelDesc:
             return None
         if self.is_stream:
             return FP6_MAX_K_SLICED if (self.dtype_bits == 4 and self.scale_mode == SCALE_PER_CHANNEL) else None
+        if self.operand_format == OPERANDS_FP6_EDGE:
+            return FP6_MAX_K
         if self.operand_format == OPERANDS_FP6:
             if self.scale_mode == SCALE_PER_CHANNEL and self.schedule == SCHEDULE_PERSISTENT:
                 return FP6_MAX_K
@@ -289,6 +298,15 @@ def _sk_desc(index, bits, layout, r, *, swiglu=False, subch=False, schedule=SCHE
         group_size_m=1, operand_format=OPERANDS_STREAM, schedule=schedule, split_k=split_k)
 
 
+def _edge_desc(index, layout, bm, *, swiglu=False):
+    # a 256-row per-channel fp6 tile's ring (_desc), at its granularity
+    return KernelDesc(
+        index=index, family=FAMILY_DENSE, dtype_bits=4, layout=layout, scale_mode=SCALE_PER_CHANNEL,
+        min_subchannel=0, max_subchannel=0, epilogue_kind=EPI_KIND_SWIGLU if swiglu else EPI_KIND_PLAIN,
+        block_m=bm, block_n=64, block_k=32, num_waves=4, num_stages=3,
+        lds_bytes=3 * (256 + 256) * 96 + MFMA32_SCALE_BYTES, group_size_m=8, operand_format=OPERANDS_FP6_EDGE)
+
+
 def _build() -> tuple[KernelDesc, ...]:
     out: list[KernelDesc] = []
 
@@ -368,10 +386,19 @@ def _build() -> tuple[KernelDesc, ...]:
                 for r in (16, 32, 64):
                     for subch in (False, True):
                         add_sk(bits, layout, r, subch=subch, split_k=split)
+    # fp6 entries for shapes that are no tile multiples (k_f6.hip)
+    for layout in (LAYOUT_NN, LAYOUT_NT, LAYOUT_TN):
+        for bm in (64, 16):
+            for swiglu in (False, True):
+                out.append(_edge_desc(len(out), layout, bm, swiglu=swiglu))
     return tuple(out)
 
 
 TABLE: tuple[KernelDesc, ...] = _build()
+
+
+# Dense entries whose operands can be converted apart from their GEMM.
+FP6_INDICES = frozenset(d.index for d in TABLE if d.family == FAMILY_DENSE and d.operand_format == OPERANDS_FP6)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -421,10 +448,81 @@ SKINNY_SUB_TOPS = {16: 96.0, 32: 184.0, 64: 152.0}
 SKINNY_SUB_MAX_M = 256
 
 
-def selection_tops(desc: KernelDesc, m: int) -> float | None:
-    """measured_tops as select ranks an entry for M rows (capi.hip
-    measured_score): the skinny subchannel tiles' figure holds up to
+# CUs of an MI355X: a round of one workgroup each (shk_table.h kF6EdgeCus).
+_CUS = 256
+
+
+def _f6_edge_us(m: int, n: int, k: int, swiglu: bool) -> float:
+    """GEMM time (us) of an FP6_EDGE per-channel call as the launcher splits
+    it (shk_table.h f6_edge_plan): 256-row tiles, half-height ones in a
+    partial last round that holds them, or 128 x 128 tiles."""
+    k1 = k / 1024.0
+    bn = 128 if swiglu else 256
+    tm, tn, tm2 = -(-m // 256), -(-n // bn), -(-m // 128)
+    rounds, rest = divmod(tm * tn, _CUS)
+    round_us = 14.0 + 4.9 * k1
+    us = round_us * (rounds + (1 if rest else 0))
+    if rest:
+        c = tn if rounds == 0 else -(-rest // tm)
+        if tm2 * c <= _CUS:
+            us = round_us * (rounds + 0.6)
+    if not swiglu:
+        small = (2.6 + 2.05 * k1) * -(-(tm2 * -(-n // 128)) // _CUS)
+        us = min(us, small)
+    return us
+
+
+PREDICT_MAX_K = 65536  # K up to which the fits of predicted_us stand
+
+_SKINNY_US = {  # (tile rows, SwiGLU): us per tile and us per tile and K value
+    (64, False): (0.005, 5.2e-6), (32, False): (0.0035, 3.75e-6), (16, False): (0.0028, 2.65e-6),
+    (64, True): (0.019, 1.1e-5), (32, True): (0.0125, 7.0e-6), (16, True): (0.0045, 4.3e-6),
+}
+
+
+def predicted_us(desc: KernelDesc, m: int, n: int, k: int) -> float | None:
+    """Predicted time of a standard int4 per-channel call on an entry, in us
+    (None for the other families and K past PREDICT_MAX_K); capi.hip computes
+    the skinny and FP6_EDGE entries' alike.  Fits to calls measured over M 64..8176 and N x K of 1024 x 4096,
+    4096 x 1024, 4096^2, 11008 x 4096, 16384 x 4096 and 8192^2:
+
+    * skinny tiles: a launch, then at least one round of tiles (few tiles
+      split K instead), each a fixed part and a part along K; the tallest
+      tile that divides M;
+    * fp6 entries: two launches, the conversion at 5 TB/s, then rounds of
+      256-row tiles (FP6) or the launcher's split (FP6_EDGE).
+
+    Measured against predicted: 512 x 4096^2 skinny 16.6 (18), 256-row fp6
+    36.7 (44), edge 24.7 (22); 8176 x 16384 x 4096 skinny 1675 (1791), edge
+    324 (300); 8192^3 fp6 277 (251)."""
+    if (desc.family != FAMILY_DENSE or desc.dtype_bits != 4 or desc.scale_mode != SCALE_PER_CHANNEL
+            or desc.schedule != SCHEDULE_STANDARD or desc.split_k > 1 or k > PREDICT_MAX_K):
+        return None
+    swiglu = desc.epilogue_kind == EPI_KIND_SWIGLU
+    if desc.operand_format == OPERANDS_STREAM:
+        r = 64 if m % 64 == 0 else (32 if m % 32 == 0 else 16)
+        base, per_k = _SKINNY_US[r, swiglu]
+        return 5.0 + max((m // r) * (n // 64), _CUS) * (base + per_k * k)
+    convert = 6.0 + 2.5e-7 * ((m + (2 * n if swiglu else n)) * k)
+    if desc.operand_format == OPERANDS_FP6_EDGE:
+        return convert + _f6_edge_us(m, n, k, swiglu)
+    if desc.operand_format == OPERANDS_FP6:
+        tiles = (m // desc.block_m) * (n // desc.block_n)
+        return convert + (14.0 + 4.9 * (k / 1024.0)) * -(-tiles // _CUS)
+    return None
+
+
+def selection_tops(desc: KernelDesc, m: int, n: int | None = None, k: int | None = None) -> float | None:
+    """The throughput by which select ranks an entry for a shape (capi.hip
+    measured_score): an int4 per-channel skinny or FP6_EDGE entry's predicted
+    one, below the FP6 entries' figures (a caller of the separate conversion
+    needs an FP6 entry where one fits); for the others, or without n and k,
+    measured_tops, where the skinny subchannel tiles' figure holds up to
     SKINNY_SUB_MAX_M rows."""
+    if n is not None and k is not None and desc.operand_format != OPERANDS_FP6:
+        us = predicted_us(desc, m, n, k)
+        if us is not None:
+            return min(3000.0, 2.0 * float(m) * float(n) * float(k) / us / 1e6)
     tops = measured_tops(desc)
     if (tops is not None and desc.operand_format == OPERANDS_STREAM and desc.scale_mode == SCALE_SUBCHANNEL
             and m > SKINNY_SUB_MAX_M):

@@ -4,8 +4,9 @@ Same selection contract as the reference's KernelRegistry (registry.py:254-352):
 candidates must match dtype, scale spec, epilogue, layout and schedule, be
 even-K, obey the split rule, and (for ``select``) accept the shape as a tile
 multiple; among them the one with the largest (measured_tops or 0,
-BLOCK_M * BLOCK_N) wins, the first on ties (the skinny subchannel tiles'
-figure counts up to kernel_table.SKINNY_SUB_MAX_M rows).  The entries come from the gfx950
+BLOCK_M * BLOCK_N) wins, the first on ties.  measured_tops is the table's
+figure for the request's shape (kernel_table.selection_tops) unless a caller
+set another.  The entries come from the gfx950
 kernel table (``kernel_table.TABLE``) instead of gfx1151 tile seeds: every
 dense table entry is registered once per epilogue and subchannel size it
 serves.
@@ -104,12 +105,12 @@ def iter_supported_kernel_metadata() -> Iterable[KernelMetadata]:
                 )
 
 
-def _selection_key(kernel: KernelMetadata, m: int) -> tuple[float, int]:
+def _selection_key(kernel: KernelMetadata, m: int, n: int | None = None, k: int | None = None) -> tuple[float, int]:
     tops = kernel.measured_tops
-    if tops is not None and kernel.table_index is not None and m > kt.SKINNY_SUB_MAX_M:
+    if kernel.table_index is not None:
         desc = kt.TABLE[kernel.table_index]
-        if desc.operand_format == kt.OPERANDS_STREAM and desc.scale_mode == kt.SCALE_SUBCHANNEL:
-            tops = None  # the skinny subchannel figure holds for few rows only (kernel_table.selection_tops)
+        if tops == kt.measured_tops(desc):  # not a caller's own figure (with_status)
+            tops = kt.selection_tops(desc, m, n, k)
     return (tops or 0.0, kernel.tile.block_m * kernel.tile.block_n)
 
 
@@ -143,6 +144,7 @@ class KernelRegistry:
         # are indexed by family.  register() clears both.
         self._families: dict[tuple, list[KernelMetadata]] | None = None
         self._selected: dict[tuple, KernelMetadata] = {}
+        self._call_kernels: dict[tuple, KernelMetadata] = {}
         for kernel in kernels:
             self.register(kernel)
 
@@ -152,6 +154,7 @@ class KernelRegistry:
         self._kernels[kernel.kernel_id] = kernel
         self._families = None
         self._selected = {}
+        self._call_kernels = {}
 
     def _family(self, dtype, scale, epilogue, layout, schedule) -> list[KernelMetadata]:
         families = self._families
@@ -203,10 +206,42 @@ class KernelRegistry:
                 f"no kernel for dtype={dtype.value}, scale={scale.label}, epilogue={epilogue.value}, "
                 f"layout={layout.value}, schedule={schedule.value}, shape=({m}, {n}, {k})"
             )
-        chosen = max(candidates, key=lambda kern: _selection_key(kern, m))
+        chosen = max(candidates, key=lambda kern: _selection_key(kern, m, n, k))
         if len(self._selected) >= 4096:  # bounded for callers that vary M call to call
             self._selected = {}
         self._selected[request] = chosen
+        return chosen
+
+    def call_kernel(self, kernel: KernelMetadata, *, m: int, n: int, k: int) -> KernelMetadata:
+        """The kernel that a whole call runs where select() picked `kernel`.
+
+        select() keeps the FP6 entries for every shape they accept, since the
+        separate conversion needs them.  A whole call is free to take any
+        entry with the same results, and on few tiles of 256 rows another one
+        is faster (512 x 4096 x 4096: FP6 36.7 us, skinny 16.6; 512 x 16384 x
+        4096: FP6 47.4, FP6_EDGE 41.9), so the smallest predicted time
+        decides (kernel_table.predicted_us).  Kernels with a figure of the
+        caller's own (with_status) stay."""
+        index = kernel.table_index
+        if index is None or kt.TABLE[index].operand_format != kt.OPERANDS_FP6:
+            return kernel
+        request = (kernel.kernel_id, m, n, k)
+        hit = self._call_kernels.get(request)
+        if hit is not None:
+            return hit
+        chosen = kernel
+        best = kt.predicted_us(kt.TABLE[index], m, n, k)
+        if best is not None and kernel.measured_tops == kt.measured_tops(kt.TABLE[index]):
+            shape = LaunchShape(m, n, k)
+            for other in self._family(kernel.a_dtype, kernel.scale, kernel.epilogue, kernel.layout, kernel.schedule):
+                if other.table_index is None or other.tile.split_k != 1 or not is_tile_multiple_shape(other, shape):
+                    continue
+                us = kt.predicted_us(kt.TABLE[other.table_index], m, n, k)
+                if us is not None and (us, -other.tile.block_m) < (best, -chosen.tile.block_m):
+                    chosen, best = other, us
+        if len(self._call_kernels) >= 4096:
+            self._call_kernels = {}
+        self._call_kernels[request] = chosen
         return chosen
 
     def select_reference(

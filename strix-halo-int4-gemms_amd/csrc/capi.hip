@@ -1,6 +1,7 @@
 // C ABI of the gfx950 quantized GEMM library: kernel table, argument
 // validation, launch geometry and error reporting.  Declarations and the
 // reference interface each symbol replaces are in include/strix_halo_gfx950.h.
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -113,6 +114,9 @@ const std::vector<Entry>& table() {
     shk::append_skinny_8_0(v);
     shk::append_skinny_8_1(v);
     shk::append_skinny_8_2(v);
+    shk::append_edge_f6(v, SHK_LAYOUT_NN);
+    shk::append_edge_f6(v, SHK_LAYOUT_NT);
+    shk::append_edge_f6(v, SHK_LAYOUT_TN);
     for (size_t i = 0; i < v.size(); ++i) v[i].d.index = (int32_t)i;
     return v;
   }();
@@ -215,8 +219,11 @@ int check_out_mode(int out_mode) {
 // nothing otherwise.
 uint64_t dense_workspace_bytes(const shk_kernel_desc& d, int32_t m, int32_t n, int32_t k) {
   if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_workspace_bytes(d, m, n, k);
-  if (d.operand_format != SHK_OPERANDS_FP6) return 0;
   const long b_cols = d.epilogue_kind == SHK_EPI_KIND_SWIGLU ? 2L * n : (long)n;
+  if (d.operand_format == SHK_OPERANDS_FP6_EDGE)
+    return shk::f6_operand_bytes(shk::f6_pad_rows(m), shk::f6_pad_k(k)) +
+           shk::f6_operand_bytes(shk::f6_pad_rows(b_cols), shk::f6_pad_k(k));
+  if (d.operand_format != SHK_OPERANDS_FP6) return 0;
   uint64_t bytes = shk::f6_operand_bytes(m, k) + shk::f6_operand_bytes(b_cols, k);
   if (d.scale_mode == SHK_SCALE_PER_CHANNEL && k > shk::F6_MAX_K) bytes += 4ull * (uint64_t)m * (uint64_t)b_cols;
   return bytes;
@@ -237,6 +244,7 @@ constexpr int kMaxInt4AccK = 131071;
 long dense_max_k(const shk_kernel_desc& d) {
   if (d.operand_format == SHK_OPERANDS_STREAM)
     return (d.dtype_bits == 4 && d.scale_mode == SHK_SCALE_PER_CHANNEL) ? shk::F6_MAX_K_SLICED : 0x7FFFFFFFL;
+  if (d.operand_format == SHK_OPERANDS_FP6_EDGE) return shk::F6_MAX_K;
   if (d.operand_format == SHK_OPERANDS_FP6)
     return (d.scale_mode == SHK_SCALE_PER_CHANNEL && d.schedule == SHK_SCHEDULE_PERSISTENT) ? shk::F6_MAX_K
                                                                                             : shk::F6_MAX_K_SLICED;
@@ -267,11 +275,14 @@ int prepare_dense(DenseCall& c, int kernel_index, Phase phase, const void* a, co
                   int32_t epilogue, int32_t out_mode, void* workspace, uint64_t workspace_bytes) {
   if (lookup(kernel_index, SHK_FAMILY_DENSE, &c.e)) return 1;
   const shk_kernel_desc& d = c.e->d;
-  const bool fp6 = d.operand_format == SHK_OPERANDS_FP6;
+  const bool edge = d.operand_format == SHK_OPERANDS_FP6_EDGE;
+  const bool fp6 = d.operand_format == SHK_OPERANDS_FP6 || edge;
   const bool stream = d.operand_format == SHK_OPERANDS_STREAM;
   const bool uses_a = phase == PHASE_ALL || phase == PHASE_CONVERT_A;
   const bool uses_b = phase == PHASE_ALL || phase == PHASE_CONVERT_B;
   const bool gemm = phase == PHASE_ALL || phase == PHASE_GEMM;
+  if (phase != PHASE_ALL && edge)
+    return fail("kernel " + std::to_string(kernel_index) + " converts its operands in the same call as its GEMM");
   if (phase != PHASE_ALL && !fp6)
     return fail("kernel " + std::to_string(kernel_index) +
                 " reads its operands directly; only fp6 entries convert them separately");
@@ -500,11 +511,40 @@ int amd_strix_halo_kernels_kernel_table_entry(int index, shk_kernel_desc* out) {
 
 namespace {
 
+// Predicted time (us) of a standard int4 per-channel call on a skinny or
+// FP6_EDGE entry, from fits to measured calls (kernel_table.predicted_us
+// states them); negative where there is none.
+constexpr long kPredictMaxK = 65536;
+double predicted_us(const shk_kernel_desc& d, long m, long n, long k) {
+  if (d.family != SHK_FAMILY_DENSE || d.dtype_bits != 4 || d.scale_mode != SHK_SCALE_PER_CHANNEL ||
+      d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1 || k > kPredictMaxK)
+    return -1.0;
+  const bool swiglu = d.epilogue_kind == SHK_EPI_KIND_SWIGLU;
+  if (d.operand_format == SHK_OPERANDS_STREAM) {
+    const long r = m % 64 == 0 ? 64 : (m % 32 == 0 ? 32 : 16);
+    const long tiles = (m / r) * (n / 64);
+    const double base = swiglu ? (r == 64 ? 0.019 : (r == 32 ? 0.0125 : 0.0045))
+                               : (r == 64 ? 0.005 : (r == 32 ? 0.0035 : 0.0028));
+    const double per_k = swiglu ? (r == 64 ? 1.1e-5 : (r == 32 ? 7.0e-6 : 4.3e-6))
+                                : (r == 64 ? 5.2e-6 : (r == 32 ? 3.75e-6 : 2.65e-6));
+    return 5.0 + (double)(tiles > 256 ? tiles : 256) * (base + per_k * (double)k);
+  }
+  if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
+  const double convert = 6.0 + 2.5e-7 * (double)((m + (swiglu ? 2 * n : n)) * k);
+  return convert + shk::f6_edge_plan(m, n, k, swiglu).us;
+}
+
 // Throughput measured on MI355X for the entries the benchmark configurations
-// time (the Python registry's kernel_table.measured_tops): the first
-// ranking key of a selection, before the tile area.
-double measured_score(const shk_kernel_desc& d, int m) {
+// time (the Python registry's kernel_table.selection_tops): the first
+// ranking key of a selection, before the tile area.  Int4 per-channel skinny
+// and FP6_EDGE entries rank by their predicted throughput for the shape,
+// below the FP6 entries where those accept it (a caller of the separate
+// conversion needs an FP6 entry).
+double measured_score(const shk_kernel_desc& d, int m, int n, int k) {
   if (d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1) return 0.0;
+  const double us = predicted_us(d, m, n, k);
+  if (us > 0.0) return std::min(3000.0, 2.0 * (double)m * (double)n * (double)k / us / 1e6);
+  if (d.operand_format == SHK_OPERANDS_FP6_EDGE) return 0.0;
   if (d.operand_format == SHK_OPERANDS_FP6) {
     if (d.scale_mode == SHK_SCALE_SUBCHANNEL) return 2001.0;
     return d.epilogue_kind == SHK_EPI_KIND_PLAIN ? 3504.0 : 3161.0;
@@ -546,6 +586,48 @@ bool accepts_shape(const shk_kernel_desc& d, int m, int n, int k, int subchannel
   return k <= dense_max_k(d);
 }
 
+// The best entry that serves a request and its shape, or -1; `direct`: of
+// those that read the packed operands (no converted workspace).
+int best_entry(int bits, int layout, int subchannel, int epilogue, int schedule, int split_k, int m, int n, int k,
+               bool direct) {
+  const auto& t = table();
+  int best = -1;
+  double best_score = -1.0;
+  long best_area = -1;
+  for (int i = 0; i < (int)t.size(); ++i) {
+    const shk_kernel_desc& d = t[i].d;
+    if (!serves_family(d, bits, layout, subchannel, epilogue, schedule, split_k)) continue;
+    if (!accepts_shape(d, m, n, k, subchannel)) continue;
+    if (direct && d.operand_format != SHK_OPERANDS_PACKED && d.operand_format != SHK_OPERANDS_STREAM) continue;
+    const double score = measured_score(d, m, n, k);
+    const long area = (long)d.block_m * d.block_n;
+    if (score > best_score || (score == best_score && area > best_area)) {
+      best = i;
+      best_score = score;
+      best_area = area;
+    }
+  }
+  return best;
+}
+
+// The entry a launch runs.  An FP6_EDGE entry without room for its converted
+// operands (`room` bytes) gives way to the best entry of its family that
+// reads the packed operands, so a caller that has no workspace is served as
+// without the FP6_EDGE entries.  Requests that the entry itself refuses keep
+// it, for its error.
+int runnable_entry(int kernel_index, int m, int n, int k, int subchannel, int epilogue, uint64_t room) {
+  const auto& t = table();
+  if (kernel_index < 0 || kernel_index >= (int)t.size()) return kernel_index;
+  const shk_kernel_desc& d = t[kernel_index].d;
+  if (d.operand_format != SHK_OPERANDS_FP6_EDGE || m <= 0 || n <= 0 || k <= 0) return kernel_index;
+  if (dense_workspace_bytes(d, m, n, k) <= room) return kernel_index;
+  if (!serves_family(d, d.dtype_bits, d.layout, subchannel, epilogue, d.schedule, 0) ||
+      !accepts_shape(d, m, n, k, subchannel))
+    return kernel_index;
+  const int other = best_entry(d.dtype_bits, d.layout, subchannel, epilogue, d.schedule, 1, m, n, k, true);
+  return other < 0 ? kernel_index : other;
+}
+
 }  // namespace
 
 int amd_strix_halo_kernels_select_dense(int32_t dtype_bits, int32_t layout, int32_t subchannel, int32_t epilogue,
@@ -564,22 +646,7 @@ int amd_strix_halo_kernels_select_dense(int32_t dtype_bits, int32_t layout, int3
   if (m <= 0 || n <= 0 || k <= 0)
     return fail("M, N, and K must be positive; got (" + std::to_string(m) + ", " + std::to_string(n) + ", " +
                 std::to_string(k) + ")");
-  const auto& t = table();
-  int best = -1;
-  double best_score = -1.0;
-  long best_area = -1;
-  for (int i = 0; i < (int)t.size(); ++i) {
-    const shk_kernel_desc& d = t[i].d;
-    if (!serves_family(d, dtype_bits, layout, subchannel, epilogue, schedule, split_k)) continue;
-    if (!accepts_shape(d, m, n, k, subchannel)) continue;
-    const double score = measured_score(d, m);
-    const long area = (long)d.block_m * d.block_n;
-    if (score > best_score || (score == best_score && area > best_area)) {
-      best = i;
-      best_score = score;
-      best_area = area;
-    }
-  }
+  const int best = best_entry(dtype_bits, layout, subchannel, epilogue, schedule, split_k, m, n, k, false);
   if (best < 0)
     return fail("no kernel for dtype_bits=" + std::to_string(dtype_bits) + ", subchannel=" +
                 std::to_string(subchannel) + ", epilogue=" + std::to_string(epilogue) + ", layout=" +
@@ -615,6 +682,7 @@ int amd_strix_halo_kernels_launch_gemm_ws(int kernel_index, int device_index, ui
                                           int32_t out_mode, void* workspace, uint64_t workspace_bytes) {
   g_last_error.clear();
   DenseCall c;
+  if (workspace == nullptr) kernel_index = runnable_entry(kernel_index, m, n, k, subchannel, epilogue, 0);
   if (prepare_dense(c, kernel_index, PHASE_ALL, a, b, a_scale, b_scale, out, m, n, k, subchannel, epilogue,
                     out_mode, workspace, workspace_bytes))
     return 1;
@@ -632,13 +700,14 @@ int amd_strix_halo_kernels_launch_gemm_noalloc(int kernel_index, int device_inde
                                                int32_t epilogue, int32_t out_mode) {
   g_last_error.clear();
   DenseCall c;
+  kernel_index = runnable_entry(kernel_index, m, n, k, subchannel, epilogue, SHK_NOALLOC_SCRATCH_BYTES);
   if (prepare_dense(c, kernel_index, PHASE_ALL, a, b, a_scale, b_scale, out, m, n, k, subchannel, epilogue,
                     out_mode, kScratchPending, SHK_NOALLOC_SCRATCH_BYTES))
     return 1;
   DeviceGuard guard(device_index);
   if (guard.error() != hipSuccess) return fail_hip("hipSetDevice", guard.error());
   const bool split_stream = c.e->d.operand_format == SHK_OPERANDS_STREAM && c.p.sk_splits > 1;
-  if (c.e->d.operand_format == SHK_OPERANDS_FP6 || split_stream) {
+  if (c.e->d.operand_format == SHK_OPERANDS_FP6 || c.e->d.operand_format == SHK_OPERANDS_FP6_EDGE || split_stream) {
     void* ptr = nullptr;
     if (scratch_address(device_index, &ptr)) return 1;
     c.p.work = static_cast<uint8_t*>(ptr);

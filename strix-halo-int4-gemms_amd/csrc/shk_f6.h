@@ -68,6 +68,11 @@ __host__ __device__ constexpr unsigned long long f6_operand_bytes(long rows, lon
   return (unsigned long long)rows * (unsigned long long)k * 3ull / 4ull;
 }
 
+// Rows and K of an operand in block format: whole 32-row panels and whole
+// 128-K stages.  The conversion fills the padding with zeros.
+__host__ __device__ constexpr long f6_pad_rows(long rows) { return (rows + 31) & ~31L; }
+__host__ __device__ constexpr long f6_pad_k(long k) { return (k + 127) & ~127L; }
+
 // One operand, or a batch of `groups` operands of the same shape (the
 // ragged path's per-expert matrices).  Rows past `rows` convert as zeros up
 // to the next 32-row panel.  K values at or past the operand's length
@@ -125,27 +130,40 @@ hipError_t launch_f6_pack2(const F6PackArgs& a, bool a_mn, const F6PackArgs& b, 
 //    odd MFMAs 1 .. 23 each carry one DMA load of stage k+3 into slot k % 3.
 // The DMA of a stage is thus issued two stages before its data is read.
 // A stage in LDS holds, per operand, eight 32-row panels of two blocks.
+//
+// 128-row tiles (C::BM == 128, MI = 2): the same columns, half the A rows.
+// A stage is 36 KiB (four A panels, eight B panels), every wave loads three
+// 1 KiB pieces of A and six of B, on the first nine of its 16 MFMAs, each
+// of which carries one or two of the 24 LDS reads.  They run the tiles of a
+// partial last round of 256-row tiles in about half its time
+// (f6_gemm_kernel).
 template <class C>
 struct F6Engine {
   static constexpr bool SWIGLU = C::SWIGLU;
   static constexpr int P = 3;
   static constexpr int NW = 4;
   static constexpr int PANEL = 2 * F6_BLOCK;     // 32 rows x 128 K: 3 KiB
-  static constexpr int OPB = 8 * PANEL;          // one operand's stage: 24 KiB
-  static constexpr int STAGE = 2 * OPB;          // 48 KiB
-  static constexpr int LDS_BYTES = P * STAGE;    // 144 KiB
-  static constexpr int DPW = STAGE / 1024 / NW;  // 12 DMA loads per wave per stage
+  static constexpr int MI = C::BM / 64;          // 32-row fragments per wave: 4 or 2
+  static constexpr int OPA = 2 * MI * PANEL;     // A's stage: 24 (12) KiB
+  static constexpr int OPB = 8 * PANEL;          // B's stage: 24 KiB
+  static constexpr int STAGE = OPA + OPB;        // 48 (36) KiB
+  static constexpr int LDS_BYTES = P * STAGE;    // 144 (108) KiB
+  static constexpr int DPW = STAGE / 1024 / NW;  // 12 (9) DMA loads per wave per stage
+  static constexpr int DPA = OPA / 1024 / NW;    // 128-row tiles: 3 of them of A, the rest of B
+  static constexpr int TICKS = 8 * MI;           // MFMAs per stage: two steps of MI x 4
+  static constexpr int READS = 4 * (MI + 4);     // LDS reads per stage
   static constexpr int TN = SWIGLU ? 64 : 128;   // output columns per wave
   static constexpr int FN = SWIGLU ? 2 : 4;      // output column fragments per wave
-  static constexpr int MI = 4;                   // 32-row fragments per wave
   static constexpr int WROWS = 32 * MI;          // output rows per wave
-  static_assert(C::BM == 256 && C::WM == 2 && C::WN == 2 && C::BROWS == 256, "256-row tiles, 2x2 waves");
+  static_assert((C::BM == 256 || C::BM == 128) && C::WM == 2 && C::WN == 2 && C::BROWS == 256,
+                "256- or 128-row tiles, 2x2 waves");
 
-  v16f acc[4][4];
-  v6i fa[2][2][4];  // [set][step][i]
-  v6i fb[2][2][4];  // [set][step][j]
+  v16f acc[MI][4];
+  v6i fa[2][2][MI];  // [set][step][i]
+  v6i fb[2][2][4];   // [set][step][j]
   uint32_t voff[DPW];
-  v4i rs;         // this wave's DMA operand (waves 0-1: A, 2-3: B)
+  v4i rs;         // this wave's DMA operand (waves 0-1: A, 2-3: B); 128-row tiles: A
+  v4i rsb;        // 128-row tiles: B
   uint32_t lds0;  // LDS address of slot 0
   int lane, wave, wm, wn;
 
@@ -162,7 +180,7 @@ struct F6Engine {
     }
   };
 
-  __device__ __forceinline__ int out_row(int i) const { return wm * 128 + 32 * i + (lane & 31); }
+  __device__ __forceinline__ int out_row(int i) const { return wm * WROWS + 32 * i + (lane & 31); }
   // first of the four columns of fragment j (< FN), register group q
   __device__ __forceinline__ int out_col(int j, int q) const { return wn * TN + 32 * j + 8 * q + 4 * (lane >> 5); }
   // the exact integer sum of accumulator register x of [i][j], as fp32 / int32
@@ -190,33 +208,49 @@ struct F6Engine {
     wn = wave / 2;
     lds0 = lds_address(smem);
     const unsigned long long panel_bytes = (unsigned long long)kb * F6_BLOCK;
+    const unsigned long long first_a = (unsigned long long)(m0 / 32) * panel_bytes + (unsigned long long)kb0 * F6_BLOCK;
+    const unsigned long long first_b = (unsigned long long)bt * 8 * panel_bytes + (unsigned long long)kb0 * F6_BLOCK;
+    if constexpr (MI == 2) {
+      rs = buffer_words(a6 + first_a, a_bytes - first_a);
+      rsb = buffer_words(b6 + first_b, b_bytes - first_b);
+      // load c fills 1 KiB piece DPA*wave + c of A, or (DPW - DPA)*wave + c - DPA of B
+#pragma unroll
+      for (int c = 0; c < DPW; ++c) {
+        const uint32_t o = 1024u * (c < DPA ? DPA * wave + c : (DPW - DPA) * wave + c - DPA) + 16u * lane;
+        voff[c] = (o / PANEL) * (uint32_t)panel_bytes + o % PANEL;
+      }
+      return;
+    }
     const bool is_a = wave < 2;
-    const unsigned long long first =
-        (is_a ? (unsigned long long)(m0 / 32) : (unsigned long long)bt * 8) * panel_bytes +
-        (unsigned long long)kb0 * F6_BLOCK;
+    const unsigned long long first = is_a ? first_a : first_b;
     rs = buffer_words((is_a ? a6 : b6) + first, (is_a ? a_bytes : b_bytes) - first);
     // DMA load c of this wave fills stage bytes [1024 * (DPW*wave + c), +1024):
     // panel o / PANEL of the operand, byte o % PANEL of its two blocks
 #pragma unroll
     for (int c = 0; c < DPW; ++c) {
-      const uint32_t o = 1024u * (DPW * wave + c) + 16u * lane - (is_a ? 0u : (uint32_t)OPB);
+      const uint32_t o = 1024u * (DPW * wave + c) + 16u * lane - (is_a ? 0u : (uint32_t)OPA);
       voff[c] = (o / PANEL) * (uint32_t)panel_bytes + o % PANEL;
     }
+  }
+  // LDS offset in a stage of this wave's DMA load c
+  __device__ __forceinline__ uint32_t dma_offset(int c) const {
+    if constexpr (MI == 2) return c < DPA ? 1024u * (DPA * wave + c) : OPA + 1024u * ((DPW - DPA) * wave + c - DPA);
+    return 1024u * (DPW * wave + c);
   }
 
   __device__ __forceinline__ Reads reads_of_slot(int slot) const {
     const uint32_t s = lds0 + (uint32_t)slot * STAGE;
-    const uint32_t a = s + 4u * wm * PANEL, b = s + OPB + 4u * wn * PANEL;
+    const uint32_t a = s + (uint32_t)(MI * PANEL) * wm, b = s + OPA + 4u * wn * PANEL;
     return Reads{a + 16u * lane, a + 1024u + 8u * lane, b + 16u * lane, b + 1024u + 8u * lane};
   }
 
-  // LDS read Q (0..31) of a stage into set S: per step, the fragments in the
-  // order of their first use (A0, B0..B3, A1..A3), each as its 16-byte then
-  // its 8-byte part.
+  // LDS read Q (0..READS-1) of a stage into set S: per step, the fragments in
+  // the order of their first use (A0, B0..B3, A1..A3), each as its 16-byte
+  // then its 8-byte part.
   template <int S, int Q>
   __device__ __forceinline__ void read(const Reads& r) {
-    constexpr int ST = Q / 16;
-    constexpr int F = (Q % 16) / 2;
+    constexpr int ST = Q / (READS / 2);
+    constexpr int F = (Q % (READS / 2)) / 2;
     constexpr bool IS_A = F == 0 || F >= 5;
     constexpr int IDX = F == 0 ? 0 : (F >= 5 ? F - 4 : F - 1);
     constexpr int OFF = IDX * PANEL + ST * F6_BLOCK;
@@ -237,8 +271,9 @@ struct F6Engine {
   }
 
   // MFMA T (0..31) of a stage on set S (step T/16, A fragment (T%16)/4, B
-  // fragment T%4), fused with DMA load (T-1)/2 of the stage for odd T < 24,
-  // followed by LDS read T of the next stage.  Every stage runs the same
+  // fragment T%4), fused with DMA load (T-1)/2 of the stage for odd T < 24
+  // (128-row tiles: load T for T < 9 of the 16), followed by LDS read T (and
+  // T + 16) of the next stage.  Every stage runs the same
   // sequence with no branch: a branch around an asm MFMA or LDS read would
   // let the register allocator copy an accumulator or fragment between the
   // asm statements, and the copy would read a value the hardware has not
@@ -247,41 +282,43 @@ struct F6Engine {
   // 0 as the C operand and define the accumulators, so no VALU write ever
   // precedes an MFMA's read of them (see run()).
   template <int S, int T, bool FIRST>
-  __device__ __forceinline__ void tick(const Reads& r, const v4i& rs_st, uint32_t so, uint32_t m0) {
-    constexpr int ST = T / 16, I = (T % 16) / 4, J = T % 4;
-    if constexpr (FIRST && T < 16 && T % 2 == 1 && T < 2 * DPW) {
-      constexpr int c = T / 2;
+  __device__ __forceinline__ void tick(const Reads& r, const v4i& rs_st, const v4i& rsb_st, uint32_t so, uint32_t slot0) {
+    constexpr int ST = T / (4 * MI), I = (T % (4 * MI)) / 4, J = T % 4;
+    constexpr bool LOAD = MI == 4 ? T % 2 == 1 && T < 2 * DPW : T < DPW;
+    constexpr int c = !LOAD ? 0 : (MI == 4 ? T / 2 : T);  // the DMA load
+    const v4i& rl = MI == 2 && c >= DPA ? rsb_st : rs_st;
+    if constexpr (FIRST && ST == 0 && LOAD) {
       asm volatile(
           "v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, 0 cbsz:2 blgp:2\n\t"
           "buffer_load_dwordx4 %3, %4, %5 offen lds"
           : "=a"(acc[I][J])
-          : "v"(fb[S][ST][J]), "v"(fa[S][ST][I]), "v"(voff[c]), "s"(rs_st), "s"(so), "{m0}"(m0 + 1024u * c)
+          : "v"(fb[S][ST][J]), "v"(fa[S][ST][I]), "v"(voff[c]), "s"(rl), "s"(so), "{m0}"(slot0 + dma_offset(c))
           : "memory");
-    } else if constexpr (FIRST && T < 16) {
+    } else if constexpr (FIRST && ST == 0) {
       asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, 0 cbsz:2 blgp:2"
                    : "=a"(acc[I][J])
                    : "v"(fb[S][ST][J]), "v"(fa[S][ST][I]));
-    } else if constexpr (T % 2 == 1 && T < 2 * DPW) {
-      constexpr int c = T / 2;
+    } else if constexpr (LOAD) {
       // the compiler writes M0 before the statement; the MFMA is the wait
       // state the LDS-DMA load needs after that write
       asm volatile(
           "v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0 cbsz:2 blgp:2\n\t"
           "buffer_load_dwordx4 %3, %4, %5 offen lds"
           : "+a"(acc[I][J])
-          : "v"(fb[S][ST][J]), "v"(fa[S][ST][I]), "v"(voff[c]), "s"(rs_st), "s"(so), "{m0}"(m0 + 1024u * c)
+          : "v"(fb[S][ST][J]), "v"(fa[S][ST][I]), "v"(voff[c]), "s"(rl), "s"(so), "{m0}"(slot0 + dma_offset(c))
           : "memory");
     } else {
       asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0 cbsz:2 blgp:2"
                    : "+a"(acc[I][J])
                    : "v"(fb[S][ST][J]), "v"(fa[S][ST][I]));
     }
-    read<1 - S, T>(r);
+    if constexpr (T < READS) read<1 - S, T>(r);
+    if constexpr (T + TICKS < READS) read<1 - S, T + TICKS>(r);
   }
   template <int S, bool FIRST, int... T>
-  __device__ __forceinline__ void ticks(const Reads& r, const v4i& rs_st, uint32_t so, uint32_t m0,
-                                        std::integer_sequence<int, T...>) {
-    (tick<S, T, FIRST>(r, rs_st, so, m0), ...);
+  __device__ __forceinline__ void ticks(const Reads& r, const v4i& rs_st, const v4i& rsb_st, uint32_t so,
+                                        uint32_t slot0, std::integer_sequence<int, T...>) {
+    (tick<S, T, FIRST>(r, rs_st, rsb_st, so, slot0), ...);
   }
   template <int S, int... Q>
   __device__ __forceinline__ void reads(const Reads& r, std::integer_sequence<int, Q...>) {
@@ -304,11 +341,18 @@ struct F6Engine {
   __device__ __forceinline__ void fence() {
     static_assert(N == 4 || N == 7, "wait states");
 #define SHK_F6_ACC(i) "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3])
-    if constexpr (N == 4)
-      asm volatile("s_nop 4" : SHK_F6_ACC(0), SHK_F6_ACC(1), SHK_F6_ACC(2), SHK_F6_ACC(3));
-    else
-      asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
-                   : SHK_F6_ACC(0), SHK_F6_ACC(1), SHK_F6_ACC(2), SHK_F6_ACC(3));
+    if constexpr (MI == 4) {
+      if constexpr (N == 4)
+        asm volatile("s_nop 4" : SHK_F6_ACC(0), SHK_F6_ACC(1), SHK_F6_ACC(2), SHK_F6_ACC(3));
+      else
+        asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
+                     : SHK_F6_ACC(0), SHK_F6_ACC(1), SHK_F6_ACC(2), SHK_F6_ACC(3));
+    } else {
+      if constexpr (N == 4)
+        asm volatile("s_nop 4" : SHK_F6_ACC(0), SHK_F6_ACC(1));
+      else
+        asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" : SHK_F6_ACC(0), SHK_F6_ACC(1));
+    }
 #undef SHK_F6_ACC
   }
 
@@ -318,9 +362,14 @@ struct F6Engine {
   // operand here, so none is copied before the data is in.
   template <int S, int ST>
   __device__ __forceinline__ void frag_fence() {
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(fa[S][ST][0]), "+v"(fa[S][ST][1]), "+v"(fa[S][ST][2]), "+v"(fa[S][ST][3]),
-                   "+v"(fb[S][ST][0]), "+v"(fb[S][ST][1]), "+v"(fb[S][ST][2]), "+v"(fb[S][ST][3])::"memory");
+    if constexpr (MI == 4)
+      asm volatile("s_waitcnt lgkmcnt(0)"
+                   : "+v"(fa[S][ST][0]), "+v"(fa[S][ST][1]), "+v"(fa[S][ST][2]), "+v"(fa[S][ST][3]),
+                     "+v"(fb[S][ST][0]), "+v"(fb[S][ST][1]), "+v"(fb[S][ST][2]), "+v"(fb[S][ST][3])::"memory");
+    else
+      asm volatile("s_waitcnt lgkmcnt(0)"
+                   : "+v"(fa[S][ST][0]), "+v"(fa[S][ST][1]), "+v"(fb[S][ST][0]), "+v"(fb[S][ST][1]),
+                     "+v"(fb[S][ST][2]), "+v"(fb[S][ST][3])::"memory");
   }
 
   // Stage k on set S.  Top: this wave's DMA of stage k+1 has landed (that
@@ -331,16 +380,17 @@ struct F6Engine {
   // `rs_end`, a resource of zero records: they return zeros without touching
   // memory, into a slot that holds no live data.
   template <int S, bool FIRST = false>
-  __device__ __forceinline__ void stage(const Reads& r, int k, int nst, int slot, const v4i& rs_end) {
+  __device__ __forceinline__ void stage(const Reads& r, int k, int nst, int slot, const v4i& rs_end,
+                                        const v4i& rsb_end) {
     wait_vmcnt<DPW>();
     frag_fence<S, 0>();
     frag_fence<S, 1>();
     asm volatile("s_barrier" ::: "memory");
     const bool live = k + 3 < nst;
     const v4i rs_st = live ? rs : rs_end;
+    const v4i rsb_st = MI == 2 ? (live ? rsb : rsb_end) : rs_st;
     const uint32_t so = live ? (uint32_t)(k + 3) * PANEL : 0u;
-    ticks<S, FIRST>(r, rs_st, so, lds0 + (uint32_t)slot * STAGE + 1024u * DPW * wave,
-                    std::make_integer_sequence<int, 32>{});
+    ticks<S, FIRST>(r, rs_st, rsb_st, so, lds0 + (uint32_t)slot * STAGE, std::make_integer_sequence<int, TICKS>{});
   }
   // Moves the read slot one ahead (wrapping after slot 2) and the stage slot.
   static __device__ __forceinline__ void advance(Reads& r, int& slot) {
@@ -358,7 +408,7 @@ struct F6Engine {
   __device__ __forceinline__ void run(int nst) {
     if (nst <= 0) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -367,26 +417,29 @@ struct F6Engine {
       return;
     }
     const v4i rs_end = v4i{rs.x, rs.y, 0, rs.w};
+    const v4i rsb_end = MI == 2 ? v4i{rsb.x, rsb.y, 0, rsb.w} : rs_end;
     // stages 0..2 (zeros past the last stage), then stage 0 into set 0
 #pragma unroll
     for (int st = 0; st < 3; ++st)
 #pragma unroll
-      for (int c = 0; c < DPW; ++c)
-        lds_dma16(st < nst ? rs : rs_end, voff[c], st < nst ? (uint32_t)st * PANEL : 0u,
-                  lds0 + (uint32_t)st * STAGE + 1024u * (DPW * wave + c));
+      for (int c = 0; c < DPW; ++c) {
+        const bool from_b = MI == 2 && c >= DPA;
+        lds_dma16(st < nst ? (from_b ? rsb : rs) : (from_b ? rsb_end : rs_end), voff[c],
+                  st < nst ? (uint32_t)st * PANEL : 0u, lds0 + (uint32_t)st * STAGE + dma_offset(c));
+      }
     wait_vmcnt<2 * DPW>();
     asm volatile("s_barrier" ::: "memory");
-    reads<0>(reads_of_slot(0), std::make_integer_sequence<int, 32>{});
+    reads<0>(reads_of_slot(0), std::make_integer_sequence<int, READS>{});
     // r: read slot of stage k+1; slot: slot of stage k
     Reads r = reads_of_slot(1);
     int slot = 0;
-    stage<0, true>(r, 0, nst, slot, rs_end);
+    stage<0, true>(r, 0, nst, slot, rs_end, rsb_end);
     advance(r, slot);
     int k = 1;
     for (; k + 2 <= nst; k += 2) {
-      stage<1>(r, k, nst, slot, rs_end);
+      stage<1>(r, k, nst, slot, rs_end, rsb_end);
       advance(r, slot);
-      stage<0>(r, k + 1, nst, slot, rs_end);
+      stage<0>(r, k + 1, nst, slot, rs_end, rsb_end);
       advance(r, slot);
     }
     // The last stage's reads fetch a stale slot into the set that no MFMA
@@ -399,7 +452,7 @@ struct F6Engine {
     frag_fence<1, 1>();
     fence<7>();
     if (k < nst) {
-      stage<1>(r, k, nst, slot, rs_end);
+      stage<1>(r, k, nst, slot, rs_end, rsb_end);
       frag_fence<0, 0>();
       frag_fence<0, 1>();
       fence<7>();
@@ -420,9 +473,9 @@ __device__ __forceinline__ float f6_bf16_at(const uint2& w, int t) {
 // Where the epilogue of a 32x32 engine writes.  Element (r, c) of the
 // output is at out + r * ld + c (elements); B scale of column c at
 // b_scale[c], the SwiGLU gate's at b_scale[n + c].  A dense tile is written
-// whole; with MASK (the ragged kernels) only rows [row_lo, row_hi) and
-// columns below col_hi are, and B scales of columns at or past col_hi are
-// not read.
+// whole; with MASK (the ragged kernels and the edge tiles of dense calls)
+// only rows [row_lo, row_hi) and columns below col_hi are, and no B scale
+// past the buffer's end is read.
 struct OutView {
   void* out;
   const uint16_t* b_scale;
@@ -487,10 +540,11 @@ __device__ __forceinline__ void f6_epilogue(const E& e, const OutView& o, int m0
                     e.acc_int(i, j, 4 * q + 3)},
                 r, off, soff, 0);
           if constexpr (C::SWIGLU) {
-            __builtin_amdgcn_raw_buffer_store_b128(
-                v4i{e.acc_int(i, j + 2, 4 * q), e.acc_int(i, j + 2, 4 * q + 1), e.acc_int(i, j + 2, 4 * q + 2),
-                    e.acc_int(i, j + 2, 4 * q + 3)},
-                r, off + (uint32_t)o.n * ESZ, soff, 0);
+            if (in)
+              __builtin_amdgcn_raw_buffer_store_b128(
+                  v4i{e.acc_int(i, j + 2, 4 * q), e.acc_int(i, j + 2, 4 * q + 1), e.acc_int(i, j + 2, 4 * q + 2),
+                      e.acc_int(i, j + 2, 4 * q + 3)},
+                  r, off + (uint32_t)o.n * ESZ, soff, 0);
           }
         } else {
           float v[4];
@@ -662,7 +716,7 @@ __device__ __forceinline__ void mfma32_prefetch_b_scales(const E& e, const OutVi
     const int c0 = n0 + e.wn * E::TN;  // the window's first column
     const int lane = e.lane;
     const int col = C::SWIGLU ? c0 + 2 * (lane & 31) + (lane >> 5) * o.n : c0 + 2 * lane;
-    const unsigned long long cols = MASK ? (unsigned long long)o.col_hi : (C::SWIGLU ? 2ull : 1ull) * o.n;
+    const unsigned long long cols = MASK && !C::SWIGLU ? (unsigned long long)o.col_hi : (C::SWIGLU ? 2ull : 1ull) * o.n;
     lds_dma4(buffer_words(o.b_scale, 2 * cols), 2u * (uint32_t)col, 0u, slot);
   }
 }
@@ -692,7 +746,6 @@ __device__ __forceinline__ void mfma32_read_b_scales(const E& e, const uint8_t* 
 template <class C, int MODE, int EPI, bool MASK = false, class E>
 __device__ __forceinline__ void mfma32_finish(const E& e, const OutView& o, uint8_t* smem, int m0, int n0,
                                               const float (&sa)[4]) {
-  static_assert(!(MASK && C::SWIGLU), "masked tiles are plain");
   if constexpr (MODE == OUT_I32) {
     const uint2 none[4][4] = {};
     f6_epilogue<C, OUT_I32, EPI_NONE, false, MASK>(e, o, m0, n0, sa, none);
@@ -744,37 +797,50 @@ __device__ __forceinline__ void f6_add_i32(const E& e, int32_t* out, int ld, int
   }
 }
 
-// One output tile of the fp6 GEMM: tile index `tile` in the XCD-aware order
-// of dense_tile_coords.  OUT_I32_ADD: K slice blockIdx.y of F6_MAX_K values
-// (the last one shorter), added into the int32 buffer p.out ([M, b_cols]).
-template <class C, int MODE, int EPI, bool PERSIST = false>
-__device__ __forceinline__ void f6_gemm_tile(const DenseArgs& p, uint8_t* smem, int tile) {
+// One output tile of the fp6 GEMM at rows m0 and column tile tn.
+// OUT_I32_ADD: K slice blockIdx.y of F6_MAX_K values (the last one shorter),
+// added into the int32 buffer p.out ([M, b_cols]).
+// MASK: M, N and K need not be multiples of the tile.  Panels past an
+// operand's last row read as zeros through the buffer's range, K is padded
+// with zeros in the blocks, and the stores stop at row M and column N.
+template <class C, int MODE, int EPI, bool PERSIST = false, bool MASK = false>
+__device__ __forceinline__ void f6_gemm_at(const DenseArgs& p, uint8_t* smem, int m0, int tn) {
   using E = F6Engine<C>;
   constexpr bool RAW = MODE == OUT_I32 || MODE == OUT_I32_ADD;
-  const int tiles_m = p.M / C::BM;
-  const int tiles_n = p.N / C::BN;
-  int tm, tn;
-  dense_tile_coords(tile, tiles_m, tiles_n, p.group_m, tm, tn);
-  const int m0 = tm * C::BM;
   const int n0 = tn * C::BN;
   int k0 = 0, klen = p.K;
   if constexpr (MODE == OUT_I32_ADD) {
     k0 = (int)blockIdx.y * F6_MAX_K;
     klen = min(F6_MAX_K, p.K - k0);
   }
+  const long rows_a = MASK ? f6_pad_rows(p.M) : p.M, rows_b = MASK ? f6_pad_rows(p.b_cols) : p.b_cols;
+  const int kpad = MASK ? (int)f6_pad_k(p.K) : p.K;
   E e;
-  e.template setup<PERSIST>(smem, p.a, p.b, m0, tn, p.K / 64, f6_operand_bytes(p.M, p.K),
-                            f6_operand_bytes(p.b_cols, p.K), k0 / 64);
-  float sa[4];
+  e.template setup<PERSIST>(smem, p.a, p.b, m0, tn, kpad / 64, f6_operand_bytes(rows_a, kpad),
+                            f6_operand_bytes(rows_b, kpad), k0 / 64);
+  float sa[4] = {};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) sa[i] = RAW ? 0.0f : load_bf16(p.a_scale + m0 + e.out_row(i));
+  for (int i = 0; i < E::MI; ++i) {
+    const int m = MASK ? min(m0 + e.out_row(i), p.M - 1) : m0 + e.out_row(i);
+    sa[i] = RAW ? 0.0f : load_bf16(p.a_scale + m);
+  }
   const OutView o = dense_view<C, RAW ? OUT_I32 : MODE>(p);
-  if constexpr (!RAW) mfma32_prefetch_b_scales<C, MODE>(e, o, n0, e.lds0 + E::LDS_BYTES + 256u * e.wave);
-  e.run(klen / 128);
+  if constexpr (!RAW) mfma32_prefetch_b_scales<C, MODE, MASK>(e, o, n0, e.lds0 + E::LDS_BYTES + 256u * e.wave);
+  const int nst = (MASK ? kpad : klen) / 128;
+  if constexpr (MASK) __builtin_assume(nst > 0);
+  e.run(nst);
   if constexpr (MODE == OUT_I32_ADD)
     f6_add_i32<C>(e, static_cast<int32_t*>(p.out), p.b_cols, p.N, m0, n0);
   else
-    mfma32_finish<C, MODE, EPI>(e, o, smem, m0, n0, sa);
+    mfma32_finish<C, MODE, EPI, MASK>(e, o, smem, m0, n0, sa);
+}
+
+// Tile index `tile` in the XCD-aware order of dense_tile_coords.
+template <class C, int MODE, int EPI, bool PERSIST = false>
+__device__ __forceinline__ void f6_gemm_tile(const DenseArgs& p, uint8_t* smem, int tile) {
+  int tm, tn;
+  dense_tile_coords(tile, p.M / C::BM, p.N / C::BN, p.group_m, tm, tn);
+  f6_gemm_at<C, MODE, EPI, PERSIST>(p, smem, tm * C::BM, tn);
 }
 
 // One kernel per output mode and epilogue (chosen by the host), so that
@@ -783,6 +849,29 @@ template <class C, int MODE, int EPI>
 __global__ __launch_bounds__(256) void f6_gemm_kernel(const DenseArgs p) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[F6Engine<C>::LDS_BYTES + MFMA32_SCALE_BYTES];
   f6_gemm_tile<C, MODE, EPI>(p, smem, blockIdx.x);
+}
+
+// The 128-row tile of a 256-row fp6 configuration.
+template <class C>
+using F6Half = Cfg<4, true, true, 128, C::BN, C::BK, 2, 2, C::SWIGLU, false, C::MK, false, 0>;
+
+// The same tiles for any M, N and K (see f6_gemm_at's MASK).  The column
+// tiles from main_n on (the host's split, f6_edge_split) run last, as tiles
+// of 128 rows.
+template <class C, int MODE, int EPI>
+__global__ __launch_bounds__(256) void f6_edge_gemm(const DenseArgs p) {
+  __shared__ __attribute__((aligned(16))) uint8_t smem[F6Engine<C>::LDS_BYTES + MFMA32_SCALE_BYTES];
+  const int tiles_m = (p.M + C::BM - 1) / C::BM, tiles_n = (p.N + C::BN - 1) / C::BN;
+  const int main_n = p.split_tn;
+  const int main_tiles = tiles_m * main_n;
+  int tm, tn;
+  if ((int)blockIdx.x >= main_tiles) {
+    dense_tile_coords((int)blockIdx.x - main_tiles, (p.M + 127) / 128, tiles_n - main_n, p.group_m, tm, tn);
+    f6_gemm_at<F6Half<C>, MODE, EPI, false, true>(p, smem, tm * 128, main_n + tn);
+    return;
+  }
+  dense_tile_coords(blockIdx.x, tiles_m, main_n, p.group_m, tm, tn);
+  f6_gemm_at<C, MODE, EPI, false, true>(p, smem, tm * C::BM, tn);
 }
 
 // Persistent schedule: gridDim.x workgroups (a multiple of 8, at most one

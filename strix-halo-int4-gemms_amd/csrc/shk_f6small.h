@@ -33,7 +33,7 @@ namespace shk {
 template <class C, int PS = 3>
 struct F6SmallEngine {
   static constexpr int P = PS;                      // ring slots
-  static_assert(P == 2 || P == 3, "two or three ring slots");
+  static_assert(P >= 2 && P <= 6, "two to six ring slots");
   static constexpr int NW = 4;
   static constexpr int PANEL = 2 * F6_BLOCK;        // 32 rows x 128 K: 3 KiB
   static constexpr int OPB = 4 * PANEL;             // one operand's stage: 12 KiB
@@ -302,7 +302,7 @@ __device__ __forceinline__ void f6s_read_b_scales(const E& e, const uint8_t* slo
 // faster per call with a three-slot ring, 1.2 us with a two-slot one).
 // With two slots the 4-byte outputs (64 KiB for the four waves) stage in
 // two passes.
-template <int MODE, bool NO_NAN, bool MASK, class E>
+template <int MODE, bool NO_NAN, bool MASK, int EPI = EPI_NONE, class E>
 __device__ __forceinline__ void f6s_store(const E& e, const OutView& o, uint8_t* smem, int m0, int n0,
                                           const float (&sa)[2], const uint2 (&sb)[2][4]) {
   constexpr int ESZ = MODE == OUT_BF16 ? 2 : 4;
@@ -353,6 +353,7 @@ __device__ __forceinline__ void f6s_store(const E& e, const OutView& o, uint8_t*
             } else {
               float x = e.acc_value(i, j, 4 * q + t) * sa[i];
               x = x * s4[t];
+              if constexpr (EPI == EPI_RELU2) x = apply_epi(x, EPI_RELU2);
               w[t] = __float_as_uint(x);
             }
           }
@@ -391,7 +392,7 @@ __device__ __forceinline__ void f6s_store(const E& e, const OutView& o, uint8_t*
 // lane's two rows, B scales from the wave's slot past the ring; bf16 with
 // the hardware conversion when every scale is below 2^48 in magnitude
 // (then |acc| < 2^31 keeps each product finite: no NaN).
-template <int MODE, bool MASK, class E>
+template <int MODE, bool MASK, int EPI = EPI_NONE, class E>
 __device__ __forceinline__ void f6s_finish(const E& e, const OutView& o, uint8_t* smem, int m0, int n0,
                                            const float (&sa)[2]) {
   uint2 sb[2][4];
@@ -405,7 +406,7 @@ __device__ __forceinline__ void f6s_finish(const E& e, const OutView& o, uint8_t
   }
   f6s_read_b_scales(e, smem + E::LDS_BYTES + 256 * e.wave, sb);
   if constexpr (MODE == OUT_F32) {
-    f6s_store<OUT_F32, false, MASK>(e, o, smem, m0, n0, sa, sb);
+    f6s_store<OUT_F32, false, MASK, EPI>(e, o, smem, m0, n0, sa, sb);
   } else {
     constexpr uint32_t F32_LIM = (127u + 48u) << 23, BF16_LIM = (127u + 48u) << 7;
     bool bounded = (__float_as_uint(sa[0]) & 0x7F800000u) < F32_LIM && (__float_as_uint(sa[1]) & 0x7F800000u) < F32_LIM;
@@ -417,8 +418,8 @@ __device__ __forceinline__ void f6s_finish(const E& e, const OutView& o, uint8_t
         bounded = bounded && (w.x & 0x7F80u) < BF16_LIM && (w.x & 0x7F800000u) < (BF16_LIM << 16) &&
                   (w.y & 0x7F80u) < BF16_LIM && (w.y & 0x7F800000u) < (BF16_LIM << 16);
       }
-    if (__all(bounded)) f6s_store<OUT_BF16, true, MASK>(e, o, smem, m0, n0, sa, sb);
-    else f6s_store<OUT_BF16, false, MASK>(e, o, smem, m0, n0, sa, sb);
+    if (__all(bounded)) f6s_store<OUT_BF16, true, MASK, EPI>(e, o, smem, m0, n0, sa, sb);
+    else f6s_store<OUT_BF16, false, MASK, EPI>(e, o, smem, m0, n0, sa, sb);
   }
 }
 

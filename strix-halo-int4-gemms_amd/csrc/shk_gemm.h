@@ -375,13 +375,15 @@ struct DenseArgs {
 };
 
 // Tile order: workgroups are dispatched round-robin over the 8 XCDs, so the
-// linear id is first remapped to give each XCD a contiguous range, then
-// grouped GROUP_M rows at a time so concurrently running tiles on one XCD
-// share A rows and B columns in that XCD's L2.
+// linear id is first remapped to give each XCD a contiguous range (x * q +
+// min(x, r) + [0, q + (x < r)) of 8q + r tiles), then grouped GROUP_M rows
+// at a time so concurrently running tiles on one XCD share A rows and B
+// columns in that XCD's L2.
 __device__ __forceinline__ void dense_tile_coords(int pid, int tiles_m, int tiles_n, int group_m, int& tm,
                                                   int& tn) {
   const int total = tiles_m * tiles_n;
-  if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
+  const int x = pid & 7, q = total >> 3, r = total & 7;
+  pid = x * q + min(x, r) + (pid >> 3);
   const int per_group = group_m * tiles_n;
   const int grp = pid / per_group;
   const int first_m = grp * group_m;

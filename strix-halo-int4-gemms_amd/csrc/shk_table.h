@@ -31,12 +31,16 @@ hipError_t launch_dense_t(const DenseArgs& a, dim3 grid, hipStream_t s) {
 // fp6 path.  f6_convert_operand converts A (operand 0) or B (operand 1) of
 // a dense call into its part of the workspace (A first, then B); the GEMM
 // then reads both parts.
+// (The FP6 entries' M, b_cols and K are tile multiples, which the padding
+// leaves as they are; the FP6_EDGE entries' are not.)
+inline uint8_t* f6_work_b(const DenseArgs& a) {
+  return a.work + f6_operand_bytes(f6_pad_rows(a.M), f6_pad_k(a.K));
+}
 inline F6PackArgs f6_pack_args(const DenseArgs& a, int operand, bool swiglu) {
-  const int kb = a.K / 64;
+  const int kb = (int)(f6_pad_k(a.K) / 64);
   // dense operands are validated 16-byte aligned
   if (operand == 0) return F6PackArgs{a.a, a.work, a.lda, a.M, kb, 0, 1, 0, 0, nullptr, a.K, 16};
-  return F6PackArgs{a.b,    a.work + f6_operand_bytes(a.M, a.K), a.ldb, a.b_cols, kb, swiglu ? a.N : 0, 1, 0, 0,
-                    nullptr, a.K, 16};
+  return F6PackArgs{a.b, f6_work_b(a), a.ldb, a.b_cols, kb, swiglu ? a.N : 0, 1, 0, 0, nullptr, a.K, 16};
 }
 inline bool f6_mn_major(const DenseArgs& a, int operand) {
   return operand == 0 ? a.layout == SHK_LAYOUT_TN : a.layout != SHK_LAYOUT_NT;
@@ -44,6 +48,53 @@ inline bool f6_mn_major(const DenseArgs& a, int operand) {
 inline hipError_t f6_convert_operand(const DenseArgs& a, int operand, bool swiglu, hipStream_t s) {
   return launch_f6_pack(f6_pack_args(a, operand, swiglu), f6_mn_major(a, operand), s);
 }
+// How an FP6_EDGE per-channel call runs: 128 x 128 tiles in rings of `slots`
+// (plain epilogues), or, with slots 0, 256-row tiles of which the last
+// `half_columns` column tiles run as 128-row tiles; `tiles` workgroups.
+//
+// The 256-row tile reads half the bytes per product, one workgroup a CU; the
+// small one fills the chip on small grids and has a short epilogue.  Both
+// costs are fits to a sweep of M 192..8176 over N x K of 1024 x 4096, 4096 x
+// 1024, 4096^2, 11008 x 4096, 16384 x 4096 and 8192^2 (us): a round of 256
+// large tiles 14 + 4.9 K/1024, 256 small tiles 2.6 + 2.05 K/1024.  Measured
+// on both sides of the line, call with conversion, small and large tiles:
+// 1008 x 4096^2 26.1 and 31.6 us, 4160 x 4096 x 1024 30.6 and 37.7, 1008 x
+// 11008 x 4096 46.9 and 47.0, 1008 x 16384 x 4096 64.0 and 58.7, 8176 x
+// 8192^2 369 and 295.
+//
+// Half-height tiles run a partial last round in about 0.6 of its time where
+// all of them fit one round of the chip: 1008 x 11008 x 4096 SwiGLU, 344
+// tiles, 85.3 -> 80.2 us; 512 x 4096^2 SwiGLU, 64 tiles, 39.7 -> 31.8.
+struct F6EdgePlan {
+  int slots;
+  int half_columns;
+  long tiles;
+  double us;  // the GEMM's predicted time
+};
+constexpr long kF6EdgeCus = 256;
+inline F6EdgePlan f6_edge_plan(long m, long n, long k, bool swiglu) {
+  const double k1 = (double)k / 1024.0;
+  const long bn = swiglu ? 128 : 256;
+  const long tm = (m + 255) / 256, tn = (n + bn - 1) / bn, tm2 = (m + 127) / 128;
+  const long tiles = tm * tn, rounds = tiles / kF6EdgeCus, rest = tiles % kF6EdgeCus;
+  const double round_us = 14.0 + 4.9 * k1;
+  F6EdgePlan p{0, 0, tiles, round_us * (double)(rounds + (rest > 0 ? 1 : 0))};
+  if (rest > 0) {
+    const long c = rounds == 0 ? tn : (rest + tm - 1) / tm;
+    if (tm2 * c <= kF6EdgeCus) {
+      p.half_columns = (int)c;
+      p.tiles = tm * (tn - c) + tm2 * c;
+      p.us = round_us * ((double)rounds + 0.6);
+    }
+  }
+  if (!swiglu) {
+    const long small = tm2 * ((n + 127) / 128);
+    const double us = (2.6 + 2.05 * k1) * (double)((small + kF6EdgeCus - 1) / kF6EdgeCus);
+    if (us <= p.us) p = F6EdgePlan{small <= 2 * kF6EdgeCus ? 3 : 2, 0, small, us};
+  }
+  return p;
+}
+
 // Large-K per-channel fp6 calls (K > F6_MAX_K): the int32 sums of the K
 // slices go to the workspace past both converted operands, [M, b_cols]
 // int32, which f6_large_k_begin clears and f6_large_k_end turns into the
@@ -297,6 +348,9 @@ inline unsigned long long sk_counter_bytes(const shk_kernel_desc& d, long m, lon
 // (append_dense_f6(layout), append_dense_dma_<bits>_<layout>,
 // append_dense_<bits>_<layout>, append_ragged_<layout>).
 void append_dense_f6(std::vector<Entry>& t, int layout);
+// fp6 entries for shapes that are no multiple of the fp6 tiles (k_f6.hip),
+// after the skinny entries.
+void append_edge_f6(std::vector<Entry>& t, int layout);
 void append_dense_dma_4_0(std::vector<Entry>& t);
 void append_dense_dma_4_1(std::vector<Entry>& t);
 void append_dense_dma_4_2(std::vector<Entry>& t);

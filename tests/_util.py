@@ -46,3 +46,10 @@ def dense_case(seed: int, *, bits: int, layout: str, m: int, n: int, k: int, sub
 
 def max_ulp(a_bits, b_bits) -> int:
     return int(ref.bf16_ulp_diff(a_bits, b_bits).max()) if np.size(a_bits) else 0
+
+
+def spec_of(sub):
+    """The ScaleSpec of a scale group size (None or 0: per-channel)."""
+    import amd_strix_halo_kernels as shk
+
+    return shk.ScaleSpec(shk.ScaleMode.SUBCHANNEL, sub) if sub else shk.ScaleSpec(shk.ScaleMode.PER_CHANNEL)

@@ -1,0 +1,65 @@
+"""Host-side checks of the FP6_EDGE entries: the library's workspace and
+selection equal the Python mirror, and the entries are chosen where their
+predicted time is the smallest."""
+
+from __future__ import annotations
+
+import ctypes
+import itertools
+
+import pytest
+
+import amd_strix_halo_kernels as shk
+from amd_strix_halo_kernels import kernel_table as kt
+from amd_strix_halo_kernels import native
+from tests._util import spec_of
+
+EDGES = [d for d in kt.TABLE if d.operand_format == kt.OPERANDS_FP6_EDGE]
+
+
+def test_edge_workspace_is_the_padded_operands():
+    lib = native.load_dispatch_library()
+    out = ctypes.c_uint64()
+    for d in EDGES:
+        cols = 2 if d.epilogue_kind == kt.EPI_KIND_SWIGLU else 1
+        for m, n, k in ((16, 64, 64), (48, 192, 192), (1008, 11008, 4096), (64, 64, kt.FP6_MAX_K)):
+            assert lib.amd_strix_halo_kernels_gemm_workspace_bytes(d.index, m, n, k, ctypes.byref(out)) == 0
+            kw = (k + 127) // 128 * 128
+            need = ((m + 31) // 32 * 32 + n * cols) * kw * 3 // 4
+            assert out.value == need == d.workspace_bytes(m, n, k)
+
+
+@pytest.mark.parametrize("sub", [0, 64, 128])
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+def test_selection_by_predicted_time_matches_the_library(sub, epilogue):
+    """registry.select and the library's select_dense agree over shapes on
+    both sides of every tile's line; a whole call runs the entry with the
+    smallest predicted time, an FP6 entry among them."""
+    epi = {"none": kt.EPILOGUE_NONE, "swiglu": kt.EPILOGUE_SWIGLU}[epilogue]
+    reg = shk.default_registry
+    formats = set()
+    for m, n, k in itertools.product((16, 48, 64, 320, 512, 1008, 1056, 2048, 4160, 8176),
+                                     (64, 1024, 4096, 11008, 16384), (64, 128, 1024, 4096, 8192, 14336)):
+        if sub and k % sub:
+            continue
+        kern = reg.select(dtype=shk.OperandDType.INT4, scale=spec_of(sub), epilogue=shk.Epilogue(epilogue), m=m, n=n,
+                          k=k, split_k=1)
+        got = native.select_dense_index(dtype_bits=4, layout=kt.LAYOUT_NN, subchannel=sub, epilogue=epi, schedule=0,
+                                        split_k=1, m=m, n=n, k=k)
+        assert got == kern.table_index, (m, n, k)
+        fitting = [e for e in kt.TABLE if e.layout == kt.LAYOUT_NN and e.epilogue_kind == kt.TABLE[got].epilogue_kind
+                   and m % e.block_m == 0 and n % e.block_n == 0 and k % e.block_k == 0]
+        if any(e.operand_format == kt.OPERANDS_FP6 and e.scale_mode == kt.TABLE[got].scale_mode for e in fitting):
+            assert kt.TABLE[got].operand_format == kt.OPERANDS_FP6
+        d = kt.TABLE[reg.call_kernel(kern, m=m, n=n, k=k).table_index]
+        formats.add(d.operand_format)
+        us = kt.predicted_us(d, m, n, k)
+        if us is not None:
+            assert us <= min(t for e in fitting if (t := kt.predicted_us(e, m, n, k)) is not None)
+    if not sub:
+        assert formats == {kt.OPERANDS_STREAM, kt.OPERANDS_FP6, kt.OPERANDS_FP6_EDGE}
+
+
+def test_edge_entries_bound_k():
+    for d in EDGES:
+        assert d.max_k == kt.FP6_MAX_K and not d.supports_k(kt.FP6_MAX_K + 64)
