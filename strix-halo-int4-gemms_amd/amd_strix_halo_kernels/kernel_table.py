@@ -298,13 +298,16 @@ def _sk_desc(index, bits, layout, r, *, swiglu=False, subch=False, schedule=SCHE
         group_size_m=1, operand_format=OPERANDS_STREAM, schedule=schedule, split_k=split_k)
 
 
-def _edge_desc(index, layout, bm, *, swiglu=False):
-    # a 256-row per-channel fp6 tile's ring (_desc), at its granularity
+def _edge_desc(index, layout, bm, *, swiglu=False, subch=False):
+    # the ring of the largest kernel the entry may launch (the 256-row
+    # per-channel tile, the subchannel tile; _desc), at its granularity
     return KernelDesc(
-        index=index, family=FAMILY_DENSE, dtype_bits=4, layout=layout, scale_mode=SCALE_PER_CHANNEL,
-        min_subchannel=0, max_subchannel=0, epilogue_kind=EPI_KIND_SWIGLU if swiglu else EPI_KIND_PLAIN,
-        block_m=bm, block_n=64, block_k=32, num_waves=4, num_stages=3,
-        lds_bytes=3 * (256 + 256) * 96 + MFMA32_SCALE_BYTES, group_size_m=8, operand_format=OPERANDS_FP6_EDGE)
+        index=index, family=FAMILY_DENSE, dtype_bits=4, layout=layout,
+        scale_mode=SCALE_SUBCHANNEL if subch else SCALE_PER_CHANNEL, min_subchannel=32 if subch else 0,
+        max_subchannel=256 if subch else 0, epilogue_kind=EPI_KIND_SWIGLU if swiglu else EPI_KIND_PLAIN,
+        block_m=bm, block_n=64, block_k=64 if subch else 32, num_waves=4, num_stages=3,
+        lds_bytes=3 * (128 + 128) * 96 + 8 * 1024 if subch else 3 * (256 + 256) * 96 + MFMA32_SCALE_BYTES,
+        group_size_m=8, operand_format=OPERANDS_FP6_EDGE)
 
 
 def _build() -> tuple[KernelDesc, ...]:
@@ -386,11 +389,12 @@ def _build() -> tuple[KernelDesc, ...]:
                 for r in (16, 32, 64):
                     for subch in (False, True):
                         add_sk(bits, layout, r, subch=subch, split_k=split)
-    # fp6 entries for shapes that are no tile multiples (k_f6.hip)
+    # fp6 entries for shapes that are no tile multiples (k_f6edge.hip)
     for layout in (LAYOUT_NN, LAYOUT_NT, LAYOUT_TN):
         for bm in (64, 16):
-            for swiglu in (False, True):
-                out.append(_edge_desc(len(out), layout, bm, swiglu=swiglu))
+            for subch in (False, True):
+                for swiglu in (False, True):
+                    out.append(_edge_desc(len(out), layout, bm, swiglu=swiglu, subch=subch))
     return tuple(out)
 
 
@@ -478,32 +482,54 @@ _SKINNY_US = {  # (tile rows, SwiGLU): us per tile and us per tile and K value
     (64, False): (0.005, 5.2e-6), (32, False): (0.0035, 3.75e-6), (16, False): (0.0028, 2.65e-6),
     (64, True): (0.019, 1.1e-5), (32, True): (0.0125, 7.0e-6), (16, True): (0.0045, 4.3e-6),
 }
+# subchannel, by group size: us per product on the 32-row skinny tiles (plain,
+# SwiGLU); a 128 x 128 fp6 tile's fixed us and us per K value
+_SKINNY_SUB_US = {32: (2.9e-8, 2.3e-8), 64: (1.5e-8, 1.2e-8), 128: (1.07e-8, 0.74e-8), 256: (0.85e-8, 0.65e-8)}
+_F6_SUB_US = {32: (5.0, 0.0215), 64: (5.0, 0.0125), 128: (5.0, 0.0061), 256: (3.5, 0.0038)}
 
 
-def predicted_us(desc: KernelDesc, m: int, n: int, k: int) -> float | None:
-    """Predicted time of a standard int4 per-channel call on an entry, in us
-    (None for the other families and K past PREDICT_MAX_K); capi.hip computes
-    the skinny and FP6_EDGE entries' alike.  Fits to calls measured over M 64..8176 and N x K of 1024 x 4096,
-    4096 x 1024, 4096^2, 11008 x 4096, 16384 x 4096 and 8192^2:
+def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = None) -> float | None:
+    """Predicted time of a standard int4 call on an entry, in us (None for the
+    other families and K past PREDICT_MAX_K); capi.hip computes the skinny
+    and FP6_EDGE entries' alike.  Fits to calls measured over M 16..8176 and
+    N x K of 1024 x 4096, 4096 x 1024, 4096^2, 11008 x 4096, 16384 x 4096 and
+    8192^2:
 
-    * skinny tiles: a launch, then at least one round of tiles (few tiles
-      split K instead), each a fixed part and a part along K; the tallest
-      tile that divides M;
+    * skinny per-channel tiles: a launch, then at least one round of tiles
+      (few tiles split K instead), each a fixed part and a part along K; the
+      tallest tile that divides M;
+    * skinny subchannel tiles: a launch and the products;
     * fp6 entries: two launches, the conversion at 5 TB/s, then rounds of
-      256-row tiles (FP6) or the launcher's split (FP6_EDGE).
+      tiles: per-channel 256-row tiles (FP6) or the launcher's split
+      (FP6_EDGE); subchannel 128 x 128 tiles, two a CU (1.3 times one).
 
-    Measured against predicted: 512 x 4096^2 skinny 16.6 (18), 256-row fp6
-    36.7 (44), edge 24.7 (22); 8176 x 16384 x 4096 skinny 1675 (1791), edge
-    324 (300); 8192^3 fp6 277 (251)."""
-    if (desc.family != FAMILY_DENSE or desc.dtype_bits != 4 or desc.scale_mode != SCALE_PER_CHANNEL
-            or desc.schedule != SCHEDULE_STANDARD or desc.split_k > 1 or k > PREDICT_MAX_K):
+    Measured against predicted, per-channel: 512 x 4096^2 skinny 16.6 (18),
+    256-row fp6 36.7 (44), edge 24.7 (22); 8176 x 16384 x 4096 skinny 1675
+    (1791), edge 324 (300); 8192^3 fp6 277 (251).  Groups of 128: 64 x 4096^2
+    skinny 17.5 (17), edge 42.3 (40); 320 x 16384 x 4096 skinny 221 (236),
+    edge 59.7 (62); 4160 x 8192^2 edge 397 (388)."""
+    if (desc.family != FAMILY_DENSE or desc.dtype_bits != 4 or desc.schedule != SCHEDULE_STANDARD
+            or desc.split_k > 1 or k > PREDICT_MAX_K):
         return None
     swiglu = desc.epilogue_kind == EPI_KIND_SWIGLU
+    cols = 2 * n if swiglu else n
+    convert = 6.0 + 2.5e-7 * ((m + cols) * k)
+    if desc.scale_mode == SCALE_SUBCHANNEL:
+        if sub not in _F6_SUB_US:
+            return None
+        if desc.operand_format == OPERANDS_STREAM:
+            tall = {32: 1.0, 64: 1.25, 16: 1.5}[desc.block_m]
+            return 6.0 + _SKINNY_SUB_US[sub][swiglu] * tall * (m * cols * k)
+        if not desc.needs_workspace:
+            return None
+        fixed, per_k = _F6_SUB_US[sub]
+        tiles = -(-m // 128) * (-(-n // 64) if swiglu else -(-n // 128))
+        rounds = 1.0 if tiles <= _CUS else 1.3 * -(-tiles // (2 * _CUS))
+        return convert + (fixed + per_k * k) * rounds
     if desc.operand_format == OPERANDS_STREAM:
         r = 64 if m % 64 == 0 else (32 if m % 32 == 0 else 16)
         base, per_k = _SKINNY_US[r, swiglu]
         return 5.0 + max((m // r) * (n // 64), _CUS) * (base + per_k * k)
-    convert = 6.0 + 2.5e-7 * ((m + (2 * n if swiglu else n)) * k)
     if desc.operand_format == OPERANDS_FP6_EDGE:
         return convert + _f6_edge_us(m, n, k, swiglu)
     if desc.operand_format == OPERANDS_FP6:
@@ -512,17 +538,19 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int) -> float | None:
     return None
 
 
-def selection_tops(desc: KernelDesc, m: int, n: int | None = None, k: int | None = None) -> float | None:
+def selection_tops(desc: KernelDesc, m: int, n: int | None = None, k: int | None = None,
+                   sub: int | None = None) -> float | None:
     """The throughput by which select ranks an entry for a shape (capi.hip
-    measured_score): an int4 per-channel skinny or FP6_EDGE entry's predicted
-    one, below the FP6 entries' figures (a caller of the separate conversion
-    needs an FP6 entry where one fits); for the others, or without n and k,
+    measured_score): an int4 skinny or FP6_EDGE entry's predicted one, below
+    the FP6 entries' figures (a caller of the separate conversion needs an
+    FP6 entry where one fits); for the others, or without n and k,
     measured_tops, where the skinny subchannel tiles' figure holds up to
     SKINNY_SUB_MAX_M rows."""
     if n is not None and k is not None and desc.operand_format != OPERANDS_FP6:
-        us = predicted_us(desc, m, n, k)
+        us = predicted_us(desc, m, n, k, sub)
         if us is not None:
-            return min(3000.0, 2.0 * float(m) * float(n) * float(k) / us / 1e6)
+            cap = 2000.0 if desc.scale_mode == SCALE_SUBCHANNEL else 3000.0
+            return min(cap, 2.0 * float(m) * float(n) * float(k) / us / 1e6)
     tops = measured_tops(desc)
     if (tops is not None and desc.operand_format == OPERANDS_STREAM and desc.scale_mode == SCALE_SUBCHANNEL
             and m > SKINNY_SUB_MAX_M):

@@ -110,7 +110,7 @@ def _selection_key(kernel: KernelMetadata, m: int, n: int | None = None, k: int 
     if kernel.table_index is not None:
         desc = kt.TABLE[kernel.table_index]
         if tops == kt.measured_tops(desc):  # not a caller's own figure (with_status)
-            tops = kt.selection_tops(desc, m, n, k)
+            tops = kt.selection_tops(desc, m, n, k, kernel.scale.subchannel_size)
     return (tops or 0.0, kernel.tile.block_m * kernel.tile.block_n)
 
 
@@ -219,7 +219,8 @@ class KernelRegistry:
         separate conversion needs them.  A whole call is free to take any
         entry with the same results, and on few tiles of 256 rows another one
         is faster (512 x 4096 x 4096: FP6 36.7 us, skinny 16.6; 512 x 16384 x
-        4096: FP6 47.4, FP6_EDGE 41.9), so the smallest predicted time
+        4096: FP6 47.4, FP6_EDGE 41.9; groups of 128, 128 x 1024 x 4096: FP6
+        37.8, skinny 12.7), so the smallest predicted time
         decides (kernel_table.predicted_us).  Kernels with a figure of the
         caller's own (with_status) stay."""
         index = kernel.table_index
@@ -230,13 +231,14 @@ class KernelRegistry:
         if hit is not None:
             return hit
         chosen = kernel
-        best = kt.predicted_us(kt.TABLE[index], m, n, k)
+        sub = kernel.scale.subchannel_size
+        best = kt.predicted_us(kt.TABLE[index], m, n, k, sub)
         if best is not None and kernel.measured_tops == kt.measured_tops(kt.TABLE[index]):
             shape = LaunchShape(m, n, k)
             for other in self._family(kernel.a_dtype, kernel.scale, kernel.epilogue, kernel.layout, kernel.schedule):
                 if other.table_index is None or other.tile.split_k != 1 or not is_tile_multiple_shape(other, shape):
                     continue
-                us = kt.predicted_us(kt.TABLE[other.table_index], m, n, k)
+                us = kt.predicted_us(kt.TABLE[other.table_index], m, n, k, sub)
                 if us is not None and (us, -other.tile.block_m) < (best, -chosen.tile.block_m):
                     chosen, best = other, us
         if len(self._call_kernels) >= 4096:

@@ -64,6 +64,7 @@ def translation_units() -> list[tuple[str, Path, list[str]]]:
     # fp6 path: the GEMM keeps 256 accumulators like the DMA objects; the
     # operand conversion is compiled with the default scheduler.
     units.append(("dense_f6", CSRC / "k_f6.hip", list(DMA_FLAGS)))
+    units.append(("edge_f6", CSRC / "k_f6edge.hip", list(DMA_FLAGS)))
     units.append(("f6pack", CSRC / "k_f6pack.hip", []))
     units.append(("ragged_f6", CSRC / "k_f6ragged.hip", list(DMA_FLAGS)))
     units.append(("quant", CSRC / "k_quant.hip", []))

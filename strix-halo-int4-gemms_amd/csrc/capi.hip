@@ -511,15 +511,32 @@ int amd_strix_halo_kernels_kernel_table_entry(int index, shk_kernel_desc* out) {
 
 namespace {
 
-// Predicted time (us) of a standard int4 per-channel call on a skinny or
-// FP6_EDGE entry, from fits to measured calls (kernel_table.predicted_us
-// states them); negative where there is none.
+// Predicted time (us) of a standard int4 call on a skinny or FP6_EDGE entry,
+// from fits to measured calls (kernel_table.predicted_us states them);
+// negative where there is none.
 constexpr long kPredictMaxK = 65536;
-double predicted_us(const shk_kernel_desc& d, long m, long n, long k) {
-  if (d.family != SHK_FAMILY_DENSE || d.dtype_bits != 4 || d.scale_mode != SHK_SCALE_PER_CHANNEL ||
-      d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1 || k > kPredictMaxK)
+double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
+  if (d.family != SHK_FAMILY_DENSE || d.dtype_bits != 4 || d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1 ||
+      k > kPredictMaxK)
     return -1.0;
   const bool swiglu = d.epilogue_kind == SHK_EPI_KIND_SWIGLU;
+  const long cols = swiglu ? 2 * n : n;
+  const double convert = 6.0 + 2.5e-7 * (double)((m + cols) * k);
+  if (d.scale_mode == SHK_SCALE_SUBCHANNEL) {
+    const int s = sub == 32 ? 0 : (sub == 64 ? 1 : (sub == 128 ? 2 : 3));
+    if (d.operand_format == SHK_OPERANDS_STREAM) {
+      static constexpr double plain[4] = {2.9e-8, 1.5e-8, 1.07e-8, 0.85e-8};
+      static constexpr double gated[4] = {2.3e-8, 1.2e-8, 0.74e-8, 0.65e-8};
+      const double tall = d.block_m == 32 ? 1.0 : (d.block_m == 64 ? 1.25 : 1.5);
+      return 6.0 + (swiglu ? gated[s] : plain[s]) * tall * (double)(m * cols * k);
+    }
+    if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
+    static constexpr double fixed[4] = {5.0, 5.0, 5.0, 3.5};
+    static constexpr double per_k[4] = {0.0215, 0.0125, 0.0061, 0.0038};
+    const long tiles = ((m + 127) / 128) * (swiglu ? (n + 63) / 64 : (n + 127) / 128);
+    const double rounds = tiles <= 256 ? 1.0 : 1.3 * (double)((tiles + 511) / 512);
+    return convert + (fixed[s] + per_k[s] * (double)k) * rounds;
+  }
   if (d.operand_format == SHK_OPERANDS_STREAM) {
     const long r = m % 64 == 0 ? 64 : (m % 32 == 0 ? 32 : 16);
     const long tiles = (m / r) * (n / 64);
@@ -530,20 +547,21 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k) {
     return 5.0 + (double)(tiles > 256 ? tiles : 256) * (base + per_k * (double)k);
   }
   if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
-  const double convert = 6.0 + 2.5e-7 * (double)((m + (swiglu ? 2 * n : n)) * k);
   return convert + shk::f6_edge_plan(m, n, k, swiglu).us;
 }
 
 // Throughput measured on MI355X for the entries the benchmark configurations
 // time (the Python registry's kernel_table.selection_tops): the first
-// ranking key of a selection, before the tile area.  Int4 per-channel skinny
+// ranking key of a selection, before the tile area.  Int4 skinny
 // and FP6_EDGE entries rank by their predicted throughput for the shape,
 // below the FP6 entries where those accept it (a caller of the separate
 // conversion needs an FP6 entry).
-double measured_score(const shk_kernel_desc& d, int m, int n, int k) {
+double measured_score(const shk_kernel_desc& d, int m, int n, int k, int subchannel) {
   if (d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1) return 0.0;
-  const double us = predicted_us(d, m, n, k);
-  if (us > 0.0) return std::min(3000.0, 2.0 * (double)m * (double)n * (double)k / us / 1e6);
+  const double us = predicted_us(d, m, n, k, subchannel);
+  if (us > 0.0)
+    return std::min(d.scale_mode == SHK_SCALE_SUBCHANNEL ? 2000.0 : 3000.0,
+                    2.0 * (double)m * (double)n * (double)k / us / 1e6);
   if (d.operand_format == SHK_OPERANDS_FP6_EDGE) return 0.0;
   if (d.operand_format == SHK_OPERANDS_FP6) {
     if (d.scale_mode == SHK_SCALE_SUBCHANNEL) return 2001.0;
@@ -599,7 +617,7 @@ int best_entry(int bits, int layout, int subchannel, int epilogue, int schedule,
     if (!serves_family(d, bits, layout, subchannel, epilogue, schedule, split_k)) continue;
     if (!accepts_shape(d, m, n, k, subchannel)) continue;
     if (direct && d.operand_format != SHK_OPERANDS_PACKED && d.operand_format != SHK_OPERANDS_STREAM) continue;
-    const double score = measured_score(d, m, n, k);
+    const double score = measured_score(d, m, n, k, subchannel);
     const long area = (long)d.block_m * d.block_n;
     if (score > best_score || (score == best_score && area > best_area)) {
       best = i;

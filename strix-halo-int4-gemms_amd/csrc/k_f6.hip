@@ -5,7 +5,6 @@
 // layout (NN, NT, TN), which differ in how the operands are converted.
 // Compiled with the iterative ILP scheduler, which keeps the accumulators in
 // place (k_dense.hip).
-#include "shk_f6small.h"
 #include "shk_f6sub.h"
 #include "shk_table.h"
 
@@ -75,84 +74,6 @@ Entry f6sub_entry(int layout) {
   d.lds_bytes = f6_sub_lds_bytes<CSub>();
   d.operand_format = SHK_OPERANDS_FP6;
   return Entry{d, &launch_f6sub, nullptr, nullptr, &launch_f6sub_gemm};
-}
-
-// ---------------------------------------------------------------------------
-// Edge entries (SHK_OPERANDS_FP6_EDGE): any M and N that are multiples of 16
-// and 64, and K of 32 (subchannel: 64).  Same conversion and MFMA tiles as
-// the FP6 entries; the converted operands are padded to whole 32-row panels
-// and 128-K stages, and the stores stop at M and N.
-
-// Per-channel 128 x 128 tile (shk_f6small.h): P ring slots, so three
-// workgroups a CU with two slots and two with three.  One workgroup alone on
-// a CU waits for its loads at every second stage with two slots: 256 tiles
-// of K = 4096 (1008 x 4096) 31.3 us a call, with three slots 26.1, with six
-// 26.6; from 384 tiles on two and three are within 2%.
-using CSmall = Cfg<4, true, true, 128, 128, 128, 2, 2, false, false, 64, false, 0>;
-
-template <int MODE, int EPI, int P>
-__global__ __launch_bounds__(256, P == 2 ? 3 : (P == 3 ? 2 : 1)) void f6_small_edge_kernel(const DenseArgs p) {
-  using E = F6SmallEngine<CSmall, P>;
-  __shared__ __attribute__((aligned(16))) uint8_t smem[E::LDS_BYTES + MFMA32_SCALE_BYTES];
-  int tm, tn;
-  dense_tile_coords(blockIdx.x, (p.M + 127) / 128, (p.N + 127) / 128, p.group_m, tm, tn);
-  const int m0 = 128 * tm, n0 = 128 * tn;
-  const int kpad = (int)f6_pad_k(p.K);
-  E e;
-  e.setup(smem, p.a, p.b, m0, n0, kpad / 64, f6_operand_bytes(f6_pad_rows(p.M), kpad),
-          f6_operand_bytes(f6_pad_rows(p.N), kpad));
-  float sa[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    sa[i] = MODE == OUT_I32 ? 0.0f : load_bf16(p.a_scale + min(m0 + e.out_row(i), p.M - 1));
-  const OutView o{p.out, p.b_scale, p.N, p.M, p.N, 0, p.M, p.N};
-  mfma32_prefetch_b_scales<CSmall, MODE, true>(e, o, n0, e.lds0 + E::LDS_BYTES + 256u * e.wave);
-  e.run(kpad / 128);
-  f6s_finish<MODE, true, EPI>(e, o, smem, m0, n0, sa);
-}
-
-template <bool SWIGLU, int MODE, int EPI>
-void launch_edge(const DenseArgs& a, hipStream_t s) {
-  constexpr int BN = SWIGLU ? 128 : 256;
-  DenseArgs g = a;
-  const int tiles_n = (g.N + BN - 1) / BN;
-  const F6EdgePlan plan = f6_edge_plan(g.M, g.N, g.K, SWIGLU);
-  if constexpr (!SWIGLU) {
-    if (plan.slots) {
-      const dim3 grid((unsigned)plan.tiles);
-      if (plan.slots == 2) hipLaunchKernelGGL((f6_small_edge_kernel<MODE, EPI, 2>), grid, dim3(256), 0, s, g);
-      else hipLaunchKernelGGL((f6_small_edge_kernel<MODE, EPI, 3>), grid, dim3(256), 0, s, g);
-      return;
-    }
-  }
-  g.split_tn = tiles_n - plan.half_columns;
-  hipLaunchKernelGGL((f6_edge_gemm<C<BN, SWIGLU>, MODE, EPI>), dim3((unsigned)plan.tiles), dim3(256), 0, s, g);
-}
-template <bool SWIGLU>
-hipError_t launch_f6_edge(const DenseArgs& a, dim3, hipStream_t s) {
-  hipError_t err = launch_f6_pack2(f6_pack_args(a, 0, SWIGLU), f6_mn_major(a, 0), f6_pack_args(a, 1, SWIGLU),
-                                   f6_mn_major(a, 1), s, nullptr, true);
-  if (err != hipSuccess) return err;
-  DenseArgs g = a;
-  g.a = a.work;
-  g.b = f6_work_b(a);
-  const bool relu2 = !SWIGLU && a.epilogue == EPI_RELU2;
-  constexpr int R2 = SWIGLU ? EPI_NONE : EPI_RELU2;
-  if (a.out_mode == OUT_I32) launch_edge<SWIGLU, OUT_I32, EPI_NONE>(g, s);
-  else if (a.out_mode == OUT_F32) relu2 ? launch_edge<SWIGLU, OUT_F32, R2>(g, s) : launch_edge<SWIGLU, OUT_F32, EPI_NONE>(g, s);
-  else relu2 ? launch_edge<SWIGLU, OUT_BF16, R2>(g, s) : launch_edge<SWIGLU, OUT_BF16, EPI_NONE>(g, s);
-  return hipGetLastError();
-}
-template <int BN, bool SWIGLU>
-Entry edge_entry(int layout, int bm) {
-  shk_kernel_desc d = desc_of<C<BN, SWIGLU>>(SHK_FAMILY_DENSE, layout, 8);
-  d.block_m = bm;
-  d.block_n = 64;
-  d.block_k = 32;
-  d.num_stages = F6Engine<C<BN, SWIGLU>>::P;
-  d.lds_bytes = F6Engine<C<BN, SWIGLU>>::LDS_BYTES + MFMA32_SCALE_BYTES;
-  d.operand_format = SHK_OPERANDS_FP6_EDGE;
-  return Entry{d, &launch_f6_edge<SWIGLU>, nullptr, nullptr, nullptr};
 }
 
 // Large-K per-channel calls: clearing the int32 workspace, and the pass
@@ -249,13 +170,6 @@ void append_dense_f6(std::vector<Entry>& t, int layout) {
   t.push_back(f6_entry<C<256, false>>(layout));
   t.push_back(f6_entry<C<128, true>>(layout));
   t.push_back(f6sub_entry(layout));
-}
-
-void append_edge_f6(std::vector<Entry>& t, int layout) {
-  for (int bm : {64, 16}) {
-    t.push_back(edge_entry<256, false>(layout, bm));
-    t.push_back(edge_entry<128, true>(layout, bm));
-  }
 }
 
 void append_persistent_f6(std::vector<Entry>& t, int layout) {

@@ -42,14 +42,12 @@ __device__ __forceinline__ void f6_store_lane(uint8_t* block, int lane, const v6
   *reinterpret_cast<uint2*>(block + 1024 + 8 * lane) = make_uint2(y[4], y[5]);
 }
 
-// Source row of packed row r.  For SwiGLU B the packed rows of each 256-row
-// tile (output columns 128t .. 128t+127) are, per 128-row half h (one wave
-// column of the GEMM tile), 64 up columns followed by the same 64 gate
-// columns: 128t + 64h + q (q < 64) and N + 128t + 64h + q - 64.
-__device__ __forceinline__ int f6_src_row(int r, int swiglu_n) {
+// Source row of packed row r.  SwiGLU B's packed rows alternate between 2^sh
+// up columns and the same 2^sh gate columns (sh = 6: a wave column of the
+// 256-row tile; 5: of the 128-row subchannel tile).
+__device__ __forceinline__ int f6_src_row(int r, int swiglu_n, int sh) {
   if (swiglu_n == 0) return r;
-  const int t = r >> 8, h = (r >> 7) & 1, q = r & 127;
-  return 128 * t + 64 * h + (q & 63) + (q >= 64 ? swiglu_n : 0);
+  return ((r >> (sh + 1)) << sh) + (r & ((1 << sh) - 1)) + ((r >> sh) & 1) * swiglu_n;
 }
 
 // Logical K length of operand g.
@@ -123,7 +121,7 @@ __device__ __forceinline__ void pack_kmajor_nb(const F6PackArgs& p, int wg) {
     const int r = 32 * panel + (lane & 31);
     const int k0 = 64 * kb + 32 * (lane >> 5);
     if (live[b] && r < p.rows && k0 < len) {
-      const uint8_t* q = src + (long)f6_src_row(r, p.swiglu_n) * p.ld + 32L * kb + 16 * (lane >> 5);
+      const uint8_t* q = src + (long)f6_src_row(r, p.swiglu_n, p.swiglu_shift) * p.ld + 32L * kb + 16 * (lane >> 5);
       const int keep = len - k0;  // K values of the 32 to keep
       // bytes holding any of them (the source row ends within the length)
       x[b] = f6_load(q, p.vec, (keep + 1) / 2);
@@ -173,7 +171,7 @@ __device__ __forceinline__ void pack_mnmajor(const F6PackArgs& p, int wg, uint8_
   const int tid = threadIdx.x;
   const int u = tid & 15;  // 16-row unit of the tile
   const int r0 = F6_TILE * t + 16 * u;
-  const long col = f6_src_row(r0, p.swiglu_n);
+  const long col = f6_src_row(r0, p.swiglu_n, p.swiglu_shift);
   const uint8_t* src = p.src + g * p.src_group;
   uint4 x[kKW][2];
 #pragma unroll

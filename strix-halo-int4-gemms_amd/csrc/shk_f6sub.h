@@ -97,10 +97,11 @@ struct F6SubEngine {
   static constexpr int LDS_BYTES = RING + 4 * SCALE_SLOT;
   static constexpr int OPW = STAGE / 1024 / NW;     // 6 operand loads per wave per stage
   static constexpr int DPW = OPW + 1;               // and one scale load
-  static constexpr int TN = 64;                     // output columns per wave
-  static constexpr int FN = 2;
-  static_assert(C::BM == 128 && C::BROWS == 128 && C::WM == 2 && C::WN == 2 && C::SUBCH && !C::SWIGLU,
-                "128 x 128 tiles of 2 x 2 waves, subchannel, plain epilogue");
+  static constexpr bool SWIGLU = C::SWIGLU;
+  static constexpr int TP = 64;                     // packed B rows per wave
+  static constexpr int TN = SWIGLU ? 32 : 64;       // output columns per wave (SwiGLU: j = 0 up, 1 gate)
+  static_assert(C::BM == 128 && C::BROWS == 128 && C::WM == 2 && C::WN == 2 && C::SUBCH,
+                "128 x 128 tiles of 2 x 2 waves, subchannel");
   static constexpr int SPG = 2;                     // stages per group of 256 K
 
   v16f acc[2][2];
@@ -120,9 +121,14 @@ struct F6SubEngine {
   bool all_fast;
 
   __device__ __forceinline__ int out_row(int i) const { return wm * 64 + 32 * i + (lane & 31); }
-  __device__ __forceinline__ int out_col(int j, int q) const { return wn * TN + 32 * j + 8 * q + 4 * (lane >> 5); }
+  __device__ __forceinline__ int out_col(int j, int q) const {
+    return wn * TN + (SWIGLU ? 0 : 32 * j) + 8 * q + 4 * (lane >> 5);
+  }
+  // the same columns as packed B rows of the tile
+  __device__ __forceinline__ int packed_col(int j, int q) const { return wn * TP + 32 * j + 8 * q + 4 * (lane >> 5); }
 
-  // a6 / b6: block-format operands; tile rows m0 (A) and n0 (B).
+  // a6 / b6: block-format operands; tile rows m0 (A) and n0 (packed B rows,
+  // columns of B; SwiGLU: 32 up columns, then the same 32 gate columns).
   __device__ __forceinline__ void setup(uint8_t* smem, const uint8_t* a6, const uint8_t* b6, int m0_, int n0,
                                         int kb, unsigned long long a_bytes, unsigned long long b_bytes,
                                         const uint16_t* a_scale, const uint16_t* b_scale, int m_rows, int n_cols,
@@ -151,7 +157,8 @@ struct F6SubEngine {
       sbase = (m0 + 64 * wave + lane) * g;
     } else {
       rss = buffer_words(b_scale, 2ull * (unsigned long long)g * n_cols);
-      sbase = 2 * (n0 + 2 * lane);
+      const int c = n0 + 2 * lane;  // the lane's packed B rows c, c + 1
+      sbase = 2 * (SWIGLU ? 32 * (c >> 6) + (c & 31) + ((c >> 5) & 1) * (n_cols / 2) : c);
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -372,7 +379,7 @@ struct F6SubEngine {
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      sb_bits[j] = *reinterpret_cast<const uint16_t*>(sl + 512 + 2 * (wn * TN + 32 * j + (lane & 31)));
+      sb_bits[j] = *reinterpret_cast<const uint16_t*>(sl + 512 + 2 * (wn * TP + 32 * j + (lane & 31)));
   }
 
   __device__ __forceinline__ void fold(const uint8_t* smem, int g) {
@@ -393,7 +400,7 @@ struct F6SubEngine {
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const uint2 w = *reinterpret_cast<const uint2*>(sl + 512 + 2 * out_col(j, q));
+        const uint2 w = *reinterpret_cast<const uint2*>(sl + 512 + 2 * packed_col(j, q));
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -509,10 +516,11 @@ struct F6SubEngine64 {
   static constexpr int LDS_BYTES = RING + SCALE_SLOTS * SCALE_SLOT;
   static constexpr int OPW = STAGE / 1024 / NW;     // 3 operand loads per wave per stage
   static constexpr int DPW = OPW + 1;               // and one scale load
-  static constexpr int TN = 64;                     // output columns per wave
-  static constexpr int FN = 2;
-  static_assert(C::BM == 128 && C::BROWS == 128 && C::WM == 2 && C::WN == 2 && C::SUBCH && !C::SWIGLU,
-                "128 x 128 tiles of 2 x 2 waves, subchannel, plain epilogue");
+  static constexpr bool SWIGLU = C::SWIGLU;
+  static constexpr int TP = 64;                     // packed B rows per wave
+  static constexpr int TN = SWIGLU ? 32 : 64;       // output columns per wave (SwiGLU: j = 0 up, 1 gate)
+  static_assert(C::BM == 128 && C::BROWS == 128 && C::WM == 2 && C::WN == 2 && C::SUBCH,
+                "128 x 128 tiles of 2 x 2 waves, subchannel");
   static_assert(SPG == 0 || SPG == 1 || SPG == 2 || SPG == 4, "groups of 32, 64, 128 or 256 K");
 
   v16f acc[2][2];
@@ -538,9 +546,14 @@ struct F6SubEngine64 {
   int fold_last;
 
   __device__ __forceinline__ int out_row(int i) const { return wm * 64 + 32 * i + (lane & 31); }
-  __device__ __forceinline__ int out_col(int j, int q) const { return wn * TN + 32 * j + 8 * q + 4 * (lane >> 5); }
+  __device__ __forceinline__ int out_col(int j, int q) const {
+    return wn * TN + (SWIGLU ? 0 : 32 * j) + 8 * q + 4 * (lane >> 5);
+  }
+  // the same columns as packed B rows of the tile
+  __device__ __forceinline__ int packed_col(int j, int q) const { return wn * TP + 32 * j + 8 * q + 4 * (lane >> 5); }
 
-  // a6 / b6: block-format operands; tile rows m0 (A) and n0 (B).
+  // a6 / b6: block-format operands; tile rows m0 (A) and n0 (packed B rows,
+  // columns of B; SwiGLU: 32 up columns, then the same 32 gate columns).
   __device__ __forceinline__ void setup(uint8_t* smem, const uint8_t* a6, const uint8_t* b6, int m0_, int n0,
                                         int kb, unsigned long long a_bytes, unsigned long long b_bytes,
                                         const uint16_t* a_scale, const uint16_t* b_scale, int m_rows, int n_cols,
@@ -569,9 +582,10 @@ struct F6SubEngine64 {
       sbase = (m0 + 64 * wave + lane) * g;
     } else {
       rss = buffer_words(b_scale, 2ull * (unsigned long long)g * n_cols);
-      sbase = 2 * (n0 + 2 * lane);
+      const int c = n0 + 2 * lane;  // the lane's packed B rows c, c + 1
+      sbase = 2 * (SWIGLU ? 32 * (c >> 6) + (c & 31) + ((c >> 5) & 1) * (n_cols / 2) : c);
     }
-    // (G is a multiple of 4 with groups of 32, so row * G is even)
+    // (G is even with groups of 32, so row * G is even)
     if constexpr (HALF) sbase = is_a ? 2 * sbase : sbase + (wave == 3 ? sb_row : 0);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -844,7 +858,7 @@ struct F6SubEngine64 {
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      sb_bits[j] = *reinterpret_cast<const uint16_t*>(sbl + 2 * (wn * TN + 32 * j + (lane & 31)));
+      sb_bits[j] = *reinterpret_cast<const uint16_t*>(sbl + 2 * (wn * TP + 32 * j + (lane & 31)));
     auto in_range = [](uint32_t b) {
       return (b & 0x7FFFu) == 0u || (((b >> 7) & 0xFFu) - (127u - 60u)) < 108u;
     };
@@ -865,7 +879,7 @@ struct F6SubEngine64 {
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const uint2 w = *reinterpret_cast<const uint2*>(sbl + 2 * out_col(j, q));
+        const uint2 w = *reinterpret_cast<const uint2*>(sbl + 2 * packed_col(j, q));
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1050,6 +1064,96 @@ __device__ __forceinline__ void f6sub_store_words(const E& e, const OutView& o, 
       }
 }
 
+// The SwiGLU results of a wave's 64 rows x 32 columns, up * silu(gate) of the
+// totals of j = 0 and 1, for the four columns of register group q of row
+// block i: the hardware exp2 / reciprocal path where every gate of the
+// group's eight outputs a lane is in its range, in every lane (as the
+// per-channel epilogue chooses).
+template <class E>
+__device__ __forceinline__ void f6sub_swiglu(const E& e, int q, float (&v)[2][4]) {
+  float gmax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) gmax = __builtin_fmaxf(gmax, __builtin_fabsf(e.tot[i][1][4 * q + t]));
+  const bool fast = __all(gmax <= SWIGLU_FAST_MAX);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float up = e.tot[i][0][4 * q + t], gate = e.tot[i][1][4 * q + t];
+      v[i][t] = fast ? swiglu_fast(up, gate) : swiglu(up, gate);
+    }
+}
+
+// Stores a SwiGLU tile, rows below o.row_hi and columns below o.col_hi (a
+// multiple of 32).  bf16 goes through the wave's 4 KiB region of the idle
+// ring (unit u, columns 8u .. 8u+7, of row r at r * 64 + 16 * (u ^ ((r / 2) %
+// 4))) and leaves as 64-byte row segments; fp32 and the int32 sums (MODE
+// OUT_I32: [M, 2N], up then gate) as four columns per store.
+template <int MODE, bool NO_NAN, class E>
+__device__ __forceinline__ void f6sub_store_swiglu(const E& e, const OutView& o, uint8_t* smem, int m0, int n0) {
+  constexpr int ESZ = MODE == OUT_BF16 ? 2 : 4;
+  const uint32_t ldo = (uint32_t)o.ld;
+  const unsigned long long first = (unsigned long long)m0 * ldo + n0;
+  const rsrc_t rs =
+      make_rsrc(static_cast<uint8_t*>(o.out) + first * ESZ, ((unsigned long long)o.rows * ldo - first) * ESZ);
+  const int lane = e.lane;
+  const bool col_ok = n0 + e.wn * 32 < o.col_hi;
+  if constexpr (MODE == OUT_BF16) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    uint8_t* region = smem + (size_t)e.wave * 64 * 64;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v[2][4];
+      f6sub_swiglu(e, q, v);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        uint32_t lo, hi;
+        if constexpr (NO_NAN) {
+          lo = pack_bf16x2_nonan(v[i][0], v[i][1]);
+          hi = pack_bf16x2_nonan(v[i][2], v[i][3]);
+        } else {
+          lo = f32_to_bf16_rne(v[i][0]) | (f32_to_bf16_rne(v[i][1]) << 16);
+          hi = f32_to_bf16_rne(v[i][2]) | (f32_to_bf16_rne(v[i][3]) << 16);
+        }
+        const int r = 32 * i + (lane & 31);
+        *reinterpret_cast<uint2*>(region + r * 64 + 16 * (q ^ ((r >> 1) & 3)) + 8 * (lane >> 5)) = make_uint2(lo, hi);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int rr = lane / 4, u = lane % 4;
+    const uint32_t voff = ((uint32_t)(e.wm * 64 + rr) * ldo + (uint32_t)(e.wn * 32 + 8 * u)) * 2u;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int r = 16 * t + rr;
+      const uint4 x = *reinterpret_cast<const uint4*>(region + r * 64 + 16 * (u ^ ((r >> 1) & 3)));
+      if (col_ok && m0 + e.wm * 64 + r < o.row_hi)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, x), rs, voff, (uint32_t)(16 * t) * ldo * 2u, 0);
+    }
+  } else {
+    const uint32_t voff = ((uint32_t)e.out_row(0) * ldo + (uint32_t)e.out_col(0, 0)) * 4u;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v[2][4];
+      if constexpr (MODE == OUT_F32) f6sub_swiglu(e, q, v);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (!(col_ok && m0 + e.out_row(i) < o.row_hi)) continue;
+        const uint32_t soff = (uint32_t)(32 * i) * ldo * 4u;
+#pragma unroll
+        for (int j = 0; j < (MODE == OUT_I32 ? 2 : 1); ++j) {
+          v4i w;
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            w[t] = __float_as_int(MODE == OUT_I32 ? e.tot[i][j][4 * q + t] : v[i][t]);
+          __builtin_amdgcn_raw_buffer_store_b128(w, rs, voff + (uint32_t)(8 * q + j * o.n) * 4u, soff, 0);
+        }
+      }
+    }
+  }
+}
+
 // The engine for groups of S = 32 * G32: the 128-K-stage engine for 256,
 // the 64-K-stage one for 32, 64 and 128 (G32 / 2 stages per group; 0: two
 // groups per stage).
@@ -1062,32 +1166,45 @@ constexpr int f6_sub_lds_bytes() {
                                                                        : F6SubEngine64<C, 0>::LDS_BYTES;
 }
 
-// One 128 x 128 output tile of the subchannel GEMM over fp6 blocks (p.a /
-// p.b point at the converted A and B); G32 = S / 32.
-template <class C, int MODE, int EPI, int G32>
+// One output tile of the subchannel GEMM over fp6 blocks (p.a / p.b point at
+// the converted A and B): 128 rows and 128 packed B rows, 64 output columns
+// for SwiGLU; G32 = S / 32.  MASK: M and N need not be multiples of the tile,
+// nor K of 128 (it is one of S and of 64; the blocks are padded with zeros,
+// and a stage past the last one loads zeros).  SwiGLU tiles are MASK tiles.
+template <class C, int MODE, int EPI, int G32, bool MASK = false>
 __device__ __forceinline__ void f6_sub_tile(const DenseArgs& p, uint8_t* smem, int tile) {
   static_assert(G32 == 1 || G32 == 2 || G32 == 4 || G32 == 8, "groups of 32, 64, 128 or 256");
+  static_assert(MASK || !C::SWIGLU, "SwiGLU tiles are masked");
   using E = F6SubEngineFor<C, G32>;
-  const int tiles_m = p.M / C::BM;
-  const int tiles_n = p.N / C::BN;
+  const int tiles_m = MASK ? (p.M + C::BM - 1) / C::BM : p.M / C::BM;
+  const int tiles_n = MASK ? (p.N + C::BN - 1) / C::BN : p.N / C::BN;
   int tm, tn;
   dense_tile_coords(tile, tiles_m, tiles_n, p.group_m, tm, tn);
   const int m0 = tm * C::BM;
   const int n0 = tn * C::BN;
+  const int kpad = MASK ? (int)f6_pad_k(p.K) : p.K;
+  const int b_cols = C::SWIGLU ? p.b_cols : p.N;
+  const long rows_a = MASK ? f6_pad_rows(p.M) : p.M, rows_b = MASK ? f6_pad_rows(b_cols) : b_cols;
   E e;
-  e.setup(smem, p.a, p.b, m0, n0, p.K / 64, f6_operand_bytes(p.M, p.K), f6_operand_bytes(p.N, p.K), p.a_scale,
-          p.b_scale, p.M, p.N, p.K / p.subchannel);
+  e.setup(smem, p.a, p.b, m0, tn * C::BROWS, kpad / 64, f6_operand_bytes(rows_a, kpad),
+          f6_operand_bytes(rows_b, kpad), p.a_scale, p.b_scale, p.M, b_cols, p.K / p.subchannel);
   e.template run<MODE == OUT_I32>(smem, p.K / (G32 == 8 ? 128 : 64));
+  if constexpr (C::SWIGLU) {
+    const OutView o{p.out, p.b_scale, MODE == OUT_I32 ? 2 * p.N : p.N, p.M, p.N, 0, p.M, p.N};
+    if (MODE != OUT_BF16 || e.all_fast) f6sub_store_swiglu<MODE, true>(e, o, smem, m0, n0);
+    else f6sub_store_swiglu<MODE, false>(e, o, smem, m0, n0);
+    return;
+  }
   const OutView o{p.out, p.b_scale, p.N, p.M, p.N, 0, p.M, p.N};
   if constexpr (MODE == OUT_I32) {
-    f6sub_store_words(e, o, m0, n0, [&](int i, int j, int x) { return __float_as_int(e.tot[i][j][x]); });
+    f6sub_store_words<MASK>(e, o, m0, n0, [&](int i, int j, int x) { return __float_as_int(e.tot[i][j][x]); });
   } else if constexpr (MODE == OUT_F32) {
-    f6sub_store_words(e, o, m0, n0,
-                      [&](int i, int j, int x) { return __float_as_int(apply_epi(e.tot[i][j][x], EPI)); });
+    f6sub_store_words<MASK>(e, o, m0, n0,
+                            [&](int i, int j, int x) { return __float_as_int(apply_epi(e.tot[i][j][x], EPI)); });
   } else {
     auto val = [&](int i, int j, int x) { return apply_epi(e.tot[i][j][x], EPI); };
-    if (e.all_fast) f6sub_store_bf16<true>(e, o, smem, m0, n0, val);
-    else f6sub_store_bf16<false>(e, o, smem, m0, n0, val);
+    if (e.all_fast) f6sub_store_bf16<true, MASK>(e, o, smem, m0, n0, val);
+    else f6sub_store_bf16<false, MASK>(e, o, smem, m0, n0, val);
   }
 }
 
@@ -1097,6 +1214,13 @@ template <class C, int MODE, int EPI, int G32>
 __global__ __launch_bounds__(256, 2) void f6_sub_kernel(const DenseArgs p) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[F6SubEngineFor<C, G32>::LDS_BYTES];
   f6_sub_tile<C, MODE, EPI, G32>(p, smem, blockIdx.x);
+}
+
+// The same tiles for any M, N and K (f6_sub_tile's MASK).
+template <class C, int MODE, int EPI, int G32>
+__global__ __launch_bounds__(256, 2) void f6_sub_edge_kernel(const DenseArgs p) {
+  __shared__ __attribute__((aligned(16))) uint8_t smem[F6SubEngineFor<C, G32>::LDS_BYTES];
+  f6_sub_tile<C, MODE, EPI, G32, true>(p, smem, blockIdx.x);
 }
 
 // Persistent schedule (as f6_gemm_persistent): gridDim.x workgroups stride

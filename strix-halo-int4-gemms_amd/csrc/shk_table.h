@@ -348,7 +348,7 @@ inline unsigned long long sk_counter_bytes(const shk_kernel_desc& d, long m, lon
 // (append_dense_f6(layout), append_dense_dma_<bits>_<layout>,
 // append_dense_<bits>_<layout>, append_ragged_<layout>).
 void append_dense_f6(std::vector<Entry>& t, int layout);
-// fp6 entries for shapes that are no multiple of the fp6 tiles (k_f6.hip),
+// fp6 entries for shapes that are no multiple of the fp6 tiles (k_f6edge.hip),
 // after the skinny entries.
 void append_edge_f6(std::vector<Entry>& t, int layout);
 void append_dense_dma_4_0(std::vector<Entry>& t);

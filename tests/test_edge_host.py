@@ -29,7 +29,7 @@ def test_edge_workspace_is_the_padded_operands():
             assert out.value == need == d.workspace_bytes(m, n, k)
 
 
-@pytest.mark.parametrize("sub", [0, 64, 128])
+@pytest.mark.parametrize("sub", [0, 32, 64, 128, 256])
 @pytest.mark.parametrize("epilogue", ["none", "swiglu"])
 def test_selection_by_predicted_time_matches_the_library(sub, epilogue):
     """registry.select and the library's select_dense agree over shapes on
@@ -53,13 +53,42 @@ def test_selection_by_predicted_time_matches_the_library(sub, epilogue):
             assert kt.TABLE[got].operand_format == kt.OPERANDS_FP6
         d = kt.TABLE[reg.call_kernel(kern, m=m, n=n, k=k).table_index]
         formats.add(d.operand_format)
-        us = kt.predicted_us(d, m, n, k)
+        us = kt.predicted_us(d, m, n, k, sub)
         if us is not None:
-            assert us <= min(t for e in fitting if (t := kt.predicted_us(e, m, n, k)) is not None)
-    if not sub:
+            assert us <= min(t for e in fitting if e.scale_mode == d.scale_mode and (t := kt.predicted_us(e, m, n, k, sub)) is not None)
+    if not sub or epilogue == "none":
         assert formats == {kt.OPERANDS_STREAM, kt.OPERANDS_FP6, kt.OPERANDS_FP6_EDGE}
 
 
 def test_edge_entries_bound_k():
     for d in EDGES:
         assert d.max_k == kt.FP6_MAX_K and not d.supports_k(kt.FP6_MAX_K + 64)
+
+
+@pytest.fixture(scope="module")
+def edge_assembly(tmp_path_factory):
+    import shutil
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    sys.path.insert(0, str(Path(__file__).resolve().parents[1] / "strix-halo-int4-gemms_amd"))
+    import build
+
+    if shutil.which(build.hipcc()) is None and not Path(build.hipcc()).exists():
+        pytest.skip("hipcc is not available")
+    src, extra = next((s, e) for n, s, e in build.translation_units() if n == "edge_f6")
+    dst = tmp_path_factory.mktemp("asm") / "edge_f6.s"
+    r = subprocess.run([build.hipcc(), *build.HIP_FLAGS, *extra, "--offload-device-only", "-S", str(src), "-o",
+                        str(dst)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return dst.read_text()
+
+
+def test_no_hazard_in_the_edge_kernels(edge_assembly):
+    """No register of an LDS read or asm MFMA in flight is touched, and no
+    asm load reads an SGPR a VALU instruction has just written."""
+    from tests._asm_check import inflight_lds_hazards, sgpr_vmem_hazards
+
+    assert not inflight_lds_hazards(edge_assembly)
+    assert not sgpr_vmem_hazards(edge_assembly)

@@ -60,6 +60,55 @@ def test_edges_of_the_tiles_match_the_oracle(layout, epilogue, m, n, k, device):
     assert max_ulp(got, want) <= 2 if epilogue == "swiglu" else np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("epilogue", ["none", "relu2", "swiglu"])
+@pytest.mark.parametrize("sub", [32, 64, 128, 256])
+@pytest.mark.parametrize("m,n,groups", [(16, 64, 1), (48, 192, 3), (144, 320, 6), (272, 128, 11)])
+def test_subchannel_edges_match_the_oracle(layout, epilogue, sub, m, n, groups, device):
+    """The subchannel tile at its edges: one to eleven groups (odd stage
+    counts, K no multiple of 128), scales over three decades, every output."""
+    k = -(-groups * sub // 64) * 64
+    case = dense_case(stable_seed("edge-sub", layout, epilogue, sub, m, n, k), bits=4, layout=layout, m=m, n=n, k=k,
+                      subchannel=sub, swiglu=epilogue == "swiglu", scale_lo=1e-4, scale_hi=0.1)
+    kernel = _kernel(kt.OPERANDS_FP6_EDGE, layout, epilogue, sub, m)
+    print(f"case {kernel.kernel_id} shape=({m},{n},{k})", flush=True)
+    a, b, sa, sb = _operands(case, device)
+    out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=device)
+    native.launch_generated_kernel(a, b, kernel=kernel, a_scale=sa, b_scale=sb, c=out[:m])
+    raw = native.launch_generated_kernel_i32(a, b, kernel=kernel, a_scale=sa, b_scale=sb)
+    torch.cuda.synchronize()
+    assert bool((out[m] == 7.0).all()), "rows past M written"
+    assert np.array_equal(raw.cpu().numpy(), ref.int_matmul(case[0], case[1]))
+    want = ref.reference_gemm_bf16(case[2], case[3], bits=4, layout=layout, a_scale=case[4], b_scale=case[5],
+                                   subchannel=sub, epilogue=epilogue)
+    got = bf16_bits(torch, out[:m])
+    assert max_ulp(got, want) <= 2 if epilogue == "swiglu" else np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+@pytest.mark.parametrize("sub", [32, 64, 128, 256])
+def test_subchannel_edges_with_special_scales(sub, epilogue, device):
+    """Scales outside the fast fold's range (subnormal, huge, infinite, NaN,
+    signed zeros): the reference's order, NaN canonical."""
+    m, n, k = 80, 128, 512
+    case = list(dense_case(stable_seed("edge-special", sub, epilogue), bits=4, layout="nn", m=m, n=n, k=k,
+                           subchannel=sub, swiglu=epilogue == "swiglu"))
+    r = ref.rng(stable_seed("edge-special-scales", sub))
+    special = np.array([0x0001, 0x0080, 0x7F7F, 0x7F80, 0xFF80, 0x7FC1, 0x0000, 0x8000, 0x2000, 0xBF80], np.uint16)
+    for i in (4, 5):
+        flat = case[i].reshape(-1)
+        flat[::7] = special[r.integers(0, special.size, flat[::7].size)]
+    kernel = _kernel(kt.OPERANDS_FP6_EDGE, "nn", epilogue, sub, m)
+    a, b, sa, sb = _operands(case, device)
+    got = bf16_bits(torch, shk.explicit_mm(a, b, kernel=kernel, a_scale=sa, b_scale=sb))
+    with np.errstate(all="ignore"):
+        want = ref.reference_gemm_bf16(case[2], case[3], bits=4, layout="nn", a_scale=case[4], b_scale=case[5],
+                                       subchannel=sub, epilogue=epilogue)
+    nan = (want & 0x7FFF) > 0x7F80
+    assert np.array_equal(got[nan], want[nan])
+    assert max_ulp(got[~nan], want[~nan]) <= 2 if epilogue == "swiglu" else np.array_equal(got, want)
+
+
 # (epilogue, m, n, k): 128 x 128 tiles in two-slot rings (720 of them); all
 # half-height (144 x 32704: 256 tiles of 128 rows), a whole round of large
 # tiles then half-height ones (plain: 257 tiles; SwiGLU: 2 x 130), whole
