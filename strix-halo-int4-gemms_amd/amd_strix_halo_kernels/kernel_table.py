@@ -188,18 +188,75 @@ SK_TARGET_UNITS = 256
 
 
 def _sk_geometry(r: int, swiglu: bool, subch: bool) -> tuple[int, int]:
-    """(ring depth, LDS bytes) of a skinny tile of r rows (SkCfg)."""
+    """(listed ring depth, LDS bytes) of a skinny tile of r rows (SkCfg)."""
     bn = SK_BN_SUBCH if subch else SK_BN
     wcols = 2 * bn if swiglu else bn
     stage = r * 64 + wcols * 64 + ((r // 16) * 256 + 256 if subch else 0)
     tiles = (r // 16) * (wcols // 16)
     ch = (4 if tiles == 1 else 2 if tiles == 2 else 1) if subch else 0  # groups per wave and round
     chain = 2 * SK_NW * ch * tiles * 1024  # two rounds of scaled partials
-    budget = 79872 - chain
+    alone = SK_NW * 2 * stage > 79872 - chain  # one workgroup a CU: a deeper ring, listed as 2
+    budget = (153600 if alone else 79872) - chain
     depth = 4 if SK_NW * 4 * stage <= budget else (3 if SK_NW * 3 * stage <= budget else 2)
     ring = SK_NW * depth * stage
     red = 0 if subch else SK_NW * (wcols // 16) * 1024
-    return depth, max(ring, red) + chain
+    return 2 if alone else depth, max(ring, red) + chain
+
+
+def _sk_needed_splits(bits: int, k: int) -> int:
+    need = 1
+    if bits == 4:
+        while need * 4 * 1023 < -(-k // 128):
+            need *= 2
+    return need
+
+
+def _sk_splits(bits: int, tiles: int, k: int) -> int:
+    nst = -(-k // (128 if bits == 4 else 64))
+    s = 1
+    while s * 2 <= 16 and tiles * s * 2 <= SK_TARGET_UNITS and nst >= 16 * s:
+        s *= 2
+    return max(s, _sk_needed_splits(bits, k))
+
+
+# (bits, SwiGLU): per tile height 16, 32, 64 the us of a call (fixed, and per
+# round of 256 workgroups at 4096 K each) and whether rounds count whole.
+_SK_FITS = {
+    (4, False): ((3.6, 3.38, False), (3.4, 4.8, False), (4.8, 6.07, False)),
+    (4, True): ((7.0, 4.6, False), (3.0, 10.5, True), (3.0, 15.5, True)),
+    (8, False): ((3.8, 5.2, False), (3.5, 6.45, False), (4.5, 8.0, False)),
+    (8, True): ((15.3, 7.7, False), (12.0, 12.5, True), (12.0, 15.0, True)),
+}
+
+
+@functools.lru_cache(maxsize=4096)
+def sk_plan(bits: int, subch: bool, swiglu: bool, m: int, n: int, k: int) -> tuple[int, float]:
+    """(tile rows, predicted us) of a standard skinny call of M rows
+    (shk_table.h sk_plan, which states the fits); us 0 for subchannel."""
+    if subch:
+        return (16 if m <= (32 if swiglu else 16) else 32), 0.0
+    best = (16, -1.0)
+    for i, (a, b, whole) in enumerate(_SK_FITS[bits, swiglu]):
+        rows = 16 << i
+        if i > 0 and m <= rows // 2:
+            break
+        tiles = -(-m // rows) * (n // SK_BN)
+        s = _sk_splits(bits, tiles, k)
+        units = tiles * s
+        rounds = 1.0 if units <= 256 else (float(-(-units // 256)) if whole else units / 256.0)
+        us = a + (float(rows // 16 * (2 if swiglu else 1)) if s > 1 else 0.0) + b * (k / s / 4096.0) * rounds
+        if best[1] < 0.0 or us < best[1]:
+            best = (rows, us)
+    return best
+
+
+def _sk_tile_rows(desc: "KernelDesc", m: int, n: int, k: int) -> int:
+    """Rows of a skinny entry's tiles: the standard entries' as sk_plan picks
+    them, the split-K and persistent entries' their block_m."""
+    if desc.schedule != SCHEDULE_STANDARD or desc.split_k > 1:
+        return desc.block_m
+    return sk_plan(desc.dtype_bits, desc.scale_mode == SCALE_SUBCHANNEL, desc.epilogue_kind == EPI_KIND_SWIGLU,
+                   m, n, k)[0]
 
 
 def sk_split_count(desc: "KernelDesc", m: int, n: int, k: int, with_workspace: bool = True) -> int:
@@ -209,19 +266,10 @@ def sk_split_count(desc: "KernelDesc", m: int, n: int, k: int, with_workspace: b
     1023 stages of 128 K.  Without a workspace 1, or 0 if K needs a split."""
     if desc.scale_mode == SCALE_SUBCHANNEL:
         return 1
-    ks = 128 if desc.dtype_bits == 4 else 64
-    nst = -(-k // ks)
-    need = 1
-    if desc.dtype_bits == 4:
-        while need * 4 * 1023 < nst:
-            need *= 2
     if not with_workspace:
-        return 1 if need == 1 else 0
-    tiles = (m // desc.block_m) * (n // desc.block_n)
-    s = 1
-    while s * 2 <= 16 and tiles * s * 2 <= SK_TARGET_UNITS and nst >= 16 * s:
-        s *= 2
-    return max(s, need)
+        return 1 if _sk_needed_splits(desc.dtype_bits, k) == 1 else 0
+    rows = _sk_tile_rows(desc, m, n, k)
+    return _sk_splits(desc.dtype_bits, -(-m // rows) * (n // desc.block_n), k)
 
 
 def sk_workspace_bytes(desc: "KernelDesc", m: int, n: int, k: int) -> int:
@@ -230,9 +278,10 @@ def sk_workspace_bytes(desc: "KernelDesc", m: int, n: int, k: int) -> int:
     s = sk_split_count(desc, m, n, k, True)
     if s <= 1:
         return 0
-    tiles = (m // desc.block_m) * (n // desc.block_n)
+    rows = _sk_tile_rows(desc, m, n, k)
+    tiles = -(-m // rows) * (n // desc.block_n)
     cf = 2 if desc.epilogue_kind == EPI_KIND_SWIGLU else 1
-    return ((tiles * 4 + 255) & ~255) + tiles * s * (desc.block_n // 16) * (desc.block_m // 16) * cf * 1024
+    return ((tiles * 4 + 255) & ~255) + tiles * s * (desc.block_n // 16) * (rows // 16) * cf * 1024
 
 
 def _desc(index, family, bits, layout, *, bm, bn, bk, wm, wn, swiglu=False, subch=False, mk=64, group_m=8, pipe=0,
@@ -478,10 +527,6 @@ def _f6_edge_us(m: int, n: int, k: int, swiglu: bool) -> float:
 
 PREDICT_MAX_K = 65536  # K up to which the fits of predicted_us stand
 
-_SKINNY_US = {  # (tile rows, SwiGLU): us per tile and us per tile and K value
-    (64, False): (0.005, 5.2e-6), (32, False): (0.0035, 3.75e-6), (16, False): (0.0028, 2.65e-6),
-    (64, True): (0.019, 1.1e-5), (32, True): (0.0125, 7.0e-6), (16, True): (0.0045, 4.3e-6),
-}
 # subchannel, by group size: us per product on the 32-row skinny tiles (plain,
 # SwiGLU); a 128 x 128 fp6 tile's fixed us and us per K value
 _SKINNY_SUB_US = {32: (2.9e-8, 2.3e-8), 64: (1.5e-8, 1.2e-8), 128: (1.07e-8, 0.74e-8), 256: (0.85e-8, 0.65e-8)}
@@ -495,17 +540,15 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
     N x K of 1024 x 4096, 4096 x 1024, 4096^2, 11008 x 4096, 16384 x 4096 and
     8192^2:
 
-    * skinny per-channel tiles: a launch, then at least one round of tiles
-      (few tiles split K instead), each a fixed part and a part along K; the
-      tallest tile that divides M;
+    * skinny per-channel tiles: sk_plan;
     * skinny subchannel tiles: a launch and the products;
     * fp6 entries: two launches, the conversion at 5 TB/s, then rounds of
       tiles: per-channel 256-row tiles (FP6) or the launcher's split
       (FP6_EDGE); subchannel 128 x 128 tiles, two a CU (1.3 times one).
 
-    Measured against predicted, per-channel: 512 x 4096^2 skinny 16.6 (18),
-    256-row fp6 36.7 (44), edge 24.7 (22); 8176 x 16384 x 4096 skinny 1675
-    (1791), edge 324 (300); 8192^3 fp6 277 (251).  Groups of 128: 64 x 4096^2
+    Measured against predicted, per-channel: 512 x 4096^2 skinny 16.6 (17),
+    256-row fp6 36.7 (44), edge 24.7 (22); 8176 x 16384 x 4096 skinny 64-row
+    tiles 810 (793), edge 324 (300); 8192^3 fp6 277 (251).  Groups of 128: 64 x 4096^2
     skinny 17.5 (17), edge 42.3 (40); 320 x 16384 x 4096 skinny 221 (236),
     edge 59.7 (62); 4160 x 8192^2 edge 397 (388)."""
     if (desc.family != FAMILY_DENSE or desc.dtype_bits != 4 or desc.schedule != SCHEDULE_STANDARD
@@ -518,8 +561,9 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
         if sub not in _F6_SUB_US:
             return None
         if desc.operand_format == OPERANDS_STREAM:
-            tall = {32: 1.0, 64: 1.25, 16: 1.5}[desc.block_m]
-            return 6.0 + _SKINNY_SUB_US[sub][swiglu] * tall * (m * cols * k)
+            low = 1.5 if sk_plan(4, True, swiglu, m, n, k)[0] == 16 else 1.0
+            rank = {32: 1.0, 64: 1.001, 16: 1.002}[desc.block_m]  # the same tiles; the 32-row entry first
+            return 6.0 + _SKINNY_SUB_US[sub][swiglu] * low * rank * (m * cols * k)
         if not desc.needs_workspace:
             return None
         fixed, per_k = _F6_SUB_US[sub]
@@ -527,9 +571,7 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
         rounds = 1.0 if tiles <= _CUS else 1.3 * -(-tiles // (2 * _CUS))
         return convert + (fixed + per_k * k) * rounds
     if desc.operand_format == OPERANDS_STREAM:
-        r = 64 if m % 64 == 0 else (32 if m % 32 == 0 else 16)
-        base, per_k = _SKINNY_US[r, swiglu]
-        return 5.0 + max((m // r) * (n // 64), _CUS) * (base + per_k * k)
+        return sk_plan(4, False, swiglu, m, n, k)[1]
     if desc.operand_format == OPERANDS_FP6_EDGE:
         return convert + _f6_edge_us(m, n, k, swiglu)
     if desc.operand_format == OPERANDS_FP6:

@@ -527,8 +527,10 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
     if (d.operand_format == SHK_OPERANDS_STREAM) {
       static constexpr double plain[4] = {2.9e-8, 1.5e-8, 1.07e-8, 0.85e-8};
       static constexpr double gated[4] = {2.3e-8, 1.2e-8, 0.74e-8, 0.65e-8};
-      const double tall = d.block_m == 32 ? 1.0 : (d.block_m == 64 ? 1.25 : 1.5);
-      return 6.0 + (swiglu ? gated[s] : plain[s]) * tall * (double)(m * cols * k);
+      const double low = shk::sk_plan(4, true, swiglu, m, n, k).rows == 16 ? 1.5 : 1.0;
+      // (the entries run the same tiles; the 32-row one ranks first)
+      const double rank = d.block_m == 32 ? 1.0 : (d.block_m == 64 ? 1.001 : 1.002);
+      return 6.0 + (swiglu ? gated[s] : plain[s]) * low * rank * (double)(m * cols * k);
     }
     if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
     static constexpr double fixed[4] = {5.0, 5.0, 5.0, 3.5};
@@ -537,15 +539,7 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
     const double rounds = tiles <= 256 ? 1.0 : 1.3 * (double)((tiles + 511) / 512);
     return convert + (fixed[s] + per_k[s] * (double)k) * rounds;
   }
-  if (d.operand_format == SHK_OPERANDS_STREAM) {
-    const long r = m % 64 == 0 ? 64 : (m % 32 == 0 ? 32 : 16);
-    const long tiles = (m / r) * (n / 64);
-    const double base = swiglu ? (r == 64 ? 0.019 : (r == 32 ? 0.0125 : 0.0045))
-                               : (r == 64 ? 0.005 : (r == 32 ? 0.0035 : 0.0028));
-    const double per_k = swiglu ? (r == 64 ? 1.1e-5 : (r == 32 ? 7.0e-6 : 4.3e-6))
-                                : (r == 64 ? 5.2e-6 : (r == 32 ? 3.75e-6 : 2.65e-6));
-    return 5.0 + (double)(tiles > 256 ? tiles : 256) * (base + per_k * (double)k);
-  }
+  if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_plan(4, false, swiglu, m, n, k).us;
   if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
   return convert + shk::f6_edge_plan(m, n, k, swiglu).us;
 }
@@ -736,7 +730,7 @@ int amd_strix_halo_kernels_launch_gemm_noalloc(int kernel_index, int device_inde
   if (split_stream) {
     // the partial slots are written before they are read; only the counters
     // must start at zero (256-byte multiple, below the scratch size)
-    const unsigned n16 = (unsigned)(shk::sk_counter_bytes(c.e->d, m, n) / 16);
+    const unsigned n16 = (unsigned)(shk::sk_counter_bytes(c.e->d, m, n, k) / 16);
     hipLaunchKernelGGL(shk::clear_counters_kernel, dim3((n16 + 255) / 256), dim3(256), 0, s,
                        reinterpret_cast<int4*>(c.p.work), n16);
     const hipError_t cerr = hipGetLastError();

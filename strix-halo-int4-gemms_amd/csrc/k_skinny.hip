@@ -39,6 +39,22 @@ hipError_t launch_sk_t(const DenseArgs& a, dim3 grid, hipStream_t s) {
   hipLaunchKernelGGL(sk_gemm_kernel<C>, dim3(sk_units<C>(a, grid)), dim3(C::NT), 0, s, a);
   return hipGetLastError();
 }
+// A standard entry: tiles of the rows that sk_plan picks, masked where M is
+// no multiple of them.
+template <class T>
+hipError_t launch_sk_rows(const DenseArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)((a.M + T::R - 1) / T::R) * (unsigned)(a.N / T::BN));
+  if (a.M % T::R == 0) return launch_sk_t<T>(a, grid, s);
+  hipLaunchKernelGGL((sk_gemm_kernel<T, true>), dim3(sk_units<T>(a, grid)), dim3(T::NT), 0, s, a);
+  return hipGetLastError();
+}
+template <bool SWIGLU, bool SUBCH>
+hipError_t launch_sk_plan(const DenseArgs& a, dim3, hipStream_t s) {
+  const int rows = sk_plan(kBits, SUBCH, SWIGLU, a.M, a.N, a.K).rows;
+  if (rows == 16) return launch_sk_rows<SC<16, SWIGLU, SUBCH>>(a, s);
+  if (SUBCH || rows == 32) return launch_sk_rows<SC<32, SWIGLU, SUBCH>>(a, s);
+  return launch_sk_rows<SC<64, SWIGLU, SUBCH>>(a, s);
+}
 template <class C>
 hipError_t launch_sk_persistent_t(const DenseArgs& a, dim3 grid, hipStream_t s) {
   return launch_persistent<&sk_gemm_kernel<C>>(a, sk_units<C>(a, grid), C::NT, s);
@@ -59,7 +75,7 @@ Entry sk_entry(int schedule, int split) {
   d.block_n = C::BN;
   d.block_k = 32;
   d.num_waves = C::NW;
-  d.num_stages = C::D;
+  d.num_stages = C::LISTED_D;
   d.lds_bytes = C::LDS_BYTES;
   d.group_size_m = 1;
   d.operand_format = SHK_OPERANDS_STREAM;
@@ -69,12 +85,19 @@ Entry sk_entry(int schedule, int split) {
                nullptr, nullptr};
 }
 
+template <int R, bool SWIGLU, bool SUBCH>
+Entry sk_rows_entry() {
+  Entry e = sk_entry<SC<R, SWIGLU, SUBCH>>(SHK_SCHEDULE_STANDARD, 1);
+  e.dense = &launch_sk_plan<SWIGLU, SUBCH>;
+  return e;
+}
+
 template <int R>
 void append_tiles(std::vector<Entry>& t) {
-  t.push_back(sk_entry<SC<R, false, false>>(SHK_SCHEDULE_STANDARD, 1));
-  t.push_back(sk_entry<SC<R, true, false>>(SHK_SCHEDULE_STANDARD, 1));
-  t.push_back(sk_entry<SC<R, false, true>>(SHK_SCHEDULE_STANDARD, 1));
-  t.push_back(sk_entry<SC<R, true, true>>(SHK_SCHEDULE_STANDARD, 1));
+  t.push_back(sk_rows_entry<R, false, false>());
+  t.push_back(sk_rows_entry<R, true, false>());
+  t.push_back(sk_rows_entry<R, false, true>());
+  t.push_back(sk_rows_entry<R, true, true>());
 }
 
 void append_all(std::vector<Entry>& t) {

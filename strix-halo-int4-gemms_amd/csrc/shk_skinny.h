@@ -74,13 +74,15 @@ constexpr int SK_BN = 64;       // output columns per K-split tile
 constexpr int SK_MAX_WAVE_STAGES_I4 = 1023;
 
 // Ring depth: the deepest of 4, 3, 2 stage slots whose rings fit the LDS
-// budget: 78 KiB for four waves (two workgroups share a CU where the tile
-// allows), 150 KiB for eight or more (one workgroup per CU).
+// budget: 78 KiB for four waves, so that two workgroups share a CU; where two
+// slots already exceed that (SwiGLU tiles of 32 and 64 rows), and for eight
+// or more waves, 150 KiB, one workgroup per CU.
 constexpr int sk_stage_bytes(int r, int wcols, bool subch) {
   return r * 64 + wcols * 64 + (subch ? (r / 16) * 256 + 256 : 0);
 }
 constexpr int sk_ring_depth(int stage, int nw, int reserved = 0) {
-  const int budget = (nw >= 8 ? 153600 : 79872) - reserved;  // reserved: LDS the tile uses beside the rings
+  const bool alone = nw >= 8 || nw * 2 * stage > 79872 - reserved;
+  const int budget = (alone ? 153600 : 79872) - reserved;  // reserved: LDS the tile uses beside the rings
   return nw * 4 * stage <= budget ? 4 : (nw * 3 * stage <= budget ? 3 : 2);
 }
 
@@ -124,6 +126,8 @@ struct SkCfg {
   static constexpr int CH = !GSPLIT ? 0 : (RT * CT == 1 ? 4 : (RT * CT == 2 ? 2 : 1));
   static constexpr int CHAIN = GSPLIT ? 2 * NW * CH * RT * CT * 1024 : 0;
   static constexpr int D = DEPTH_ > 0 ? DEPTH_ : sk_ring_depth(STAGE, NW, CHAIN);
+  // the depth the table lists (part of the kernel id): that of a shared CU
+  static constexpr int LISTED_D = NW * 2 * STAGE > 79872 - CHAIN ? 2 : D;
   static constexpr int RING = NW * D * STAGE;
   static constexpr int RED = KSPLIT ? NW * CT * 1024 : 0;  // one row tile of the cross-wave sum
   static constexpr int LDS_BYTES = (RING > RED ? RING : RED) + CHAIN;
@@ -375,7 +379,7 @@ struct SkScales {
   __device__ __forceinline__ void load(const DenseArgs& p, int m0, int n0, int wave, int lane) {
     const int g = lane >> 4;
 #pragma unroll
-    for (int rt = 0; rt < C::RT; ++rt) sa[rt] = load_bf16(p.a_scale + m0 + 16 * rt + (lane & 15));
+    for (int rt = 0; rt < C::RT; ++rt) sa[rt] = load_bf16(p.a_scale + min(m0 + 16 * rt + (lane & 15), p.M - 1));
 #pragma unroll
     for (int f = 0; f < C::FT; ++f) {
       const int n = n0 + (C::KSPLIT ? 16 * wave : C::WOUT * wave + 16 * f) + 4 * g;
@@ -390,7 +394,7 @@ struct SkScales {
   }
 };
 
-template <class C>
+template <class C, bool MASK>
 __device__ __forceinline__ void sk_unit_pc(const DenseArgs& p, uint8_t* smem, int* last_flag, int lane, int wave,
                                            int tm, int tn, int split, int splits, int tile) {
   SkEngine<C> e(p, smem, lane, wave, tm * C::R, tn * C::BN);
@@ -483,11 +487,12 @@ __device__ __forceinline__ void sk_unit_pc(const DenseArgs& p, uint8_t* smem, in
     // exact int32 partials: slot (tile, split) of the workspace after the
     // counters; finalizer wave w's part is RT x FC tiles of 64 lanes x 16 bytes
     int* counters = reinterpret_cast<int*>(p.work);
-    const long counter_bytes = ((long)(p.M / C::R) * (p.N / C::BN) * 4 + 255) & ~255L;
+    const int tiles = (MASK ? (p.M + C::R - 1) / C::R : p.M / C::R) * (p.N / C::BN);
+    const long counter_bytes = ((long)tiles * 4 + 255) & ~255L;
     constexpr long WAVE_BYTES = (long)C::RT * C::FC * 1024;
     constexpr long SLOT_BYTES = C::NFIN * WAVE_BYTES;
     const uint8_t* parts = p.work + counter_bytes;
-    const long ws_bytes = counter_bytes + ((long)(p.M / C::R) * (p.N / C::BN)) * splits * SLOT_BYTES;
+    const long ws_bytes = counter_bytes + (long)tiles * splits * SLOT_BYTES;
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(parts), 0, (int)(ws_bytes - counter_bytes), 0x00020000);
     const uint32_t mine_off = (uint32_t)(((long)tile * splits + split) * SLOT_BYTES + wave * WAVE_BYTES);
@@ -558,6 +563,7 @@ __device__ __forceinline__ void sk_unit_pc(const DenseArgs& p, uint8_t* smem, in
 #pragma unroll
     for (int rt = 0; rt < C::RT; ++rt) {
       const int m = e.m0 + 16 * rt + (lane & 15);
+      if (MASK && m >= p.M) continue;
       float up[4], gt[4];
       int iu[4], ig[4];
       const float sa = scl.sa[rt];
@@ -630,7 +636,7 @@ __device__ __forceinline__ void sk_scale_group(const DenseArgs& p, const uint8_t
   }
 }
 
-template <class C>
+template <class C, bool MASK>
 __device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, int lane, int wave, int tm, int tn) {
   static_assert(C::GSPLIT && C::NW == 4, "four waves take the groups in turn");
   SkEngine<C> e(p, smem, lane, wave, tm * C::R, tn * C::BN);
@@ -781,6 +787,7 @@ __device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, in
     for (int ot = 0; ot < OT; ++ot) {
       const int m = e.m0 + 16 * rt + (lane & 15);
       const int n = e.n0 + 16 * ot + 4 * lg;
+      if (MASK && m >= p.M) continue;
       float up[4], gt[4];
       int iu[4], ig[4];
 #pragma unroll
@@ -798,13 +805,16 @@ __device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, in
 // striding over the units (persistent schedule).  Units are (split, column
 // tile, row tile) with the row tile fastest, so the workgroups reading the
 // same B columns run together on one XCD.
-template <class C>
+// MASK: M need not be a multiple of R.  A rows past M read zeros through the
+// buffer range (MN-major A: the next K row's values, whose products go to
+// rows that are not stored).
+template <class C, bool MASK = false>
 __global__ __launch_bounds__(C::NT) void sk_gemm_kernel(const DenseArgs p) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[C::LDS_BYTES];
   __shared__ int last_flag;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tiles_m = p.M / C::R, tiles = tiles_m * (p.N / C::BN);
+  const int tiles_m = MASK ? (p.M + C::R - 1) / C::R : p.M / C::R, tiles = tiles_m * (p.N / C::BN);
   const int splits = C::SUBCH ? 1 : p.sk_splits;
   const int units = tiles * splits;
   for (int u = blockIdx.x; u < units; u += gridDim.x) {
@@ -812,9 +822,9 @@ __global__ __launch_bounds__(C::NT) void sk_gemm_kernel(const DenseArgs p) {
     const int split = lu / tiles, t = lu - split * tiles;
     const int tn = t / tiles_m, tm = t - tn * tiles_m;
     if constexpr (C::SUBCH)
-      sk_unit_sc<C>(p, smem, lane, wave, tm, tn);
+      sk_unit_sc<C, MASK>(p, smem, lane, wave, tm, tn);
     else
-      sk_unit_pc<C>(p, smem, &last_flag, lane, wave, tm, tn, split, splits, tn * tiles_m + tm);
+      sk_unit_pc<C, MASK>(p, smem, &last_flag, lane, wave, tm, tn, split, splits, tn * tiles_m + tm);
     __syncthreads();
   }
 }

@@ -310,38 +310,100 @@ Entry bwd_entry(int layout) {
 // 8.8 us against 9.9 us for four, each K split adding a tail of device-scope
 // round trips) while every wave keeps at least two stages, at most 16;
 // and for int4 at least as many as keep each wave's x256 int32 sum within
-// 1023 stages of 128 K (up to 64 at K = 2^24).  Without a workspace only
-// one, or 0 when K needs more.  Subchannel tiles always use one.
+// 1023 stages of 128 K (up to 64 at K = 2^24).  Subchannel tiles always use
+// one.
 constexpr int kSkTargetUnits = 256;
-inline int sk_split_count(const shk_kernel_desc& d, long m, long n, long k, bool with_workspace) {
-  if (d.scale_mode == SHK_SCALE_SUBCHANNEL) return 1;
-  const long ks = d.dtype_bits == 4 ? 128 : 64;
-  const long nst = (k + ks - 1) / ks;
+inline int sk_needed_splits(int bits, long k) {
   long need = 1;
-  if (d.dtype_bits == 4)
-    while (need * 4L * 1023L < nst) need *= 2;
-  if (!with_workspace) return need == 1 ? 1 : 0;
-  const long tiles = (m / d.block_m) * (n / d.block_n);
+  if (bits == 4)
+    while (need * 4L * 1023L < (k + 127) / 128) need *= 2;
+  return (int)need;
+}
+inline int sk_splits(int bits, long tiles, long k) {
+  const long nst = bits == 4 ? (k + 127) / 128 : (k + 63) / 64;
   long s = 1;
   while (s * 2 <= 16 && tiles * s * 2 <= kSkTargetUnits && nst >= 16L * s) s *= 2;
+  const long need = sk_needed_splits(bits, k);
   return (int)(s > need ? s : need);
+}
+
+// Rows of the tiles that a standard skinny call of M rows runs, whatever the
+// entry's block_m: 16, 32 or 64, masked to M.  A taller tile reads B fewer
+// times and keeps the matrix cores busier per byte; a lower one gives a small
+// N more workgroups and computes fewer rows that are not there.
+//
+// Per-channel: the smallest predicted time (us) a + b * (K per workgroup /
+// 4096) * rounds of 256 workgroups, whole rounds for the SwiGLU tiles of 32
+// and 64 rows, which run one workgroup a CU, and with K split one more for
+// every 16 rows (up and gate) of partials.  The
+// figures are fits to calls of M 32..400 on N x K of 11008 x 4096, 8192^2,
+// 4096^2 and 1024 x 4096.  Measured, 16, 32 and 64 rows: int8 SwiGLU 48 x
+// 11008 x 4096 29.9, 32.5, 25.7 us, 400 rows 153, 124, 97; int4 SwiGLU 112
+// rows 29.6, 33.7, 34.7; int4 plain 112 x 8192^2 27.7, 21.9, 17.7, 48 x
+// 4096^2 7.0, 8.3, 10.5.
+//
+// Subchannel (16 columns a tile, so many tiles): 32 rows from 17 rows on
+// (SwiGLU from 33); groups of 128, 48 x 4096^2: 19.9, 16.3, 19.6, 400 rows
+// 110, 80, 124.
+struct SkPlan {
+  int rows;
+  double us;
+};
+inline SkPlan sk_plan(int bits, bool subch, bool swiglu, long m, long n, long k) {
+  if (subch) return SkPlan{m <= (swiglu ? 32 : 16) ? 16 : 32, 0.0};
+  struct Fit {
+    double a, b;
+    bool whole;
+  };
+  static constexpr Fit fits[2][2][3] = {
+      {{{3.6, 3.38, false}, {3.4, 4.8, false}, {4.8, 6.07, false}}, {{7.0, 4.6, false}, {3.0, 10.5, true}, {3.0, 15.5, true}}},
+      {{{3.8, 5.2, false}, {3.5, 6.45, false}, {4.5, 8.0, false}}, {{15.3, 7.7, false}, {12.0, 12.5, true}, {12.0, 15.0, true}}}};
+  SkPlan best{16, -1.0};
+  for (int i = 0; i < 3; ++i) {
+    const int rows = 16 << i;
+    if (i > 0 && m <= rows / 2) break;
+    const Fit& f = fits[bits == 8][swiglu][i];
+    const long tiles = ((m + rows - 1) / rows) * (n / 64);
+    const int s = sk_splits(bits, tiles, k);
+    const long units = tiles * s;
+    const double rounds = units <= 256 ? 1.0 : (f.whole ? (double)((units + 255) / 256) : (double)units / 256.0);
+    const double us = f.a + (s > 1 ? (double)(rows / 16 * (swiglu ? 2 : 1)) : 0.0) + f.b * ((double)k / (double)s / 4096.0) * rounds;
+    if (best.us < 0.0 || us < best.us) best = SkPlan{rows, us};
+  }
+  return best;
+}
+// Rows of a table entry's tiles: the split-K and persistent entries keep
+// their block_m.
+inline int sk_tile_rows(const shk_kernel_desc& d, long m, long n, long k) {
+  if (d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1) return d.block_m;
+  return sk_plan(d.dtype_bits, d.scale_mode == SHK_SCALE_SUBCHANNEL, d.epilogue_kind == SHK_EPI_KIND_SWIGLU, m, n, k).rows;
+}
+inline long sk_tiles(const shk_kernel_desc& d, long m, long n, long k) {
+  const long r = sk_tile_rows(d, m, n, k);
+  return ((m + r - 1) / r) * (n / d.block_n);
+}
+// Workgroups sharing a tile's K; without a workspace one, or 0 when K needs
+// more.
+inline int sk_split_count(const shk_kernel_desc& d, long m, long n, long k, bool with_workspace) {
+  if (d.scale_mode == SHK_SCALE_SUBCHANNEL) return 1;
+  if (!with_workspace) return sk_needed_splits(d.dtype_bits, k) == 1 ? 1 : 0;
+  return sk_splits(d.dtype_bits, sk_tiles(d, m, n, k), k);
 }
 // Workspace of a skinny launch with more than one split: the tiles' arrival
 // counters, padded to 256 bytes, then an exact int32 partial of every (tile,
 // split).  All of it is zero before the first launch and every launch leaves
 // what it used zero, whatever the shapes of the launches that share it.
+inline unsigned long long sk_counter_bytes(const shk_kernel_desc& d, long m, long n, long k) {
+  return (unsigned long long)((sk_tiles(d, m, n, k) * 4 + 255) & ~255L);
+}
 inline unsigned long long sk_workspace_bytes(const shk_kernel_desc& d, long m, long n, long k) {
   const int s = sk_split_count(d, m, n, k, true);
   if (s <= 1) return 0;
-  const long tiles = (m / d.block_m) * (n / d.block_n);
   const long cf = d.epilogue_kind == SHK_EPI_KIND_SWIGLU ? 2 : 1;
-  // per (tile, split): (block_n / 16) output column tiles x (block_m / 16)
-  // row tiles x (up, gate) x 1 KiB
-  return (unsigned long long)((tiles * 4 + 255) & ~255L) +
-         (unsigned long long)tiles * s * (d.block_n / 16) * (d.block_m / 16) * cf * 1024;
-}
-inline unsigned long long sk_counter_bytes(const shk_kernel_desc& d, long m, long n) {
-  return (unsigned long long)((((m / d.block_m) * (n / d.block_n)) * 4 + 255) & ~255L);
+  // per (tile, split): (block_n / 16) output column tiles x (rows / 16) row
+  // tiles x (up, gate) x 1 KiB
+  return sk_counter_bytes(d, m, n, k) + (unsigned long long)sk_tiles(d, m, n, k) * s * (d.block_n / 16) *
+                                            (sk_tile_rows(d, m, n, k) / 16) * cf * 1024;
 }
 
 // Each kernel translation unit appends its entries in a fixed order

@@ -1,0 +1,68 @@
+"""The skinny tiles' row heights (shk_table.h sk_plan): a call of M rows runs
+16-, 32- or 64-row tiles masked to M, whatever block_m its entry has.  Every
+output against the CPU oracle; the row below the output stays untouched."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle import ref
+from tests._util import bf16_bits, dense_case, max_ulp, spec_of, stable_seed, to_dev
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+import amd_strix_halo_kernels as shk  # noqa: E402
+from amd_strix_halo_kernels import kernel_table as kt  # noqa: E402
+from amd_strix_halo_kernels import native  # noqa: E402
+
+
+def _check(bits, layout, epilogue, sub, m, n, k, device, rows):
+    swiglu = epilogue == "swiglu"
+    assert kt.sk_plan(bits, bool(sub), swiglu, m, n, k)[0] == rows
+    a_q, b_q, a_arg, b_arg, sa, sb = dense_case(stable_seed("rows", bits, layout, epilogue, sub, m, n, k), bits=bits,
+                                                layout=layout, m=m, n=n, k=k, subchannel=sub or None, swiglu=swiglu)
+    a, b, ta, tb = (to_dev(torch, x, device) for x in (a_arg, b_arg, sa, sb))
+    kernel = next(x for x in shk.default_registry.all() if kt.TABLE[x.table_index].is_stream
+                  and x.tile.block_m == 16 and x.scale == spec_of(sub) and x.epilogue.value == epilogue
+                  and x.layout.value == layout and x.tile.split_k == 1 and kt.TABLE[x.table_index].dtype_bits == bits
+                  and x.schedule is shk.KernelSchedule.STANDARD)
+    print(f"case {kernel.kernel_id} shape=({m},{n},{k}) rows={rows}", flush=True)
+    out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=device)
+    for _ in range(2):  # a split launch leaves its workspace zero for the next
+        native.launch_generated_kernel(a, b, kernel=kernel, a_scale=ta, b_scale=tb, c=out[:m])
+    raw = native.launch_generated_kernel_i32(a, b, kernel=kernel, a_scale=ta, b_scale=tb)
+    torch.cuda.synchronize()
+    assert bool((out[m] == 7.0).all()), "rows past M written"
+    assert np.array_equal(raw.cpu().numpy(), ref.int_matmul(a_q, b_q))
+    want = ref.reference_gemm_bf16(a_arg, b_arg, bits=bits, layout=layout, a_scale=sa, b_scale=sb,
+                                   subchannel=sub or None, epilogue=epilogue)
+    got = bf16_bits(torch, out[:m])
+    assert max_ulp(got, want) <= 2 if swiglu else np.array_equal(got, want)
+
+
+# (bits, epilogue, rows, m, n, k): masked and whole tiles of each height,
+# with and without K split over workgroups
+_PLANS = [
+    (4, "none", 64, 112, 8192, 2080), (4, "none", 64, 192, 8192, 2080), (4, "none", 32, 48, 512, 96),
+    (4, "none", 32, 144, 512, 8192), (8, "none", 64, 112, 8192, 1024), (8, "none", 32, 144, 512, 4096),
+    (8, "none", 32, 48, 512, 96), (4, "swiglu", 64, 272, 2048, 96), (4, "swiglu", 64, 192, 4096, 96),
+    (4, "swiglu", 32, 48, 512, 2080), (8, "swiglu", 64, 272, 2048, 96), (8, "swiglu", 64, 272, 512, 8192),
+    (8, "swiglu", 32, 48, 512, 1024),
+]
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("bits,epilogue,rows,m,n,k", _PLANS)
+def test_every_height_matches_the_oracle(bits, epilogue, rows, m, n, k, layout, device):
+    _check(bits, layout, epilogue, 0, m, n, k, device, rows)
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("sub", [32, 64, 128, 256])
+@pytest.mark.parametrize("epilogue,m", [("none", 48), ("none", 64), ("swiglu", 80)])
+def test_subchannel_32_row_tiles_match_the_oracle(bits, sub, epilogue, m, layout, device):
+    _check(bits, layout, epilogue, sub, m, 192, 5 * sub, device, 32)
