@@ -19,6 +19,11 @@
 // a multiple of 128.  Workspace: A as round32(M) rows x Kw, then per group
 // B as round32(N) rows x Kw.
 //
+// Any group sizes are safe to run: the host's check of their sum may finish
+// while the kernels run (ragged.py), so a task past the rows of lhs returns,
+// rows past M are never stored (the output buffer's range), and the
+// backward's lengths are clamped to the K capacity.
+//
 // Subchannel forward: the same tasks and converted operands on the 128 x 128
 // subchannel tile of shk_f6sub.h (groups of 32 to 256 added into fp32 in
 // group order, api.py:311-325 as ragged.py applies it), two workgroups per
@@ -75,6 +80,7 @@ __global__ __launch_bounds__(256, 3) void f6_ragged_fwd_kernel(const RaggedFwdAr
   const int tn = w - task * tiles_n;
   const int4 t = *reinterpret_cast<const int4*>(p.tasks + 4 * task);
   const int g = t.x, m0 = t.y;
+  if (m0 < 0 || m0 >= p.M) return;  // group sizes that do not sum to M: the task holds no row of lhs
   const int kw = round128(p.K);
   const unsigned long long a_bytes = f6_operand_bytes(round32(p.M), kw);
   const unsigned long long b_bytes = f6_operand_bytes(round32(p.N), kw);
@@ -123,6 +129,7 @@ __global__ __launch_bounds__(256, 2) void f6_ragged_sub_fwd_kernel(const RaggedF
   const int tn = w - task * tiles_n;
   const int4 t = *reinterpret_cast<const int4*>(p.tasks + 4 * task);
   const int g = t.x, m0 = t.y, n0 = tn * kTile;
+  if (m0 < 0 || m0 >= p.M) return;  // as in f6_ragged_fwd_kernel
   const int kw = round256(p.K);
   const unsigned long long a_bytes = f6_operand_bytes(round32(p.M), kw);
   const unsigned long long b_bytes = f6_operand_bytes(round32(p.N), kw);
