@@ -39,7 +39,7 @@ hipError_t launch_sk_t(const DenseArgs& a, dim3 grid, hipStream_t s) {
   hipLaunchKernelGGL(sk_gemm_kernel<C>, dim3(sk_units<C>(a, grid)), dim3(C::NT), 0, s, a);
   return hipGetLastError();
 }
-// A standard entry: tiles of the rows that sk_plan picks, masked where M is
+// A standard entry: tiles of the rows that sk_plan picked, masked where M is
 // no multiple of them.
 template <class T>
 hipError_t launch_sk_rows(const DenseArgs& a, hipStream_t s) {
@@ -50,7 +50,11 @@ hipError_t launch_sk_rows(const DenseArgs& a, hipStream_t s) {
 }
 template <bool SWIGLU, bool SUBCH>
 hipError_t launch_sk_plan(const DenseArgs& a, dim3, hipStream_t s) {
-  const int rows = sk_plan(kBits, SUBCH, SWIGLU, a.M, a.N, a.K).rows;
+  const int rows = a.sk_rows;
+  if constexpr (SUBCH && !SWIGLU) {
+    using T = SkCfg<kBits, kLayout, 16, false, true, 16, 8>;
+    if (rows == 16 && a.subchannel >= T::KS) return launch_sk_rows<T>(a, s);
+  }
   if (rows == 16) return launch_sk_rows<SC<16, SWIGLU, SUBCH>>(a, s);
   if (SUBCH || rows == 32) return launch_sk_rows<SC<32, SWIGLU, SUBCH>>(a, s);
   return launch_sk_rows<SC<64, SWIGLU, SUBCH>>(a, s);

@@ -372,6 +372,7 @@ struct DenseArgs {
   uint8_t* work;     // fp6 path: caller workspace for the converted operands
   int split_tn;      // int8 256-row tiles: first column tile run as 128-row tiles (0: none)
   int sk_splits;     // skinny per-channel tiles: workgroups sharing a tile's K (1: none)
+  int sk_rows;       // skinny tiles: rows of a tile (sk_plan)
 };
 
 // Tile order: workgroups are dispatched round-robin over the 8 XCDs, so the

@@ -81,7 +81,7 @@ constexpr int sk_stage_bytes(int r, int wcols, bool subch) {
   return r * 64 + wcols * 64 + (subch ? (r / 16) * 256 + 256 : 0);
 }
 constexpr int sk_ring_depth(int stage, int nw, int reserved = 0) {
-  const bool alone = nw >= 8 || nw * 2 * stage > 79872 - reserved;
+  const bool alone = nw > 8 || nw * 2 * stage > 79872 - reserved;
   const int budget = (alone ? 153600 : 79872) - reserved;  // reserved: LDS the tile uses beside the rings
   return nw * 4 * stage <= budget ? 4 : (nw * 3 * stage <= budget ? 3 : 2);
 }
@@ -123,7 +123,7 @@ struct SkCfg {
   // GSPLIT: each wave takes CH consecutive groups per round; two rounds'
   // scaled partials, one 16 x 16 tile (1 KiB) per wave, group, row tile and
   // B column tile, follow the rings
-  static constexpr int CH = !GSPLIT ? 0 : (RT * CT == 1 ? 4 : (RT * CT == 2 ? 2 : 1));
+  static constexpr int CH = !GSPLIT ? 0 : (NW == 8 ? 1 : (RT * CT == 1 ? 4 : (RT * CT == 2 ? 2 : 1)));
   static constexpr int CHAIN = GSPLIT ? 2 * NW * CH * RT * CT * 1024 : 0;
   static constexpr int D = DEPTH_ > 0 ? DEPTH_ : sk_ring_depth(STAGE, NW, CHAIN);
   // the depth the table lists (part of the kernel id): that of a shared CU
@@ -588,18 +588,26 @@ __device__ __forceinline__ void sk_unit_pc(const DenseArgs& p, uint8_t* smem, in
 }
 
 // ---------------------------------------------------------------------------
-// Subchannel tile (GSPLIT): the four waves share the tile's 16 output
+// Subchannel tile (GSPLIT): the NW = 4 or 8 waves share the tile's 16 output
 // columns (and the gate's 16 for SwiGLU) and take its groups in chunks of
-// CH consecutive groups: in round r, wave w multiplies chunk 4r + w (its
+// CH consecutive groups: in round r, wave w multiplies chunk NW r + w (its
 // stages, or for chunks shorter than a stage its groups' steps of one
 // stage, the A fragments of the other lanes zeroed for groups of 32) and
 // scales each group's integer partial,
 // x = (float(sum_g) * a_scale[m, g]) * b_scale[g, n] (api.py:311-325).  The
-// round's 4 CH values of x go through LDS; after the round's barrier wave 0
+// round's NW CH values of x go through LDS; after the round's barrier wave 0
 // adds them into the totals in group order, which is the reference's order
 // of the sums (the raw mode adds the integer partials).  Wave 0 stores the
 // tile.
 
+// Eight waves, one group each per round, for 16 rows and groups of a whole
+// stage or more (128, 256; int8 also 64): a wave waits on memory, LDS and
+// dependent VALU results for half of its cycles, and four waves a SIMD in
+// place of two fill more of them (16 x 8192^2, groups of 128: 23.6 -> 21.6
+// us B MN-major, 18.5 -> 15.3 K-major; 256: 21.3 -> 19.6, 15.0 -> 13.7).
+// Shorter groups would load every stage once per group: four waves (groups
+// of 64: 28.4 us with four, 31.5 with eight).
+//
 // x of one group from its integer partials and the scales in the stage slot
 // (j: the group's slot among the stage's scales; odd_a[rt]: whether the
 // lane's a_scale element of group 0 is the high half of its dword).
@@ -638,7 +646,8 @@ __device__ __forceinline__ void sk_scale_group(const DenseArgs& p, const uint8_t
 
 template <class C, bool MASK>
 __device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, int lane, int wave, int tm, int tn) {
-  static_assert(C::GSPLIT && C::NW == 4, "four waves take the groups in turn");
+  static_assert(C::GSPLIT && (C::NW == 4 || C::NW == 8), "four or eight waves take the groups in turn");
+  constexpr int NWSH = C::NW == 8 ? 3 : 2;  // log2(NW)
   SkEngine<C> e(p, smem, lane, wave, tm * C::R, tn * C::BN);
   constexpr int KSH = C::BITS == 4 ? 7 : 6;  // log2(KS)
   static_assert((1 << KSH) == C::KS, "stage K");
@@ -652,12 +661,12 @@ __device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, in
   const int lsh = sh + CHSH;                    // log2 of a chunk's K
   const int spc_sh = lsh > KSH ? lsh - KSH : 0;
   const int spc = 1 << spc_sh;                  // stages per chunk (a chunk shorter than a stage: 1)
-  const int rounds = (nch + 3) >> 2;
-  const int my_chunks = wave < nch ? ((nch - 1 - wave) >> 2) + 1 : 0;
+  const int rounds = (nch + C::NW - 1) >> NWSH;
+  const int my_chunks = wave < nch ? ((nch - 1 - wave) >> NWSH) + 1 : 0;
   const int n_i = my_chunks << spc_sh;          // this wave's stages
   const int lg = lane >> 4;
   // this wave's stage i: stage i % spc of chunk 4 (i / spc) + wave
-  auto stage_of = [&](int i) { return (((4 * (i >> spc_sh) + wave) << lsh) >> KSH) + (i & (spc - 1)); };
+  auto stage_of = [&](int i) { return ((((i >> spc_sh) * C::NW + wave) << lsh) >> KSH) + (i & (spc - 1)); };
   uint8_t* chain = smem + (C::LDS_BYTES - C::CHAIN);
   auto chain_at = [&](int par, int w, int cg, int rt, int c) {
     return chain + ((((par * C::NW + w) * CH + cg) * C::RT + rt) * C::CT + c) * 1024 + 16 * lane;
@@ -714,7 +723,7 @@ __device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, in
   clear(acc);
   int i = 0;
   for (int r = 0; r < rounds; ++r) {
-    const int k = 4 * r + wave;  // this wave's chunk: groups [k CH, (k + 1) CH)
+    const int k = C::NW * r + wave;  // this wave's chunk: groups [k CH, (k + 1) CH)
     const int par = r & 1;
     if (k < nch) {
       for (int j = 0; j < spc; ++j, ++i) {
@@ -757,10 +766,10 @@ __device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, in
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (wave == 0) {
 #pragma unroll
-      for (int w = 0; w < 4; ++w)
+      for (int w = 0; w < C::NW; ++w)
 #pragma unroll
         for (int cg = 0; cg < CH; ++cg) {
-          if ((((4 * r + w) << CHSH) + cg) >= G) continue;
+          if ((((C::NW * r + w) << CHSH) + cg) >= G) continue;
 #pragma unroll
           for (int rt = 0; rt < C::RT; ++rt)
 #pragma unroll

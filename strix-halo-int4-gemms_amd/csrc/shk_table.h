@@ -378,32 +378,34 @@ inline int sk_tile_rows(const shk_kernel_desc& d, long m, long n, long k) {
   if (d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1) return d.block_m;
   return sk_plan(d.dtype_bits, d.scale_mode == SHK_SCALE_SUBCHANNEL, d.epilogue_kind == SHK_EPI_KIND_SWIGLU, m, n, k).rows;
 }
-inline long sk_tiles(const shk_kernel_desc& d, long m, long n, long k) {
-  const long r = sk_tile_rows(d, m, n, k);
-  return ((m + r - 1) / r) * (n / d.block_n);
-}
-// Workgroups sharing a tile's K; without a workspace one, or 0 when K needs
-// more.
-inline int sk_split_count(const shk_kernel_desc& d, long m, long n, long k, bool with_workspace) {
-  if (d.scale_mode == SHK_SCALE_SUBCHANNEL) return 1;
-  if (!with_workspace) return sk_needed_splits(d.dtype_bits, k) == 1 ? 1 : 0;
-  return sk_splits(d.dtype_bits, sk_tiles(d, m, n, k), k);
-}
-// Workspace of a skinny launch with more than one split: the tiles' arrival
-// counters, padded to 256 bytes, then an exact int32 partial of every (tile,
-// split).  All of it is zero before the first launch and every launch leaves
-// what it used zero, whatever the shapes of the launches that share it.
-inline unsigned long long sk_counter_bytes(const shk_kernel_desc& d, long m, long n, long k) {
-  return (unsigned long long)((sk_tiles(d, m, n, k) * 4 + 255) & ~255L);
-}
-inline unsigned long long sk_workspace_bytes(const shk_kernel_desc& d, long m, long n, long k) {
-  const int s = sk_split_count(d, m, n, k, true);
-  if (s <= 1) return 0;
-  const long cf = d.epilogue_kind == SHK_EPI_KIND_SWIGLU ? 2 : 1;
-  // per (tile, split): (block_n / 16) output column tiles x (rows / 16) row
-  // tiles x (up, gate) x 1 KiB
-  return sk_counter_bytes(d, m, n, k) + (unsigned long long)sk_tiles(d, m, n, k) * s * (d.block_n / 16) *
-                                            (sk_tile_rows(d, m, n, k) / 16) * cf * 1024;
+// A skinny call: its tile rows, the workgroups sharing a tile's K (without a
+// workspace one, or 0 when K needs more; subchannel tiles always one), and
+// with more than one split its workspace: the tiles' arrival counters, padded
+// to 256 bytes, then an exact int32 partial of every (tile, split).  All of
+// it is zero before the first launch and every launch leaves what it used
+// zero, whatever the shapes of the launches that share it.
+struct SkCall {
+  int rows, splits;
+  unsigned long long counter_bytes, workspace_bytes;  // 0 unsplit
+};
+inline SkCall sk_call(const shk_kernel_desc& d, long m, long n, long k, bool with_workspace) {
+  SkCall c{sk_tile_rows(d, m, n, k), 1, 0, 0};
+  if (d.scale_mode == SHK_SCALE_SUBCHANNEL) return c;
+  if (!with_workspace) {
+    if (sk_needed_splits(d.dtype_bits, k) != 1) c.splits = 0;
+    return c;
+  }
+  const long tiles = ((m + c.rows - 1) / c.rows) * (n / d.block_n);
+  c.splits = sk_splits(d.dtype_bits, tiles, k);
+  if (c.splits > 1) {
+    const long cf = d.epilogue_kind == SHK_EPI_KIND_SWIGLU ? 2 : 1;
+    c.counter_bytes = (unsigned long long)((tiles * 4 + 255) & ~255L);
+    // per (tile, split): (block_n / 16) output column tiles x (rows / 16) row
+    // tiles x (up, gate) x 1 KiB
+    c.workspace_bytes =
+        c.counter_bytes + (unsigned long long)tiles * c.splits * (d.block_n / 16) * (c.rows / 16) * cf * 1024;
+  }
+  return c;
 }
 
 // Each kernel translation unit appends its entries in a fixed order
