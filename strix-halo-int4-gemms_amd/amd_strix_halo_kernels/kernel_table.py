@@ -544,13 +544,14 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
     * skinny subchannel tiles: a launch and the products;
     * fp6 entries: two launches, the conversion at 5 TB/s, then rounds of
       tiles: per-channel 256-row tiles (FP6) or the launcher's split
-      (FP6_EDGE); subchannel 128 x 128 tiles, two a CU (1.3 times one).
+      (FP6_EDGE); subchannel 128 x 128 tiles, two a CU (1.3 times one; 1.1
+      beside half-height tiles, which alone take 0.8).
 
     Measured against predicted, per-channel: 512 x 4096^2 skinny 16.6 (17),
     256-row fp6 36.7 (44), edge 24.7 (22); 8176 x 16384 x 4096 skinny 64-row
     tiles 810 (793), edge 324 (300); 8192^3 fp6 277 (251).  Groups of 128: 64 x 4096^2
-    skinny 17.5 (17), edge 42.3 (40); 320 x 16384 x 4096 skinny 221 (236),
-    edge 59.7 (62); 4160 x 8192^2 edge 397 (388)."""
+    skinny 17.5 (17), edge 37.5 (34); 320 x 16384 x 4096 skinny 221 (236),
+    edge 56.5 (57); 4160 x 4096^2 edge 116 (132)."""
     if (desc.family != FAMILY_DENSE or desc.dtype_bits != 4 or desc.schedule != SCHEDULE_STANDARD
             or desc.split_k > 1 or k > PREDICT_MAX_K):
         return None
@@ -567,8 +568,13 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
         if not desc.needs_workspace:
             return None
         fixed, per_k = _F6_SUB_US[sub]
-        tiles = -(-m // 128) * (-(-n // 64) if swiglu else -(-n // 128))
-        rounds = 1.0 if tiles <= _CUS else 1.3 * -(-tiles // (2 * _CUS))
+        columns = -(-n // 64) if swiglu else -(-n // 128)
+        whole, tiles = (m + 63) // 128 * columns, -(-m // 128) * columns  # the others half as high
+        rounds = 1.0
+        if tiles > _CUS:
+            rounds = 1.1 if whole <= _CUS and tiles <= 2 * _CUS else 1.3 * -(-(whole + tiles) // (4 * _CUS))
+        if whole == 0:
+            rounds *= 0.8
         return convert + (fixed + per_k * k) * rounds
     if desc.operand_format == OPERANDS_STREAM:
         return sk_plan(4, False, swiglu, m, n, k)[1]

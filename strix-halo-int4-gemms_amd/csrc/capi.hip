@@ -537,8 +537,11 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
     if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
     static constexpr double fixed[4] = {5.0, 5.0, 5.0, 3.5};
     static constexpr double per_k[4] = {0.0215, 0.0125, 0.0061, 0.0038};
-    const long tiles = ((m + 127) / 128) * (swiglu ? (n + 63) / 64 : (n + 127) / 128);
-    const double rounds = tiles <= 256 ? 1.0 : 1.3 * (double)((tiles + 511) / 512);
+    const long cols_t = swiglu ? (n + 63) / 64 : (n + 127) / 128;
+    const long whole = (m + 63) / 128 * cols_t, tiles = (m + 127) / 128 * cols_t;  // the others half as high
+    double rounds = 1.0;
+    if (tiles > 256) rounds = whole <= 256 && tiles <= 512 ? 1.1 : 1.3 * (double)((whole + tiles + 1023) / 1024);
+    if (whole == 0) rounds *= 0.8;
     return convert + (fixed[s] + per_k[s] * (double)k) * rounds;
   }
   if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_plan(4, false, swiglu, m, n, k).us;

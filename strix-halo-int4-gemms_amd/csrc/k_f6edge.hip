@@ -67,6 +67,7 @@ using CSub = Cfg<4, true, true, 128, SWIGLU ? 64 : 128, 128, 2, 2, SWIGLU, true,
 template <bool SWIGLU, int MODE, int EPI>
 void launch_sub_edge(const DenseArgs& g, hipStream_t s) {
   using T = CSub<SWIGLU>;
+  // (whole tile rows, and one more for the rows left over)
   const dim3 grid((unsigned)(((g.M + T::BM - 1) / T::BM) * ((g.N + T::BN - 1) / T::BN)));
   if (g.subchannel == 32) hipLaunchKernelGGL((f6_sub_edge_kernel<T, MODE, EPI, 1>), grid, dim3(256), 0, s, g);
   else if (g.subchannel == 64) hipLaunchKernelGGL((f6_sub_edge_kernel<T, MODE, EPI, 2>), grid, dim3(256), 0, s, g);

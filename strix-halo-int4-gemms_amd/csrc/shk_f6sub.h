@@ -69,14 +69,15 @@ namespace shk {
 // is exact in fp32.  sa_bits / sb_bits: the bf16 bits of the lane's scales
 // (rows out_row(0), out_row(1); columns 32j + lane % 32).
 typedef float f6_v32f __attribute__((ext_vector_type(32)));
-__device__ __forceinline__ void f6sub_fold_fast(const v16f (&acc)[2][2], float (&tot)[2][2][16], int lane,
-                                                const uint32_t (&sa_bits)[2], const uint32_t (&sb_bits)[2]) {
-  const float av = __uint_as_float((lane < 32 ? sa_bits[0] : sa_bits[1]) << 16);
+template <int MI>
+__device__ __forceinline__ void f6sub_fold_fast(const v16f (&acc)[MI][2], float (&tot)[MI][2][16], int lane,
+                                                const uint32_t (&sa_bits)[MI], const uint32_t (&sb_bits)[2]) {
+  const float av = __uint_as_float((lane < 32 ? sa_bits[0] : sa_bits[MI - 1]) << 16);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const f6_v32f ab = __builtin_amdgcn_mfma_f32_32x32x1f32(__uint_as_float(sb_bits[j] << 16), av, f6_v32f{}, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float x = acc[i][j][r] * ab[16 * i + r];
@@ -85,8 +86,9 @@ __device__ __forceinline__ void f6sub_fold_fast(const v16f (&acc)[2][2], float (
   }
 }
 
-template <class C>
+template <class C, int MI_ = 2>
 struct F6SubEngine {
+  static constexpr int MI = MI_;                    // 32-row blocks per wave
   static constexpr int P = 3;                       // ring slots
   static constexpr int NW = 4;
   static constexpr int PANEL = 2 * F6_BLOCK;        // 32 rows x 128 K: 3 KiB
@@ -104,9 +106,9 @@ struct F6SubEngine {
                 "128 x 128 tiles of 2 x 2 waves, subchannel");
   static constexpr int SPG = 2;                     // stages per group of 256 K
 
-  v16f acc[2][2];
-  float tot[2][2][16];
-  v6i fa[2][2][2];  // [set][step][i]
+  v16f acc[MI][2];
+  float tot[MI][2][16];
+  v6i fa[2][2][MI];  // [set][step][i]
   v6i fb[2][2][2];  // [set][step][j]
   uint32_t voff[OPW];
   v4i rs;        // operand DMA resource (waves 0-1: A, 2-3: B)
@@ -120,7 +122,7 @@ struct F6SubEngine {
   // products below 2^110 in magnitude, so none is NaN
   bool all_fast;
 
-  __device__ __forceinline__ int out_row(int i) const { return wm * 64 + 32 * i + (lane & 31); }
+  __device__ __forceinline__ int out_row(int i) const { return wm * (32 * MI) + 32 * i + (lane & 31); }
   __device__ __forceinline__ int out_col(int j, int q) const {
     return wn * TN + (SWIGLU ? 0 : 32 * j) + 8 * q + 4 * (lane >> 5);
   }
@@ -161,7 +163,7 @@ struct F6SubEngine {
       sbase = 2 * (SWIGLU ? 32 * (c >> 6) + (c & 31) + ((c >> 5) & 1) * (n_cols / 2) : c);
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -194,7 +196,7 @@ struct F6SubEngine {
   // (panel i adds PANEL * i, step 1 adds one block)
   __device__ __forceinline__ Reads reads_of_slot(int slot) const {
     const uint32_t s = lds0 + (uint32_t)slot * STAGE;
-    const uint32_t a = s + 2u * wm * PANEL, b = s + OPB + 2u * wn * PANEL;
+    const uint32_t a = s + (uint32_t)MI * wm * PANEL, b = s + OPB + 2u * wn * PANEL;
     return Reads{a + 16u * lane, a + 1024u + 8u * lane, b + 16u * lane, b + 1024u + 8u * lane};
   }
 
@@ -208,7 +210,8 @@ struct F6SubEngine {
     constexpr bool IS_A = F == 0 || F == 3;
     constexpr int IDX = F == 0 ? 0 : (F == 3 ? 1 : F - 1);
     constexpr int OFF = IDX * PANEL + ST * F6_BLOCK;
-    v6i& dst = IS_A ? fa[S][ST][IDX] : fb[S][ST][IDX];
+    if constexpr (IS_A && IDX >= MI) return;
+    v6i& dst = IS_A ? fa[S][ST][IDX % MI] : fb[S][ST][IDX];
     if constexpr (Q % 2 == 0) {
       v4i x;
       asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(x) : "v"(IS_A ? r.a16 : r.b16), "i"(OFF));
@@ -240,6 +243,20 @@ struct F6SubEngine {
                                        const v4i& rss_st, uint32_t svo, uint32_t sm0, int s8) {
     constexpr int ST = T / 4, I = (T % 4) / 2, J = T % 2;
     constexpr bool Z = ZERO && ST == 0;
+    if constexpr (I >= MI) {
+      // one row block a wave: the tick has its loads only (with the wait
+      // states after the M0 write, as in lds_dma16)
+      if constexpr (T < OPW)
+        asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                     :
+                     : "v"(voff[T]), "s"(rs_st), "s"(so), "{m0}"(m0_st + 1024u * T)
+                     : "memory");
+      else if constexpr (T == OPW && !ZERO)
+        asm volatile("s_nop 4\n\tbuffer_load_dword %0, %1, 0 offen lds"
+                     :
+                     : "v"(svo), "s"(rss_st), "{m0}"(sm0)
+                     : "memory");
+    } else
     // the compiler writes M0 before each statement; the MFMA is the wait
     // state the LDS-DMA load needs after that write
     if constexpr (T < OPW) {
@@ -297,7 +314,11 @@ struct F6SubEngine {
   template <int N>
   __device__ __forceinline__ void fence() {
     static_assert(N == 4 || N == 7, "wait states");
-    if constexpr (N == 4)
+    if constexpr (MI == 1 && N == 4)
+      asm volatile("s_nop 4" : "+v"(acc[0][0]), "+v"(acc[0][1]));
+    else if constexpr (MI == 1)
+      asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(acc[0][0]), "+v"(acc[0][1]));
+    else if constexpr (N == 4)
       asm volatile("s_nop 4" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[1][0]), "+v"(acc[1][1]));
     else
       asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
@@ -309,6 +330,11 @@ struct F6SubEngine {
   // operand here, so none is copied before the data is in.
   template <int S>
   __device__ __forceinline__ void frag_fence() {
+    if constexpr (MI == 1)
+      asm volatile("s_waitcnt lgkmcnt(0)"
+                   : "+v"(fa[S][0][0]), "+v"(fb[S][0][0]), "+v"(fb[S][0][1]), "+v"(fa[S][1][0]), "+v"(fb[S][1][0]),
+                     "+v"(fb[S][1][1])::"memory");
+    else
     asm volatile("s_waitcnt lgkmcnt(0)"
                  : "+v"(fa[S][0][0]), "+v"(fa[S][0][1]), "+v"(fb[S][0][0]), "+v"(fb[S][0][1]), "+v"(fa[S][1][0]),
                    "+v"(fa[S][1][1]), "+v"(fb[S][1][0]), "+v"(fb[S][1][1])::"memory");
@@ -367,11 +393,11 @@ struct F6SubEngine {
   // window.  Read at the top of the group's last stage (after its barrier,
   // so the DMA that loaded them is complete and visible), so that their
   // latency passes under that stage's MFMAs.
-  uint32_t sa_bits[2], sb_bits[2];
+  uint32_t sa_bits[MI], sb_bits[2];
   __device__ __forceinline__ void load_scales(const uint8_t* smem, int g) {
     const uint8_t* sl = smem + RING + (g & 3) * SCALE_SLOT;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < MI; ++i) {
       const int row = out_row(i);
       const uint32_t w = *reinterpret_cast<const uint32_t*>(sl + 4 * row);
       const int e = (m0 + row) * groups + g;
@@ -387,22 +413,22 @@ struct F6SubEngine {
     auto in_range = [](uint32_t b) {
       return (b & 0x7FFFu) == 0u || (((b >> 7) & 0xFFu) - (127u - 60u)) < 108u;
     };
-    const bool ok = in_range(sa_bits[0]) && in_range(sa_bits[1]) && in_range(sb_bits[0]) && in_range(sb_bits[1]);
+    const bool ok = in_range(sa_bits[0]) && in_range(sa_bits[MI - 1]) && in_range(sb_bits[0]) && in_range(sb_bits[1]);
     if (__all(ok)) {
       f6sub_fold_fast(acc, tot, lane, sa_bits, sb_bits);
       return;
     }
     all_fast = false;
-    float sa[2];
+    float sa[MI];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) sa[i] = __uint_as_float(sa_bits[i] << 16);
+    for (int i = 0; i < MI; ++i) sa[i] = __uint_as_float(sa_bits[i] << 16);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const uint2 w = *reinterpret_cast<const uint2*>(sl + 512 + 2 * packed_col(j, q));
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
             float x = acc[i][j][4 * q + t] * sa[i];
@@ -416,7 +442,7 @@ struct F6SubEngine {
   // which then hold int32 bit patterns.
   __device__ __forceinline__ void fold_raw() {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -503,8 +529,9 @@ struct F6SubEngine {
 // folded before stage k's barrier; with two groups per stage, a slot holds
 // both groups' a_scale dwords and b_scale rows.  (The 128-K engine does not
 // fit 256 registers with a fold after every stage.)
-template <class C, int SPG>
+template <class C, int SPG, int MI_ = 2>
 struct F6SubEngine64 {
+  static constexpr int MI = MI_;                    // 32-row blocks per wave
   static constexpr int P = 6;                       // ring slots
   static constexpr int NW = 4;
   static constexpr int OPB = 4 * F6_BLOCK;          // 128 rows x 64 K: 6 KiB
@@ -523,9 +550,9 @@ struct F6SubEngine64 {
                 "128 x 128 tiles of 2 x 2 waves, subchannel");
   static_assert(SPG == 0 || SPG == 1 || SPG == 2 || SPG == 4, "groups of 32, 64, 128 or 256 K");
 
-  v16f acc[2][2];
-  float tot[2][2][16];
-  v6i fa[2][2];  // [set][i]
+  v16f acc[MI][2];
+  float tot[MI][2][16];
+  v6i fa[2][MI];  // [set][i]
   v6i fb[2][2];  // [set][j]
   uint32_t voff[OPW];
   v4i rs;        // operand DMA resource (waves 0-1: A, 2-3: B)
@@ -545,7 +572,7 @@ struct F6SubEngine64 {
   // largest int, makes every comparison with it a constant.
   int fold_last;
 
-  __device__ __forceinline__ int out_row(int i) const { return wm * 64 + 32 * i + (lane & 31); }
+  __device__ __forceinline__ int out_row(int i) const { return wm * (32 * MI) + 32 * i + (lane & 31); }
   __device__ __forceinline__ int out_col(int j, int q) const {
     return wn * TN + (SWIGLU ? 0 : 32 * j) + 8 * q + 4 * (lane >> 5);
   }
@@ -588,7 +615,7 @@ struct F6SubEngine64 {
     // (G is even with groups of 32, so row * G is even)
     if constexpr (HALF) sbase = is_a ? 2 * sbase : sbase + (wave == 3 ? sb_row : 0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -627,7 +654,7 @@ struct F6SubEngine64 {
   };
   __device__ __forceinline__ Reads reads_of_slot(int slot) const {
     const uint32_t s = lds0 + (uint32_t)slot * STAGE;
-    const uint32_t a = s + 2u * wm * F6_BLOCK, b = s + OPB + 2u * wn * F6_BLOCK;
+    const uint32_t a = s + (uint32_t)MI * wm * F6_BLOCK, b = s + OPB + 2u * wn * F6_BLOCK;
     return Reads{a + 16u * lane, a + 1024u + 8u * lane, b + 16u * lane, b + 1024u + 8u * lane};
   }
 
@@ -639,7 +666,8 @@ struct F6SubEngine64 {
     constexpr bool IS_A = F == 0 || F == 3;
     constexpr int IDX = F == 0 ? 0 : (F == 3 ? 1 : F - 1);
     constexpr int OFF = IDX * F6_BLOCK;
-    v6i& dst = IS_A ? fa[S][IDX] : fb[S][IDX];
+    if constexpr (IS_A && IDX >= MI) return;
+    v6i& dst = IS_A ? fa[S][IDX % MI] : fb[S][IDX];
     if constexpr (Q % 2 == 0) {
       v4i x;
       asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(x) : "v"(IS_A ? r.a16 : r.b16), "i"(OFF));
@@ -666,7 +694,21 @@ struct F6SubEngine64 {
   __device__ __forceinline__ void tick(const Reads& r, const v4i& rs_st, uint32_t so, uint32_t m0_st,
                                        const v4i& rss_st, uint32_t svo, uint32_t sm0, int s8) {
     constexpr int I = T / 2, J = T % 2;
-    if constexpr (PART == 2) {
+    if constexpr (I >= MI) {
+      // one row block a wave: the tick has its load only (with the wait
+      // states after the M0 write, as in lds_dma16)
+      if constexpr (PART == 2) return;
+      if constexpr (T < OPW)
+        asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                     :
+                     : "v"(voff[T]), "s"(rs_st), "s"(so), "{m0}"(m0_st + 1024u * T)
+                     : "memory");
+      else
+        asm volatile("s_nop 4\n\tbuffer_load_dword %0, %1, 0 offen lds"
+                     :
+                     : "v"(svo), "s"(rss_st), "{m0}"(sm0)
+                     : "memory");
+    } else if constexpr (PART == 2) {
       if constexpr (ZERO)
         asm volatile("v_mfma_scale_f32_32x32x64_f8f6f4 %0, %1, %2, 0, %3, %3 op_sel_hi:[0,0,0] cbsz:2 blgp:2"
                      : "+v"(acc[I][J])
@@ -732,7 +774,11 @@ struct F6SubEngine64 {
   template <int N>
   __device__ __forceinline__ void fence() {
     static_assert(N == 4 || N == 7, "wait states");
-    if constexpr (N == 4)
+    if constexpr (MI == 1 && N == 4)
+      asm volatile("s_nop 4" : "+v"(acc[0][0]), "+v"(acc[0][1]));
+    else if constexpr (MI == 1)
+      asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(acc[0][0]), "+v"(acc[0][1]));
+    else if constexpr (N == 4)
       asm volatile("s_nop 4" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[1][0]), "+v"(acc[1][1]));
     else
       asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
@@ -743,7 +789,7 @@ struct F6SubEngine64 {
   // compiler would give those MFMAs a second accumulator set).
   __device__ __forceinline__ void tot_fence() {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         float* t = tot[i][j];
@@ -757,7 +803,10 @@ struct F6SubEngine64 {
   // is an operand, so no copy of it is placed before this point.
   template <int S>
   __device__ __forceinline__ void frag_fence() {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[S][0]), "+v"(fa[S][1]), "+v"(fb[S][0]), "+v"(fb[S][1])::"memory");
+    if constexpr (MI == 1)
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[S][0]), "+v"(fb[S][0]), "+v"(fb[S][1])::"memory");
+    else
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[S][0]), "+v"(fa[S][1]), "+v"(fb[S][0]), "+v"(fb[S][1])::"memory");
   }
 
   // Stage k on set S (ZERO: the first stage of a group).  Past the last
@@ -848,9 +897,9 @@ struct F6SubEngine64 {
   __device__ __forceinline__ void fold(const uint8_t* smem, int g) {
     const uint8_t* sl = smem + RING + ((HALF ? g >> 1 : g) & (SCALE_SLOTS - 1)) * SCALE_SLOT;
     const uint8_t* sbl = sl + 512 + (HALF ? 256 * (g & 1) : 0);  // the group's b_scale row
-    uint32_t sa_bits[2], sb_bits[2];
+    uint32_t sa_bits[MI], sb_bits[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < MI; ++i) {
       const int row = out_row(i);
       const uint32_t w = *reinterpret_cast<const uint32_t*>(sl + 4 * row);
       const int e = (m0 + row) * groups + g;
@@ -862,7 +911,7 @@ struct F6SubEngine64 {
     auto in_range = [](uint32_t b) {
       return (b & 0x7FFFu) == 0u || (((b >> 7) & 0xFFu) - (127u - 60u)) < 108u;
     };
-    const bool ok = in_range(sa_bits[0]) & in_range(sa_bits[1]) & in_range(sb_bits[0]) & in_range(sb_bits[1]);
+    const bool ok = in_range(sa_bits[0]) & in_range(sa_bits[MI - 1]) & in_range(sb_bits[0]) & in_range(sb_bits[1]);
     if constexpr (FAST) {
       if (__all(ok)) {
         f6sub_fold_fast(acc, tot, lane, sa_bits, sb_bits);
@@ -872,16 +921,16 @@ struct F6SubEngine64 {
     } else {
       if (!__all(ok)) all_fast = false;
     }
-    float sa[2];
+    float sa[MI];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) sa[i] = __uint_as_float(sa_bits[i] << 16);
+    for (int i = 0; i < MI; ++i) sa[i] = __uint_as_float(sa_bits[i] << 16);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const uint2 w = *reinterpret_cast<const uint2*>(sbl + 2 * packed_col(j, q));
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
             float x = acc[i][j][4 * q + t] * sa[i];
@@ -895,7 +944,7 @@ struct F6SubEngine64 {
   // which then hold int32 bit patterns.
   __device__ __forceinline__ void fold_raw() {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -1011,7 +1060,7 @@ __device__ __forceinline__ void f6sub_store_bf16(const E& e, const OutView& o, u
       const int u = 4 * j + q;
       const int half = 8 * (lane >> 5);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < E::MI; ++i) {
         const int x = 4 * q;
         uint32_t lo, hi;
         if constexpr (NO_NAN) {
@@ -1029,13 +1078,13 @@ __device__ __forceinline__ void f6sub_store_bf16(const E& e, const OutView& o, u
   const unsigned long long first = (unsigned long long)m0 * ldo + n0;
   const rsrc_t rs = make_rsrc(static_cast<uint8_t*>(o.out) + first * 2, ((unsigned long long)o.rows * ldo - first) * 2);
   const int rr = lane / 8, u = lane % 8;
-  const uint32_t voff = ((uint32_t)(e.wm * 64 + rr) * ldo + (uint32_t)(e.wn * 64 + 8 * u)) * 2u;
+  const uint32_t voff = ((uint32_t)(e.wm * (32 * E::MI) + rr) * ldo + (uint32_t)(e.wn * 64 + 8 * u)) * 2u;
   const bool col_ok = !MASK || n0 + e.wn * 64 + 8 * u < o.col_hi;
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
+  for (int t = 0; t < 4 * E::MI; ++t) {
     const int r = 8 * t + rr;
     const uint4 x = *reinterpret_cast<const uint4*>(region + r * 128 + 16 * (u ^ ((r >> 1) & 7)));
-    const int row = m0 + e.wm * 64 + r;
+    const int row = m0 + e.wm * (32 * E::MI) + r;
     if (!MASK || (col_ok && row >= o.row_lo && row < o.row_hi))
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, x), rs, voff, (uint32_t)(8 * t) * ldo * 2u, 0);
   }
@@ -1054,7 +1103,7 @@ __device__ __forceinline__ void f6sub_store_words(const E& e, const OutView& o, 
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < E::MI; ++i) {
         const int x = 4 * q;
         const int row = m0 + e.out_row(i), col = n0 + e.out_col(j, q);
         if (!MASK || (row >= o.row_lo && row < o.row_hi && col < o.col_hi))
@@ -1070,15 +1119,15 @@ __device__ __forceinline__ void f6sub_store_words(const E& e, const OutView& o, 
 // group's eight outputs a lane is in its range, in every lane (as the
 // per-channel epilogue chooses).
 template <class E>
-__device__ __forceinline__ void f6sub_swiglu(const E& e, int q, float (&v)[2][4]) {
+__device__ __forceinline__ void f6sub_swiglu(const E& e, int q, float (&v)[E::MI][4]) {
   float gmax = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < E::MI; ++i)
 #pragma unroll
     for (int t = 0; t < 4; ++t) gmax = __builtin_fmaxf(gmax, __builtin_fabsf(e.tot[i][1][4 * q + t]));
   const bool fast = __all(gmax <= SWIGLU_FAST_MAX);
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < E::MI; ++i)
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const float up = e.tot[i][0][4 * q + t], gate = e.tot[i][1][4 * q + t];
@@ -1105,10 +1154,10 @@ __device__ __forceinline__ void f6sub_store_swiglu(const E& e, const OutView& o,
     uint8_t* region = smem + (size_t)e.wave * 64 * 64;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      float v[2][4];
+      float v[E::MI][4];
       f6sub_swiglu(e, q, v);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < E::MI; ++i) {
         uint32_t lo, hi;
         if constexpr (NO_NAN) {
           lo = pack_bf16x2_nonan(v[i][0], v[i][1]);
@@ -1123,22 +1172,22 @@ __device__ __forceinline__ void f6sub_store_swiglu(const E& e, const OutView& o,
       __builtin_amdgcn_sched_barrier(0);
     }
     const int rr = lane / 4, u = lane % 4;
-    const uint32_t voff = ((uint32_t)(e.wm * 64 + rr) * ldo + (uint32_t)(e.wn * 32 + 8 * u)) * 2u;
+    const uint32_t voff = ((uint32_t)(e.wm * (32 * E::MI) + rr) * ldo + (uint32_t)(e.wn * 32 + 8 * u)) * 2u;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < 2 * E::MI; ++t) {
       const int r = 16 * t + rr;
       const uint4 x = *reinterpret_cast<const uint4*>(region + r * 64 + 16 * (u ^ ((r >> 1) & 3)));
-      if (col_ok && m0 + e.wm * 64 + r < o.row_hi)
+      if (col_ok && m0 + e.wm * (32 * E::MI) + r < o.row_hi)
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, x), rs, voff, (uint32_t)(16 * t) * ldo * 2u, 0);
     }
   } else {
     const uint32_t voff = ((uint32_t)e.out_row(0) * ldo + (uint32_t)e.out_col(0, 0)) * 4u;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      float v[2][4];
+      float v[E::MI][4];
       if constexpr (MODE == OUT_F32) f6sub_swiglu(e, q, v);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < E::MI; ++i) {
         if (!(col_ok && m0 + e.out_row(i) < o.row_hi)) continue;
         const uint32_t soff = (uint32_t)(32 * i) * ldo * 4u;
 #pragma unroll
@@ -1157,8 +1206,8 @@ __device__ __forceinline__ void f6sub_store_swiglu(const E& e, const OutView& o,
 // The engine for groups of S = 32 * G32: the 128-K-stage engine for 256,
 // the 64-K-stage one for 32, 64 and 128 (G32 / 2 stages per group; 0: two
 // groups per stage).
-template <class C, int G32>
-using F6SubEngineFor = std::conditional_t<G32 == 8, F6SubEngine<C>, F6SubEngine64<C, G32 / 2>>;
+template <class C, int G32, int MI = 2>
+using F6SubEngineFor = std::conditional_t<G32 == 8, F6SubEngine<C, MI>, F6SubEngine64<C, G32 / 2, MI>>;
 // The largest LDS layout of the subchannel kernels (the table entry's).
 template <class C>
 constexpr int f6_sub_lds_bytes() {
@@ -1167,20 +1216,16 @@ constexpr int f6_sub_lds_bytes() {
 }
 
 // One output tile of the subchannel GEMM over fp6 blocks (p.a / p.b point at
-// the converted A and B): 128 rows and 128 packed B rows, 64 output columns
-// for SwiGLU; G32 = S / 32.  MASK: M and N need not be multiples of the tile,
-// nor K of 128 (it is one of S and of 64; the blocks are padded with zeros,
-// and a stage past the last one loads zeros).  SwiGLU tiles are MASK tiles.
-template <class C, int MODE, int EPI, int G32, bool MASK = false>
-__device__ __forceinline__ void f6_sub_tile(const DenseArgs& p, uint8_t* smem, int tile) {
+// the converted A and B), from row m0: 64 MI rows and 128 packed B rows, 64
+// output columns for SwiGLU; G32 = S / 32.  MASK: M and N need not be
+// multiples of the tile, nor K of 128 (it is one of S and of 64; the blocks
+// are padded with zeros, and a stage past the last one loads zeros).  SwiGLU
+// tiles are MASK tiles.
+template <class C, int MODE, int EPI, int G32, bool MASK = false, int MI = 2>
+__device__ __forceinline__ void f6_sub_tile_at(const DenseArgs& p, uint8_t* smem, int m0, int tn) {
   static_assert(G32 == 1 || G32 == 2 || G32 == 4 || G32 == 8, "groups of 32, 64, 128 or 256");
-  static_assert(MASK || !C::SWIGLU, "SwiGLU tiles are masked");
-  using E = F6SubEngineFor<C, G32>;
-  const int tiles_m = MASK ? (p.M + C::BM - 1) / C::BM : p.M / C::BM;
-  const int tiles_n = MASK ? (p.N + C::BN - 1) / C::BN : p.N / C::BN;
-  int tm, tn;
-  dense_tile_coords(tile, tiles_m, tiles_n, p.group_m, tm, tn);
-  const int m0 = tm * C::BM;
+  static_assert(MASK || (!C::SWIGLU && MI == 2), "SwiGLU and half-height tiles are masked");
+  using E = F6SubEngineFor<C, G32, MI>;
   const int n0 = tn * C::BN;
   const int kpad = MASK ? (int)f6_pad_k(p.K) : p.K;
   const int b_cols = C::SWIGLU ? p.b_cols : p.N;
@@ -1208,6 +1253,13 @@ __device__ __forceinline__ void f6_sub_tile(const DenseArgs& p, uint8_t* smem, i
   }
 }
 
+template <class C, int MODE, int EPI, int G32>
+__device__ __forceinline__ void f6_sub_tile(const DenseArgs& p, uint8_t* smem, int tile) {
+  int tm, tn;
+  dense_tile_coords(tile, p.M / C::BM, p.N / C::BN, p.group_m, tm, tn);
+  f6_sub_tile_at<C, MODE, EPI, G32>(p, smem, tm * C::BM, tn);
+}
+
 // One kernel per output mode, epilogue and group size; one workgroup per
 // tile, two workgroups per CU.
 template <class C, int MODE, int EPI, int G32>
@@ -1216,11 +1268,30 @@ __global__ __launch_bounds__(256, 2) void f6_sub_kernel(const DenseArgs p) {
   f6_sub_tile<C, MODE, EPI, G32>(p, smem, blockIdx.x);
 }
 
-// The same tiles for any M, N and K (f6_sub_tile's MASK).
+// The same tiles for any M, N and K (MASK).  Up to 64 rows left over by the
+// whole tiles run as tiles of half the height (MI = 1: 32 rows a wave, half
+// the MFMAs and folds; the loads of the absent A panels return zeros) after
+// the whole ones, so that they fill slots beside whole tiles, on the XCD of
+// their columns' whole tiles where those are a multiple of eight.  Whole
+// call, whole and half-height last tiles: 320 x 16384 x 4096, groups of 32
+// 137.6 -> 120.4 us, of 128 60.7 -> 56.5; 1072 x 4096^2, of 32 130.0 ->
+// 109.4, of 128 51.8 -> 47.9; 64 x 11008 x 4096, of 32 107.5 -> 82.0; grids
+// of at most one tile a CU are unchanged (320 x 4096^2, of 128 44.3, 44.0).
+__device__ __host__ __forceinline__ int f6_sub_whole_tiles(int m) { return (m + 63) / 128; }
 template <class C, int MODE, int EPI, int G32>
 __global__ __launch_bounds__(256, 2) void f6_sub_edge_kernel(const DenseArgs p) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[F6SubEngineFor<C, G32>::LDS_BYTES];
-  f6_sub_tile<C, MODE, EPI, G32, true>(p, smem, blockIdx.x);
+  const int tiles_m = f6_sub_whole_tiles(p.M), tiles_n = (p.N + C::BN - 1) / C::BN;
+  const int tile = blockIdx.x;
+  if (tile < tiles_m * tiles_n) {
+    int tm, tn;
+    dense_tile_coords(tile, tiles_m, tiles_n, p.group_m, tm, tn);
+    f6_sub_tile_at<C, MODE, EPI, G32, true>(p, smem, tm * C::BM, tn);
+  } else {
+    int tm, tn;
+    dense_tile_coords(tile - tiles_m * tiles_n, 1, tiles_n, 1, tm, tn);
+    f6_sub_tile_at<C, MODE, EPI, G32, true, 1>(p, smem, tiles_m * C::BM, tn);
+  }
 }
 
 // Persistent schedule (as f6_gemm_persistent): gridDim.x workgroups stride

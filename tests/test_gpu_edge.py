@@ -63,7 +63,7 @@ def test_edges_of_the_tiles_match_the_oracle(layout, epilogue, m, n, k, device):
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("epilogue", ["none", "relu2", "swiglu"])
 @pytest.mark.parametrize("sub", [32, 64, 128, 256])
-@pytest.mark.parametrize("m,n,groups", [(16, 64, 1), (48, 192, 3), (144, 320, 6), (272, 128, 11)])
+@pytest.mark.parametrize("m,n,groups", [(16, 64, 1), (48, 192, 3), (80, 128, 2), (192, 192, 5), (240, 320, 6), (272, 128, 11)])
 def test_subchannel_edges_match_the_oracle(layout, epilogue, sub, m, n, groups, device):
     """The subchannel tile at its edges: one to eleven groups (odd stage
     counts, K no multiple of 128), scales over three decades, every output."""
