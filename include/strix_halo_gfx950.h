@@ -358,7 +358,10 @@ int amd_strix_halo_kernels_launch_ragged_fwd_ws(int kernel_index, int device_ind
  * No counterpart in the reference, whose forward takes the list from
  * calculate_group_info (ragged.py:201-323) as a separate step: the fp6
  * entries build it inside their conversion launch (up to 1024 groups), so
- * a call is two launches with no host work between them.  capacity must be
+ * a call is two launches with no host work between them; where groups hold
+ * few rows (NN and NT, 16-byte aligned operands and rows) they run skinny
+ * tiles on the packed operands instead, one launch that leaves the
+ * workspace alone and gives the same results.  capacity must be
  * at least amd_strix_halo_kernels_ragged_task_capacity(m, groups, block_m,
  * align_tile) (rc 1 otherwise), the bound of any list those group sizes
  * can make, since the sizes are read on the device. */

@@ -67,6 +67,7 @@ def translation_units() -> list[tuple[str, Path, list[str]]]:
     units.append(("edge_f6", CSRC / "k_f6edge.hip", list(DMA_FLAGS)))
     units.append(("f6pack", CSRC / "k_f6pack.hip", []))
     units.append(("ragged_f6", CSRC / "k_f6ragged.hip", list(DMA_FLAGS)))
+    units.append(("ragged_skinny", CSRC / "k_ragskinny.hip", []))
     units.append(("quant", CSRC / "k_quant.hip", []))
     for layout in (0, 1, 2, 3):
         units.append((f"ragged_{layout}", CSRC / "k_ragged.hip", [f"-DSHK_LAYOUT={layout}"]))

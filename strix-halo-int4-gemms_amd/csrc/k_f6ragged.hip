@@ -19,6 +19,9 @@
 // a multiple of 128.  Workspace: A as round32(M) rows x Kw, then per group
 // B as round32(N) rows x Kw.
 //
+// Where groups hold few rows the forward runs skinny tiles on the packed
+// operands instead (k_ragskinny.hip).
+//
 // Any group sizes are safe to run: the host's check of their sum may finish
 // while the kernels run (ragged.py), so a task past the rows of lhs returns,
 // rows past M are never stored (the output buffer's range), and the
@@ -271,6 +274,7 @@ int piece_bytes(const uint8_t* src, long ld) {
 }
 
 hipError_t launch_f6_ragged_fwd(const RaggedFwdArgs& a, dim3 grid, hipStream_t s) {
+  if (const int rows = ragged_skinny_rows(a)) return launch_ragged_skinny(a, rows, s);
   const int kw = round128(a.K);
   const unsigned long long a_bytes = f6_operand_bytes(round32(a.M), kw);
   const F6PackArgs pa{a.lhs, a.work, a.lda, a.M, kw / 64, 0, 1, 0, 0, nullptr, a.K, piece_bytes(a.lhs, a.lda),
@@ -294,6 +298,7 @@ void launch_ragged_sub(const RaggedFwdArgs& a, dim3 grid, hipStream_t s) {
   else hipLaunchKernelGGL((f6_ragged_sub_fwd_kernel<MODE, 8>), grid, dim3(256), 0, s, a);
 }
 hipError_t launch_f6_ragged_sub_fwd(const RaggedFwdArgs& a, dim3 grid, hipStream_t s) {
+  if (const int rows = ragged_skinny_rows(a)) return launch_ragged_skinny(a, rows, s);
   const int kw = round256(a.K);
   const unsigned long long a_bytes = f6_operand_bytes(round32(a.M), kw);
   F6PackArgs pa{a.lhs, a.work, a.lda, a.M, kw / 64, 0, 1, 0, 0, nullptr, a.K, piece_bytes(a.lhs, a.lda),

@@ -376,13 +376,15 @@ template <class C>
 struct SkScales {
   float sa[C::RT];
   float sbu[C::FT][4], sbg[C::FT][4];
+  template <bool NMASK>
   __device__ __forceinline__ void load(const DenseArgs& p, int m0, int n0, int wave, int lane) {
     const int g = lane >> 4;
 #pragma unroll
     for (int rt = 0; rt < C::RT; ++rt) sa[rt] = load_bf16(p.a_scale + min(m0 + 16 * rt + (lane & 15), p.M - 1));
 #pragma unroll
     for (int f = 0; f < C::FT; ++f) {
-      const int n = n0 + (C::KSPLIT ? 16 * wave : C::WOUT * wave + 16 * f) + 4 * g;
+      int n = n0 + (C::KSPLIT ? 16 * wave : C::WOUT * wave + 16 * f) + 4 * g;
+      if constexpr (NMASK) n = min(n, p.N - 4);
       sk_bf16x4(*reinterpret_cast<const uint2*>(p.b_scale + n), sbu[f]);
       if constexpr (C::SWIGLU) {
         sk_bf16x4(*reinterpret_cast<const uint2*>(p.b_scale + p.N + n), sbg[f]);
@@ -394,10 +396,12 @@ struct SkScales {
   }
 };
 
-template <class C, bool MASK>
+// (m0, n0): the tile's first row and column.  NMASK: the tile may reach past
+// column N (N is then a multiple of 4).
+template <class C, bool MASK, bool NMASK = false>
 __device__ __forceinline__ void sk_unit_pc(const DenseArgs& p, uint8_t* smem, int* last_flag, int lane, int wave,
-                                           int tm, int tn, int split, int splits, int tile) {
-  SkEngine<C> e(p, smem, lane, wave, tm * C::R, tn * C::BN);
+                                           int m0, int n0, int split, int splits, int tile) {
+  SkEngine<C> e(p, smem, lane, wave, m0, n0);
   const int nst = (p.K + C::KS - 1) / C::KS;
   const int per = (nst + splits - 1) / splits;
   const int lo = split * per, hi = min(nst, lo + per);
@@ -417,7 +421,7 @@ __device__ __forceinline__ void sk_unit_pc(const DenseArgs& p, uint8_t* smem, in
   for (int i = 0; i < C::D - 1; ++i)
     if (i < mine) e.issue(lo + first + i * stride, i);
   SkScales<C> scl;
-  if (p.out_mode != OUT_I32 && wave < C::NFIN) scl.load(p, e.m0, e.n0, wave, lane);
+  if (p.out_mode != OUT_I32 && wave < C::NFIN) scl.template load<NMASK>(p, e.m0, e.n0, wave, lane);
   for (int i = 0; i < mine; ++i) {
     const bool ahead = i + C::D - 1 < mine;
     if (ahead) {
@@ -558,6 +562,7 @@ __device__ __forceinline__ void sk_unit_pc(const DenseArgs& p, uint8_t* smem, in
 #pragma unroll
   for (int f = 0; f < C::FT; ++f) {
     const int n = e.n0 + (C::KSPLIT ? 16 * wave : C::WOUT * wave + 16 * f) + 4 * g;
+    if (NMASK && n >= p.N) continue;
     const float(&sbu)[4] = scl.sbu[f];
     const float(&sbg)[4] = scl.sbg[f];
 #pragma unroll
@@ -645,10 +650,10 @@ __device__ __forceinline__ void sk_scale_group(const DenseArgs& p, const uint8_t
 }
 
 template <class C, bool MASK>
-__device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, int lane, int wave, int tm, int tn) {
+__device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, int lane, int wave, int m0, int n0) {
   static_assert(C::GSPLIT && (C::NW == 4 || C::NW == 8), "four or eight waves take the groups in turn");
   constexpr int NWSH = C::NW == 8 ? 3 : 2;  // log2(NW)
-  SkEngine<C> e(p, smem, lane, wave, tm * C::R, tn * C::BN);
+  SkEngine<C> e(p, smem, lane, wave, m0, n0);
   constexpr int KSH = C::BITS == 4 ? 7 : 6;  // log2(KS)
   static_assert((1 << KSH) == C::KS, "stage K");
   constexpr int CH = C::CH;
@@ -831,9 +836,9 @@ __global__ __launch_bounds__(C::NT) void sk_gemm_kernel(const DenseArgs p) {
     const int split = lu / tiles, t = lu - split * tiles;
     const int tn = t / tiles_m, tm = t - tn * tiles_m;
     if constexpr (C::SUBCH)
-      sk_unit_sc<C, MASK>(p, smem, lane, wave, tm, tn);
+      sk_unit_sc<C, MASK>(p, smem, lane, wave, tm * C::R, tn * C::BN);
     else
-      sk_unit_pc<C, MASK>(p, smem, &last_flag, lane, wave, tm, tn, split, splits, tn * tiles_m + tm);
+      sk_unit_pc<C, MASK>(p, smem, &last_flag, lane, wave, tm * C::R, tn * C::BN, split, splits, tn * tiles_m + tm);
     __syncthreads();
   }
 }

@@ -460,6 +460,10 @@ int max_info_groups();
 // fp6 ragged entries of one layout (k_f6ragged.hip): the forward (task
 // tile 128) and the K-ragged backward, each per-channel and subchannel.
 Entry f6_ragged_fwd_entry(int layout);
+// Rows of the skinny tiles that a ragged forward runs in place of the fp6
+// ones (k_ragskinny.hip), or 0.
+int ragged_skinny_rows(const RaggedFwdArgs& a);
+hipError_t launch_ragged_skinny(const RaggedFwdArgs& a, int rows, hipStream_t s);
 Entry f6_ragged_sub_fwd_entry(int layout);
 Entry f6_ragged_bwd_entry(int layout);
 Entry f6_ragged_sub_bwd_entry(int layout);
