@@ -219,24 +219,33 @@ def _sk_splits(bits: int, tiles: int, k: int) -> int:
     return max(s, _sk_needed_splits(bits, k))
 
 
-# (bits, SwiGLU): per tile height 16, 32, 64 the us of a call (fixed, and per
-# round of 256 workgroups at 4096 K each) and whether rounds count whole.
+# (bits, SwiGLU): per tile height 16, 32, 64 the us of a call (fixed, more for
+# a wide B, and per round of 256 workgroups at 4096 K each), the fraction of a
+# round that stays as K shrinks and whether rounds count whole.
 _SK_FITS = {
-    (4, False): ((3.6, 3.38, False), (3.4, 4.8, False), (4.8, 6.07, False)),
-    (4, True): ((7.0, 4.6, False), (3.0, 10.5, True), (3.0, 15.5, True)),
-    (8, False): ((3.8, 5.2, False), (3.5, 6.45, False), (4.5, 8.0, False)),
-    (8, True): ((15.3, 7.7, False), (12.0, 12.5, True), (12.0, 15.0, True)),
+    (4, False): ((3.6, 0.0, 3.38, 0.27, False), (3.4, 0.0, 4.8, 0.25, False), (4.8, 0.0, 6.07, 0.3, False)),
+    (4, True): ((4.0, 3.0, 4.6, 0.35, False), (5.5, 0.0, 10.5, 0.37, True), (7.5, 0.0, 15.5, 0.45, True)),
+    (8, False): ((3.8, 0.0, 5.2, 0.12, False), (4.2, 0.0, 6.45, 0.13, False), (4.5, 0.0, 8.0, 0.2, False)),
+    (8, True): ((3.2, 12.1, 7.7, 0.05, False), (3.0, 9.0, 12.5, 0.2, True), (3.0, 9.0, 15.0, 0.33, True)),
 }
 
 
 @functools.lru_cache(maxsize=4096)
-def sk_plan(bits: int, subch: bool, swiglu: bool, m: int, n: int, k: int) -> tuple[int, float]:
+def sk_plan(bits: int, sub: int, swiglu: bool, m: int, n: int, k: int) -> tuple[int, float]:
     """(tile rows, predicted us) of a standard skinny call of M rows
-    (shk_table.h sk_plan, which states the fits); us 0 for subchannel."""
-    if subch:
-        return (16 if m <= (32 if swiglu else 16) else 32), 0.0
+    (shk_table.h sk_plan, which states the fits); us 0 for subchannel (sub:
+    the group size, 0 for per-channel)."""
+    if sub > 0:
+        def load(rows: int) -> float:
+            t = -(-m // rows) * (n // 16)
+            rest = t % 512
+            return 1.0 if t <= 256 else 1.37 * (t // 512 + (0.0 if rest == 0 else 0.73 if rest <= 256 else 1.0))
+
+        tall = 1.15 if swiglu and sub >= (128 if bits == 4 else 64) else 1.45
+        return (16 if m <= 16 or load(16) <= tall * load(32) else 32), 0.0
     best = (16, -1.0)
-    for i, (a, b, whole) in enumerate(_SK_FITS[bits, swiglu]):
+    wide, k4 = min(1.0, 2.0 * n * k / 9e7), k / 4096.0
+    for i, (a, w, b, f, whole) in enumerate(_SK_FITS[bits, swiglu]):
         rows = 16 << i
         if i > 0 and m <= rows // 2:
             break
@@ -244,7 +253,8 @@ def sk_plan(bits: int, subch: bool, swiglu: bool, m: int, n: int, k: int) -> tup
         s = _sk_splits(bits, tiles, k)
         units = tiles * s
         rounds = 1.0 if units <= 256 else (float(-(-units // 256)) if whole else units / 256.0)
-        us = a + (float(rows // 16 * (2 if swiglu else 1)) if s > 1 else 0.0) + b * (k / s / 4096.0) * rounds
+        us = (a + w * wide + (float(rows // 16 * (2 if swiglu else 1)) if s > 1 else 0.0)
+              + b * (k4 / s * rounds + f * max(0.0, 1.0 - k4) * (rounds - 1.0)))
         if best[1] < 0.0 or us < best[1]:
             best = (rows, us)
     return best
@@ -255,8 +265,7 @@ def _sk_tile_rows(desc: "KernelDesc", m: int, n: int, k: int) -> int:
     them, the split-K and persistent entries' their block_m."""
     if desc.schedule != SCHEDULE_STANDARD or desc.split_k > 1:
         return desc.block_m
-    return sk_plan(desc.dtype_bits, desc.scale_mode == SCALE_SUBCHANNEL, desc.epilogue_kind == EPI_KIND_SWIGLU,
-                   m, n, k)[0]
+    return sk_plan(desc.dtype_bits, 0, desc.epilogue_kind == EPI_KIND_SWIGLU, m, n, k)[0]
 
 
 def sk_split_count(desc: "KernelDesc", m: int, n: int, k: int, with_workspace: bool = True) -> int:
@@ -529,7 +538,7 @@ PREDICT_MAX_K = 65536  # K up to which the fits of predicted_us stand
 
 # subchannel, by group size: us per product on the 32-row skinny tiles (plain,
 # SwiGLU); a 128 x 128 fp6 tile's fixed us and us per K value
-_SKINNY_SUB_US = {32: (2.9e-8, 2.3e-8), 64: (1.5e-8, 1.2e-8), 128: (1.07e-8, 0.74e-8), 256: (0.85e-8, 0.65e-8)}
+_SKINNY_SUB_US = {32: (2.78e-8, 2.24e-8), 64: (1.38e-8, 1.14e-8), 128: (0.95e-8, 0.68e-8), 256: (0.73e-8, 0.59e-8)}
 _F6_SUB_US = {32: (5.0, 0.0215), 64: (5.0, 0.0125), 128: (5.0, 0.0061), 256: (3.5, 0.0038)}
 
 
@@ -541,7 +550,7 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
     8192^2:
 
     * skinny per-channel tiles: sk_plan;
-    * skinny subchannel tiles: a launch and the products;
+    * skinny subchannel tiles: a launch, the products and the outputs;
     * fp6 entries: two launches, the conversion at 5 TB/s, then rounds of
       tiles: per-channel 256-row tiles (FP6) or the launcher's split
       (FP6_EDGE); subchannel 128 x 128 tiles, two a CU (1.3 times one; 1.1
@@ -562,9 +571,9 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
         if sub not in _F6_SUB_US:
             return None
         if desc.operand_format == OPERANDS_STREAM:
-            low = 1.5 if sk_plan(4, True, swiglu, m, n, k)[0] == 16 else 1.0
+            low = 1.5 if sk_plan(4, sub, swiglu, m, n, k)[0] == 16 else 1.0
             rank = {32: 1.0, 64: 1.001, 16: 1.002}[desc.block_m]  # the same tiles; the 32-row entry first
-            return 6.0 + _SKINNY_SUB_US[sub][swiglu] * low * rank * (m * cols * k)
+            return 6.0 + rank * (_SKINNY_SUB_US[sub][swiglu] * low * (m * cols * k) + 5e-6 * (m * n))
         if not desc.needs_workspace:
             return None
         fixed, per_k = _F6_SUB_US[sub]
@@ -577,7 +586,7 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
             rounds *= 0.8
         return convert + (fixed + per_k * k) * rounds
     if desc.operand_format == OPERANDS_STREAM:
-        return sk_plan(4, False, swiglu, m, n, k)[1]
+        return sk_plan(4, 0, swiglu, m, n, k)[1]
     if desc.operand_format == OPERANDS_FP6_EDGE:
         return convert + _f6_edge_us(m, n, k, swiglu)
     if desc.operand_format == OPERANDS_FP6:

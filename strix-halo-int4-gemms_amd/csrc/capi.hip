@@ -218,7 +218,7 @@ int check_out_mode(int out_mode) {
 // arrival counters and exact partials of a split K (shk::sk_call);
 // nothing otherwise.
 uint64_t dense_workspace_bytes(const shk_kernel_desc& d, int32_t m, int32_t n, int32_t k) {
-  if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_call(d, m, n, k, true).workspace_bytes;
+  if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_call(d, m, n, k, 0, true).workspace_bytes;
   const long b_cols = d.epilogue_kind == SHK_EPI_KIND_SWIGLU ? 2L * n : (long)n;
   if (d.operand_format == SHK_OPERANDS_FP6_EDGE)
     return shk::f6_operand_bytes(shk::f6_pad_rows(m), shk::f6_pad_k(k)) +
@@ -351,7 +351,7 @@ int prepare_dense(DenseCall& c, int kernel_index, Phase phase, const void* a, co
   if (stream && gemm) {
     // K split over workgroups only with a (zeroed-counter) workspace
     const bool with_ws = workspace != nullptr;
-    shk::SkCall call = shk::sk_call(d, m, n, k, true);
+    shk::SkCall call = shk::sk_call(d, m, n, k, subchannel, true);
     const uint64_t need = call.workspace_bytes;
     if (with_ws && workspace != kScratchPending) {
       if (workspace_bytes < need)
@@ -363,7 +363,7 @@ int prepare_dense(DenseCall& c, int kernel_index, Phase phase, const void* a, co
                   " bytes of scratch for this shape; the no-allocation entry point's scratch holds at most " +
                   std::to_string(workspace_bytes) + " bytes (use amd_strix_halo_kernels_launch_gemm_ws)");
     }
-    if (!(with_ws && need > 0)) call = shk::sk_call(d, m, n, k, false);
+    if (!(with_ws && need > 0)) call = shk::sk_call(d, m, n, k, subchannel, false);
     if (call.splits == 0)
       return fail("kernel " + std::to_string(kernel_index) + " splits K=" + std::to_string(k) +
                   " over workgroups, which needs a workspace (amd_strix_halo_kernels_launch_gemm_ws)");
@@ -527,12 +527,12 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
   if (d.scale_mode == SHK_SCALE_SUBCHANNEL) {
     const int s = sub == 32 ? 0 : (sub == 64 ? 1 : (sub == 128 ? 2 : 3));
     if (d.operand_format == SHK_OPERANDS_STREAM) {
-      static constexpr double plain[4] = {2.9e-8, 1.5e-8, 1.07e-8, 0.85e-8};
-      static constexpr double gated[4] = {2.3e-8, 1.2e-8, 0.74e-8, 0.65e-8};
-      const double low = shk::sk_plan(4, true, swiglu, m, n, k).rows == 16 ? 1.5 : 1.0;
+      static constexpr double plain[4] = {2.78e-8, 1.38e-8, 0.95e-8, 0.73e-8};
+      static constexpr double gated[4] = {2.24e-8, 1.14e-8, 0.68e-8, 0.59e-8};
+      const double low = shk::sk_plan(4, sub, swiglu, m, n, k).rows == 16 ? 1.5 : 1.0;
       // (the entries run the same tiles; the 32-row one ranks first)
       const double rank = d.block_m == 32 ? 1.0 : (d.block_m == 64 ? 1.001 : 1.002);
-      return 6.0 + (swiglu ? gated[s] : plain[s]) * low * rank * (double)(m * cols * k);
+      return 6.0 + rank * ((swiglu ? gated[s] : plain[s]) * low * (double)(m * cols * k) + 5e-6 * (double)(m * n));
     }
     if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
     static constexpr double fixed[4] = {5.0, 5.0, 5.0, 3.5};
@@ -544,7 +544,7 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
     if (whole == 0) rounds *= 0.8;
     return convert + (fixed[s] + per_k[s] * (double)k) * rounds;
   }
-  if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_plan(4, false, swiglu, m, n, k).us;
+  if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_plan(4, 0, swiglu, m, n, k).us;
   if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
   return convert + shk::f6_edge_plan(m, n, k, swiglu).us;
 }
@@ -735,7 +735,7 @@ int amd_strix_halo_kernels_launch_gemm_noalloc(int kernel_index, int device_inde
   if (split_stream) {
     // the partial slots are written before they are read; only the counters
     // must start at zero (256-byte multiple, below the scratch size)
-    const unsigned n16 = (unsigned)(shk::sk_call(c.e->d, m, n, k, true).counter_bytes / 16);
+    const unsigned n16 = (unsigned)(shk::sk_call(c.e->d, m, n, k, 0, true).counter_bytes / 16);
     hipLaunchKernelGGL(shk::clear_counters_kernel, dim3((n16 + 255) / 256), dim3(256), 0, s,
                        reinterpret_cast<int4*>(c.p.work), n16);
     const hipError_t cerr = hipGetLastError();

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "../../include/strix_halo_gfx950.h"
@@ -335,29 +336,48 @@ inline int sk_splits(int bits, long tiles, long k) {
 // Per-channel: the smallest predicted time (us) a + b * (K per workgroup /
 // 4096) * rounds of 256 workgroups, whole rounds for the SwiGLU tiles of 32
 // and 64 rows, which run one workgroup a CU, and with K split one more for
-// every 16 rows (up and gate) of partials.  The
-// figures are fits to calls of M 32..400 on N x K of 11008 x 4096, 8192^2,
-// 4096^2 and 1024 x 4096.  Measured, 16, 32 and 64 rows: int8 SwiGLU 48 x
-// 11008 x 4096 29.9, 32.5, 25.7 us, 400 rows 153, 124, 97; int4 SwiGLU 112
-// rows 29.6, 33.7, 34.7; int4 plain 112 x 8192^2 27.7, 21.9, 17.7, 48 x
-// 4096^2 7.0, 8.3, 10.5.
+// every 16 rows (up and gate) of partials; below K = 4096 a round keeps the
+// fraction f of the difference (a tile's prologue and epilogue), and `wide`
+// is what a SwiGLU call of 90 M values of B and more adds.  The figures are
+// fits to calls of M 32..1648 on N x K of 11008 x 4096, 8192^2, 4096^2, 1024
+// x 4096, 4096 x 512..2048 and 9728 x 704.  Measured, 16, 32 and 64 rows:
+// int8 SwiGLU 48 x 11008 x 4096 29.9, 32.5, 25.7 us, 400 rows 153, 124, 97;
+// int4 SwiGLU 112 rows 29.6, 33.7, 34.7, 1648 x 4864 x 704 66.8, 87.3, 73.3;
+// int4 plain 112 x 8192^2 27.7, 21.9, 17.7, 48 x 4096^2 7.0, 8.3, 10.5, 1024
+// x 4096 x 512 23.7, 17.0, 14.0.
 //
-// Subchannel (16 columns a tile, so many tiles): 32 rows from 17 rows on
-// (SwiGLU from 33); groups of 128, 48 x 4096^2: 19.9, 16.3, 19.6, 400 rows
-// 110, 80, 124.
+// Subchannel (16 columns a tile, so many tiles): rounds of 512 workgroups, a
+// last one of up to half the chip for 0.73, a grid of one a CU for 1 / 1.37;
+// a round of 32-row tiles takes 1.45 of one of 16-row tiles, 1.15 where the
+// four waves' 16-row tile is bound by its B reads (SwiGLU, groups of a stage
+// and more).  Measured, 16 and 32 rows, groups of 128: 48 x 4096^2 19.9 and
+// 16.3 us, 400 rows 110 and 80, 64 x 1024 x 4096 9.0 and 13.0, 272 x 960 x
+// 3584 16.8 and 22.7, its SwiGLU 32.2 and 29.5; groups of 64, SwiGLU, 272 x
+// 960 x 3584 37.2 and 46.1.
 struct SkPlan {
   int rows;
   double us;
 };
-inline SkPlan sk_plan(int bits, bool subch, bool swiglu, long m, long n, long k) {
-  if (subch) return SkPlan{m <= (swiglu ? 32 : 16) ? 16 : 32, 0.0};
+// `sub`: the group size, or 0 for per-channel scales.
+inline SkPlan sk_plan(int bits, int sub, bool swiglu, long m, long n, long k) {
+  if (sub > 0) {
+    auto load = [&](long rows) {
+      const long t = ((m + rows - 1) / rows) * (n / 16), rest = t % 512;
+      return t <= 256 ? 1.0 : 1.37 * ((double)(t / 512) + (rest == 0 ? 0.0 : (rest <= 256 ? 0.73 : 1.0)));
+    };
+    const double tall = swiglu && sub >= (bits == 4 ? 128 : 64) ? 1.15 : 1.45;
+    return SkPlan{m <= 16 || load(16) <= tall * load(32) ? 16 : 32, 0.0};
+  }
   struct Fit {
-    double a, b;
+    double a, wide, b, f;
     bool whole;
   };
   static constexpr Fit fits[2][2][3] = {
-      {{{3.6, 3.38, false}, {3.4, 4.8, false}, {4.8, 6.07, false}}, {{7.0, 4.6, false}, {3.0, 10.5, true}, {3.0, 15.5, true}}},
-      {{{3.8, 5.2, false}, {3.5, 6.45, false}, {4.5, 8.0, false}}, {{15.3, 7.7, false}, {12.0, 12.5, true}, {12.0, 15.0, true}}}};
+      {{{3.6, 0.0, 3.38, 0.27, false}, {3.4, 0.0, 4.8, 0.25, false}, {4.8, 0.0, 6.07, 0.3, false}},
+       {{4.0, 3.0, 4.6, 0.35, false}, {5.5, 0.0, 10.5, 0.37, true}, {7.5, 0.0, 15.5, 0.45, true}}},
+      {{{3.8, 0.0, 5.2, 0.12, false}, {4.2, 0.0, 6.45, 0.13, false}, {4.5, 0.0, 8.0, 0.2, false}},
+       {{3.2, 12.1, 7.7, 0.05, false}, {3.0, 9.0, 12.5, 0.2, true}, {3.0, 9.0, 15.0, 0.33, true}}}};
+  const double wide = std::min(1.0, 2.0 * (double)n * (double)k / 9e7), k4 = (double)k / 4096.0;
   SkPlan best{16, -1.0};
   for (int i = 0; i < 3; ++i) {
     const int rows = 16 << i;
@@ -367,16 +387,17 @@ inline SkPlan sk_plan(int bits, bool subch, bool swiglu, long m, long n, long k)
     const int s = sk_splits(bits, tiles, k);
     const long units = tiles * s;
     const double rounds = units <= 256 ? 1.0 : (f.whole ? (double)((units + 255) / 256) : (double)units / 256.0);
-    const double us = f.a + (s > 1 ? (double)(rows / 16 * (swiglu ? 2 : 1)) : 0.0) + f.b * ((double)k / (double)s / 4096.0) * rounds;
+    const double us = f.a + f.wide * wide + (s > 1 ? (double)(rows / 16 * (swiglu ? 2 : 1)) : 0.0) +
+                      f.b * (k4 / (double)s * rounds + f.f * std::max(0.0, 1.0 - k4) * (rounds - 1.0));
     if (best.us < 0.0 || us < best.us) best = SkPlan{rows, us};
   }
   return best;
 }
 // Rows of a table entry's tiles: the split-K and persistent entries keep
 // their block_m.
-inline int sk_tile_rows(const shk_kernel_desc& d, long m, long n, long k) {
+inline int sk_tile_rows(const shk_kernel_desc& d, long m, long n, long k, int sub) {
   if (d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1) return d.block_m;
-  return sk_plan(d.dtype_bits, d.scale_mode == SHK_SCALE_SUBCHANNEL, d.epilogue_kind == SHK_EPI_KIND_SWIGLU, m, n, k).rows;
+  return sk_plan(d.dtype_bits, sub, d.epilogue_kind == SHK_EPI_KIND_SWIGLU, m, n, k).rows;
 }
 // A skinny call: its tile rows, the workgroups sharing a tile's K (without a
 // workspace one, or 0 when K needs more; subchannel tiles always one), and
@@ -388,8 +409,10 @@ struct SkCall {
   int rows, splits;
   unsigned long long counter_bytes, workspace_bytes;  // 0 unsplit
 };
-inline SkCall sk_call(const shk_kernel_desc& d, long m, long n, long k, bool with_workspace) {
-  SkCall c{sk_tile_rows(d, m, n, k), 1, 0, 0};
+// `sub`: the call's group size (0 per-channel; the workspace does not depend
+// on it).
+inline SkCall sk_call(const shk_kernel_desc& d, long m, long n, long k, int sub, bool with_workspace) {
+  SkCall c{sk_tile_rows(d, m, n, k, sub), 1, 0, 0};
   if (d.scale_mode == SHK_SCALE_SUBCHANNEL) return c;
   if (!with_workspace) {
     if (sk_needed_splits(d.dtype_bits, k) != 1) c.splits = 0;

@@ -21,7 +21,7 @@ from amd_strix_halo_kernels import native  # noqa: E402
 
 def _check(bits, layout, epilogue, sub, m, n, k, device, rows):
     swiglu = epilogue == "swiglu"
-    assert kt.sk_plan(bits, bool(sub), swiglu, m, n, k)[0] == rows
+    assert kt.sk_plan(bits, sub, swiglu, m, n, k)[0] == rows
     a_q, b_q, a_arg, b_arg, sa, sb = dense_case(stable_seed("rows", bits, layout, epilogue, sub, m, n, k), bits=bits,
                                                 layout=layout, m=m, n=n, k=k, subchannel=sub or None, swiglu=swiglu)
     a, b, ta, tb = (to_dev(torch, x, device) for x in (a_arg, b_arg, sa, sb))
@@ -47,10 +47,10 @@ def _check(bits, layout, epilogue, sub, m, n, k, device, rows):
 # with and without K split over workgroups
 _PLANS = [
     (4, "none", 64, 112, 8192, 2080), (4, "none", 64, 192, 8192, 2080), (4, "none", 32, 48, 512, 96),
-    (4, "none", 32, 144, 512, 8192), (8, "none", 64, 112, 8192, 1024), (8, "none", 32, 144, 512, 4096),
-    (8, "none", 32, 48, 512, 96), (4, "swiglu", 64, 272, 2048, 96), (4, "swiglu", 64, 192, 4096, 96),
-    (4, "swiglu", 32, 48, 512, 2080), (8, "swiglu", 64, 272, 2048, 96), (8, "swiglu", 64, 272, 512, 8192),
-    (8, "swiglu", 32, 48, 512, 1024),
+    (4, "none", 32, 144, 512, 8192), (8, "none", 64, 112, 8192, 1024), (8, "none", 32, 144, 512, 8192),
+    (8, "none", 32, 112, 4096, 96), (8, "none", 64, 272, 512, 8192), (4, "swiglu", 64, 112, 8192, 96),
+    (4, "swiglu", 16, 48, 512, 2080), (8, "swiglu", 64, 272, 2048, 96), (8, "swiglu", 64, 272, 512, 8192),
+    (8, "swiglu", 32, 48, 512, 96), (8, "swiglu", 32, 48, 2048, 8192),
 ]
 
 
@@ -63,6 +63,8 @@ def test_every_height_matches_the_oracle(bits, epilogue, rows, m, n, k, layout, 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("sub", [32, 64, 128, 256])
-@pytest.mark.parametrize("epilogue,m", [("none", 48), ("none", 64), ("swiglu", 80)])
-def test_subchannel_32_row_tiles_match_the_oracle(bits, sub, epilogue, m, layout, device):
-    _check(bits, layout, epilogue, sub, m, 192, 5 * sub, device, 32)
+@pytest.mark.parametrize("epilogue,m,rows", [("none", 48, 32), ("none", 64, 32), ("swiglu", 48, 32), ("none", 32, 16)])
+def test_subchannel_32_row_tiles_match_the_oracle(bits, sub, epilogue, m, rows, layout, device):
+    """32-row tiles where they make fewer rounds of workgroups (N = 4096)."""
+    _check(bits, layout, epilogue, sub, m, 4096 if rows == 32 else 192, (2 if sub > 64 else 5) * sub // 64 * 64 or 64,
+           device, rows)
