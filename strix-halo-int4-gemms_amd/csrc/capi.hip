@@ -218,7 +218,7 @@ int check_out_mode(int out_mode) {
 // arrival counters and exact partials of a split K (shk::sk_call);
 // nothing otherwise.
 uint64_t dense_workspace_bytes(const shk_kernel_desc& d, int32_t m, int32_t n, int32_t k) {
-  if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_call(d, m, n, k, 0, true).workspace_bytes;
+  if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_call(d, m, n, k, 0).workspace_bytes;
   const long b_cols = d.epilogue_kind == SHK_EPI_KIND_SWIGLU ? 2L * n : (long)n;
   if (d.operand_format == SHK_OPERANDS_FP6_EDGE)
     return shk::f6_operand_bytes(shk::f6_pad_rows(m), shk::f6_pad_k(k)) +
@@ -351,7 +351,7 @@ int prepare_dense(DenseCall& c, int kernel_index, Phase phase, const void* a, co
   if (stream && gemm) {
     // K split over workgroups only with a (zeroed-counter) workspace
     const bool with_ws = workspace != nullptr;
-    shk::SkCall call = shk::sk_call(d, m, n, k, subchannel, true);
+    shk::SkCall call = shk::sk_call(d, m, n, k, subchannel);
     const uint64_t need = call.workspace_bytes;
     if (with_ws && workspace != kScratchPending) {
       if (workspace_bytes < need)
@@ -363,7 +363,7 @@ int prepare_dense(DenseCall& c, int kernel_index, Phase phase, const void* a, co
                   " bytes of scratch for this shape; the no-allocation entry point's scratch holds at most " +
                   std::to_string(workspace_bytes) + " bytes (use amd_strix_halo_kernels_launch_gemm_ws)");
     }
-    if (!(with_ws && need > 0)) call = shk::sk_call(d, m, n, k, subchannel, false);
+    if (!(with_ws && need > 0)) call.splits = shk::sk_direct_splits(d, k);
     if (call.splits == 0)
       return fail("kernel " + std::to_string(kernel_index) + " splits K=" + std::to_string(k) +
                   " over workgroups, which needs a workspace (amd_strix_halo_kernels_launch_gemm_ws)");
@@ -735,7 +735,7 @@ int amd_strix_halo_kernels_launch_gemm_noalloc(int kernel_index, int device_inde
   if (split_stream) {
     // the partial slots are written before they are read; only the counters
     // must start at zero (256-byte multiple, below the scratch size)
-    const unsigned n16 = (unsigned)(shk::sk_call(c.e->d, m, n, k, 0, true).counter_bytes / 16);
+    const unsigned n16 = (unsigned)(shk::sk_call(c.e->d, m, n, k, 0).counter_bytes / 16);
     hipLaunchKernelGGL(shk::clear_counters_kernel, dim3((n16 + 255) / 256), dim3(256), 0, s,
                        reinterpret_cast<int4*>(c.p.work), n16);
     const hipError_t cerr = hipGetLastError();

@@ -399,9 +399,8 @@ inline int sk_tile_rows(const shk_kernel_desc& d, long m, long n, long k, int su
   if (d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1) return d.block_m;
   return sk_plan(d.dtype_bits, sub, d.epilogue_kind == SHK_EPI_KIND_SWIGLU, m, n, k).rows;
 }
-// A skinny call: its tile rows, the workgroups sharing a tile's K (without a
-// workspace one, or 0 when K needs more; subchannel tiles always one), and
-// with more than one split its workspace: the tiles' arrival counters, padded
+// A skinny call: its tile rows, the workgroups sharing a tile's K (subchannel
+// tiles always one), and with more than one split its workspace: the tiles' arrival counters, padded
 // to 256 bytes, then an exact int32 partial of every (tile, split).  All of
 // it is zero before the first launch and every launch leaves what it used
 // zero, whatever the shapes of the launches that share it.
@@ -411,13 +410,9 @@ struct SkCall {
 };
 // `sub`: the call's group size (0 per-channel; the workspace does not depend
 // on it).
-inline SkCall sk_call(const shk_kernel_desc& d, long m, long n, long k, int sub, bool with_workspace) {
+inline SkCall sk_call(const shk_kernel_desc& d, long m, long n, long k, int sub) {
   SkCall c{sk_tile_rows(d, m, n, k, sub), 1, 0, 0};
   if (d.scale_mode == SHK_SCALE_SUBCHANNEL) return c;
-  if (!with_workspace) {
-    if (sk_needed_splits(d.dtype_bits, k) != 1) c.splits = 0;
-    return c;
-  }
   const long tiles = ((m + c.rows - 1) / c.rows) * (n / d.block_n);
   c.splits = sk_splits(d.dtype_bits, tiles, k);
   if (c.splits > 1) {
@@ -429,6 +424,11 @@ inline SkCall sk_call(const shk_kernel_desc& d, long m, long n, long k, int sub,
         c.counter_bytes + (unsigned long long)tiles * c.splits * (d.block_n / 16) * (c.rows / 16) * cf * 1024;
   }
   return c;
+}
+
+// Splits of the same call without a workspace: one, or 0 when K needs more.
+inline int sk_direct_splits(const shk_kernel_desc& d, long k) {
+  return d.scale_mode == SHK_SCALE_SUBCHANNEL || sk_needed_splits(d.dtype_bits, k) == 1 ? 1 : 0;
 }
 
 // Each kernel translation unit appends its entries in a fixed order
