@@ -1,4 +1,4 @@
-"""FP6_EDGE entries (k_f6.hip): the fp6 tiles on shapes that are no multiple
+"""FP6_EDGE entries (k_f6edge.hip): the fp6 tiles on shapes that are no multiple
 of them, against the CPU oracle and against the skinny tiles, which read the
 same operands without converting them.
 
