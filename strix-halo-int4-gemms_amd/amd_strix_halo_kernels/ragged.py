@@ -313,7 +313,8 @@ class _GroupSizesCheck:
         self._host = None
         sizes = group_sizes.detach()
         if defer and sizes.is_cuda and not torch.cuda.is_current_stream_capturing():
-            self._host = torch.empty(sizes.shape, dtype=sizes.dtype, pin_memory=True)
+            # (the caller's default device may be the GPU, whose memory cannot be pinned)
+            self._host = torch.empty(sizes.shape, dtype=sizes.dtype, device="cpu", pin_memory=True)
             self._host.copy_(sizes, non_blocking=True)
             self._event = torch.cuda.current_stream(sizes.device).record_event()
         else:

@@ -85,3 +85,19 @@ def test_capture_refuses_sizes_on_the_device(device):
         except RuntimeError:
             pass
     torch.cuda.synchronize()
+
+
+def test_calls_under_a_default_device(device):
+    """A default device of the caller's does not reach the buffer that the
+    check copies the sizes into."""
+    lhs, rhs = _operands(device)
+    gs = torch.tensor([150, 0, 50], device=device)
+    bwd = torch.randint(0, 256, (3, 96, 64), dtype=torch.uint8, device=device)
+    bwd_rhs = torch.randint(0, 256, (3, 64, 64), dtype=torch.uint8, device=device)
+    bwd_gs = torch.tensor([128, 0, 77], device=device)
+    want, want_bwd = shk.ragged_dot_int4(lhs, rhs, gs), shk.ragged_dot_int4_bwd(bwd, bwd_rhs, bwd_gs)
+    with torch.device(device):
+        assert torch.equal(shk.ragged_dot_int4(lhs, rhs, gs), want)
+        assert torch.equal(shk.ragged_dot_int4_bwd(bwd, bwd_rhs, bwd_gs), want_bwd)
+        with pytest.raises(ValueError, match="got 199"):
+            shk.ragged_dot_int4(lhs, rhs, gs - torch.tensor([1, 0, 0]))
