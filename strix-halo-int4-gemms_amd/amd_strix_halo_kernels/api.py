@@ -13,7 +13,6 @@ from __future__ import annotations
 
 from typing import Any
 
-from . import kernel_table as kt
 from .exceptions import KernelNotAvailableError
 from .metadata import (
     SUPPORTED_GEMM_LAYOUTS,
@@ -128,10 +127,8 @@ def mm(
         kernel = registry.select_reference(dtype=dtype, layout=layout, scale=scale, epilogue=epilogue,
                                            schedule=schedule)
     else:
-        kernel = registry.select(dtype=dtype, layout=layout, scale=scale, epilogue=epilogue, m=m, n=n, k=k,
-                                 schedule=schedule)
-        if kernel.table_index in kt.FP6_INDICES:
-            kernel = registry.call_kernel(kernel, m=m, n=n, k=k)
+        kernel = registry.select_call(dtype=dtype, layout=layout, scale=scale, epilogue=epilogue, m=m, n=n, k=k,
+                                      schedule=schedule)
     return explicit_mm(a, b, kernel=kernel, a_scale=a_scale, b_scale=b_scale, gate=gate,
                        use_reference=use_reference)
 
@@ -159,10 +156,8 @@ def fused_swiglu_up_gate(
         kernel = registry.select_reference(dtype=dtype, layout=layout, scale=scale, epilogue=Epilogue.SWIGLU,
                                            split_k=1)
     else:
-        kernel = registry.select(dtype=dtype, layout=layout, scale=scale, epilogue=Epilogue.SWIGLU, m=m, n=n,
-                                 k=k, split_k=1)
-        if kernel.table_index in kt.FP6_INDICES:
-            kernel = registry.call_kernel(kernel, m=m, n=n, k=k)
+        kernel = registry.select_call(dtype=dtype, layout=layout, scale=scale, epilogue=Epilogue.SWIGLU, m=m, n=n,
+                                      k=k, split_k=1)
     return explicit_mm(a, b_up_gate, kernel=kernel, a_scale=a_scale, b_scale=b_scale, use_reference=use_reference)
 
 

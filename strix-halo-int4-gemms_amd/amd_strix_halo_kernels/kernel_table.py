@@ -112,6 +112,13 @@ class KernelDesc:
     def is_stream(self) -> bool:
         return self.operand_format == OPERANDS_STREAM
 
+    @property
+    def plans_rows(self) -> bool:
+        """A skinny entry whose tiles' height is picked for each call
+        (sk_plan) from any M that is a multiple of 16; group_size_m is the
+        most 16-row blocks that a tile joins."""
+        return self.is_stream and self.group_size_m > 1
+
     def workspace_bytes(self, m: int, n: int, k: int) -> int:
         """Bytes of the workspace for shape (m, n, k): fp6 operands (FP6;
         per-channel calls with K > FP6_MAX_K add [m, b_cols] int32 sums), the
@@ -187,20 +194,21 @@ SK_BN_SUBCH = 16
 SK_TARGET_UNITS = 256
 
 
-def _sk_geometry(r: int, swiglu: bool, subch: bool) -> tuple[int, int]:
-    """(listed ring depth, LDS bytes) of a skinny tile of r rows (SkCfg)."""
+def _sk_geometry(r: int, swiglu: bool, subch: bool, *, fixed: bool = True) -> tuple[int, int]:
+    """(ring depth, LDS bytes) of a skinny tile of r rows (SkCfg), in an entry
+    of that height (`fixed`) or in one that plans its rows."""
     bn = SK_BN_SUBCH if subch else SK_BN
     wcols = 2 * bn if swiglu else bn
     stage = r * 64 + wcols * 64 + ((r // 16) * 256 + 256 if subch else 0)
     tiles = (r // 16) * (wcols // 16)
     ch = (4 if tiles == 1 else 2 if tiles == 2 else 1) if subch else 0  # groups per wave and round
     chain = 2 * SK_NW * ch * tiles * 1024  # two rounds of scaled partials
-    alone = SK_NW * 2 * stage > 79872 - chain  # one workgroup a CU: a deeper ring, listed as 2
-    budget = (153600 if alone else 79872) - chain
+    alone = SK_NW * 2 * stage > 79872 - chain  # one workgroup a CU
+    budget = (153600 if alone and not fixed else 79872) - chain
     depth = 4 if SK_NW * 4 * stage <= budget else (3 if SK_NW * 3 * stage <= budget else 2)
     ring = SK_NW * depth * stage
     red = 0 if subch else SK_NW * (wcols // 16) * 1024
-    return 2 if alone else depth, max(ring, red) + chain
+    return depth, max(ring, red) + chain
 
 
 def _sk_needed_splits(bits: int, k: int) -> int:
@@ -232,9 +240,9 @@ _SK_FITS = {
 
 @functools.lru_cache(maxsize=4096)
 def sk_plan(bits: int, sub: int, swiglu: bool, m: int, n: int, k: int) -> tuple[int, float]:
-    """(tile rows, predicted us) of a standard skinny call of M rows
-    (shk_table.h sk_plan, which states the fits); us 0 for subchannel (sub:
-    the group size, 0 for per-channel)."""
+    """(tile rows, predicted us) of a call of M rows on a skinny entry that
+    plans its rows (shk_table.h sk_plan, which states the fits); us 0 for
+    subchannel (sub: the group size, 0 for per-channel)."""
     if sub > 0:
         def load(rows: int) -> float:
             t = -(-m // rows) * (n // 16)
@@ -261,9 +269,8 @@ def sk_plan(bits: int, sub: int, swiglu: bool, m: int, n: int, k: int) -> tuple[
 
 
 def _sk_tile_rows(desc: "KernelDesc", m: int, n: int, k: int) -> int:
-    """Rows of a skinny entry's tiles: the standard entries' as sk_plan picks
-    them, the split-K and persistent entries' their block_m."""
-    if desc.schedule != SCHEDULE_STANDARD or desc.split_k > 1:
+    """Rows of a skinny entry's tiles."""
+    if not desc.plans_rows:
         return desc.block_m
     return sk_plan(desc.dtype_bits, 0, desc.epilogue_kind == EPI_KIND_SWIGLU, m, n, k)[0]
 
@@ -354,6 +361,19 @@ def _sk_desc(index, bits, layout, r, *, swiglu=False, subch=False, schedule=SCHE
         block_m=r, block_n=SK_BN_SUBCH if subch else SK_BN, block_k=32, num_waves=SK_NW, num_stages=depth,
         lds_bytes=lds,
         group_size_m=1, operand_format=OPERANDS_STREAM, schedule=schedule, split_k=split_k)
+
+
+def _sk_rows_desc(index, bits, layout, *, swiglu, subch):
+    # the figures of the tallest tile
+    r = 32 if subch else 64
+    depth, lds = _sk_geometry(r, swiglu, subch, fixed=False)
+    return KernelDesc(
+        index=index, family=FAMILY_DENSE, dtype_bits=bits, layout=layout,
+        scale_mode=SCALE_SUBCHANNEL if subch else SCALE_PER_CHANNEL,
+        min_subchannel=32 if subch else 0, max_subchannel=256 if subch else 0,
+        epilogue_kind=EPI_KIND_SWIGLU if swiglu else EPI_KIND_PLAIN, block_m=16,
+        block_n=SK_BN_SUBCH if subch else SK_BN, block_k=32, num_waves=SK_NW, num_stages=depth, lds_bytes=lds,
+        group_size_m=r // 16, operand_format=OPERANDS_STREAM)
 
 
 def _edge_desc(index, layout, bm, *, swiglu=False, subch=False):
@@ -453,14 +473,16 @@ def _build() -> tuple[KernelDesc, ...]:
             for subch in (False, True):
                 for swiglu in (False, True):
                     out.append(_edge_desc(len(out), layout, bm, swiglu=swiglu, subch=subch))
+    # skinny entries that plan their rows (k_skinny.hip sk_rows_entry)
+    for bits in (4, 8):
+        for layout in (LAYOUT_NN, LAYOUT_NT, LAYOUT_TN):
+            for subch in (False, True):
+                for swiglu in (False, True):
+                    out.append(_sk_rows_desc(len(out), bits, layout, swiglu=swiglu, subch=subch))
     return tuple(out)
 
 
 TABLE: tuple[KernelDesc, ...] = _build()
-
-
-# Dense entries whose operands can be converted apart from their GEMM.
-FP6_INDICES = frozenset(d.index for d in TABLE if d.family == FAMILY_DENSE and d.operand_format == OPERANDS_FP6)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -485,7 +507,9 @@ def measured_tops(desc: KernelDesc) -> float | None:
             return 2001.0
         return 3504.0 if desc.epilogue_kind == EPI_KIND_PLAIN else 3161.0
     if desc.operand_format == OPERANDS_STREAM:
-        return SKINNY_TOPS if desc.scale_mode == SCALE_PER_CHANNEL else SKINNY_SUB_TOPS[desc.block_m]
+        if desc.scale_mode == SCALE_PER_CHANNEL:
+            return SKINNY_TOPS
+        return SKINNY_SUB_TOPS[32 if desc.plans_rows else desc.block_m]
     if desc.dtype_bits == 8 and desc.num_stages == 4 and desc.block_m == 256:
         return 2014.0 if desc.epilogue_kind == EPI_KIND_SWIGLU else 2270.0
     return None
@@ -545,7 +569,8 @@ _F6_SUB_US = {32: (5.0, 0.0215), 64: (5.0, 0.0125), 128: (5.0, 0.0061), 256: (3.
 def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = None) -> float | None:
     """Predicted time of a standard int4 call on an entry, in us (None for the
     other families and K past PREDICT_MAX_K); capi.hip computes the skinny
-    and FP6_EDGE entries' alike.  Fits to calls measured over M 16..8176 and
+    and FP6_EDGE entries' alike, and the skinny entries of a family share the
+    planned tiles' time (among them selection_area decides).  Fits to calls measured over M 16..8176 and
     N x K of 1024 x 4096, 4096 x 1024, 4096^2, 11008 x 4096, 16384 x 4096 and
     8192^2:
 
@@ -572,7 +597,8 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
             return None
         if desc.operand_format == OPERANDS_STREAM:
             low = 1.5 if sk_plan(4, sub, swiglu, m, n, k)[0] == 16 else 1.0
-            rank = {32: 1.0, 64: 1.001, 16: 1.002}[desc.block_m]  # the same tiles; the 32-row entry first
+            # of the heights, the 32-row tile ranks first, as measured (SKINNY_SUB_TOPS)
+            rank = 1.0 if desc.plans_rows else {32: 1.0, 64: 1.001, 16: 1.002}[desc.block_m]
             return 6.0 + rank * (_SKINNY_SUB_US[sub][swiglu] * low * (m * cols * k) + 5e-6 * (m * n))
         if not desc.needs_workspace:
             return None
@@ -613,6 +639,17 @@ def selection_tops(desc: KernelDesc, m: int, n: int | None = None, k: int | None
             and m > SKINNY_SUB_MAX_M):
         return None
     return tops
+
+
+def selection_area(desc: KernelDesc, m: int) -> int:
+    """The second ranking key of select for M rows, a tile's area (capi.hip
+    selection_area).  A skinny entry that plans its rows counts as a 16-row
+    tile, just before the entry of that height; subchannel calls past
+    SKINNY_SUB_MAX_M rows find it before every skinny entry of one height."""
+    if desc.plans_rows:
+        tall = desc.scale_mode == SCALE_SUBCHANNEL and m > SKINNY_SUB_MAX_M
+        return (64 if tall else 16) * desc.block_n + 1
+    return desc.block_m * desc.block_n
 
 
 def entries(family: int) -> tuple[KernelDesc, ...]:

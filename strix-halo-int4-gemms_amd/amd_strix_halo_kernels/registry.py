@@ -35,7 +35,7 @@ from .metadata import (
     make_kernel_id,
     output_dtype_for_split_k,
 )
-from .template_config import LaunchShape, is_tile_multiple_shape
+from .template_config import slices_k
 
 _LAYOUT_OF_CODE = {kt.LAYOUT_NN: GemmLayout.NN, kt.LAYOUT_NT: GemmLayout.NT, kt.LAYOUT_TN: GemmLayout.TN,
                    kt.LAYOUT_TT: GemmLayout.TT}
@@ -105,35 +105,37 @@ def iter_supported_kernel_metadata() -> Iterable[KernelMetadata]:
                 )
 
 
-def _selection_key(kernel: KernelMetadata, m: int, n: int | None = None, k: int | None = None) -> tuple[float, int]:
-    tops = kernel.measured_tops
-    if kernel.table_index is not None:
-        desc = kt.TABLE[kernel.table_index]
-        if tops == kt.measured_tops(desc):  # not a caller's own figure (with_status)
-            tops = kt.selection_tops(desc, m, n, k, kernel.scale.subchannel_size)
-    return (tops or 0.0, kernel.tile.block_m * kernel.tile.block_n)
+class _Candidate:
+    """A kernel of a family with what decides whether it runs a shape: the
+    multiples of the launch-shape contract (template_config.py
+    tile_multiple_rejection_reasons) and its K bound, as plain numbers."""
+
+    __slots__ = ("kernel", "desc", "split_k", "block_m", "block_n", "period", "sub", "slice_sub", "max_k")
+
+    def __init__(self, kernel: KernelMetadata) -> None:
+        tile = kernel.tile
+        self.kernel = kernel
+        self.desc = None if kernel.table_index is None else kt.TABLE[kernel.table_index]
+        self.split_k = tile.split_k
+        self.block_m, self.block_n, self.period = tile.block_m, tile.block_n, tile.block_k * tile.split_k
+        subchannel = kernel.scale.mode is ScaleMode.SUBCHANNEL and kernel.scale.subchannel_size is not None
+        self.sub = kernel.scale.subchannel_size if subchannel else 1
+        self.slice_sub = self.sub if subchannel and tile.split_k > 1 and slices_k(kernel) else 1
+        # the library's bound (gfx950 accumulators and buffer offsets)
+        self.max_k = None if self.desc is None else self.desc.max_k
+
+    def accepts(self, m: int, n: int, k: int) -> bool:
+        return not (m % self.block_m or n % self.block_n or k % self.period or k % self.sub
+                    or k // self.split_k % self.slice_sub) and (self.max_k is None or k <= self.max_k)
 
 
-def _matches(kernel: KernelMetadata, dtype, scale, epilogue, layout, schedule, split_k) -> bool:
-    return (
-        kernel.a_dtype is dtype
-        and kernel.b_dtype is dtype
-        and kernel.scale == scale
-        and kernel.epilogue is epilogue
-        and kernel.layout is layout
-        and kernel.schedule is schedule
-        and not (kernel.epilogue in {Epilogue.RELU2, Epilogue.SWIGLU} and kernel.tile.split_k != 1)
-        and (split_k is None or kernel.tile.split_k == split_k)
-        and kernel.tile.even_k
-    )
-
-
-def _runs_k(kernel: KernelMetadata, k: int) -> bool:
-    """The library's K bound of the kernel's table entry (gfx950 accumulators
-    and buffer offsets); kernels without a table entry have none."""
-    if kernel.table_index is None:
-        return True
-    return kt.TABLE[kernel.table_index].supports_k(k)
+def _selection_key(c: _Candidate, m: int, n: int | None = None, k: int | None = None) -> tuple[float, int]:
+    tops, desc = c.kernel.measured_tops, c.desc
+    if desc is None:
+        return (tops or 0.0, c.block_m * c.block_n)
+    if tops == kt.measured_tops(desc):  # not a caller's own figure (with_status)
+        tops = kt.selection_tops(desc, m, n, k, c.kernel.scale.subchannel_size)
+    return (tops or 0.0, kt.selection_area(desc, m))
 
 
 class KernelRegistry:
@@ -156,14 +158,17 @@ class KernelRegistry:
         self._selected = {}
         self._call_kernels = {}
 
-    def _family(self, dtype, scale, epilogue, layout, schedule) -> list[KernelMetadata]:
+    def _family(self, dtype, scale, epilogue, layout, schedule) -> list[_Candidate]:
         families = self._families
         if families is None:
             families = {}
             for kern in self._kernels.values():
-                if kern.a_dtype is kern.b_dtype:
-                    key = (kern.a_dtype, kern.scale, kern.epilogue, kern.layout, kern.schedule)
-                    families.setdefault(key, []).append(kern)
+                if kern.a_dtype is not kern.b_dtype or not kern.tile.even_k:
+                    continue
+                if kern.epilogue in {Epilogue.RELU2, Epilogue.SWIGLU} and kern.tile.split_k != 1:
+                    continue
+                key = (kern.a_dtype, kern.scale, kern.epilogue, kern.layout, kern.schedule)
+                families.setdefault(key, []).append(_Candidate(kern))
             self._families = families
         return families.get((dtype, scale, epilogue, layout, schedule), [])
 
@@ -191,59 +196,87 @@ class KernelRegistry:
         hit = self._selected.get(request)
         if hit is not None:
             return hit
-        shape = LaunchShape(m, n, k)
         candidates = [
-            kernel
-            for kernel in self._family(dtype, scale, epilogue, layout, schedule)
-            if _matches(kernel, dtype, scale, epilogue, layout, schedule, split_k)
-            and is_tile_multiple_shape(kernel, shape)
-            and _runs_k(kernel, k)
-        ]
+            c for c in self._family(dtype, scale, epilogue, layout, schedule)
+            if (split_k is None or c.split_k == split_k) and c.accepts(m, n, k)
+        ] if m > 0 and n > 0 and k > 0 else []
         if require_compiled:
-            candidates = [c for c in candidates if c.status in {KernelStatus.COMPILED, KernelStatus.BENCHMARKED}]
+            candidates = [c for c in candidates
+                          if c.kernel.status in {KernelStatus.COMPILED, KernelStatus.BENCHMARKED}]
         if not candidates:
             raise LookupError(
                 f"no kernel for dtype={dtype.value}, scale={scale.label}, epilogue={epilogue.value}, "
                 f"layout={layout.value}, schedule={schedule.value}, shape=({m}, {n}, {k})"
             )
-        chosen = max(candidates, key=lambda kern: _selection_key(kern, m, n, k))
+        chosen = max(candidates, key=lambda c: _selection_key(c, m, n, k)).kernel
         if len(self._selected) >= 4096:  # bounded for callers that vary M call to call
             self._selected = {}
         self._selected[request] = chosen
+        return chosen
+
+    def select_call(
+        self,
+        *,
+        dtype: OperandDType,
+        scale: ScaleSpec,
+        epilogue: Epilogue,
+        m: int,
+        n: int,
+        k: int,
+        layout: GemmLayout = GemmLayout.NN,
+        split_k: int | None = None,
+        schedule: KernelSchedule = KernelSchedule.STANDARD,
+    ) -> KernelMetadata:
+        """The kernel that a whole call of a request runs: call_kernel of what
+        select() picks, in one memo lookup a call."""
+        request = (dtype, scale, epilogue, m, n, k, layout, split_k, schedule)
+        hit = self._call_kernels.get(request)
+        if hit is not None:
+            return hit
+        chosen = self.call_kernel(
+            self.select(dtype=dtype, scale=scale, epilogue=epilogue, m=m, n=n, k=k, layout=layout, split_k=split_k,
+                        schedule=schedule), m=m, n=n, k=k)
+        if getattr(self.select, "__func__", None) is KernelRegistry.select:  # another rule is asked every time
+            if len(self._call_kernels) >= 4096:
+                self._call_kernels = {}
+            self._call_kernels[request] = chosen
         return chosen
 
     def call_kernel(self, kernel: KernelMetadata, *, m: int, n: int, k: int) -> KernelMetadata:
         """The kernel that a whole call runs where select() picked `kernel`.
 
         select() keeps the FP6 entries for every shape they accept, since the
-        separate conversion needs them.  A whole call is free to take any
-        entry with the same results, and on few tiles of 256 rows another one
-        is faster (512 x 4096 x 4096: FP6 36.7 us, skinny 16.6; 512 x 16384 x
-        4096: FP6 47.4, FP6_EDGE 41.9; groups of 128, 128 x 1024 x 4096: FP6
-        37.8, skinny 12.7), so the smallest predicted time
-        decides (kernel_table.predicted_us).  Kernels with a figure of the
-        caller's own (with_status) stay."""
-        index = kernel.table_index
-        if index is None or kt.TABLE[index].operand_format != kt.OPERANDS_FP6:
+        separate conversion needs them, and the skinny entry of a single
+        height for the M of that height.  A whole call is free to take any
+        entry with the same results: of the skinny entries the one that plans
+        its rows, and where an FP6 entry fits the smallest predicted time
+        decides (kernel_table.predicted_us), since on few tiles of 256 rows
+        another one is faster (512 x 4096 x 4096: FP6 36.7 us, skinny 16.6; 512
+        x 16384 x 4096: FP6 47.4, FP6_EDGE 41.9; groups of 128, 128 x 1024 x
+        4096: FP6 37.8, skinny 12.7).  Kernels with a figure of the caller's
+        own (with_status) stay."""
+        desc = None if kernel.table_index is None else kt.TABLE[kernel.table_index]
+        fp6 = desc is not None and desc.operand_format == kt.OPERANDS_FP6
+        if not (fp6 or (desc is not None and desc.is_stream and not desc.plans_rows)):
             return kernel
-        request = (kernel.kernel_id, m, n, k)
-        hit = self._call_kernels.get(request)
-        if hit is not None:
-            return hit
+        if kernel.tile.split_k != 1 or kernel.measured_tops != kt.measured_tops(desc):
+            return kernel
         chosen = kernel
         sub = kernel.scale.subchannel_size
-        best = kt.predicted_us(kt.TABLE[index], m, n, k, sub)
-        if best is not None and kernel.measured_tops == kt.measured_tops(kt.TABLE[index]):
-            shape = LaunchShape(m, n, k)
-            for other in self._family(kernel.a_dtype, kernel.scale, kernel.epilogue, kernel.layout, kernel.schedule):
-                if other.table_index is None or other.tile.split_k != 1 or not is_tile_multiple_shape(other, shape):
-                    continue
-                us = kt.predicted_us(kt.TABLE[other.table_index], m, n, k, sub)
-                if us is not None and (us, -other.tile.block_m) < (best, -chosen.tile.block_m):
-                    chosen, best = other, us
-        if len(self._call_kernels) >= 4096:
-            self._call_kernels = {}
-        self._call_kernels[request] = chosen
+        best = kt.predicted_us(desc, m, n, k, sub)
+        for other in self._family(kernel.a_dtype, kernel.scale, kernel.epilogue, kernel.layout, kernel.schedule):
+            entry = other.desc
+            if entry is None or other.split_k != 1 or (entry.is_stream and not entry.plans_rows):
+                continue
+            if not fp6:
+                if entry.plans_rows:
+                    return other.kernel
+                continue
+            if best is None or not other.accepts(m, n, k):
+                continue
+            us = kt.predicted_us(entry, m, n, k, sub)
+            if us is not None and us < best:
+                chosen, best = other.kernel, us
         return chosen
 
     def select_reference(
@@ -257,9 +290,7 @@ class KernelRegistry:
         schedule: KernelSchedule = KernelSchedule.STANDARD,
     ) -> KernelMetadata:
         candidates = [
-            kernel
-            for kernel in self._family(dtype, scale, epilogue, layout, schedule)
-            if _matches(kernel, dtype, scale, epilogue, layout, schedule, split_k)
+            c for c in self._family(dtype, scale, epilogue, layout, schedule) if split_k is None or c.split_k == split_k
         ]
         if not candidates:
             raise LookupError(
@@ -267,7 +298,7 @@ class KernelRegistry:
                 f"epilogue={epilogue.value}, layout={layout.value}, schedule={schedule.value}"
             )
         # no shape: rank as for a large M (the skinny subchannel figure applies to few rows only)
-        return max(candidates, key=lambda kern: _selection_key(kern, 1 << 30))
+        return max(candidates, key=lambda c: _selection_key(c, 1 << 30)).kernel
 
     def with_status(self, kernel_id: str, status: KernelStatus, **updates: object) -> "KernelRegistry":
         copied = KernelRegistry(self._kernels.values())

@@ -40,13 +40,13 @@ def tile_multiple_rejection_reasons(kernel: KernelMetadata, shape: LaunchShape) 
     if kernel.scale.mode is ScaleMode.SUBCHANNEL and sub is not None and shape.k % sub:
         out.append(f"K={shape.k} is not divisible by SUBCHANNEL={sub}")
     elif (kernel.scale.mode is ScaleMode.SUBCHANNEL and sub is not None and tile.split_k > 1
-          and _slices_k(kernel) and (shape.k // tile.split_k) % sub):
+          and slices_k(kernel) and (shape.k // tile.split_k) % sub):
         # each K slice of a split-K kernel starts at a scale group boundary
         out.append(f"K/SPLIT_K={shape.k // tile.split_k} is not divisible by SUBCHANNEL={sub}")
     return tuple(out)
 
 
-def _slices_k(kernel: KernelMetadata) -> bool:
+def slices_k(kernel: KernelMetadata) -> bool:
     """Whether a split-K kernel cuts K into SPLIT_K contiguous slices (the
     gfx950 split tiles); the skinny (STREAM) split tiles fold every scale
     group of the whole K in one workgroup and need no slice boundary."""

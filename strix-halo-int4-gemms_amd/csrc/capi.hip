@@ -117,6 +117,12 @@ const std::vector<Entry>& table() {
     shk::append_edge_f6(v, SHK_LAYOUT_NN);
     shk::append_edge_f6(v, SHK_LAYOUT_NT);
     shk::append_edge_f6(v, SHK_LAYOUT_TN);
+    shk::append_skinny_rows_4_0(v);
+    shk::append_skinny_rows_4_1(v);
+    shk::append_skinny_rows_4_2(v);
+    shk::append_skinny_rows_8_0(v);
+    shk::append_skinny_rows_8_1(v);
+    shk::append_skinny_rows_8_2(v);
     for (size_t i = 0; i < v.size(); ++i) v[i].d.index = (int32_t)i;
     return v;
   }();
@@ -513,9 +519,10 @@ int amd_strix_halo_kernels_kernel_table_entry(int index, shk_kernel_desc* out) {
 
 namespace {
 
-// Predicted time (us) of a standard int4 call on a skinny or FP6_EDGE entry,
-// from fits to measured calls (kernel_table.predicted_us states them);
-// negative where there is none.
+// Predicted time (us) of a standard int4 call on the skinny tiles or an
+// FP6_EDGE entry, from fits to measured calls (kernel_table.predicted_us
+// states them); negative where there is none.  The skinny entries of a family
+// share the planned tiles' time: among them selection_area decides.
 constexpr long kPredictMaxK = 65536;
 double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
   if (d.family != SHK_FAMILY_DENSE || d.dtype_bits != 4 || d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1 ||
@@ -530,8 +537,8 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
       static constexpr double plain[4] = {2.78e-8, 1.38e-8, 0.95e-8, 0.73e-8};
       static constexpr double gated[4] = {2.24e-8, 1.14e-8, 0.68e-8, 0.59e-8};
       const double low = shk::sk_plan(4, sub, swiglu, m, n, k).rows == 16 ? 1.5 : 1.0;
-      // (the entries run the same tiles; the 32-row one ranks first)
-      const double rank = d.block_m == 32 ? 1.0 : (d.block_m == 64 ? 1.001 : 1.002);
+      // of the heights, the 32-row tile ranks first, as measured (measured_score)
+      const double rank = shk::sk_plans_rows(d) || d.block_m == 32 ? 1.0 : (d.block_m == 64 ? 1.001 : 1.002);
       return 6.0 + rank * ((swiglu ? gated[s] : plain[s]) * low * (double)(m * cols * k) + 5e-6 * (double)(m * n));
     }
     if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
@@ -569,11 +576,23 @@ double measured_score(const shk_kernel_desc& d, int m, int n, int k, int subchan
   if (d.operand_format == SHK_OPERANDS_STREAM) {  // the skinny tiles (subchannel: by tile height, up to 256 rows)
     if (d.scale_mode == SHK_SCALE_PER_CHANNEL) return 241.0;
     if (m > 256) return 0.0;
+    if (shk::sk_plans_rows(d)) return 184.0;
     return d.block_m == 16 ? 96.0 : (d.block_m == 32 ? 184.0 : 152.0);
   }
   if (d.dtype_bits == 8 && d.num_stages == 4 && d.block_m == 256)
     return d.epilogue_kind == SHK_EPI_KIND_SWIGLU ? 2014.0 : 2270.0;
   return 0.0;
+}
+
+// The second ranking key, a tile's area.  A skinny entry that plans its rows
+// counts as a 16-row tile, just before the entry of that height, so that M of
+// a multiple of 32 or 64 rows finds the entry of that height, as in the
+// reference's small-M tiles (registry.py:29, 48-77); a whole mm() call runs
+// the planned entry all the same.  Subchannel calls of more than 256 rows, for
+// which the figures of the single heights do not stand, find it first.
+long selection_area(const shk_kernel_desc& d, int m) {
+  if (shk::sk_plans_rows(d)) return (d.scale_mode == SHK_SCALE_SUBCHANNEL && m > 256 ? 64L : 16L) * d.block_n + 1;
+  return (long)d.block_m * d.block_n;
 }
 
 // Whether a dense entry serves the request's family: SwiGLU entries serve
@@ -617,7 +636,7 @@ int best_entry(int bits, int layout, int subchannel, int epilogue, int schedule,
     if (!accepts_shape(d, m, n, k, subchannel)) continue;
     if (direct && d.operand_format != SHK_OPERANDS_PACKED && d.operand_format != SHK_OPERANDS_STREAM) continue;
     const double score = measured_score(d, m, n, k, subchannel);
-    const long area = (long)d.block_m * d.block_n;
+    const long area = selection_area(d, m);
     if (score > best_score || (score == best_score && area > best_area)) {
       best = i;
       best_score = score;

@@ -9,7 +9,8 @@
 // SwiGLU tiles take K in multiples of 32, registry.py:112-176): per-channel
 // and subchannel, plain and SwiGLU, for int4 the persistent schedule
 // (registry.py:230-251, split-K variants included), and split-K 2/4/8
-// (SUPPORTED_SPLIT_K).
+// (SUPPORTED_SPLIT_K).  append_skinny_rows_<bits>_<layout>() adds, at the
+// table's end, the entries that pick their tiles' height for each call.
 #include "shk_skinny.h"
 #include "shk_table.h"
 
@@ -28,6 +29,11 @@ constexpr int kLayout = SHK_LAYOUT;
 
 template <int R, bool SWIGLU, bool SUBCH>
 using SC = SkCfg<kBits, kLayout, R, SWIGLU, SUBCH>;
+// The tiles of the entries whose block_m is their height: rings that leave
+// room for a second workgroup on the CU.
+template <int R, bool SWIGLU, bool SUBCH>
+using Fixed = SkCfg<kBits, kLayout, R, SWIGLU, SUBCH, SUBCH ? 16 : 0, SK_NW, SK_BN,
+                    SC<R, SWIGLU, SUBCH>::ALONE ? 2 : 0>;
 
 // grid.x = output tiles; per-channel tiles run sk_splits workgroups each.
 template <class C>
@@ -39,8 +45,8 @@ hipError_t launch_sk_t(const DenseArgs& a, dim3 grid, hipStream_t s) {
   hipLaunchKernelGGL(sk_gemm_kernel<C>, dim3(sk_units<C>(a, grid)), dim3(C::NT), 0, s, a);
   return hipGetLastError();
 }
-// A standard entry: tiles of the rows that sk_plan picked, masked where M is
-// no multiple of them.
+// An entry that plans its rows: tiles of the height that sk_plan picked,
+// masked where M is no multiple of it.
 template <class T>
 hipError_t launch_sk_rows(const DenseArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.M + T::R - 1) / T::R) * (unsigned)(a.N / T::BN));
@@ -79,7 +85,7 @@ Entry sk_entry(int schedule, int split) {
   d.block_n = C::BN;
   d.block_k = 32;
   d.num_waves = C::NW;
-  d.num_stages = C::LISTED_D;
+  d.num_stages = C::D;
   d.lds_bytes = C::LDS_BYTES;
   d.group_size_m = 1;
   d.operand_format = SHK_OPERANDS_STREAM;
@@ -89,19 +95,24 @@ Entry sk_entry(int schedule, int split) {
                nullptr, nullptr};
 }
 
-template <int R, bool SWIGLU, bool SUBCH>
-Entry sk_rows_entry() {
-  Entry e = sk_entry<SC<R, SWIGLU, SUBCH>>(SHK_SCHEDULE_STANDARD, 1);
-  e.dense = &launch_sk_plan<SWIGLU, SUBCH>;
-  return e;
-}
-
 template <int R>
 void append_tiles(std::vector<Entry>& t) {
-  t.push_back(sk_rows_entry<R, false, false>());
-  t.push_back(sk_rows_entry<R, true, false>());
-  t.push_back(sk_rows_entry<R, false, true>());
-  t.push_back(sk_rows_entry<R, true, true>());
+  t.push_back(sk_entry<Fixed<R, false, false>>(SHK_SCHEDULE_STANDARD, 1));
+  t.push_back(sk_entry<Fixed<R, true, false>>(SHK_SCHEDULE_STANDARD, 1));
+  t.push_back(sk_entry<Fixed<R, false, true>>(SHK_SCHEDULE_STANDARD, 1));
+  t.push_back(sk_entry<Fixed<R, true, true>>(SHK_SCHEDULE_STANDARD, 1));
+}
+
+// Any M that is a multiple of 16: group_size_m is the most 16-row blocks that
+// a tile joins, and the figures are those of that tile.
+template <bool SWIGLU, bool SUBCH>
+Entry sk_rows_entry() {
+  constexpr int R = SUBCH ? 32 : 64;
+  Entry e = sk_entry<SC<R, SWIGLU, SUBCH>>(SHK_SCHEDULE_STANDARD, 1);
+  e.d.block_m = 16;
+  e.d.group_size_m = R / 16;
+  e.dense = &launch_sk_plan<SWIGLU, SUBCH>;
+  return e;
 }
 
 void append_all(std::vector<Entry>& t) {
@@ -112,21 +123,21 @@ void append_all(std::vector<Entry>& t) {
     // the reference's persistent int4 tiles are its NONE tiles, split-K
     // variants included (registry.py:230-251)
     for (int split : {1, 2, 4, 8}) {
-      t.push_back(sk_entry<SC<16, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<SC<16, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<SC<32, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<SC<32, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<SC<64, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<SC<64, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<Fixed<16, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<Fixed<16, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<Fixed<32, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<Fixed<32, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<Fixed<64, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<Fixed<64, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
     }
   }
   for (int split : {2, 4, 8}) {
-    t.push_back(sk_entry<SC<16, false, false>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<SC<16, false, true>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<SC<32, false, false>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<SC<32, false, true>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<SC<64, false, false>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<SC<64, false, true>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<Fixed<16, false, false>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<Fixed<16, false, true>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<Fixed<32, false, false>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<Fixed<32, false, true>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<Fixed<64, false, false>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<Fixed<64, false, true>>(SHK_SCHEDULE_STANDARD, split));
   }
 }
 
@@ -134,6 +145,13 @@ void append_all(std::vector<Entry>& t) {
 
 #define SHK_CAT3(a, b, c) a##b##_##c
 #define SHK_APPEND_NAME(b, l) SHK_CAT3(append_skinny_, b, l)
+#define SHK_APPEND_ROWS_NAME(b, l) SHK_CAT3(append_skinny_rows_, b, l)
 void SHK_APPEND_NAME(SHK_BITS, SHK_LAYOUT)(std::vector<Entry>& t) { append_all(t); }
+void SHK_APPEND_ROWS_NAME(SHK_BITS, SHK_LAYOUT)(std::vector<Entry>& t) {
+  t.push_back(sk_rows_entry<false, false>());
+  t.push_back(sk_rows_entry<true, false>());
+  t.push_back(sk_rows_entry<false, true>());
+  t.push_back(sk_rows_entry<true, true>());
+}
 
 }  // namespace shk

@@ -74,15 +74,15 @@ constexpr int SK_BN = 64;       // output columns per K-split tile
 constexpr int SK_MAX_WAVE_STAGES_I4 = 1023;
 
 // Ring depth: the deepest of 4, 3, 2 stage slots whose rings fit the LDS
-// budget: 78 KiB for four waves, so that two workgroups share a CU; where two
-// slots already exceed that (SwiGLU tiles of 32 and 64 rows), and for eight
-// or more waves, 150 KiB, one workgroup per CU.
+// budget: 78 KiB, so that two workgroups share a CU, or 150 KiB where two
+// slots already exceed that (SwiGLU tiles of 32 and 64 rows).
 constexpr int sk_stage_bytes(int r, int wcols, bool subch) {
   return r * 64 + wcols * 64 + (subch ? (r / 16) * 256 + 256 : 0);
 }
+// (reserved: LDS the tile uses beside the rings)
+constexpr bool sk_alone(int stage, int nw, int reserved) { return nw * 2 * stage > 79872 - reserved; }
 constexpr int sk_ring_depth(int stage, int nw, int reserved = 0) {
-  const bool alone = nw > 8 || nw * 2 * stage > 79872 - reserved;
-  const int budget = (alone ? 153600 : 79872) - reserved;  // reserved: LDS the tile uses beside the rings
+  const int budget = (sk_alone(stage, nw, reserved) ? 153600 : 79872) - reserved;
   return nw * 4 * stage <= budget ? 4 : (nw * 3 * stage <= budget ? 3 : 2);
 }
 
@@ -126,8 +126,7 @@ struct SkCfg {
   static constexpr int CH = !GSPLIT ? 0 : (NW == 8 ? 1 : (RT * CT == 1 ? 4 : (RT * CT == 2 ? 2 : 1)));
   static constexpr int CHAIN = GSPLIT ? 2 * NW * CH * RT * CT * 1024 : 0;
   static constexpr int D = DEPTH_ > 0 ? DEPTH_ : sk_ring_depth(STAGE, NW, CHAIN);
-  // the depth the table lists (part of the kernel id): that of a shared CU
-  static constexpr int LISTED_D = NW * 2 * STAGE > 79872 - CHAIN ? 2 : D;
+  static constexpr bool ALONE = sk_alone(STAGE, NW, CHAIN);  // one workgroup a CU, whatever the depth
   static constexpr int RING = NW * D * STAGE;
   static constexpr int RED = KSPLIT ? NW * CT * 1024 : 0;  // one row tile of the cross-wave sum
   static constexpr int LDS_BYTES = (RING > RED ? RING : RED) + CHAIN;
@@ -670,7 +669,7 @@ __device__ __forceinline__ void sk_unit_sc(const DenseArgs& p, uint8_t* smem, in
   const int my_chunks = wave < nch ? ((nch - 1 - wave) >> NWSH) + 1 : 0;
   const int n_i = my_chunks << spc_sh;          // this wave's stages
   const int lg = lane >> 4;
-  // this wave's stage i: stage i % spc of chunk 4 (i / spc) + wave
+  // this wave's stage i: stage i % spc of chunk NW (i / spc) + wave
   auto stage_of = [&](int i) { return ((((i >> spc_sh) * C::NW + wave) << lsh) >> KSH) + (i & (spc - 1)); };
   uint8_t* chain = smem + (C::LDS_BYTES - C::CHAIN);
   auto chain_at = [&](int par, int w, int cg, int rt, int c) {

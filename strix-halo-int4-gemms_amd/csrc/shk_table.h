@@ -328,10 +328,15 @@ inline int sk_splits(int bits, long tiles, long k) {
   return (int)(s > need ? s : need);
 }
 
-// Rows of the tiles that a standard skinny call of M rows runs, whatever the
-// entry's block_m: 16, 32 or 64, masked to M.  A taller tile reads B fewer
-// times and keeps the matrix cores busier per byte; a lower one gives a small
-// N more workgroups and computes fewer rows that are not there.
+// Whether a skinny entry plans its tiles' rows for each call (k_skinny.hip
+// sk_rows_entry); the other entries' tiles are block_m rows.
+inline bool sk_plans_rows(const shk_kernel_desc& d) {
+  return d.operand_format == SHK_OPERANDS_STREAM && d.group_size_m > 1;
+}
+// The tile rows such an entry takes for a call of M rows: 16, 32 or 64,
+// masked to M.  A taller tile reads B fewer times and keeps the matrix cores
+// busier per byte; a lower one gives a small N more workgroups and computes
+// fewer rows that are not there.
 //
 // Per-channel: the smallest predicted time (us) a + b * (K per workgroup /
 // 4096) * rounds of 256 workgroups, whole rounds for the SwiGLU tiles of 32
@@ -393,10 +398,9 @@ inline SkPlan sk_plan(int bits, int sub, bool swiglu, long m, long n, long k) {
   }
   return best;
 }
-// Rows of a table entry's tiles: the split-K and persistent entries keep
-// their block_m.
+// Rows of a table entry's tiles.
 inline int sk_tile_rows(const shk_kernel_desc& d, long m, long n, long k, int sub) {
-  if (d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1) return d.block_m;
+  if (!sk_plans_rows(d)) return d.block_m;
   return sk_plan(d.dtype_bits, sub, d.epilogue_kind == SHK_EPI_KIND_SWIGLU, m, n, k).rows;
 }
 // A skinny call: its tile rows, the workgroups sharing a tile's K (subchannel
@@ -470,11 +474,17 @@ void append_split_8_2(std::vector<Entry>& t);
 // the per-channel and subchannel tiles, plain and SwiGLU; for int4 the
 // persistent plain tiles, split-K 1/2/4/8; then split-K 2/4/8 plain tiles.
 void append_skinny_4_0(std::vector<Entry>& t);
+void append_skinny_rows_4_0(std::vector<Entry>& t);
 void append_skinny_4_1(std::vector<Entry>& t);
+void append_skinny_rows_4_1(std::vector<Entry>& t);
 void append_skinny_4_2(std::vector<Entry>& t);
+void append_skinny_rows_4_2(std::vector<Entry>& t);
 void append_skinny_8_0(std::vector<Entry>& t);
+void append_skinny_rows_8_0(std::vector<Entry>& t);
 void append_skinny_8_1(std::vector<Entry>& t);
+void append_skinny_rows_8_1(std::vector<Entry>& t);
 void append_skinny_8_2(std::vector<Entry>& t);
+void append_skinny_rows_8_2(std::vector<Entry>& t);
 void append_ragged_0(std::vector<Entry>& t);
 void append_ragged_1(std::vector<Entry>& t);
 void append_ragged_2(std::vector<Entry>& t);

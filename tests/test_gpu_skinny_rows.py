@@ -1,6 +1,7 @@
-"""The skinny tiles' row heights (shk_table.h sk_plan): a call of M rows runs
-16-, 32- or 64-row tiles masked to M, whatever block_m its entry has.  Every
-output against the CPU oracle; the row below the output stays untouched."""
+"""The skinny entries that plan their rows (shk_table.h sk_plan): a call of M
+rows runs 16-, 32- or 64-row tiles masked to M.  Every output against the CPU
+oracle; the row below the output stays untouched, and the workspace of a split
+K is left zero."""
 
 from __future__ import annotations
 
@@ -19,16 +20,16 @@ from amd_strix_halo_kernels import kernel_table as kt  # noqa: E402
 from amd_strix_halo_kernels import native  # noqa: E402
 
 
-def _check(bits, layout, epilogue, sub, m, n, k, device, rows):
+def _check(bits, layout, epilogue, sub, m, n, k, device, rows, splits=None):
     swiglu = epilogue == "swiglu"
     assert kt.sk_plan(bits, sub, swiglu, m, n, k)[0] == rows
     a_q, b_q, a_arg, b_arg, sa, sb = dense_case(stable_seed("rows", bits, layout, epilogue, sub, m, n, k), bits=bits,
                                                 layout=layout, m=m, n=n, k=k, subchannel=sub or None, swiglu=swiglu)
     a, b, ta, tb = (to_dev(torch, x, device) for x in (a_arg, b_arg, sa, sb))
-    kernel = next(x for x in shk.default_registry.all() if kt.TABLE[x.table_index].is_stream
-                  and x.tile.block_m == 16 and x.scale == spec_of(sub) and x.epilogue.value == epilogue
-                  and x.layout.value == layout and x.tile.split_k == 1 and kt.TABLE[x.table_index].dtype_bits == bits
-                  and x.schedule is shk.KernelSchedule.STANDARD)
+    kernel = next(x for x in shk.default_registry.all() if kt.TABLE[x.table_index].plans_rows
+                  and x.scale == spec_of(sub) and x.epilogue.value == epilogue and x.layout.value == layout
+                  and kt.TABLE[x.table_index].dtype_bits == bits)
+    assert splits is None or kt.sk_split_count(kt.TABLE[kernel.table_index], m, n, k) == splits
     print(f"case {kernel.kernel_id} shape=({m},{n},{k}) rows={rows}", flush=True)
     out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=device)
     for _ in range(2):  # a split launch leaves its workspace zero for the next
@@ -36,6 +37,8 @@ def _check(bits, layout, epilogue, sub, m, n, k, device, rows):
     raw = native.launch_generated_kernel_i32(a, b, kernel=kernel, a_scale=ta, b_scale=tb)
     torch.cuda.synchronize()
     assert bool((out[m] == 7.0).all()), "rows past M written"
+    work = native._SPLIT_WORKSPACES.get((device.index or 0, torch.cuda.current_stream(device).cuda_stream))
+    assert work is None or int(work.count_nonzero()) == 0
     assert np.array_equal(raw.cpu().numpy(), ref.int_matmul(a_q, b_q))
     want = ref.reference_gemm_bf16(a_arg, b_arg, bits=bits, layout=layout, a_scale=sa, b_scale=sb,
                                    subchannel=sub or None, epilogue=epilogue)
@@ -68,3 +71,21 @@ def test_subchannel_32_row_tiles_match_the_oracle(bits, sub, epilogue, m, rows, 
     """32-row tiles where they make fewer rounds of workgroups (N = 4096)."""
     _check(bits, layout, epilogue, sub, m, 4096 if rows == 32 else 192, (2 if sub > 64 else 5) * sub // 64 * 64 or 64,
            device, rows)
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,n,k", [(64, 6720, 13632), (480, 896, 13824)])
+def test_int4_64_row_tiles_with_k_split(m, n, k, layout, device):
+    """64-row tiles, whole and masked, of which two workgroups share the K."""
+    _check(4, layout, "none", 0, m, n, k, device, 64, splits=2)
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("sub", [32, 64, 128, 256])
+@pytest.mark.parametrize("epilogue,m,groups", [("none", 48, 9), ("none", 64, 37), ("swiglu", 48, 37), ("swiglu", 64, 9)])
+def test_subchannel_32_row_tiles_over_several_rounds(bits, sub, epilogue, m, groups, layout, device):
+    """More scale groups than the waves of a 32-row tile take in one round (8,
+    SwiGLU 4): the totals carry over, in group order."""
+    k = -(-groups * sub // 64) * 64
+    _check(bits, layout, epilogue, sub, m, 3072, k, device, 32)

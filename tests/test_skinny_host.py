@@ -172,3 +172,64 @@ def test_workspace_bytes_match_the_library():
                 continue
             assert lib.amd_strix_halo_kernels_gemm_workspace_bytes(d.index, m, n, k, ctypes.byref(out)) == 0
             assert out.value == d.workspace_bytes(m, n, k), (d, m, n, k)
+
+
+def test_entries_of_one_height_run_it():
+    """A skinny entry's block_m is the height of its tiles: the library sizes
+    the partials of a split K by it, whatever height a call of that shape
+    would plan.  One more entry a family plans its rows, and whole calls run it."""
+    lib = native.load_dispatch_library()
+    out = ctypes.c_uint64()
+    shapes = ((64, 128, 8192 + 32), (192, 64, 8192), (64, 8192, 8192), (64, 512, 1 << 20))
+    planned = 0
+    for d in kt.TABLE:
+        if not d.is_stream or d.scale_mode != kt.SCALE_PER_CHANNEL:
+            continue
+        cols = 2 if d.epilogue_kind == kt.EPI_KIND_SWIGLU else 1
+        for m, n, k in shapes:
+            rows = d.block_m
+            if d.plans_rows:
+                rows = kt.sk_plan(d.dtype_bits, 0, cols == 2, m, n, k)[0]
+                planned += rows != 16
+            tiles = -(-m // rows) * (n // 64)
+            splits = kt.sk_split_count(d, m, n, k)
+            need = 0 if splits <= 1 else (tiles * 4 + 255) // 256 * 256 + tiles * splits * rows * 64 * cols * 4
+            assert lib.amd_strix_halo_kernels_gemm_workspace_bytes(d.index, m, n, k, ctypes.byref(out)) == 0
+            assert out.value == need == d.workspace_bytes(m, n, k), (d, m, n, k)
+    assert planned
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("sub", [None, 32, 128])
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+def test_whole_calls_run_the_entry_that_plans_its_rows(bits, sub, epilogue):
+    """select() returns the entry whose height M is, a whole call the planned
+    one; where no height of 32 or 64 divides M both do."""
+    dtype = shk.OperandDType.INT4 if bits == 4 else shk.OperandDType.INT8
+    spec = shk.ScaleSpec(shk.ScaleMode.SUBCHANNEL, sub) if sub else shk.ScaleSpec(shk.ScaleMode.PER_CHANNEL)
+    request = dict(dtype=dtype, scale=spec, epilogue=shk.Epilogue(epilogue), n=128, k=128, split_k=1)
+    reg = shk.default_registry
+    for m in (16, 32, 48, 80):
+        picked = reg.select(m=m, **request)
+        assert picked.tile.block_m == (32 if m == 32 else 16)
+        assert kt.TABLE[picked.table_index].plans_rows == (m != 32)
+        for _ in range(2):
+            call = reg.select_call(m=m, **request)
+            assert kt.TABLE[call.table_index].plans_rows and call.epilogue.value == epilogue and call.scale == spec
+    # a figure of the caller's own keeps the kernel it was set for
+    picked = reg.select(m=32, **request)
+    own = reg.with_status(picked.kernel_id, picked.status, measured_tops=9e9)
+    assert own.select_call(m=32, **request).kernel_id == picked.kernel_id
+
+
+def test_the_registry_accepts_by_the_launch_shape_contract():
+    """The registry's quick acceptance equals the contract that launches check
+    (template_config.py) and the entry's K bound, for every kernel."""
+    from amd_strix_halo_kernels.registry import _Candidate
+    from amd_strix_halo_kernels.template_config import LaunchShape, is_tile_multiple_shape
+
+    for kernel in shk.default_registry.all():
+        c = _Candidate(kernel)
+        for m, n, k in itertools.product((16, 40, 64, 256), (16, 64, 320), (32, 96, 128, 192, 512, 131072, 1 << 25)):
+            want = is_tile_multiple_shape(kernel, LaunchShape(m, n, k)) and kt.TABLE[kernel.table_index].supports_k(k)
+            assert c.accepts(m, n, k) == want, (kernel.kernel_id, m, n, k)
