@@ -194,17 +194,15 @@ SK_BN_SUBCH = 16
 SK_TARGET_UNITS = 256
 
 
-def _sk_geometry(r: int, swiglu: bool, subch: bool, *, fixed: bool = True) -> tuple[int, int]:
-    """(ring depth, LDS bytes) of a skinny tile of r rows (SkCfg), in an entry
-    of that height (`fixed`) or in one that plans its rows."""
+def _sk_geometry(r: int, swiglu: bool, subch: bool) -> tuple[int, int]:
+    """(ring depth, LDS bytes) of a skinny tile of r rows (SkCfg)."""
     bn = SK_BN_SUBCH if subch else SK_BN
     wcols = 2 * bn if swiglu else bn
     stage = r * 64 + wcols * 64 + ((r // 16) * 256 + 256 if subch else 0)
     tiles = (r // 16) * (wcols // 16)
     ch = (4 if tiles == 1 else 2 if tiles == 2 else 1) if subch else 0  # groups per wave and round
     chain = 2 * SK_NW * ch * tiles * 1024  # two rounds of scaled partials
-    alone = SK_NW * 2 * stage > 79872 - chain  # one workgroup a CU
-    budget = (153600 if alone and not fixed else 79872) - chain
+    budget = 79872 - chain
     depth = 4 if SK_NW * 4 * stage <= budget else (3 if SK_NW * 3 * stage <= budget else 2)
     ring = SK_NW * depth * stage
     red = 0 if subch else SK_NW * (wcols // 16) * 1024
@@ -366,7 +364,7 @@ def _sk_desc(index, bits, layout, r, *, swiglu=False, subch=False, schedule=SCHE
 def _sk_rows_desc(index, bits, layout, *, swiglu, subch):
     # the figures of the tallest tile
     r = 32 if subch else 64
-    depth, lds = _sk_geometry(r, swiglu, subch, fixed=False)
+    depth, lds = _sk_geometry(r, swiglu, subch)
     return KernelDesc(
         index=index, family=FAMILY_DENSE, dtype_bits=bits, layout=layout,
         scale_mode=SCALE_SUBCHANNEL if subch else SCALE_PER_CHANNEL,

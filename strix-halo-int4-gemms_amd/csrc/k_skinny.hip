@@ -29,11 +29,6 @@ constexpr int kLayout = SHK_LAYOUT;
 
 template <int R, bool SWIGLU, bool SUBCH>
 using SC = SkCfg<kBits, kLayout, R, SWIGLU, SUBCH>;
-// The tiles of the entries whose block_m is their height: rings that leave
-// room for a second workgroup on the CU.
-template <int R, bool SWIGLU, bool SUBCH>
-using Fixed = SkCfg<kBits, kLayout, R, SWIGLU, SUBCH, SUBCH ? 16 : 0, SK_NW, SK_BN,
-                    SC<R, SWIGLU, SUBCH>::ALONE ? 2 : 0>;
 
 // grid.x = output tiles; per-channel tiles run sk_splits workgroups each.
 template <class C>
@@ -62,8 +57,10 @@ hipError_t launch_sk_plan(const DenseArgs& a, dim3, hipStream_t s) {
     if (rows == 16 && a.subchannel >= T::KS) return launch_sk_rows<T>(a, s);
   }
   if (rows == 16) return launch_sk_rows<SC<16, SWIGLU, SUBCH>>(a, s);
-  if (SUBCH || rows == 32) return launch_sk_rows<SC<32, SWIGLU, SUBCH>>(a, s);
-  return launch_sk_rows<SC<64, SWIGLU, SUBCH>>(a, s);
+  if constexpr (!SUBCH) {
+    if (rows == 64) return launch_sk_rows<SC<64, SWIGLU, SUBCH>>(a, s);
+  }
+  return launch_sk_rows<SC<32, SWIGLU, SUBCH>>(a, s);
 }
 template <class C>
 hipError_t launch_sk_persistent_t(const DenseArgs& a, dim3 grid, hipStream_t s) {
@@ -97,10 +94,10 @@ Entry sk_entry(int schedule, int split) {
 
 template <int R>
 void append_tiles(std::vector<Entry>& t) {
-  t.push_back(sk_entry<Fixed<R, false, false>>(SHK_SCHEDULE_STANDARD, 1));
-  t.push_back(sk_entry<Fixed<R, true, false>>(SHK_SCHEDULE_STANDARD, 1));
-  t.push_back(sk_entry<Fixed<R, false, true>>(SHK_SCHEDULE_STANDARD, 1));
-  t.push_back(sk_entry<Fixed<R, true, true>>(SHK_SCHEDULE_STANDARD, 1));
+  t.push_back(sk_entry<SC<R, false, false>>(SHK_SCHEDULE_STANDARD, 1));
+  t.push_back(sk_entry<SC<R, true, false>>(SHK_SCHEDULE_STANDARD, 1));
+  t.push_back(sk_entry<SC<R, false, true>>(SHK_SCHEDULE_STANDARD, 1));
+  t.push_back(sk_entry<SC<R, true, true>>(SHK_SCHEDULE_STANDARD, 1));
 }
 
 // Any M that is a multiple of 16: group_size_m is the most 16-row blocks that
@@ -123,21 +120,21 @@ void append_all(std::vector<Entry>& t) {
     // the reference's persistent int4 tiles are its NONE tiles, split-K
     // variants included (registry.py:230-251)
     for (int split : {1, 2, 4, 8}) {
-      t.push_back(sk_entry<Fixed<16, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<Fixed<16, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<Fixed<32, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<Fixed<32, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<Fixed<64, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
-      t.push_back(sk_entry<Fixed<64, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<SC<16, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<SC<16, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<SC<32, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<SC<32, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<SC<64, false, false>>(SHK_SCHEDULE_PERSISTENT, split));
+      t.push_back(sk_entry<SC<64, false, true>>(SHK_SCHEDULE_PERSISTENT, split));
     }
   }
   for (int split : {2, 4, 8}) {
-    t.push_back(sk_entry<Fixed<16, false, false>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<Fixed<16, false, true>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<Fixed<32, false, false>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<Fixed<32, false, true>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<Fixed<64, false, false>>(SHK_SCHEDULE_STANDARD, split));
-    t.push_back(sk_entry<Fixed<64, false, true>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<SC<16, false, false>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<SC<16, false, true>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<SC<32, false, false>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<SC<32, false, true>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<SC<64, false, false>>(SHK_SCHEDULE_STANDARD, split));
+    t.push_back(sk_entry<SC<64, false, true>>(SHK_SCHEDULE_STANDARD, split));
   }
 }
 

@@ -73,16 +73,16 @@ constexpr int SK_BN = 64;       // output columns per K-split tile
 // for K below 131072, i.e. at most 1023 stages of 128 K per wave and split.
 constexpr int SK_MAX_WAVE_STAGES_I4 = 1023;
 
-// Ring depth: the deepest of 4, 3, 2 stage slots whose rings fit the LDS
-// budget: 78 KiB, so that two workgroups share a CU, or 150 KiB where two
-// slots already exceed that (SwiGLU tiles of 32 and 64 rows).
+// Ring depth: the deepest of 4, 3, 2 stage slots whose rings fit 78 KiB of
+// LDS, so that two workgroups share a CU.  Two slots of the SwiGLU tiles of 32
+// and 64 rows already exceed that; a third is no gain there (int4, one CU's
+// workgroup with two and three slots: 1024 x 3840 x 4096 57.0 and 64.4 us, 64
+// x 9088 x 2112 11.8 and 12.8, 32 x 12224 x 9472 23.4 and 23.8).
 constexpr int sk_stage_bytes(int r, int wcols, bool subch) {
   return r * 64 + wcols * 64 + (subch ? (r / 16) * 256 + 256 : 0);
 }
-// (reserved: LDS the tile uses beside the rings)
-constexpr bool sk_alone(int stage, int nw, int reserved) { return nw * 2 * stage > 79872 - reserved; }
 constexpr int sk_ring_depth(int stage, int nw, int reserved = 0) {
-  const int budget = (sk_alone(stage, nw, reserved) ? 153600 : 79872) - reserved;
+  const int budget = 79872 - reserved;  // reserved: LDS the tile uses beside the rings
   return nw * 4 * stage <= budget ? 4 : (nw * 3 * stage <= budget ? 3 : 2);
 }
 
@@ -126,7 +126,6 @@ struct SkCfg {
   static constexpr int CH = !GSPLIT ? 0 : (NW == 8 ? 1 : (RT * CT == 1 ? 4 : (RT * CT == 2 ? 2 : 1)));
   static constexpr int CHAIN = GSPLIT ? 2 * NW * CH * RT * CT * 1024 : 0;
   static constexpr int D = DEPTH_ > 0 ? DEPTH_ : sk_ring_depth(STAGE, NW, CHAIN);
-  static constexpr bool ALONE = sk_alone(STAGE, NW, CHAIN);  // one workgroup a CU, whatever the depth
   static constexpr int RING = NW * D * STAGE;
   static constexpr int RED = KSPLIT ? NW * CT * 1024 : 0;  // one row tile of the cross-wave sum
   static constexpr int LDS_BYTES = (RING > RED ? RING : RED) + CHAIN;
