@@ -225,52 +225,80 @@ def _sk_splits(bits: int, tiles: int, k: int) -> int:
     return max(s, _sk_needed_splits(bits, k))
 
 
-# (bits, SwiGLU): per tile height 16, 32, 64 the us of a call (fixed, more for
-# a wide B, and per round of 256 workgroups at 4096 K each), the fraction of a
-# round that stays as K shrinks and whether rounds count whole.
-_SK_FITS = {
-    (4, False): ((3.6, 0.0, 3.38, 0.27, False), (3.4, 0.0, 4.8, 0.25, False), (4.8, 0.0, 6.07, 0.3, False)),
-    (4, True): ((4.0, 3.0, 4.6, 0.35, False), (5.5, 0.0, 10.5, 0.37, True), (7.5, 0.0, 15.5, 0.45, True)),
-    (8, False): ((3.8, 0.0, 5.2, 0.12, False), (4.2, 0.0, 6.45, 0.13, False), (4.5, 0.0, 8.0, 0.2, False)),
-    (8, True): ((3.2, 12.1, 7.7, 0.05, False), (3.0, 9.0, 12.5, 0.2, True), (3.0, 9.0, 15.0, 0.33, True)),
-}
+# Time fits of the skinny tiles by [8-bit][SwiGLU][16, 32, 64 rows], and for
+# subchannel [8-bit][SwiGLU][groups of a stage or more][16, 32 rows]
+# (shk_table.h sk_plan, which states the terms).
+_SK_FIT = ((((3.76, 2.96, 0.96, 3.11, 0.2, 0.77, 0.1, 1.39, 0.88),
+             (3.91, 4.12, 1.8, 2.72, 0.16, 0.54, 0.65, 1.07, 1.19),
+             (4.89, 5.84, 2.69, 3.29, 0.33, 1.19, 0.64, 0.1, 1.64)),
+            ((3.91, 5.25, 4.09, 1.05, 0.67, 0.92, 0.07, 1.09, 1.19),
+             (4.97, 6.96, 6.16, 0.83, 1.12, 0.51, 3.21, 0.32, 1.55),
+             (6.94, 9.81, 8.75, 0.0, 0.81, 0.14, 5.91, 1.36, 2.78))),
+           (((3.71, 3.68, 4.83, 0.45, 0.0, 0.41, 0.0, 3.55, 1.02),
+             (3.64, 5.78, 5.15, 2.5, 0.0, 0.55, 0.0, 3.24, 1.09),
+             (4.16, 8.21, 7.34, 4.93, 0.0, 0.77, 0.0, 2.21, 1.59)),
+            ((2.87, 10.23, 6.51, 4.32, 1.34, 0.51, 0.0, 3.5, 1.14),
+             (3.74, 11.02, 7.83, 4.71, 2.69, 0.0, 2.68, 3.73, 1.71),
+             (5.52, 14.08, 12.06, 1.6, 1.05, 0.14, 4.59, 2.99, 2.72))))
+_SK_SUB_FIT = (((((3.5, 2.26, 3.42, 2.89, 3.49, 1.45, 0.15, 0.89, 0.44, 0.13),
+                  (3.48, 0.06, 6.6, 0.44, 6.75, 1.04, 0.47, 0.98, 0.0, 0.05)),
+                 ((3.63, 1.63, 1.64, 2.68, 1.95, 0.89, 0.77, 0.72, 1.53, 0.6),
+                  (3.84, 4.06, 3.62, 4.79, 3.72, 1.07, 0.55, 1.02, 0.79, 0.37))),
+                (((3.84, 0.47, 6.04, 0.29, 6.52, 0.39, 0.71, 1.01, 0.96, 0.62),
+                  (3.78, 0.14, 10.11, 0.68, 10.49, 0.0, 1.15, 1.06, 0.74, 0.64)),
+                 ((4.0, 3.09, 4.1, 5.12, 3.22, 1.21, 0.64, 0.97, 2.21, 1.16),
+                  (3.86, 4.44, 6.46, 6.36, 5.75, 2.24, 0.0, 1.03, 1.13, 0.8)))),
+               ((((3.59, 0.0, 3.86, 0.0, 4.24, 0.0, 0.56, 0.91, 1.52, 0.59),
+                  (3.41, 0.0, 5.68, 0.0, 6.02, 0.0, 0.84, 0.94, 1.15, 0.48)),
+                 ((3.42, 2.59, 1.44, 4.91, 1.73, 1.86, 0.55, 0.57, 4.23, 1.94),
+                  (3.84, 5.39, 3.26, 9.06, 2.89, 2.21, 0.0, 0.84, 2.47, 1.64))),
+                (((3.86, 0.0, 5.44, 0.0, 5.84, 0.0, 0.82, 1.02, 2.57, 0.75),
+                  (3.38, 0.0, 9.69, 0.0, 10.3, 0.0, 1.15, 0.91, 3.97, 1.54)),
+                 ((3.9, 4.15, 2.68, 9.52, 1.89, 2.21, 1.68, 0.63, 6.05, 4.11),
+                  (3.31, 6.32, 6.61, 11.59, 3.82, 2.14, 0.0, 0.74, 5.02, 3.92)))))
 
 
 @functools.lru_cache(maxsize=4096)
-def sk_plan(bits: int, sub: int, swiglu: bool, m: int, n: int, k: int) -> tuple[int, float]:
+def sk_plan(bits: int, sub: int, swiglu: bool, m: int, n: int, k: int, layout: int = LAYOUT_NN) -> tuple[int, float]:
     """(tile rows, predicted us) of a call of M rows on a skinny entry that
-    plans its rows (shk_table.h sk_plan, which states the fits); us 0 for
-    subchannel (sub: the group size, 0 for per-channel)."""
-    if sub > 0:
-        def load(rows: int) -> float:
-            t = -(-m // rows) * (n // 16)
-            rest = t % 512
-            return 1.0 if t <= 256 else 1.37 * (t // 512 + (0.0 if rest == 0 else 0.73 if rest <= 256 else 1.0))
-
-        tall = 1.15 if swiglu and sub >= (128 if bits == 4 else 64) else 1.45
-        return (16 if m <= 16 or load(16) <= tall * load(32) else 32), 0.0
-    best = (16, -1.0)
-    wide, k4 = min(1.0, 2.0 * n * k / 9e7), k / 4096.0
-    for i, (a, w, b, f, whole) in enumerate(_SK_FITS[bits, swiglu]):
+    plans its rows (shk_table.h sk_plan, which states the fits); sub: the
+    group size, 0 for per-channel scales."""
+    best, whole = (16, -1.0), (16, -1.0)
+    for i in range(2 if sub else 3):
         rows = 16 << i
         if i > 0 and m <= rows // 2:
             break
-        tiles = -(-m // rows) * (n // SK_BN)
-        s = _sk_splits(bits, tiles, k)
-        units = tiles * s
-        rounds = 1.0 if units <= 256 else (float(-(-units // 256)) if whole else units / 256.0)
-        us = (a + w * wide + (float(rows // 16 * (2 if swiglu else 1)) if s > 1 else 0.0)
-              + b * (k4 / s * rounds + f * max(0.0, 1.0 - k4) * (rounds - 1.0)))
+        tiles = -(-m // rows) * (n // (SK_BN_SUBCH if sub else SK_BN))
+        s = 1 if sub else _sk_splits(bits, tiles, k)
+        u = tiles * s
+        w = k / s / 4096.0
+        second = u > 256
+        past = u / 256.0 - 1.0 if second else 0.0
+        wm, w2, twice = w * (1.0 + past), w if second else 0.0, (u - 1) // 512
+        a_mn, b_mn = wm if layout == LAYOUT_TN else 0.0, wm if layout == LAYOUT_NN else 0.0
+        if sub:
+            g = k / sub / 32.0
+            fit = _SK_SUB_FIT[bits == 8][swiglu][sub >= (128 if bits == 4 else 64)][i]
+            terms = (1.0, w, g, w * twice, g * twice, w2, g if second else 0.0, past, a_mn, b_mn)
+        else:
+            fit = _SK_FIT[bits == 8][swiglu][i]
+            rounds = (u - 1) // 256
+            terms = (1.0, w, w * rounds, w * twice, w2, past, float(rounds), a_mn, float(s.bit_length() - 1))
+        us = 0.0
+        for f, x in zip(fit, terms):
+            us += f * x
         if best[1] < 0.0 or us < best[1]:
             best = (rows, us)
-    return best
+        if m % rows == 0:
+            whole = (rows, us)
+    return whole if whole[1] <= 1.05 * best[1] else best
 
 
 def _sk_tile_rows(desc: "KernelDesc", m: int, n: int, k: int) -> int:
     """Rows of a skinny entry's tiles."""
     if not desc.plans_rows:
         return desc.block_m
-    return sk_plan(desc.dtype_bits, 0, desc.epilogue_kind == EPI_KIND_SWIGLU, m, n, k)[0]
+    return sk_plan(desc.dtype_bits, 0, desc.epilogue_kind == EPI_KIND_SWIGLU, m, n, k, desc.layout)[0]
 
 
 def sk_split_count(desc: "KernelDesc", m: int, n: int, k: int, with_workspace: bool = True) -> int:
@@ -558,32 +586,39 @@ def _f6_edge_us(m: int, n: int, k: int, swiglu: bool) -> float:
 
 PREDICT_MAX_K = 65536  # K up to which the fits of predicted_us stand
 
-# subchannel, by group size: us per product on the 32-row skinny tiles (plain,
-# SwiGLU); a 128 x 128 fp6 tile's fixed us and us per K value
-_SKINNY_SUB_US = {32: (2.78e-8, 2.24e-8), 64: (1.38e-8, 1.14e-8), 128: (0.95e-8, 0.68e-8), 256: (0.73e-8, 0.59e-8)}
+# subchannel: a 128 x 128 fp6 tile's fixed us and us per K value by group
+# size; the 64 x 64 tile's us by [SwiGLU][NN, NT, TN] for a round of 256 tiles
+# (constant, K / 1024, K / 8 groups) and for the tiles past it (the same)
+_PACKED_SUB_US = (
+    ((3.18, 9.2, 3.26, 2.83, 1.36, 0.9), (2.93, 4.84, 3.42, 1.47, 1.31, 0.83), (3.4, 12.61, 3.5, 4.53, 2.14, 1.09)),
+    ((2.87, 11.52, 5.56, 7.46, 3.23, 0.79), (3.64, 7.13, 5.28, 1.63, 3.65, 1.59), (3.4, 15.99, 5.23, 0.0, 5.86, 0.0)),
+)
 _F6_SUB_US = {32: (5.0, 0.0215), 64: (5.0, 0.0125), 128: (5.0, 0.0061), 256: (3.5, 0.0038)}
 
 
 def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = None) -> float | None:
     """Predicted time of a standard int4 call on an entry, in us (None for the
-    other families and K past PREDICT_MAX_K); capi.hip computes the skinny
-    and FP6_EDGE entries' alike, and the skinny entries of a family share the
-    planned tiles' time (among them selection_area decides).  Fits to calls measured over M 16..8176 and
-    N x K of 1024 x 4096, 4096 x 1024, 4096^2, 11008 x 4096, 16384 x 4096 and
-    8192^2:
+    other families and K past PREDICT_MAX_K); capi.hip computes the skinny,
+    FP6_EDGE and 64 x 64 entries' alike, and the skinny entries of a family
+    share the planned tiles' time (among them selection_area decides):
 
-    * skinny per-channel tiles: sk_plan;
-    * skinny subchannel tiles: a launch, the products and the outputs;
+    * skinny tiles: sk_plan;
+    * the subchannel 64 x 64 tile on the packed operands, past
+      SKINNY_SUB_MAX_M rows (below them the skinny tiles' figures stand):
+      linear in K, groups and tiles past a round, by layout;
     * fp6 entries: two launches, the conversion at 5 TB/s, then rounds of
       tiles: per-channel 256-row tiles (FP6) or the launcher's split
       (FP6_EDGE); subchannel 128 x 128 tiles, two a CU (1.3 times one; 1.1
       beside half-height tiles, which alone take 0.8).
 
-    Measured against predicted, per-channel: 512 x 4096^2 skinny 16.6 (17),
-    256-row fp6 36.7 (44), edge 24.7 (22); 8176 x 16384 x 4096 skinny 64-row
-    tiles 810 (793), edge 324 (300); 8192^3 fp6 277 (251).  Groups of 128: 64 x 4096^2
-    skinny 17.5 (17), edge 37.5 (34); 320 x 16384 x 4096 skinny 221 (236),
-    edge 56.5 (57); 4160 x 4096^2 edge 116 (132)."""
+    Fitted to calls drawn over M 16..8192, N 512..16384 and K 512..14336 in
+    every layout, each entry measured (us): the predicted choice takes 1.1%
+    (per-channel), 0.6% (subchannel) and 1.7, 0.4% (SwiGLU) more than the best
+    of the entries, and of 3978 calls 24 take 3% more than on the entry that
+    the figures alone, without predictions, rank first.  Groups of 64, 1536 x
+    704 x 768 NT: 64 x 64 tile 12.4, edge 18.1, skinny 24.6; groups of 128, 320
+    x 16384 x 4096 skinny 221, edge 56.5; per-channel 8176 x 16384 x 4096
+    skinny 810, edge 324."""
     if (desc.family != FAMILY_DENSE or desc.dtype_bits != 4 or desc.schedule != SCHEDULE_STANDARD
             or desc.split_k > 1 or k > PREDICT_MAX_K):
         return None
@@ -593,11 +628,20 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
     if desc.scale_mode == SCALE_SUBCHANNEL:
         if sub not in _F6_SUB_US:
             return None
-        if desc.operand_format == OPERANDS_STREAM:
-            low = 1.5 if sk_plan(4, sub, swiglu, m, n, k)[0] == 16 else 1.0
+        if desc.is_stream:
             # of the heights, the 32-row tile ranks first, as measured (SKINNY_SUB_TOPS)
             rank = 1.0 if desc.plans_rows else {32: 1.0, 64: 1.001, 16: 1.002}[desc.block_m]
-            return 6.0 + rank * (_SKINNY_SUB_US[sub][swiglu] * low * (m * cols * k) + 5e-6 * (m * n))
+            return rank * sk_plan(4, sub, swiglu, m, n, k, desc.layout)[1]
+        if desc.operand_format == OPERANDS_PACKED:
+            if desc.block_m != 64 or desc.block_n != 64 or m <= SKINNY_SUB_MAX_M:
+                return None
+            u = float((m // 64) * (n // 64))
+            past = u / 256.0 - 1.0 if u > 256.0 else 0.0
+            w, g = k / 1024.0, k / sub / 8.0
+            us = 0.0
+            for f, x in zip(_PACKED_SUB_US[swiglu][desc.layout], (1.0, w, g, w * past, g * past, past)):
+                us += f * x
+            return us
         if not desc.needs_workspace:
             return None
         fixed, per_k = _F6_SUB_US[sub]
@@ -610,7 +654,7 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
             rounds *= 0.8
         return convert + (fixed + per_k * k) * rounds
     if desc.operand_format == OPERANDS_STREAM:
-        return sk_plan(4, 0, swiglu, m, n, k)[1]
+        return sk_plan(4, 0, swiglu, m, n, k, desc.layout)[1]
     if desc.operand_format == OPERANDS_FP6_EDGE:
         return convert + _f6_edge_us(m, n, k, swiglu)
     if desc.operand_format == OPERANDS_FP6:
@@ -627,7 +671,7 @@ def selection_tops(desc: KernelDesc, m: int, n: int | None = None, k: int | None
     FP6 entry where one fits); for the others, or without n and k,
     measured_tops, where the skinny subchannel tiles' figure holds up to
     SKINNY_SUB_MAX_M rows."""
-    if n is not None and k is not None and desc.operand_format != OPERANDS_FP6:
+    if n is not None and k is not None and desc.dtype_bits == 4 and desc.operand_format != OPERANDS_FP6:
         us = predicted_us(desc, m, n, k, sub)
         if us is not None:
             cap = 2000.0 if desc.scale_mode == SCALE_SUBCHANNEL else 3000.0

@@ -110,7 +110,8 @@ class _Candidate:
     multiples of the launch-shape contract (template_config.py
     tile_multiple_rejection_reasons) and its K bound, as plain numbers."""
 
-    __slots__ = ("kernel", "desc", "split_k", "block_m", "block_n", "period", "sub", "slice_sub", "max_k")
+    __slots__ = ("kernel", "desc", "split_k", "block_m", "block_n", "period", "sub", "slice_sub", "max_k", "table_figure",
+                 "area")
 
     def __init__(self, kernel: KernelMetadata) -> None:
         tile = kernel.tile
@@ -123,6 +124,9 @@ class _Candidate:
         self.slice_sub = self.sub if subchannel and tile.split_k > 1 and slices_k(kernel) else 1
         # the library's bound (gfx950 accumulators and buffer offsets)
         self.max_k = None if self.desc is None else self.desc.max_k
+        # whether measured_tops is the table's, not a caller's own (with_status)
+        self.table_figure = self.desc is not None and kernel.measured_tops == kt.measured_tops(self.desc)
+        self.area = None if self.desc is not None and self.desc.plans_rows else tile.block_m * tile.block_n
 
     def accepts(self, m: int, n: int, k: int) -> bool:
         return not (m % self.block_m or n % self.block_n or k % self.period or k % self.sub
@@ -130,12 +134,10 @@ class _Candidate:
 
 
 def _selection_key(c: _Candidate, m: int, n: int | None = None, k: int | None = None) -> tuple[float, int]:
-    tops, desc = c.kernel.measured_tops, c.desc
-    if desc is None:
-        return (tops or 0.0, c.block_m * c.block_n)
-    if tops == kt.measured_tops(desc):  # not a caller's own figure (with_status)
-        tops = kt.selection_tops(desc, m, n, k, c.kernel.scale.subchannel_size)
-    return (tops or 0.0, kt.selection_area(desc, m))
+    tops = c.kernel.measured_tops
+    if c.table_figure:
+        tops = kt.selection_tops(c.desc, m, n, k, c.kernel.scale.subchannel_size)
+    return (tops or 0.0, c.area or kt.selection_area(c.desc, m))
 
 
 class KernelRegistry:
@@ -249,17 +251,17 @@ class KernelRegistry:
         separate conversion needs them, and the skinny entry of a single
         height for the M of that height.  A whole call is free to take any
         entry with the same results: of the skinny entries the one that plans
-        its rows, and where an FP6 entry fits the smallest predicted time
-        decides (kernel_table.predicted_us), since on few tiles of 256 rows
-        another one is faster (512 x 4096 x 4096: FP6 36.7 us, skinny 16.6; 512
-        x 16384 x 4096: FP6 47.4, FP6_EDGE 41.9; groups of 128, 128 x 1024 x
-        4096: FP6 37.8, skinny 12.7).  Kernels with a figure of the caller's
-        own (with_status) stay."""
+        its rows, and where an FP6 entry fits the smallest predicted time of
+        the entries with its operand alignment (kernel_table.predicted_us),
+        since on few tiles of 256 rows another one is faster (512 x 4096 x
+        4096: FP6 36.7 us, skinny 16.6; 512 x 16384 x 4096: FP6 47.4, FP6_EDGE
+        41.9; groups of 128, 128 x 1024 x 4096: FP6 37.8, skinny 12.7).
+        Kernels with a figure of the caller's own (with_status) stay."""
         desc = None if kernel.table_index is None else kt.TABLE[kernel.table_index]
         fp6 = desc is not None and desc.operand_format == kt.OPERANDS_FP6
         if not (fp6 or (desc is not None and desc.is_stream and not desc.plans_rows)):
             return kernel
-        if kernel.tile.split_k != 1 or kernel.measured_tops != kt.measured_tops(desc):
+        if kernel.tile.split_k != 1 or kernel.measured_tops != kt.measured_tops(desc):  # as _Candidate.table_figure
             return kernel
         chosen = kernel
         sub = kernel.scale.subchannel_size
@@ -272,7 +274,7 @@ class KernelRegistry:
                 if entry.plans_rows:
                     return other.kernel
                 continue
-            if best is None or not other.accepts(m, n, k):
+            if best is None or entry.operand_format == kt.OPERANDS_PACKED or not other.accepts(m, n, k):
                 continue
             us = kt.predicted_us(entry, m, n, k, sub)
             if us is not None and us < best:

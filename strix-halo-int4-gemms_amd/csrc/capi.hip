@@ -519,8 +519,8 @@ int amd_strix_halo_kernels_kernel_table_entry(int index, shk_kernel_desc* out) {
 
 namespace {
 
-// Predicted time (us) of a standard int4 call on the skinny tiles or an
-// FP6_EDGE entry, from fits to measured calls (kernel_table.predicted_us
+// Predicted time (us) of a standard int4 call on the skinny tiles, an FP6_EDGE
+// entry or the subchannel 64 x 64 tile, from fits to measured calls (kernel_table.predicted_us
 // states them); negative where there is none.  The skinny entries of a family
 // share the planned tiles' time: among them selection_area decides.
 constexpr long kPredictMaxK = 65536;
@@ -532,15 +532,26 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
   const long cols = swiglu ? 2 * n : n;
   const double convert = 6.0 + 2.5e-7 * (double)((m + cols) * k);
   if (d.scale_mode == SHK_SCALE_SUBCHANNEL) {
-    const int s = sub == 32 ? 0 : (sub == 64 ? 1 : (sub == 128 ? 2 : 3));
     if (d.operand_format == SHK_OPERANDS_STREAM) {
-      static constexpr double plain[4] = {2.78e-8, 1.38e-8, 0.95e-8, 0.73e-8};
-      static constexpr double gated[4] = {2.24e-8, 1.14e-8, 0.68e-8, 0.59e-8};
-      const double low = shk::sk_plan(4, sub, swiglu, m, n, k).rows == 16 ? 1.5 : 1.0;
       // of the heights, the 32-row tile ranks first, as measured (measured_score)
       const double rank = shk::sk_plans_rows(d) || d.block_m == 32 ? 1.0 : (d.block_m == 64 ? 1.001 : 1.002);
-      return 6.0 + rank * ((swiglu ? gated[s] : plain[s]) * low * (double)(m * cols * k) + 5e-6 * (double)(m * n));
+      return rank * shk::sk_plan(4, sub, swiglu, d.layout, m, n, k).us;
     }
+    if (d.operand_format == SHK_OPERANDS_PACKED) {
+      if (d.block_m != 64 || d.block_n != 64 || m <= 256) return -1.0;
+      static constexpr double fits[2][3][6] = {  // [SwiGLU][NN, NT, TN]
+          {{3.18, 9.2, 3.26, 2.83, 1.36, 0.9}, {2.93, 4.84, 3.42, 1.47, 1.31, 0.83}, {3.4, 12.61, 3.5, 4.53, 2.14, 1.09}},
+          {{2.87, 11.52, 5.56, 7.46, 3.23, 0.79},
+           {3.64, 7.13, 5.28, 1.63, 3.65, 1.59},
+           {3.4, 15.99, 5.23, 0.0, 5.86, 0.0}}};
+      const double u = (double)((m / 64) * (n / 64)), past = u > 256.0 ? u / 256.0 - 1.0 : 0.0;
+      const double w = (double)k / 1024.0, g = (double)k / (double)sub / 8.0;
+      const double x[6] = {1.0, w, g, w * past, g * past, past};
+      double us = 0.0;
+      for (int j = 0; j < 6; ++j) us += fits[swiglu][d.layout][j] * x[j];
+      return us;
+    }
+    const int s = sub == 32 ? 0 : (sub == 64 ? 1 : (sub == 128 ? 2 : 3));
     if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
     static constexpr double fixed[4] = {5.0, 5.0, 5.0, 3.5};
     static constexpr double per_k[4] = {0.0215, 0.0125, 0.0061, 0.0038};
@@ -551,7 +562,7 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
     if (whole == 0) rounds *= 0.8;
     return convert + (fixed[s] + per_k[s] * (double)k) * rounds;
   }
-  if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_plan(4, 0, swiglu, m, n, k).us;
+  if (d.operand_format == SHK_OPERANDS_STREAM) return shk::sk_plan(4, 0, swiglu, d.layout, m, n, k).us;
   if (d.operand_format != SHK_OPERANDS_FP6_EDGE) return -1.0;
   return convert + shk::f6_edge_plan(m, n, k, swiglu).us;
 }

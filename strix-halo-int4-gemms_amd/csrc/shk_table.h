@@ -334,74 +334,98 @@ inline bool sk_plans_rows(const shk_kernel_desc& d) {
   return d.operand_format == SHK_OPERANDS_STREAM && d.group_size_m > 1;
 }
 // The tile rows such an entry takes for a call of M rows: 16, 32 or 64,
-// masked to M.  A taller tile reads B fewer times and keeps the matrix cores
-// busier per byte; a lower one gives a small N more workgroups and computes
-// fewer rows that are not there.
+// masked to M (subchannel 16 or 32).  A taller tile reads B fewer times and
+// keeps the matrix cores busier per byte; a lower one gives a small N more
+// workgroups and computes fewer rows that are not there.
 //
-// Per-channel: the smallest predicted time (us) a + b * (K per workgroup /
-// 4096) * rounds of 256 workgroups, whole rounds for the SwiGLU tiles of 32
-// and 64 rows, which run one workgroup a CU, and with K split one more for
-// every 16 rows (up and gate) of partials; below K = 4096 a round keeps the
-// fraction f of the difference (a tile's prologue and epilogue), and `wide`
-// is what a SwiGLU call of 90 M values of B and more adds.  The figures are
-// fits to calls of M 32..1648 on N x K of 11008 x 4096, 8192^2, 4096^2, 1024
-// x 4096, 4096 x 512..2048 and 9728 x 704.  Measured, 16, 32 and 64 rows:
-// int8 SwiGLU 48 x 11008 x 4096 29.9, 32.5, 25.7 us, 400 rows 153, 124, 97;
-// int4 SwiGLU 112 rows 29.6, 33.7, 34.7, 1648 x 4864 x 704 66.8, 87.3, 73.3;
-// int4 plain 112 x 8192^2 27.7, 21.9, 17.7, 48 x 4096^2 7.0, 8.3, 10.5, 1024
-// x 4096 x 512 23.7, 17.0, 14.0.
-//
-// Subchannel (16 columns a tile, so many tiles): rounds of 512 workgroups, a
-// last one of up to half the chip for 0.73, a grid of one a CU for 1 / 1.37;
-// a round of 32-row tiles takes 1.45 of one of 16-row tiles, 1.15 where the
-// four waves' 16-row tile is bound by its B reads (SwiGLU, groups of a stage
-// and more).  Measured, 16 and 32 rows, groups of 128: 48 x 4096^2 19.9 and
-// 16.3 us, 400 rows 110 and 80, 64 x 1024 x 4096 9.0 and 13.0, 272 x 960 x
-// 3584 16.8 and 22.7, its SwiGLU 32.2 and 29.5; groups of 64, SwiGLU, 272 x
-// 960 x 3584 37.2 and 46.1.
+// The height of the smallest predicted time, but the tallest that divides M
+// where that is within 5%, the fits' own error: whole tiles need no mask and
+// a height that changes little is not worth a wrong guess.  The time (us) is
+// linear in what a launch of u workgroups, each with w = K / 4096 of its part
+// of K and g = K / 32 groups, takes on 256 CUs: one round, whether there is a
+// second, how many whole rounds of 256 and of 512 (two a CU), the workgroups
+// past the first 256, MN-major A and B (16-byte pieces of a row an
+// instruction), and the doublings of K's split.  Fitted to 4500 calls drawn
+// over M 16..8192, N 512..16384, K 512..14336 in all layouts and widths,
+// every height measured: median error 4%, a tenth above 11%.  Measured, 16,
+// 32 and 64 rows: int8 SwiGLU 48 x 11008 x 4096 NT 29.9, 32.5, 25.7 us; 288 x
+// 1088 x 4480 with A MN-major 28.8, 20.0 and 24.5; int4 SwiGLU 64 x 12224 x
+// 6208 31.6, 32.0, 25.4; int4 plain 112 x 8192^2 27.7, 21.9, 17.7; 32 x 10688
+// x 12224 22.7, 17.0.  16 and 32 rows, groups of 128: 400 x 4096^2 110 and 80
+// us, 48 x 16064 x 5120 NT 46.5 and 53.0.
 struct SkPlan {
   int rows;
   double us;
 };
+constexpr int kSkTerms = 9;      // constant, w, w rounds, w double rounds, w second, past, rounds, A MN, log2 splits
+constexpr int kSkSubTerms = 10;  // constant, w, g, w and g double rounds, w and g second, past, A MN, B MN
+// [8-bit][SwiGLU][16, 32, 64 rows]
+constexpr double kSkFit[2][2][3][kSkTerms] = {
+    {{{3.76, 2.96, 0.96, 3.11, 0.2, 0.77, 0.1, 1.39, 0.88},
+       {3.91, 4.12, 1.8, 2.72, 0.16, 0.54, 0.65, 1.07, 1.19},
+       {4.89, 5.84, 2.69, 3.29, 0.33, 1.19, 0.64, 0.1, 1.64}},
+      {{3.91, 5.25, 4.09, 1.05, 0.67, 0.92, 0.07, 1.09, 1.19},
+       {4.97, 6.96, 6.16, 0.83, 1.12, 0.51, 3.21, 0.32, 1.55},
+       {6.94, 9.81, 8.75, 0.0, 0.81, 0.14, 5.91, 1.36, 2.78}}},
+     {{{3.71, 3.68, 4.83, 0.45, 0.0, 0.41, 0.0, 3.55, 1.02},
+       {3.64, 5.78, 5.15, 2.5, 0.0, 0.55, 0.0, 3.24, 1.09},
+       {4.16, 8.21, 7.34, 4.93, 0.0, 0.77, 0.0, 2.21, 1.59}},
+      {{2.87, 10.23, 6.51, 4.32, 1.34, 0.51, 0.0, 3.5, 1.14},
+       {3.74, 11.02, 7.83, 4.71, 2.69, 0.0, 2.68, 3.73, 1.71},
+       {5.52, 14.08, 12.06, 1.6, 1.05, 0.14, 4.59, 2.99, 2.72}}}};
+// [8-bit][SwiGLU][groups of a stage or more][16, 32 rows]
+constexpr double kSkSubFit[2][2][2][2][kSkSubTerms] = {
+    {{{{3.5, 2.26, 3.42, 2.89, 3.49, 1.45, 0.15, 0.89, 0.44, 0.13},
+       {3.48, 0.06, 6.6, 0.44, 6.75, 1.04, 0.47, 0.98, 0.0, 0.05}},
+      {{3.63, 1.63, 1.64, 2.68, 1.95, 0.89, 0.77, 0.72, 1.53, 0.6},
+       {3.84, 4.06, 3.62, 4.79, 3.72, 1.07, 0.55, 1.02, 0.79, 0.37}}},
+     {{{3.84, 0.47, 6.04, 0.29, 6.52, 0.39, 0.71, 1.01, 0.96, 0.62},
+       {3.78, 0.14, 10.11, 0.68, 10.49, 0.0, 1.15, 1.06, 0.74, 0.64}},
+      {{4.0, 3.09, 4.1, 5.12, 3.22, 1.21, 0.64, 0.97, 2.21, 1.16},
+       {3.86, 4.44, 6.46, 6.36, 5.75, 2.24, 0.0, 1.03, 1.13, 0.8}}}},
+    {{{{3.59, 0.0, 3.86, 0.0, 4.24, 0.0, 0.56, 0.91, 1.52, 0.59},
+       {3.41, 0.0, 5.68, 0.0, 6.02, 0.0, 0.84, 0.94, 1.15, 0.48}},
+      {{3.42, 2.59, 1.44, 4.91, 1.73, 1.86, 0.55, 0.57, 4.23, 1.94},
+       {3.84, 5.39, 3.26, 9.06, 2.89, 2.21, 0.0, 0.84, 2.47, 1.64}}},
+     {{{3.86, 0.0, 5.44, 0.0, 5.84, 0.0, 0.82, 1.02, 2.57, 0.75},
+       {3.38, 0.0, 9.69, 0.0, 10.3, 0.0, 1.15, 0.91, 3.97, 1.54}},
+      {{3.9, 4.15, 2.68, 9.52, 1.89, 2.21, 1.68, 0.63, 6.05, 4.11},
+       {3.31, 6.32, 6.61, 11.59, 3.82, 2.14, 0.0, 0.74, 5.02, 3.92}}}}};
 // `sub`: the group size, or 0 for per-channel scales.
-inline SkPlan sk_plan(int bits, int sub, bool swiglu, long m, long n, long k) {
-  if (sub > 0) {
-    auto load = [&](long rows) {
-      const long t = ((m + rows - 1) / rows) * (n / 16), rest = t % 512;
-      return t <= 256 ? 1.0 : 1.37 * ((double)(t / 512) + (rest == 0 ? 0.0 : (rest <= 256 ? 0.73 : 1.0)));
-    };
-    const double tall = swiglu && sub >= (bits == 4 ? 128 : 64) ? 1.15 : 1.45;
-    return SkPlan{m <= 16 || load(16) <= tall * load(32) ? 16 : 32, 0.0};
-  }
-  struct Fit {
-    double a, wide, b, f;
-    bool whole;
-  };
-  static constexpr Fit fits[2][2][3] = {
-      {{{3.6, 0.0, 3.38, 0.27, false}, {3.4, 0.0, 4.8, 0.25, false}, {4.8, 0.0, 6.07, 0.3, false}},
-       {{4.0, 3.0, 4.6, 0.35, false}, {5.5, 0.0, 10.5, 0.37, true}, {7.5, 0.0, 15.5, 0.45, true}}},
-      {{{3.8, 0.0, 5.2, 0.12, false}, {4.2, 0.0, 6.45, 0.13, false}, {4.5, 0.0, 8.0, 0.2, false}},
-       {{3.2, 12.1, 7.7, 0.05, false}, {3.0, 9.0, 12.5, 0.2, true}, {3.0, 9.0, 15.0, 0.33, true}}}};
-  const double wide = std::min(1.0, 2.0 * (double)n * (double)k / 9e7), k4 = (double)k / 4096.0;
-  SkPlan best{16, -1.0};
-  for (int i = 0; i < 3; ++i) {
+inline SkPlan sk_plan(int bits, int sub, bool swiglu, int layout, long m, long n, long k) {
+  const double a_mn = layout == SHK_LAYOUT_TN ? 1.0 : 0.0, b_mn = layout == SHK_LAYOUT_NN ? 1.0 : 0.0;
+  SkPlan best{16, -1.0}, whole{16, -1.0};
+  for (int i = 0; i < (sub > 0 ? 2 : 3); ++i) {
     const int rows = 16 << i;
     if (i > 0 && m <= rows / 2) break;
-    const Fit& f = fits[bits == 8][swiglu][i];
-    const long tiles = ((m + rows - 1) / rows) * (n / 64);
-    const int s = sk_splits(bits, tiles, k);
-    const long units = tiles * s;
-    const double rounds = units <= 256 ? 1.0 : (f.whole ? (double)((units + 255) / 256) : (double)units / 256.0);
-    const double us = f.a + f.wide * wide + (s > 1 ? (double)(rows / 16 * (swiglu ? 2 : 1)) : 0.0) +
-                      f.b * (k4 / (double)s * rounds + f.f * std::max(0.0, 1.0 - k4) * (rounds - 1.0));
+    const long tiles = (m + rows - 1) / rows * (sub > 0 ? n / 16 : n / 64);
+    const int s = sub > 0 ? 1 : sk_splits(bits, tiles, k);
+    const double u = (double)(tiles * s), w = (double)k / (double)s / 4096.0;
+    const bool second = tiles * s > 256;
+    const double past = second ? u / 256.0 - 1.0 : 0.0, wm = w * (1.0 + past), w2 = second ? w : 0.0;
+    const double twice = (double)((tiles * s - 1) / 512);  // double rounds past the first
+    double us = 0.0;
+    if (sub > 0) {
+      const double g = (double)k / (double)sub / 32.0;
+      const double x[kSkSubTerms] = {1.0, w, g, w * twice, g * twice, w2, second ? g : 0.0, past, wm * a_mn, wm * b_mn};
+      const double* f = kSkSubFit[bits == 8][swiglu][sub >= (bits == 4 ? 128 : 64)][i];
+      for (int j = 0; j < kSkSubTerms; ++j) us += f[j] * x[j];
+    } else {
+      int halvings = 0;
+      while ((1 << halvings) < s) ++halvings;
+      const double rounds = (double)((tiles * s - 1) / 256);
+      const double x[kSkTerms] = {1.0, w, w * rounds, w * twice, w2, past, rounds, wm * a_mn, (double)halvings};
+      for (int j = 0; j < kSkTerms; ++j) us += kSkFit[bits == 8][swiglu][i][j] * x[j];
+    }
     if (best.us < 0.0 || us < best.us) best = SkPlan{rows, us};
+    if (m % rows == 0) whole = SkPlan{rows, us};
   }
-  return best;
+  return whole.us <= 1.05 * best.us ? whole : best;
 }
 // Rows of a table entry's tiles.
 inline int sk_tile_rows(const shk_kernel_desc& d, long m, long n, long k, int sub) {
   if (!sk_plans_rows(d)) return d.block_m;
-  return sk_plan(d.dtype_bits, sub, d.epilogue_kind == SHK_EPI_KIND_SWIGLU, m, n, k).rows;
+  return sk_plan(d.dtype_bits, sub, d.epilogue_kind == SHK_EPI_KIND_SWIGLU, d.layout, m, n, k).rows;
 }
 // A skinny call: its tile rows, the workgroups sharing a tile's K (subchannel
 // tiles always one), and with more than one split its workspace: the tiles' arrival counters, padded

@@ -55,9 +55,25 @@ def test_selection_by_predicted_time_matches_the_library(sub, epilogue):
         formats.add(d.operand_format)
         us = kt.predicted_us(d, m, n, k, sub)
         if us is not None:
-            assert us <= min(t for e in fitting if e.scale_mode == d.scale_mode and (t := kt.predicted_us(e, m, n, k, sub)) is not None)
+            picked_fp6 = kt.TABLE[got].operand_format == kt.OPERANDS_FP6  # such a call keeps to 16-byte operands
+            assert us <= min(t for e in fitting if e.scale_mode == d.scale_mode
+                             and not (picked_fp6 and e.operand_format == kt.OPERANDS_PACKED)
+                             and (t := kt.predicted_us(e, m, n, k, sub)) is not None)
     if not sub or epilogue == "none":
-        assert formats == {kt.OPERANDS_STREAM, kt.OPERANDS_FP6, kt.OPERANDS_FP6_EDGE}
+        assert formats - {kt.OPERANDS_PACKED} == {kt.OPERANDS_STREAM, kt.OPERANDS_FP6, kt.OPERANDS_FP6_EDGE}
+        assert sub or kt.OPERANDS_PACKED not in formats
+
+
+@pytest.mark.parametrize("m,n,k,sub,layout,fmt", [
+    (1536, 704, 768, 64, "nt", kt.OPERANDS_PACKED),  # 12.4 us; edge 18.1, skinny 24.6
+    (1216, 896, 640, 128, "nt", kt.OPERANDS_PACKED),  # 9.0; 12.7, 17.4
+    (320, 5952, 1728, 32, "nt", kt.OPERANDS_PACKED),  # 39.3; 53.6, 110
+    (1344, 5952, 4096, 128, "nn", kt.OPERANDS_FP6_EDGE), (256, 704, 768, 64, "nt", kt.OPERANDS_STREAM),
+])
+def test_the_64_row_subchannel_tile_runs_where_it_is_fastest(m, n, k, sub, layout, fmt):
+    kern = shk.default_registry.select_call(dtype=shk.OperandDType.INT4, scale=spec_of(sub), epilogue=shk.Epilogue.NONE,
+                                            m=m, n=n, k=k, layout=shk.GemmLayout(layout))
+    assert kt.TABLE[kern.table_index].operand_format == fmt
 
 
 def test_edge_entries_bound_k():

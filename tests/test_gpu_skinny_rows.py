@@ -5,6 +5,8 @@ K is left zero."""
 
 from __future__ import annotations
 
+import itertools
+
 import numpy as np
 import pytest
 
@@ -22,7 +24,7 @@ from amd_strix_halo_kernels import native  # noqa: E402
 
 def _check(bits, layout, epilogue, sub, m, n, k, device, rows, splits=None):
     swiglu = epilogue == "swiglu"
-    assert kt.sk_plan(bits, sub, swiglu, m, n, k)[0] == rows
+    assert kt.sk_plan(bits, sub, swiglu, m, n, k, kt.LAYOUT_CODES[layout])[0] == rows
     a_q, b_q, a_arg, b_arg, sa, sb = dense_case(stable_seed("rows", bits, layout, epilogue, sub, m, n, k), bits=bits,
                                                 layout=layout, m=m, n=n, k=k, subchannel=sub or None, swiglu=swiglu)
     a, b, ta, tb = (to_dev(torch, x, device) for x in (a_arg, b_arg, sa, sb))
@@ -46,31 +48,43 @@ def _check(bits, layout, epilogue, sub, m, n, k, device, rows, splits=None):
     assert max_ulp(got, want) <= 2 if swiglu else np.array_equal(got, want)
 
 
-# (bits, epilogue, rows, m, n, k): masked and whole tiles of each height,
-# with and without K split over workgroups
-_PLANS = [
-    (4, "none", 64, 112, 8192, 2080), (4, "none", 64, 192, 8192, 2080), (4, "none", 32, 48, 512, 96),
-    (4, "none", 32, 144, 512, 8192), (8, "none", 64, 112, 8192, 1024), (8, "none", 32, 144, 512, 8192),
-    (8, "none", 32, 112, 4096, 96), (8, "none", 64, 272, 512, 8192), (4, "swiglu", 64, 112, 8192, 96),
-    (4, "swiglu", 16, 48, 512, 2080), (8, "swiglu", 64, 272, 2048, 96), (8, "swiglu", 64, 272, 512, 8192),
-    (8, "swiglu", 32, 48, 512, 96), (8, "swiglu", 32, 48, 2048, 8192),
-]
+def _shape(bits, sub, swiglu, layout, rows, masked, split, groups=None):
+    """The least work whose plan is tiles of `rows` rows, masked or whole, with
+    or without K split over workgroups."""
+    code = kt.LAYOUT_CODES[layout]
+    ks = [groups * sub + (32 if groups * sub % 64 else 0)] if sub else [96, 160, 544, 1056, 2080, 4128, 8192, 13632]
+    shapes = sorted(itertools.product(range(16, 305, 16), (64, 192, 512, 1024, 2048, 3072, 4096, 8192), ks),
+                    key=lambda s: s[0] * s[1] * s[2])
+    for m, n, k in shapes:
+        if bool(m % rows) != masked or kt.sk_plan(bits, sub, swiglu, m, n, k, code)[0] != rows:
+            continue
+        if sub or (kt._sk_splits(bits, -(-m // rows) * (n // 64), k) > 1) == split:
+            return m, n, k
+    raise LookupError
 
 
+# every height masked and whole, with K split where a plan of the height splits it
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
-@pytest.mark.parametrize("bits,epilogue,rows,m,n,k", _PLANS)
-def test_every_height_matches_the_oracle(bits, epilogue, rows, m, n, k, layout, device):
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+@pytest.mark.parametrize("rows,masked,split", [(16, False, False), (16, False, True), (32, True, False), (32, False, False),
+                                               (32, True, True), (64, True, False), (64, False, False), (64, True, True)])
+def test_every_height_matches_the_oracle(bits, epilogue, rows, masked, split, layout, device):
+    m, n, k = _shape(bits, 0, epilogue == "swiglu", layout, rows, masked, split)
     _check(bits, layout, epilogue, 0, m, n, k, device, rows)
 
 
+# one to three groups, and more than the waves of a tile take in one round (16
+# rows 8 or 16 groups, 32 rows 8, SwiGLU 4): the totals carry over in group order
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("sub", [32, 64, 128, 256])
-@pytest.mark.parametrize("epilogue,m,rows", [("none", 48, 32), ("none", 64, 32), ("swiglu", 48, 32), ("none", 32, 16)])
-def test_subchannel_32_row_tiles_match_the_oracle(bits, sub, epilogue, m, rows, layout, device):
-    """32-row tiles where they make fewer rounds of workgroups (N = 4096)."""
-    _check(bits, layout, epilogue, sub, m, 4096 if rows == 32 else 192, (2 if sub > 64 else 5) * sub // 64 * 64 or 64,
-           device, rows)
+@pytest.mark.parametrize("epilogue,rows,masked,groups", [("none", 16, False, 2), ("none", 32, True, 2), ("none", 32, True, 9),
+                                                         ("none", 32, False, 37), ("swiglu", 32, True, 37),
+                                                         ("swiglu", 32, False, 9)])
+def test_subchannel_heights_match_the_oracle(bits, sub, epilogue, rows, masked, groups, layout, device):
+    m, n, k = _shape(bits, sub, epilogue == "swiglu", layout, rows, masked, False, groups)
+    _check(bits, layout, epilogue, sub, m, n, k, device, rows)
 
 
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
@@ -78,14 +92,3 @@ def test_subchannel_32_row_tiles_match_the_oracle(bits, sub, epilogue, m, rows, 
 def test_int4_64_row_tiles_with_k_split(m, n, k, layout, device):
     """64-row tiles, whole and masked, of which two workgroups share the K."""
     _check(4, layout, "none", 0, m, n, k, device, 64, splits=2)
-
-
-@pytest.mark.parametrize("layout", ["nn", "nt"])
-@pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("sub", [32, 64, 128, 256])
-@pytest.mark.parametrize("epilogue,m,groups", [("none", 48, 9), ("none", 64, 37), ("swiglu", 48, 37), ("swiglu", 64, 9)])
-def test_subchannel_32_row_tiles_over_several_rounds(bits, sub, epilogue, m, groups, layout, device):
-    """More scale groups than the waves of a 32-row tile take in one round (8,
-    SwiGLU 4): the totals carry over, in group order."""
-    k = -(-groups * sub // 64) * 64
-    _check(bits, layout, epilogue, sub, m, 3072, k, device, 32)

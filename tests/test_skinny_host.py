@@ -189,7 +189,7 @@ def test_entries_of_one_height_run_it():
         for m, n, k in shapes:
             rows = d.block_m
             if d.plans_rows:
-                rows = kt.sk_plan(d.dtype_bits, 0, cols == 2, m, n, k)[0]
+                rows = kt.sk_plan(d.dtype_bits, 0, cols == 2, m, n, k, d.layout)[0]
                 planned += rows != 16
             tiles = -(-m // rows) * (n // 64)
             splits = kt.sk_split_count(d, m, n, k)
