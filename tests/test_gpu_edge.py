@@ -4,7 +4,8 @@ same operands without converting them.
 
 int32 sums are whole numbers and equal; per-channel bf16 results scale the
 same integers in the same order and equal bit for bit; SwiGLU goes through
-exp and stays within 2 bf16 ulp."""
+exp and stays within 2 bf16 ulp of the oracle, and equals the skinny tiles',
+which take the same expf and division."""
 
 from __future__ import annotations
 
@@ -130,6 +131,33 @@ def test_every_tile_split_equals_the_skinny_tiles(epilogue, m, n, k, device):
     assert torch.equal(raws[0], raws[1])
     got, want = (bf16_bits(torch, o) for o in outs)
     assert max_ulp(got, want) <= 2 if epilogue == "swiglu" else np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("mode", [kt.OUT_BF16, kt.OUT_F32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("sub", [None, 32, 64, 128, 256])
+def test_swiglu_equals_the_skinny_tiles_bit_for_bit(sub, mode, device):
+    """Edge and skinny tiles share shapes, so a call must not lose precision by
+    which of them it runs: the same scaled sums through the same expf and
+    division, for gates of both signs up to some hundred."""
+    m, n, k = 208, 192, 768
+    case = dense_case(stable_seed("edge-swiglu", sub, mode), bits=4, layout="nn", m=m, n=n, k=k, subchannel=sub,
+                      swiglu=True, scale_lo=0.02, scale_hi=0.2)
+    a, b, sa, sb = _operands(case, device)
+    lib = native.load_dispatch_library()
+    outs = []
+    for fmt in (kt.OPERANDS_FP6_EDGE, kt.OPERANDS_STREAM):
+        kernel = _kernel(fmt, "nn", "swiglu", sub, m)
+        out = torch.zeros((m, n), dtype=torch.bfloat16 if mode == kt.OUT_BF16 else torch.float32, device=device)
+        nbytes = native.gemm_workspace_bytes(kernel, m, n, k)
+        work = torch.zeros(max(nbytes, 16), dtype=torch.uint8, device=device)
+        rc = lib.amd_strix_halo_kernels_launch_gemm_ws(
+            kernel.table_index, 0, torch.cuda.current_stream().cuda_stream, a.data_ptr(), b.data_ptr(), sa.data_ptr(),
+            sb.data_ptr(), out.data_ptr(), m, n, k, sub or 0, kt.EPILOGUE_SWIGLU, mode, work.data_ptr(), nbytes)
+        torch.cuda.synchronize()
+        assert rc == 0, lib.amd_strix_halo_kernels_last_error()
+        outs.append(out)
+    assert float(outs[0].float().abs().max()) > 100.0
+    assert torch.equal(outs[0], outs[1])
 
 
 @pytest.mark.parametrize("epilogue", ["none", "swiglu"])
