@@ -216,6 +216,19 @@ int amd_strix_halo_kernels_launch_gemm(int kernel_index, int device_index, uintp
                                        int32_t k, int32_t subchannel, int32_t epilogue,
                                        int32_t out_mode);
 
+/* The entry that amd_strix_halo_kernels_launch_gemm_ws runs for these
+ * arguments (workspace: null or not), written to *index; nothing is launched.
+ * It is kernel_index itself but for FP6_EDGE entries and STREAM entries that
+ * plan their rows: the former give way to an entry that needs no workspace
+ * where there is none, and both, where a or b is not 16-byte aligned, to the
+ * PACKED entry that serves the shape if that is the one
+ * amd_strix_halo_kernels_select_dense would pick without them (its MN-major
+ * operands need 8 bytes).  Returns 0, or 1 for a bad index.  No counterpart in
+ * the reference. */
+int amd_strix_halo_kernels_launched_entry(int kernel_index, const void* a, const void* b, int32_t m, int32_t n,
+                                          int32_t k, int32_t subchannel, int32_t epilogue, const void* workspace,
+                                          int32_t* index);
+
 /* Workspace bytes a dense entry needs for shape (m, n, k) (0 for PACKED
  * entries), written to *bytes.  Returns 0, or 1 for a bad index or shape.
  * No counterpart in the reference, whose gfx1151 kernels read int4 operands

@@ -81,6 +81,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.amd_strix_halo_kernels_select_dense.restype = I
     lib.amd_strix_halo_kernels_launch_gemm.argtypes = [I, I, U, P, P, P, P, P, I32, I32, I32, I32, I32, I32]
     lib.amd_strix_halo_kernels_launch_gemm.restype = I
+    lib.amd_strix_halo_kernels_launched_entry.argtypes = [I, P, P, I32, I32, I32, I32, I32, P, ctypes.POINTER(I32)]
+    lib.amd_strix_halo_kernels_launched_entry.restype = I
     lib.amd_strix_halo_kernels_gemm_workspace_bytes.argtypes = [I, I32, I32, I32, ctypes.POINTER(ctypes.c_uint64)]
     lib.amd_strix_halo_kernels_gemm_workspace_bytes.restype = I
     lib.amd_strix_halo_kernels_launch_gemm_ws.argtypes = [I, I, U, P, P, P, P, P, I32, I32, I32, I32, I32, I32, P,

@@ -568,18 +568,9 @@ double predicted_us(const shk_kernel_desc& d, long m, long n, long k, int sub) {
 }
 
 // Throughput measured on MI355X for the entries the benchmark configurations
-// time (the Python registry's kernel_table.selection_tops): the first
-// ranking key of a selection, before the tile area.  Int4 skinny
-// and FP6_EDGE entries rank by their predicted throughput for the shape,
-// below the FP6 entries where those accept it (a caller of the separate
-// conversion needs an FP6 entry).
-double measured_score(const shk_kernel_desc& d, int m, int n, int k, int subchannel) {
-  if (d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1) return 0.0;
-  const double us = predicted_us(d, m, n, k, subchannel);
-  if (us > 0.0)
-    return std::min(d.scale_mode == SHK_SCALE_SUBCHANNEL ? 2000.0 : 3000.0,
-                    2.0 * (double)m * (double)n * (double)k / us / 1e6);
-  if (d.operand_format == SHK_OPERANDS_FP6_EDGE) return 0.0;
+// time (kernel_table.measured_tops).
+double measured_figure(const shk_kernel_desc& d, int m) {
+  if (d.schedule != SHK_SCHEDULE_STANDARD || d.split_k > 1 || d.operand_format == SHK_OPERANDS_FP6_EDGE) return 0.0;
   if (d.operand_format == SHK_OPERANDS_FP6) {
     if (d.scale_mode == SHK_SCALE_SUBCHANNEL) return 2001.0;
     return d.epilogue_kind == SHK_EPI_KIND_PLAIN ? 3504.0 : 3161.0;
@@ -593,6 +584,18 @@ double measured_score(const shk_kernel_desc& d, int m, int n, int k, int subchan
   if (d.dtype_bits == 8 && d.num_stages == 4 && d.block_m == 256)
     return d.epilogue_kind == SHK_EPI_KIND_SWIGLU ? 2014.0 : 2270.0;
   return 0.0;
+}
+
+// The first ranking key of a selection (kernel_table.selection_tops), before
+// the tile area: int4 entries with a predicted time for the shape rank by it,
+// below the FP6 entries where those accept it (a caller of the separate
+// conversion needs an FP6 entry), the others by their figure.
+double measured_score(const shk_kernel_desc& d, int m, int n, int k, int subchannel) {
+  const double us = predicted_us(d, m, n, k, subchannel);
+  if (us > 0.0)
+    return std::min(d.scale_mode == SHK_SCALE_SUBCHANNEL ? 2000.0 : 3000.0,
+                    2.0 * (double)m * (double)n * (double)k / us / 1e6);
+  return measured_figure(d, m);
 }
 
 // The second ranking key, a tile's area.  A skinny entry that plans its rows
@@ -633,10 +636,16 @@ bool accepts_shape(const shk_kernel_desc& d, int m, int n, int k, int subchannel
   return k <= dense_max_k(d);
 }
 
-// The best entry that serves a request and its shape, or -1; `direct`: of
-// those that read the packed operands (no converted workspace).
+// Which entries best_entry considers.
+enum Among {
+  ALL,
+  DIRECT,   // those that read the packed operands (no converted workspace)
+  FIGURES,  // as before entries had predicted times: no FP6_EDGE ones, no planned rows, ranked by their figures
+};
+
+// The best entry that serves a request and its shape, or -1.
 int best_entry(int bits, int layout, int subchannel, int epilogue, int schedule, int split_k, int m, int n, int k,
-               bool direct) {
+               Among among) {
   const auto& t = table();
   int best = -1;
   double best_score = -1.0;
@@ -645,8 +654,10 @@ int best_entry(int bits, int layout, int subchannel, int epilogue, int schedule,
     const shk_kernel_desc& d = t[i].d;
     if (!serves_family(d, bits, layout, subchannel, epilogue, schedule, split_k)) continue;
     if (!accepts_shape(d, m, n, k, subchannel)) continue;
-    if (direct && d.operand_format != SHK_OPERANDS_PACKED && d.operand_format != SHK_OPERANDS_STREAM) continue;
-    const double score = measured_score(d, m, n, k, subchannel);
+    const bool edge = d.operand_format == SHK_OPERANDS_FP6_EDGE;
+    if (among == DIRECT && (edge || d.operand_format == SHK_OPERANDS_FP6)) continue;
+    if (among == FIGURES && (edge || shk::sk_plans_rows(d))) continue;
+    const double score = among == FIGURES ? measured_figure(d, m) : measured_score(d, m, n, k, subchannel);
     const long area = selection_area(d, m);
     if (score > best_score || (score == best_score && area > best_area)) {
       best = i;
@@ -657,22 +668,31 @@ int best_entry(int bits, int layout, int subchannel, int epilogue, int schedule,
   return best;
 }
 
-// The entry a launch runs.  An FP6_EDGE entry without room for its converted
-// operands (`room` bytes) gives way to the best entry of its family that
-// reads the packed operands, so a caller that has no workspace is served as
-// without the FP6_EDGE entries.  Requests that the entry itself refuses keep
+// The entry a launch runs.  Two kinds of entries give way to another of their
+// family, so that what a call may bring does not depend on which entry is
+// predicted fastest for its shape; requests that the entry itself refuses keep
 // it, for its error.
-int runnable_entry(int kernel_index, int m, int n, int k, int subchannel, int epilogue, uint64_t room) {
+//  * An FP6_EDGE entry without room for its converted operands (`room` bytes)
+//    to the best entry that reads the packed operands.
+//  * An FP6_EDGE entry or a skinny one that plans its rows, whose operands are
+//    not both 16-byte aligned, to the entry that the figures alone rank first,
+//    if that is a PACKED one: its MN-major operands need 8 bytes.
+int runnable_entry(int kernel_index, const void* a, const void* b, int m, int n, int k, int subchannel, int epilogue,
+                   uint64_t room) {
   const auto& t = table();
   if (kernel_index < 0 || kernel_index >= (int)t.size()) return kernel_index;
   const shk_kernel_desc& d = t[kernel_index].d;
-  if (d.operand_format != SHK_OPERANDS_FP6_EDGE || m <= 0 || n <= 0 || k <= 0) return kernel_index;
-  if (dense_workspace_bytes(d, m, n, k) <= room) return kernel_index;
+  const bool edge = d.operand_format == SHK_OPERANDS_FP6_EDGE;
+  if ((!edge && !shk::sk_plans_rows(d)) || m <= 0 || n <= 0 || k <= 0) return kernel_index;
+  const bool fits = !edge || dense_workspace_bytes(d, m, n, k) <= room, whole = aligned(a, 16) && aligned(b, 16);
+  if (fits && whole) return kernel_index;
   if (!serves_family(d, d.dtype_bits, d.layout, subchannel, epilogue, d.schedule, 0) ||
       !accepts_shape(d, m, n, k, subchannel))
     return kernel_index;
-  const int other = best_entry(d.dtype_bits, d.layout, subchannel, epilogue, d.schedule, 1, m, n, k, true);
-  return other < 0 ? kernel_index : other;
+  const int other = best_entry(d.dtype_bits, d.layout, subchannel, epilogue, d.schedule, 1, m, n, k,
+                               whole ? DIRECT : FIGURES);
+  if (other < 0 || (!whole && t[other].d.operand_format != SHK_OPERANDS_PACKED)) return kernel_index;
+  return other;
 }
 
 }  // namespace
@@ -693,7 +713,7 @@ int amd_strix_halo_kernels_select_dense(int32_t dtype_bits, int32_t layout, int3
   if (m <= 0 || n <= 0 || k <= 0)
     return fail("M, N, and K must be positive; got (" + std::to_string(m) + ", " + std::to_string(n) + ", " +
                 std::to_string(k) + ")");
-  const int best = best_entry(dtype_bits, layout, subchannel, epilogue, schedule, split_k, m, n, k, false);
+  const int best = best_entry(dtype_bits, layout, subchannel, epilogue, schedule, split_k, m, n, k, ALL);
   if (best < 0)
     return fail("no kernel for dtype_bits=" + std::to_string(dtype_bits) + ", subchannel=" +
                 std::to_string(subchannel) + ", epilogue=" + std::to_string(epilogue) + ", layout=" +
@@ -715,6 +735,16 @@ int amd_strix_halo_kernels_gemm_workspace_bytes(int kernel_index, int32_t m, int
   return 0;
 }
 
+int amd_strix_halo_kernels_launched_entry(int kernel_index, const void* a, const void* b, int32_t m, int32_t n, int32_t k,
+                                          int32_t subchannel, int32_t epilogue, const void* workspace,
+                                          int32_t* index) {
+  g_last_error.clear();
+  if (index == nullptr) return fail("index must be non-null");
+  if (kernel_index < 0 || kernel_index >= (int)table().size()) return fail("kernel index out of range");
+  *index = runnable_entry(kernel_index, a, b, m, n, k, subchannel, epilogue, workspace ? UINT64_MAX : 0);
+  return 0;
+}
+
 int amd_strix_halo_kernels_launch_gemm(int kernel_index, int device_index, uintptr_t stream, const void* a,
                                        const void* b, const void* a_scale, const void* b_scale, void* out,
                                        int32_t m, int32_t n, int32_t k, int32_t subchannel, int32_t epilogue,
@@ -729,7 +759,7 @@ int amd_strix_halo_kernels_launch_gemm_ws(int kernel_index, int device_index, ui
                                           int32_t out_mode, void* workspace, uint64_t workspace_bytes) {
   g_last_error.clear();
   DenseCall c;
-  if (workspace == nullptr) kernel_index = runnable_entry(kernel_index, m, n, k, subchannel, epilogue, 0);
+  kernel_index = runnable_entry(kernel_index, a, b, m, n, k, subchannel, epilogue, workspace ? UINT64_MAX : 0);
   if (prepare_dense(c, kernel_index, PHASE_ALL, a, b, a_scale, b_scale, out, m, n, k, subchannel, epilogue,
                     out_mode, workspace, workspace_bytes))
     return 1;
@@ -747,7 +777,7 @@ int amd_strix_halo_kernels_launch_gemm_noalloc(int kernel_index, int device_inde
                                                int32_t epilogue, int32_t out_mode) {
   g_last_error.clear();
   DenseCall c;
-  kernel_index = runnable_entry(kernel_index, m, n, k, subchannel, epilogue, SHK_NOALLOC_SCRATCH_BYTES);
+  kernel_index = runnable_entry(kernel_index, a, b, m, n, k, subchannel, epilogue, SHK_NOALLOC_SCRATCH_BYTES);
   if (prepare_dense(c, kernel_index, PHASE_ALL, a, b, a_scale, b_scale, out, m, n, k, subchannel, epilogue,
                     out_mode, kScratchPending, SHK_NOALLOC_SCRATCH_BYTES))
     return 1;

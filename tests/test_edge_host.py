@@ -76,6 +76,41 @@ def test_the_64_row_subchannel_tile_runs_where_it_is_fastest(m, n, k, sub, layou
     assert kt.TABLE[kern.table_index].operand_format == fmt
 
 
+def _launched(index, m, n, k, sub, epilogue=kt.EPILOGUE_NONE, a=1 << 20, b=1 << 20, workspace=1 << 20):
+    lib = native.load_dispatch_library()
+    out = ctypes.c_int32(-1)
+    assert lib.amd_strix_halo_kernels_launched_entry(index, a, b, m, n, k, sub, epilogue, workspace, ctypes.byref(out)) == 0
+    return out.value
+
+
+@pytest.mark.parametrize("epilogue", ["none", "swiglu"])
+@pytest.mark.parametrize("sub", [0, 32, 128])
+def test_operands_at_8_bytes_run_where_the_64_row_tile_does(sub, epilogue):
+    """Shapes that the 64 x 64 tile serves by its figures (subchannel, past 256
+    rows, no fp6 tile) take MN-major operands at 8 bytes, as that tile does,
+    whichever entry is predicted fastest for them; the others refuse them."""
+    reg = shk.default_registry
+    epi = {"none": kt.EPILOGUE_NONE, "swiglu": kt.EPILOGUE_SWIGLU}[epilogue]
+    served = 0
+    for m, n, k in itertools.product((64, 256, 320, 512, 576, 1008, 4160), (64, 192, 1024, 16384), (128, 576, 4096)):
+        if sub and k % sub:
+            continue
+        kern = reg.select_call(dtype=shk.OperandDType.INT4, scale=spec_of(sub), epilogue=shk.Epilogue(epilogue), m=m,
+                               n=n, k=k)
+        index = kern.table_index
+        assert _launched(index, m, n, k, sub, epi) == index
+        fp6 = epilogue == "none" and m % 128 == 0 and n % 128 == 0 and k % 128 == 0
+        if kt.TABLE[index].operand_format == kt.OPERANDS_FP6 or fp6:
+            continue
+        for a, b in (((1 << 20) + 8, 1 << 20), (1 << 20, (1 << 20) + 8)):
+            got = kt.TABLE[_launched(index, m, n, k, sub, epi, a, b)]
+            packed = sub and m > 256 and m % 64 == 0 and k % 64 == 0
+            assert (got.operand_format == kt.OPERANDS_PACKED) == bool(packed), (m, n, k, got)
+            assert m % got.block_m == 0 and n % got.block_n == 0 and k % got.block_k == 0
+            served += bool(packed)
+    assert bool(served) == bool(sub)
+
+
 def test_edge_entries_bound_k():
     for d in EDGES:
         assert d.max_k == kt.FP6_MAX_K and not d.supports_k(kt.FP6_MAX_K + 64)

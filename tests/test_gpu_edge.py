@@ -133,6 +133,33 @@ def test_every_tile_split_equals_the_skinny_tiles(epilogue, m, n, k, device):
     assert max_ulp(got, want) <= 2 if epilogue == "swiglu" else np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("layout", ["nn", "tn"])
+@pytest.mark.parametrize("m,n,k,sub", [(320, 1024, 640, 128), (1344, 192, 576, 64), (320, 64, 256, 32)])
+def test_calls_with_operands_at_8_bytes(m, n, k, sub, layout, device):
+    """An MN-major operand that starts 8 bytes past a 16-byte boundary, as a
+    view into a larger buffer may: the 64 x 64 tile's calls take it, with the
+    bits of the aligned call."""
+    case = dense_case(stable_seed("edge-8", m, n, k, layout), bits=4, layout=layout, m=m, n=n, k=k, subchannel=sub,
+                      swiglu=False)
+    a, b, sa, sb = _operands(case, device)
+
+    def moved(t):
+        buf = torch.empty(t.numel() + 16, dtype=t.dtype, device=device)
+        view = buf[8:8 + t.numel()].view(t.shape)
+        view.copy_(t)
+        assert view.data_ptr() % 16 == 8
+        return view
+
+    kw = dict(a_scale=sa, b_scale=sb, layout=shk.GemmLayout(layout), scale=spec_of(sub))
+    want = shk.mm(a, b, **kw)
+    assert torch.equal(shk.mm(a, moved(b), **kw), want)
+    if layout == "tn":
+        assert torch.equal(shk.mm(moved(a), moved(b), **kw), want)
+    else:
+        with pytest.raises(RuntimeError, match="16-byte aligned A"):
+            shk.mm(moved(a), b, **kw)
+
+
 @pytest.mark.parametrize("mode", [kt.OUT_BF16, kt.OUT_F32], ids=["bf16", "f32"])
 @pytest.mark.parametrize("sub", [None, 32, 64, 128, 256])
 def test_swiglu_equals_the_skinny_tiles_bit_for_bit(sub, mode, device):
