@@ -78,7 +78,9 @@ extern "C" {
 #define SHK_OPERANDS_PACKED 0
 #define SHK_OPERANDS_FP6 1
 /* STREAM entries (block_m 16, 32, 64; block_k 32) read the packed operands
- * straight from HBM like PACKED ones.  Per-channel calls may split a tile's
+ * straight from HBM like PACKED ones.  Those with group_size_m above 1 pick
+ * their tiles' height for each call, up to that many 16-row blocks, and mask
+ * the rows past M (M a multiple of 16); the others' tiles are block_m rows.  Per-channel calls may split a tile's
  * K over several workgroups that add exact int32 partials; they do so only
  * with a workspace of amd_strix_halo_kernels_gemm_workspace_bytes() bytes
  * (0 when the shape needs no split), which must be zero before the first
@@ -93,11 +95,12 @@ extern "C" {
 /* FP6_EDGE entries (int4; block_m 16 or 64, block_n 64) run the fp6 tiles on
  * shapes that are no multiple of them: the operands are converted with their
  * rows padded to 32 and K to 128, and the output stops at M and N.  They take
- * a workspace as FP6 entries do, of 3/4 byte per padded value, and K up to
- * 262144; the conversion is part of the launch.  Launched without a workspace
- * (or, by the no-allocation entry point, with one that does not fit its
- * scratch), the call runs on the best entry of the same family that needs
- * none; the results are the same. */
+ * a caller's workspace as FP6 entries do, of 3/4 byte per padded value, and K
+ * up to 262144; the conversion is part of the launch.  Launched without a
+ * workspace, or through the no-allocation entry point, whose scratch array
+ * they do not use, the call runs on the best entry of the same family that
+ * needs none (amd_strix_halo_kernels_launched_entry); the results are the
+ * same. */
 #define SHK_OPERANDS_FP6_EDGE 3
 
 /* Tile schedules of a dense entry (reference metadata.KernelSchedule,
@@ -261,7 +264,8 @@ int amd_strix_halo_kernels_launch_gemm_ws(int kernel_index, int device_index, ui
  * instead of a caller workspace; STREAM entries that split K keep their
  * arrival counters and partials there and clear the counters with a small
  * kernel on `stream` before the GEMM (two launches); PACKED entries need
- * none and run as amd_strix_halo_kernels_launch_gemm.  The array is reserved
+ * none and run as amd_strix_halo_kernels_launch_gemm, FP6_EDGE entries as
+ * there too.  The array is reserved
  * on every device where the library's code object is loaded, whether or not
  * this entry point is called.  The call allocates and frees nothing (its
  * first call on a device looks the array's address up once).  Shapes whose

@@ -339,6 +339,10 @@ int prepare_dense(DenseCall& c, int kernel_index, Phase phase, const void* a, co
                 (split > 1 ? " per K slice (K/SPLIT_K); got K/SPLIT_K=" + std::to_string(k / split)
                            : "; got " + std::to_string(k)));
   }
+  if (edge && workspace == kScratchPending) {  // (kept only where it refuses the call)
+    workspace = nullptr;
+    workspace_bytes = 0;
+  }
   if (fp6 && workspace == kScratchPending) {
     // the no-allocation entry point: the library's scratch array, whose
     // device address the caller fills in after validation
@@ -672,26 +676,34 @@ int best_entry(int bits, int layout, int subchannel, int epilogue, int schedule,
 // family, so that what a call may bring does not depend on which entry is
 // predicted fastest for its shape; requests that the entry itself refuses keep
 // it, for its error.
-//  * An FP6_EDGE entry without room for its converted operands (`room` bytes)
-//    to the best entry that reads the packed operands.
+//  * An FP6_EDGE entry without a caller's workspace to the best entry that
+//    reads the packed operands.  (The library's scratch array is not taken for
+//    it: calls on two streams that need no scratch by their shape may overlap.)
 //  * An FP6_EDGE entry or a skinny one that plans its rows, whose operands are
 //    not both 16-byte aligned, to the entry that the figures alone rank first,
 //    if that is a PACKED one: its MN-major operands need 8 bytes.
 int runnable_entry(int kernel_index, const void* a, const void* b, int m, int n, int k, int subchannel, int epilogue,
-                   uint64_t room) {
+                   bool workspace) {
   const auto& t = table();
   if (kernel_index < 0 || kernel_index >= (int)t.size()) return kernel_index;
   const shk_kernel_desc& d = t[kernel_index].d;
   const bool edge = d.operand_format == SHK_OPERANDS_FP6_EDGE;
   if ((!edge && !shk::sk_plans_rows(d)) || m <= 0 || n <= 0 || k <= 0) return kernel_index;
-  const bool fits = !edge || dense_workspace_bytes(d, m, n, k) <= room, whole = aligned(a, 16) && aligned(b, 16);
+  const bool fits = !edge || workspace, whole = aligned(a, 16) && aligned(b, 16);
   if (fits && whole) return kernel_index;
   if (!serves_family(d, d.dtype_bits, d.layout, subchannel, epilogue, d.schedule, 0) ||
       !accepts_shape(d, m, n, k, subchannel))
     return kernel_index;
-  const int other = best_entry(d.dtype_bits, d.layout, subchannel, epilogue, d.schedule, 1, m, n, k,
-                               whole ? DIRECT : FIGURES);
-  if (other < 0 || (!whole && t[other].d.operand_format != SHK_OPERANDS_PACKED)) return kernel_index;
+  auto best = [&](Among among) {
+    return best_entry(d.dtype_bits, d.layout, subchannel, epilogue, d.schedule, 1, m, n, k, among);
+  };
+  if (!whole) {
+    const int other = best(FIGURES);
+    if (other >= 0 && t[other].d.operand_format == SHK_OPERANDS_PACKED) return other;
+    if (fits) return kernel_index;
+  }
+  const int other = best(DIRECT);
+  if (other < 0) return kernel_index;
   return other;
 }
 
@@ -741,7 +753,7 @@ int amd_strix_halo_kernels_launched_entry(int kernel_index, const void* a, const
   g_last_error.clear();
   if (index == nullptr) return fail("index must be non-null");
   if (kernel_index < 0 || kernel_index >= (int)table().size()) return fail("kernel index out of range");
-  *index = runnable_entry(kernel_index, a, b, m, n, k, subchannel, epilogue, workspace ? UINT64_MAX : 0);
+  *index = runnable_entry(kernel_index, a, b, m, n, k, subchannel, epilogue, workspace != nullptr);
   return 0;
 }
 
@@ -759,7 +771,7 @@ int amd_strix_halo_kernels_launch_gemm_ws(int kernel_index, int device_index, ui
                                           int32_t out_mode, void* workspace, uint64_t workspace_bytes) {
   g_last_error.clear();
   DenseCall c;
-  kernel_index = runnable_entry(kernel_index, a, b, m, n, k, subchannel, epilogue, workspace ? UINT64_MAX : 0);
+  kernel_index = runnable_entry(kernel_index, a, b, m, n, k, subchannel, epilogue, workspace != nullptr);
   if (prepare_dense(c, kernel_index, PHASE_ALL, a, b, a_scale, b_scale, out, m, n, k, subchannel, epilogue,
                     out_mode, workspace, workspace_bytes))
     return 1;
@@ -777,14 +789,14 @@ int amd_strix_halo_kernels_launch_gemm_noalloc(int kernel_index, int device_inde
                                                int32_t epilogue, int32_t out_mode) {
   g_last_error.clear();
   DenseCall c;
-  kernel_index = runnable_entry(kernel_index, a, b, m, n, k, subchannel, epilogue, SHK_NOALLOC_SCRATCH_BYTES);
+  kernel_index = runnable_entry(kernel_index, a, b, m, n, k, subchannel, epilogue, false);
   if (prepare_dense(c, kernel_index, PHASE_ALL, a, b, a_scale, b_scale, out, m, n, k, subchannel, epilogue,
                     out_mode, kScratchPending, SHK_NOALLOC_SCRATCH_BYTES))
     return 1;
   DeviceGuard guard(device_index);
   if (guard.error() != hipSuccess) return fail_hip("hipSetDevice", guard.error());
   const bool split_stream = c.e->d.operand_format == SHK_OPERANDS_STREAM && c.p.sk_splits > 1;
-  if (c.e->d.operand_format == SHK_OPERANDS_FP6 || c.e->d.operand_format == SHK_OPERANDS_FP6_EDGE || split_stream) {
+  if (c.e->d.operand_format == SHK_OPERANDS_FP6 || split_stream) {
     void* ptr = nullptr;
     if (scratch_address(device_index, &ptr)) return 1;
     c.p.work = static_cast<uint8_t*>(ptr);

@@ -111,6 +111,29 @@ def test_operands_at_8_bytes_run_where_the_64_row_tile_does(sub, epilogue):
     assert bool(served) == bool(sub)
 
 
+def test_edge_entries_leave_the_scratch_array_alone():
+    """Without a caller's workspace, as through the no-allocation entry point,
+    an FP6_EDGE entry gives way for every shape, also one whose converted
+    operands would fit the scratch array: the array is shared by a device's
+    calls, and these shapes' calls may overlap."""
+    for d in EDGES:
+        sub = d.max_subchannel
+        epi = kt.EPILOGUE_SWIGLU if d.epilogue_kind == kt.EPI_KIND_SWIGLU else kt.EPILOGUE_NONE
+        for m, n, k in ((64, 64, 256), (1088, 11008, 4096)):
+            assert d.workspace_bytes(m, n, k) <= kt.NOALLOC_SCRATCH_BYTES
+            assert _launched(d.index, m, n, k, sub, epi) == d.index
+            for b in (1 << 20, (1 << 20) + 8):
+                got = kt.TABLE[_launched(d.index, m, n, k, sub, epi, b=b, workspace=None)]
+                assert not got.needs_workspace and got.layout == d.layout and got.epilogue_kind == d.epilogue_kind
+    # refused requests are refused before anything runs
+    lib = native.load_dispatch_library()
+    d, p = EDGES[0], 1 << 20
+    for m, b, message in ((72, p, b"not divisible"), (64, p + 4, b"aligned B")):
+        rc = lib.amd_strix_halo_kernels_launch_gemm_noalloc(d.index, 0, 0, p, b, p, p, p, m, 64, 256, 0,
+                                                            kt.EPILOGUE_NONE, kt.OUT_BF16)
+        assert rc == 1 and message in lib.amd_strix_halo_kernels_last_error()
+
+
 def test_edge_entries_bound_k():
     for d in EDGES:
         assert d.max_k == kt.FP6_MAX_K and not d.supports_k(kt.FP6_MAX_K + 64)
