@@ -390,6 +390,15 @@ int amd_strix_halo_kernels_launch_ragged_fwd_grouped(int kernel_index, int devic
                                                      int32_t k_packed, int32_t groups, int32_t subchannel,
                                                      int32_t out_mode, void* workspace, uint64_t workspace_bytes);
 
+/* The rows of the skinny tiles that amd_strix_halo_kernels_launch_ragged_fwd_grouped
+ * runs for these arguments (16, 32 or 64), or 0 where it runs the entry's own
+ * tiles; nothing is launched.  lhs and rhs are looked at for their alignment
+ * and may not be null.  Returns 0, or 1 with an error.  No counterpart in the
+ * reference. */
+int amd_strix_halo_kernels_ragged_fwd_rows(int kernel_index, const void* lhs, const void* rhs, int32_t m, int32_t n,
+                                           int32_t k_packed, int32_t groups, int32_t subchannel, int32_t* rows);
+
+
 /* ---- ragged backward --------------------------------------------------------
  * Replaces amd_strix_halo_kernels_launch_ragged_bwd_hsaco (dispatch.cpp:391-457)
  * as called by native.launch_ragged_bwd_kernel (native.py:603-667).

@@ -115,6 +115,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.amd_strix_halo_kernels_launch_ragged_fwd_grouped.argtypes = [I, I, U, P, P, P, P, P, I32, P, P, I32, P, I32,
                                                                      I32, I32, I32, I32, I32, P, ctypes.c_uint64]
     lib.amd_strix_halo_kernels_launch_ragged_fwd_grouped.restype = I
+    lib.amd_strix_halo_kernels_ragged_fwd_rows.argtypes = [I, P, P, I32, I32, I32, I32, I32, ctypes.POINTER(I32)]
+    lib.amd_strix_halo_kernels_ragged_fwd_rows.restype = I
     lib.amd_strix_halo_kernels_launch_ragged_bwd_ws.argtypes = [I, I, U, P, P, P, P, P, P, I32, I32, I32, I32, I32,
                                                                 I32, I32, P, ctypes.c_uint64]
     lib.amd_strix_halo_kernels_launch_ragged_bwd_ws.restype = I
@@ -638,6 +640,20 @@ def _ragged_workspace(torch, desc, like, m, n, k_packed, groups, stream, head: i
     if buf is not None and stream is not None:
         buf.record_stream(stream)
     return buf, nbytes
+
+
+def ragged_fwd_rows(lhs: Any, rhs: Any, *, layout: GemmLayout, subchannel: int | None, rows: int, cols: int,
+                    k_packed: int, groups: int, library_path=None) -> int:
+    """Rows of the skinny tiles that the fp6 ragged forward runs for a call
+    (operands, or their addresses), 0 where it runs its own."""
+    lib = _verified_library(library_path)
+    desc = kt.find_ragged(kt.FAMILY_RAGGED_FWD, layout=kt.LAYOUT_CODES[layout.value], subchannel=subchannel,
+                          block_m=kt.RAGGED_FP6_BLOCK_M, fp6=True)
+    out = ctypes.c_int32(-1)
+    a, b = (x if isinstance(x, int) else x.data_ptr() for x in (lhs, rhs))
+    _check(lib, lib.amd_strix_halo_kernels_ragged_fwd_rows(desc.index, a, b, rows, cols, k_packed, groups,
+                                                           subchannel or 0, ctypes.byref(out)))
+    return int(out.value)
 
 
 def launch_ragged_fwd(

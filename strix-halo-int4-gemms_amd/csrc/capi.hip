@@ -1005,6 +1005,28 @@ int amd_strix_halo_kernels_launch_ragged_fwd_ws(int kernel_index, int device_ind
                     capacity, out, m, n, k_packed, groups, subchannel, out_mode, workspace, workspace_bytes, nullptr);
 }
 
+int amd_strix_halo_kernels_ragged_fwd_rows(int kernel_index, const void* lhs, const void* rhs, int32_t m, int32_t n,
+                                           int32_t k_packed, int32_t groups, int32_t subchannel, int32_t* rows) {
+  g_last_error.clear();
+  const Entry* e = nullptr;
+  if (lookup(kernel_index, SHK_FAMILY_RAGGED_FWD, &e)) return 1;
+  if (rows == nullptr) return fail("rows must be non-null");
+  if (m <= 0 || n <= 0 || k_packed <= 0 || groups <= 0) return fail("sizes must be positive");
+  if (check_subchannel(e->d, subchannel)) return 1;
+  shk::RaggedFwdArgs p{};
+  p.lhs = static_cast<const uint8_t*>(lhs);
+  p.rhs = static_cast<const uint8_t*>(rhs);
+  p.M = m;
+  p.N = n;
+  p.K = 2 * k_packed;
+  p.groups = groups;
+  p.subchannel = subchannel;
+  p.layout = e->d.layout;
+  p.job.sizes = reinterpret_cast<const int32_t*>(lhs);  // (the rule asks only whether the call builds its list)
+  *rows = e->d.operand_format == SHK_OPERANDS_FP6 && groups <= shk::kFusedTaskGroups ? shk::ragged_skinny_rows(p) : 0;
+  return 0;
+}
+
 int amd_strix_halo_kernels_launch_ragged_fwd_grouped(int kernel_index, int device_index, uintptr_t stream,
                                                      const void* lhs, const void* rhs, const void* a_scale,
                                                      const void* b_scale, const int32_t* group_sizes,

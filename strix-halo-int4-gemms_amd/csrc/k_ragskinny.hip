@@ -113,12 +113,14 @@ __global__ __launch_bounds__(T::NT) void ragged_skinny_kernel(const RaggedFwdArg
     sk_unit_pc<T, true, true>(q, smem, &last_flag, lane, wave, row, tn * T::BN, 0, 1, 0);
 }
 
+// Workgroups of a launch of tiles of `rows` rows and `bn` columns: every
+// group's last block may be partial; one more builds the task list.
+long workgroups(const RaggedFwdArgs& a, int rows, int bn) {
+  return ((long)a.groups + a.M / rows) * ((a.N + bn - 1) / bn) + 1;
+}
 template <class T>
 hipError_t launch(const RaggedFwdArgs& a, hipStream_t s) {
-  // every group's last block may be partial
-  const long tasks = (long)a.groups + a.M / T::R;
-  const long tiles_n = (a.N + T::BN - 1) / T::BN;
-  hipLaunchKernelGGL(ragged_skinny_kernel<T>, dim3((unsigned)(tasks * tiles_n + 1)), dim3(T::NT), 0, s, a);
+  hipLaunchKernelGGL(ragged_skinny_kernel<T>, dim3((unsigned)workgroups(a, T::R, T::BN)), dim3(T::NT), 0, s, a);
   return hipGetLastError();
 }
 
@@ -131,8 +133,6 @@ hipError_t launch_rows(const RaggedFwdArgs& a, int rows, hipStream_t s) {
   if (rows == 16) return launch<C<LAYOUT, 16, false>>(a, s);
   return rows == 32 ? launch<C<LAYOUT, 32, false>>(a, s) : launch<C<LAYOUT, 64, false>>(a, s);
 }
-
-}  // namespace
 
 // What the host knows is the rows of all groups, so the rule goes by their
 // average r = M / groups, and by R-row tasks of groups * (r / R + 1/2).  Calls
@@ -153,14 +153,13 @@ hipError_t launch_rows(const RaggedFwdArgs& a, int rows, hipStream_t s) {
 //    1024 x 2048 89.8 and 104.6; r = 16: 131 and 105.
 // The path is taken where its prediction is 1.15 (subchannel 1.1) times
 // shorter, since uneven groups make more tasks than the average does.
-int ragged_skinny_rows(const RaggedFwdArgs& a) {
+int predicted_rows(const RaggedFwdArgs& a) {
   const bool nt = a.layout == SHK_LAYOUT_NT;
   if (a.job.sizes == nullptr || a.groups > kFusedTaskGroups || (a.layout != SHK_LAYOUT_NN && !nt)) return 0;
   // 16-byte pieces of both operands, 32-bit offsets
   auto aligned16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (!aligned16(a.lhs) || !aligned16(a.rhs) || a.K < 32 || a.K % 32 || a.N % 16) return 0;
   if (a.M > 65536 || a.K > 65536 || (long)a.N * a.K > (1L << 32)) return 0;
-  if (((long)a.groups + a.M / 16) * (a.N / 16) > (1L << 30)) return 0;
   const double g = a.groups, n = a.N, k = a.K, r = a.M / g;
   const double convert = 6.0 + 2.5e-7 * (a.M + g * n) * k;
   auto tasks = [&](int rows) { return std::max(std::min(g, (double)a.M), g * (r / rows + 0.5)); };
@@ -180,6 +179,17 @@ int ragged_skinny_rows(const RaggedFwdArgs& a) {
   const double low = 6.0 + 1.35 * product[i] * 16 * tasks(16) * n * k;
   const double high = 6.0 + product[i] * 32 * tasks(32) * n * k;
   return 1.1 * std::min(low, high) < fp6 ? (low <= high ? 16 : 32) : 0;
+}
+
+}  // namespace
+
+// The predicted choice, unless its grid is more than a launch can hold: below
+// 2^32 work-items, of at most 512 a workgroup (many experts with a very wide
+// N; the fp6 tiles are 128 columns wide).
+int ragged_skinny_rows(const RaggedFwdArgs& a) {
+  const int rows = predicted_rows(a);
+  const int bn = a.subchannel > 0 ? 16 : SK_BN, threads = rows == 16 && a.subchannel >= 128 ? 512 : 64 * SK_NW;
+  return rows && workgroups(a, rows, bn) * threads < (1L << 32) ? rows : 0;
 }
 
 hipError_t launch_ragged_skinny(const RaggedFwdArgs& a, int rows, hipStream_t s) {
