@@ -196,12 +196,13 @@ def _ragged_int_reference(a_q, b_q, sizes):
 
 
 @pytest.mark.parametrize("groups,align", [(5, 32), (37, 64), (1100, 32)])
-@pytest.mark.parametrize("fp6", [True, False], ids=["fp6", "packed"])
-def test_grouped_forward_builds_the_oracle_task_list(groups, align, fp6, device):
+@pytest.mark.parametrize("fp6,n", [(True, 64), (True, 72), (False, 64)], ids=["skinny", "fp6", "packed"])
+def test_grouped_forward_builds_the_oracle_task_list(groups, align, fp6, n, device):
     """amd_strix_halo_kernels_launch_ragged_fwd_grouped: the task list it
-    leaves in the caller's buffer (built inside the fp6 conversion launch for
-    up to 1024 groups, by the stand-alone launch otherwise) is the oracle's
-    calculate_group_info, and the output is the oracle's forward."""
+    leaves in the caller's buffer (built inside the fp6 conversion launch, or
+    by a workgroup of the skinny tiles, for up to 1024 groups, by the
+    stand-alone launch otherwise) is the oracle's calculate_group_info, and
+    the output is the oracle's forward."""
     import ctypes
 
     from amd_strix_halo_kernels import kernel_table as kt
@@ -209,7 +210,7 @@ def test_grouped_forward_builds_the_oracle_task_list(groups, align, fp6, device)
     r = ref.rng(stable_seed("grouped", groups, align, fp6))
     sizes = r.integers(0, 90, size=groups)
     sizes[r.integers(0, groups)] = 0
-    m, k, n = int(sizes.sum()) + 3, 128, 64
+    m, k = int(sizes.sum()) + 3, 128
     a_q, b_q, sa, sb = _fwd_case(stable_seed("grouped-op", groups), m, k, n, list(sizes), SCALES[0])
     tile = kt.RAGGED_FP6_BLOCK_M if fp6 else 64
     desc = kt.find_ragged(kt.FAMILY_RAGGED_FWD, layout=kt.LAYOUT_NN, subchannel=None, block_m=tile, fp6=fp6)
@@ -217,6 +218,10 @@ def test_grouped_forward_builds_the_oracle_task_list(groups, align, fp6, device)
     lhs, rhs = _pack_fwd(a_q, b_q, shk.GemmLayout.NN)
     lhs_d, rhs_d = to_dev(torch, lhs, device), to_dev(torch, rhs, device)
     sa_d, sb_d = to_dev(torch, sa, device), to_dev(torch, sb, device)
+    if fp6:
+        rows = native.ragged_fwd_rows(lhs_d, rhs_d, layout=shk.GemmLayout.NN, subchannel=None, rows=m, cols=n,
+                                      k_packed=k // 2, groups=groups)
+        assert (rows > 0) == (n % 16 == 0 and groups <= 1024)
     gs = torch.tensor(sizes, dtype=torch.int32, device=device)
     cap = kt.ragged_task_capacity(m, groups, tile)
     tasks = torch.full((cap, 4), -5, dtype=torch.int32, device=device)

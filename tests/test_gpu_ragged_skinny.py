@@ -16,6 +16,7 @@ torch = pytest.importorskip("torch")
 
 import amd_strix_halo_kernels as shk  # noqa: E402
 from amd_strix_halo_kernels import kernel_table as kt  # noqa: E402
+from amd_strix_halo_kernels import native  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -40,6 +41,9 @@ def test_ragged_skinny_tiles_match_the_oracle(name, sub, layout, device):
     print(f"case ragged skinny {layout.value} S={sub} {name} m={m}", flush=True)
     want = ref.ragged_fwd_reference(a_q, b_q, np.array(sizes), sa, sb, subchannel=sub)
     rows = sum(sizes)
+    picked = native.ragged_fwd_rows(1 << 20, 1 << 20, layout=layout, subchannel=sub, rows=m, cols=n, k_packed=k // 2,
+                                    groups=len(sizes))
+    assert picked > 0  # (freshly allocated operands are aligned)
 
     def run(mode):
         return _run_fwd_native(device, a_q, b_q, sizes, sa, sb, layout, kt.RAGGED_FP6_BLOCK_M, mode, fp6=True,
@@ -70,6 +74,9 @@ def test_both_ragged_paths_give_the_same_bits(sub, device):
     spec = shk.ScaleSpec(shk.ScaleMode.SUBCHANNEL, sub) if sub else shk.ScaleSpec(shk.ScaleMode.PER_CHANNEL)
     moved = torch.empty(lhs.numel() + 8, dtype=torch.uint8, device=device)[8:].view_as(lhs)
     moved.copy_(lhs)
+    picked = [native.ragged_fwd_rows(x, rhs, layout=shk.GemmLayout.NN, subchannel=sub, rows=rows, cols=n,
+                                     k_packed=k // 2, groups=groups) for x in (lhs, moved)]
+    assert picked[0] == 16 and picked[1] == 0
     for dtype in (torch.bfloat16, torch.float32):
         print(f"case ragged paths S={sub} {dtype}", flush=True)
         a = shk.ragged_dot_int4(lhs, rhs, sizes, a_scale=sa, b_scale=sb, scale=spec, output_dtype=dtype)
