@@ -268,6 +268,8 @@ def sk_plan(bits: int, sub: int, swiglu: bool, m: int, n: int, k: int, layout: i
         rows = 16 << i
         if i > 0 and m <= rows // 2:
             break
+        if not sub and m % rows and _sk_needed_splits(bits, k) > 1:
+            continue
         tiles = -(-m // rows) * (n // (SK_BN_SUBCH if sub else SK_BN))
         s = 1 if sub else _sk_splits(bits, tiles, k)
         u = tiles * s

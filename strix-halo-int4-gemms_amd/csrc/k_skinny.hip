@@ -11,6 +11,8 @@
 // (registry.py:230-251, split-K variants included), and split-K 2/4/8
 // (SUPPORTED_SPLIT_K).  append_skinny_rows_<bits>_<layout>() adds, at the
 // table's end, the entries that pick their tiles' height for each call.
+#include <algorithm>
+
 #include "shk_skinny.h"
 #include "shk_table.h"
 
@@ -30,14 +32,17 @@ constexpr int kLayout = SHK_LAYOUT;
 template <int R, bool SWIGLU, bool SUBCH>
 using SC = SkCfg<kBits, kLayout, R, SWIGLU, SUBCH>;
 
-// grid.x = output tiles; per-channel tiles run sk_splits workgroups each.
+// grid.x = output tiles; per-channel tiles run sk_splits workgroups each.  A
+// launch holds fewer than 2^32 work-items: past 2^22 workgroups (a multiple of
+// the XCDs) they stride over the units.
+constexpr unsigned kSkMaxGrid = 1u << 22;
 template <class C>
 unsigned sk_units(const DenseArgs& a, dim3 grid) {
   return grid.x * (unsigned)(C::SUBCH ? 1 : (a.sk_splits > 0 ? a.sk_splits : 1));
 }
 template <class C>
 hipError_t launch_sk_t(const DenseArgs& a, dim3 grid, hipStream_t s) {
-  hipLaunchKernelGGL(sk_gemm_kernel<C>, dim3(sk_units<C>(a, grid)), dim3(C::NT), 0, s, a);
+  hipLaunchKernelGGL(sk_gemm_kernel<C>, dim3(std::min(sk_units<C>(a, grid), kSkMaxGrid)), dim3(C::NT), 0, s, a);
   return hipGetLastError();
 }
 // An entry that plans its rows: tiles of the height that sk_plan picked,
@@ -46,7 +51,8 @@ template <class T>
 hipError_t launch_sk_rows(const DenseArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.M + T::R - 1) / T::R) * (unsigned)(a.N / T::BN));
   if (a.M % T::R == 0) return launch_sk_t<T>(a, grid, s);
-  hipLaunchKernelGGL((sk_gemm_kernel<T, true>), dim3(sk_units<T>(a, grid)), dim3(T::NT), 0, s, a);
+  hipLaunchKernelGGL((sk_gemm_kernel<T, true>), dim3(std::min(sk_units<T>(a, grid), kSkMaxGrid)), dim3(T::NT), 0, s,
+                     a);
   return hipGetLastError();
 }
 template <bool SWIGLU, bool SUBCH>

@@ -398,6 +398,9 @@ inline SkPlan sk_plan(int bits, int sub, bool swiglu, int layout, long m, long n
   for (int i = 0; i < (sub > 0 ? 2 : 3); ++i) {
     const int rows = 16 << i;
     if (i > 0 && m <= rows / 2) break;
+    // (where the K of one workgroup is bounded every tile keeps partials: no
+    // more of them than M has rows, so that the workspace fits where it did)
+    if (sub == 0 && m % rows != 0 && sk_needed_splits(bits, k) > 1) continue;
     const long tiles = (m + rows - 1) / rows * (sub > 0 ? n / 16 : n / 64);
     const int s = sub > 0 ? 1 : sk_splits(bits, tiles, k);
     const double u = (double)(tiles * s), w = (double)k / (double)s / 4096.0;

@@ -199,6 +199,20 @@ def test_entries_of_one_height_run_it():
     assert planned
 
 
+@pytest.mark.parametrize("layout", [kt.LAYOUT_NN, kt.LAYOUT_NT, kt.LAYOUT_TN])
+def test_planned_rows_need_no_more_workspace_past_one_workgroup_of_k(layout):
+    """int4 K past what one workgroup sums keeps int32 partials of every tile,
+    tens of MiB: an entry that plans its rows needs no more of them than the
+    entry of 16 rows, so that a call that fits the no-allocation scratch by its
+    rows fits it by its tiles."""
+    by = {d.plans_rows: d for d in kt.TABLE if d.is_stream and d.dtype_bits == 4 and d.layout == layout
+          and d.scale_mode == kt.SCALE_PER_CHANNEL and d.epilogue_kind == kt.EPI_KIND_PLAIN and d.block_m == 16
+          and d.split_k == 1 and d.schedule == kt.SCHEDULE_STANDARD}
+    for m, n, k in itertools.product((16, 48, 80, 112, 240, 1008), (64, 4800, 65536), (524288, 1 << 22, 1 << 24)):
+        assert by[True].workspace_bytes(m, n, k) <= by[False].workspace_bytes(m, n, k), (m, n, k)
+    assert by[True].workspace_bytes(48, 4800, 1 << 24) <= kt.NOALLOC_SCRATCH_BYTES
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("sub", [None, 32, 128])
 @pytest.mark.parametrize("epilogue", ["none", "swiglu"])
