@@ -7,7 +7,7 @@ another value corrupted the ragged fp6 forward's B-scale address for 16
 lanes of a wave, in a few tiles per call; the engines now name every
 fragment register in their waits.  This test compiles each translation unit
 that holds such a loop to gfx950 assembly (hipcc -S, as build.py compiles
-it) and scans it.  CPU only; about a minute."""
+it) and scans it.  CPU only; a minute or two."""
 
 from __future__ import annotations
 
@@ -24,7 +24,7 @@ from tests._asm_check import inflight_lds_hazards, sgpr_vmem_hazards
 ROOT = Path(__file__).resolve().parents[1]
 sys.path.insert(0, str(ROOT / "strix-halo-int4-gemms_amd"))
 
-UNITS = ("dense_f6", "ragged_f6", "dense_dma_4_0", "dense_dma_4_1", "dense_dma_4_2", "dense_dma_8_0", "dense_dma_8_1",
+UNITS = ("dense_f6", "edge_f6", "ragged_f6", "ragged_skinny", "dense_dma_4_0", "dense_dma_4_1", "dense_dma_4_2", "dense_dma_8_0", "dense_dma_8_1",
          "dense_dma_8_2", "skinny_4_0", "skinny_4_1", "skinny_4_2", "skinny_8_0", "skinny_8_1", "skinny_8_2")
 # every kernel unit (the SGPR-operand scan covers all of them)
 ALL_UNITS = UNITS + ("dense_4_0", "dense_4_1", "dense_4_2", "dense_8_0", "dense_8_1", "dense_8_2", "f6pack", "quant",
@@ -38,7 +38,7 @@ def assembly(tmp_path_factory):
     if shutil.which(build.hipcc()) is None and not Path(build.hipcc()).exists():
         pytest.skip("hipcc is not available")
     out = tmp_path_factory.mktemp("asm")
-    units = {name: (src, extra) for name, src, extra in build.translation_units() if name in ALL_UNITS}
+    units = {name: (src, extra) for name, src, extra in build.translation_units() if name != "capi"}
     assert set(units) == set(ALL_UNITS)
 
     def one(name):
@@ -101,6 +101,30 @@ def test_fp6_gemm_accumulators_are_written_only_by_mfmas(assembly):
             assert size and int(size.group(1)) < 64, (name, size and size.group(1))
         checked += 1
     assert checked >= 10
+
+
+def test_fp6_edge_accumulators_are_written_only_by_mfmas(assembly):
+    """The same for both tile heights of the edge GEMM, whose two K loops stand
+    in one kernel: within each run of MFMAs (none more than 120 lines from the
+    next; the epilogue between them is longer) no accumulator is written by
+    anything else and nothing goes to scratch."""
+    import re
+
+    checked = 0
+    for name, lines in _functions(assembly["edge_f6"]):
+        if "f6_edge_gemm" not in name:
+            continue
+        mf = [i for i, line in enumerate(lines) if "v_mfma" in line]
+        starts = [mf[0]] + [b for a, b in zip(mf, mf[1:]) if b - a > 120]
+        ends = [a for a, b in zip(mf, mf[1:]) if b - a > 120] + [mf[-1]]
+        assert len(starts) == 2, name
+        for a, b in zip(starts, ends):
+            bad = [lines[i].strip() for i in range(a, b)
+                   if re.search(r"v_accvgpr_(write|mov)|scratch_|^\s*v_\w+(_e\d+)?\s+a\[?\d", lines[i])
+                   and "v_mfma" not in lines[i]]
+            assert not bad, (name, bad[:4])
+        checked += 1
+    assert checked == 8
 
 
 def test_the_sgpr_scan_finds_a_reload_before_an_asm_load():
