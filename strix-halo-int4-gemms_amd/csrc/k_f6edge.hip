@@ -16,12 +16,12 @@ using C = Cfg<4, true, true, 256, BN, 128, 2, 2, SWIGLU, false, 64, false, 0>;
 // Per-channel 128 x 128 tile (shk_f6small.h): P ring slots, so three
 // workgroups a CU with two slots and two with three.  One workgroup alone on
 // a CU waits for its loads at every second stage with two slots: 256 tiles
-// of K = 4096 (1008 x 4096) 31.3 us a call, with three slots 26.1, with six
-// 26.6; from 384 tiles on two and three are within 2%.
+// of K = 4096 (1008 x 4096) 31.3 us a call, with three slots 26.1; from 384
+// tiles on two and three are within 2%.
 using CSmall = Cfg<4, true, true, 128, 128, 128, 2, 2, false, false, 64, false, 0>;
 
 template <int MODE, int EPI, int P>
-__global__ __launch_bounds__(256, P == 2 ? 3 : (P == 3 ? 2 : 1)) void f6_small_edge_kernel(const DenseArgs p) {
+__global__ __launch_bounds__(256, P == 2 ? 3 : 2) void f6_small_edge_kernel(const DenseArgs p) {
   using E = F6SmallEngine<CSmall, P>;
   __shared__ __attribute__((aligned(16))) uint8_t smem[E::LDS_BYTES + MFMA32_SCALE_BYTES];
   int tm, tn;

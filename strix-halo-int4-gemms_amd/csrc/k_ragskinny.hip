@@ -151,8 +151,10 @@ hipError_t launch_rows(const RaggedFwdArgs& a, int rows, hipStream_t s) {
 //    and 33.4; r = 64: 30.4 and 33.8; r = 1: 64 x 1024 x 2048 42.7 and 58.6;
 //    r = 16: 61.6 and 62.7; r = 32: 85.6 and 63.9.  Groups of 32: r = 4: 64 x
 //    1024 x 2048 89.8 and 104.6; r = 16: 131 and 105.
-// The path is taken where its prediction is 1.15 (subchannel 1.1) times
-// shorter, since uneven groups make more tasks than the average does.
+// The figures are fits to ragged calls, whose tiles find their rows and leave a
+// list (the dense tiles' stand at sk_plan).  The path is taken where its
+// prediction is 1.15 (subchannel 1.1) times shorter, since uneven groups make
+// more tasks than the average does.
 int predicted_rows(const RaggedFwdArgs& a) {
   const bool nt = a.layout == SHK_LAYOUT_NT;
   if (a.job.sizes == nullptr || a.groups > kFusedTaskGroups || (a.layout != SHK_LAYOUT_NN && !nt)) return 0;

@@ -860,7 +860,7 @@ template <class C>
 using F6Half = Cfg<4, true, true, 128, C::BN, C::BK, 2, 2, C::SWIGLU, false, C::MK, false, 0>;
 
 // The same tiles for any M, N and K (see f6_gemm_at's MASK).  The column
-// tiles from main_n on (the host's split, f6_edge_split) run last, as tiles
+// tiles from main_n on (the host's split, f6_edge_plan) run last, as tiles
 // of 128 rows.
 template <class C, int MODE, int EPI>
 __global__ __launch_bounds__(256) void f6_edge_gemm(const DenseArgs p) {

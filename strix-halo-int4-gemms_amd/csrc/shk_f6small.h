@@ -33,7 +33,7 @@ namespace shk {
 template <class C, int PS = 3>
 struct F6SmallEngine {
   static constexpr int P = PS;                      // ring slots
-  static_assert(P >= 2 && P <= 6, "two to six ring slots");
+  static_assert(P == 2 || P == 3, "two or three ring slots");
   static constexpr int NW = 4;
   static constexpr int PANEL = 2 * F6_BLOCK;        // 32 rows x 128 K: 3 KiB
   static constexpr int OPB = 4 * PANEL;             // one operand's stage: 12 KiB

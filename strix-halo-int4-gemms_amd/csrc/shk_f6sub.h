@@ -256,10 +256,9 @@ struct F6SubEngine {
                      :
                      : "v"(svo), "s"(rss_st), "{m0}"(sm0)
                      : "memory");
-    } else
-    // the compiler writes M0 before each statement; the MFMA is the wait
-    // state the LDS-DMA load needs after that write
-    if constexpr (T < OPW) {
+    } else if constexpr (T < OPW) {
+      // the compiler writes M0 before each statement; the MFMA is the wait
+      // state the LDS-DMA load needs after that write
       if constexpr (Z)
         asm volatile(
             "v_mfma_scale_f32_32x32x64_f8f6f4 %0, %1, %2, 0, %3, %3 op_sel_hi:[0,0,0] cbsz:2 blgp:2\n\t"
@@ -335,9 +334,9 @@ struct F6SubEngine {
                    : "+v"(fa[S][0][0]), "+v"(fb[S][0][0]), "+v"(fb[S][0][1]), "+v"(fa[S][1][0]), "+v"(fb[S][1][0]),
                      "+v"(fb[S][1][1])::"memory");
     else
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(fa[S][0][0]), "+v"(fa[S][0][1]), "+v"(fb[S][0][0]), "+v"(fb[S][0][1]), "+v"(fa[S][1][0]),
-                   "+v"(fa[S][1][1]), "+v"(fb[S][1][0]), "+v"(fb[S][1][1])::"memory");
+      asm volatile("s_waitcnt lgkmcnt(0)"
+                   : "+v"(fa[S][0][0]), "+v"(fa[S][0][1]), "+v"(fb[S][0][0]), "+v"(fb[S][0][1]), "+v"(fa[S][1][0]),
+                     "+v"(fa[S][1][1]), "+v"(fb[S][1][0]), "+v"(fb[S][1][1])::"memory");
   }
 
   // Stage k (128 K) on set S (ZERO: the first stage of a group; READ: the

@@ -609,7 +609,8 @@ __device__ __forceinline__ void sk_unit_pc(const DenseArgs& p, uint8_t* smem, in
 // place of two fill more of them (16 x 8192^2, groups of 128: 23.6 -> 21.6
 // us B MN-major, 18.5 -> 15.3 K-major; 256: 21.3 -> 19.6, 15.0 -> 13.7).
 // Shorter groups would load every stage once per group: four waves (groups
-// of 64: 28.4 us with four, 31.5 with eight).
+// of 64: 28.4 us with four, 31.5 with eight).  SwiGLU tiles, whose waves hold
+// two column tiles, run four; eight were not measured there.
 //
 // x of one group from its integer partials and the scales in the stage slot
 // (j: the group's slot among the stage's scales; odd_a[rt]: whether the
