@@ -305,7 +305,7 @@ def _sk_tile_rows(desc: "KernelDesc", m: int, n: int, k: int) -> int:
 
 def sk_split_count(desc: "KernelDesc", m: int, n: int, k: int, with_workspace: bool = True) -> int:
     """Workgroups sharing a skinny per-channel tile's K (shk_table.h
-    sk_split_count): about SK_TARGET_UNITS workgroups with at least two
+    sk_splits): about SK_TARGET_UNITS workgroups with at least two
     stages per wave, at most 16; for int4 enough to keep every wave within
     1023 stages of 128 K.  Without a workspace 1, or 0 if K needs a split."""
     if desc.scale_mode == SCALE_SUBCHANNEL:

@@ -303,7 +303,7 @@ class _GroupSizesCheck:
     stream, and finish() waits for it and raises: a call queues its kernels in
     between, so that the GPU goes on to them when the copy is done instead of
     idling for the host's part of the call (C5 forward, back-to-back calls:
-    59 -> 44 us, backward 70 -> 55).  Otherwise the check is made at once.  A
+    61 -> 46 us, backward 73 -> 59).  Otherwise the check is made at once.  A
     deferred check must not follow a write to a caller's tensor, and a stream
     under capture refuses the copy at once, as ever."""
 
