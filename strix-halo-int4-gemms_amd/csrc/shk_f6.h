@@ -643,15 +643,16 @@ __device__ __forceinline__ void mfma32_epilogue_lds(const E& e, const OutView& o
           }
         // one wave-uniform choice per 16 outputs: the hardware exp2 /
         // reciprocal path where it is accurate (fmax skips a NaN gate, which
-        // gives NaN on either path).  The edge tiles (MASK) keep expf and the
-        // division, as the skinny and register-staged tiles that share their
-        // shapes compute (1008 x 11008 x 4096, whole call: 88.6 us, 81.3 with
-        // the hardware path, whose fp32 results are up to 20 times further off).
-        if (!MASK && __all(gmax <= SWIGLU_FAST_MAX)) {
+        // gives NaN on either path).  The edge tiles (MASK) keep the precision
+        // of the skinny and register-staged tiles that share their shapes
+        // (1008 x 11008 x 4096, whole call, two boxes: 81.0 us with swiglu_fast and
+        // 87.9 with swiglu, 82.0 and 86.1 with swiglu_bounded).
+        if (__all(gmax <= SWIGLU_FAST_MAX)) {
 #pragma unroll
           for (int i = 0; i < E::MI; ++i)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) v[i][t] = swiglu_fast(up[i][t], gt[i][t]);
+            for (int t = 0; t < 4; ++t)
+              v[i][t] = MASK ? swiglu_bounded(up[i][t], gt[i][t]) : swiglu_fast(up[i][t], gt[i][t]);
         } else {
 #pragma unroll
           for (int i = 0; i < E::MI; ++i)

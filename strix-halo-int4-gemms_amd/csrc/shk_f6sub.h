@@ -1114,14 +1114,27 @@ __device__ __forceinline__ void f6sub_store_words(const E& e, const OutView& o, 
 
 // The SwiGLU results of a wave's 64 rows x 32 columns, up * silu(gate) of the
 // totals of j = 0 and 1, for the four columns of register group q of row
-// block i, with expf and the division, as the skinny and register-staged
-// tiles that share the shapes compute.
+// block i, at the precision of the skinny and register-staged tiles that share
+// the shapes: swiglu_bounded where every gate of the group's eight outputs a
+// lane is in its range, in every lane.
 template <class E>
 __device__ __forceinline__ void f6sub_swiglu(const E& e, int q, float (&v)[E::MI][4]) {
+  float gmax = 0.0f;
 #pragma unroll
   for (int i = 0; i < E::MI; ++i)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) v[i][t] = swiglu(e.tot[i][0][4 * q + t], e.tot[i][1][4 * q + t]);
+    for (int t = 0; t < 4; ++t) gmax = __builtin_fmaxf(gmax, __builtin_fabsf(e.tot[i][1][4 * q + t]));
+  if (__all(gmax <= SWIGLU_FAST_MAX)) {
+#pragma unroll
+    for (int i = 0; i < E::MI; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) v[i][t] = swiglu_bounded(e.tot[i][0][4 * q + t], e.tot[i][1][4 * q + t]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < E::MI; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) v[i][t] = swiglu(e.tot[i][0][4 * q + t], e.tot[i][1][4 * q + t]);
+  }
 }
 
 // Stores a SwiGLU tile, rows below o.row_hi and columns below o.col_hi (a

@@ -4,8 +4,8 @@ same operands without converting them.
 
 int32 sums are whole numbers and equal; per-channel bf16 results scale the
 same integers in the same order and equal bit for bit; SwiGLU goes through
-exp and stays within 2 bf16 ulp of the oracle, and equals the skinny tiles',
-which take the same expf and division."""
+exp and stays within 2 bf16 ulp of the oracle and one fp32 ulp of the skinny
+tiles."""
 
 from __future__ import annotations
 
@@ -162,10 +162,12 @@ def test_calls_with_operands_at_8_bytes(m, n, k, sub, layout, device):
 
 @pytest.mark.parametrize("mode", [kt.OUT_BF16, kt.OUT_F32], ids=["bf16", "f32"])
 @pytest.mark.parametrize("sub", [None, 32, 64, 128, 256])
-def test_swiglu_equals_the_skinny_tiles_bit_for_bit(sub, mode, device):
+def test_swiglu_is_as_precise_as_the_skinny_tiles(sub, mode, device):
     """Edge and skinny tiles share shapes, so a call must not lose precision by
-    which of them it runs: the same scaled sums through the same expf and
-    division, for gates of both signs up to some hundred."""
+    which of them it runs: the same scaled sums, gates of both signs up to some
+    hundred.  Both quotients round correctly but where the edge tile's last
+    rounding is a near tie (4 gates in 10^7): the fp32 results differ by one
+    ulp there, and up times them may by one more."""
     m, n, k = 208, 192, 768
     case = dense_case(stable_seed("edge-swiglu", sub, mode), bits=4, layout="nn", m=m, n=n, k=k, subchannel=sub,
                       swiglu=True, scale_lo=0.02, scale_hi=0.2)
@@ -184,7 +186,11 @@ def test_swiglu_equals_the_skinny_tiles_bit_for_bit(sub, mode, device):
         assert rc == 0, lib.amd_strix_halo_kernels_last_error()
         outs.append(out)
     assert float(outs[0].float().abs().max()) > 100.0
-    assert torch.equal(outs[0], outs[1])
+    if mode == kt.OUT_BF16:
+        assert torch.equal(outs[0], outs[1])
+    else:
+        ulps = (outs[0].view(torch.int32) - outs[1].view(torch.int32)).abs()
+        assert int(ulps.max()) <= 2 and float((ulps > 0).float().mean()) <= 1e-4
 
 
 @pytest.mark.parametrize("epilogue", ["none", "swiglu"])
