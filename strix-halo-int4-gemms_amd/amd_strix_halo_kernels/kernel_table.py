@@ -614,9 +614,9 @@ def predicted_us(desc: KernelDesc, m: int, n: int, k: int, sub: int | None = Non
       beside half-height tiles, which alone take 0.8).
 
     Fitted to calls drawn over M 16..8192, N 512..16384 and K 512..14336 in
-    every layout, each entry measured (us): the predicted choice takes 1.1%
-    (per-channel), 0.6% (subchannel) and 1.7, 0.4% (SwiGLU) more than the best
-    of the entries, and of 3978 calls 24 take 3% more than on the entry that
+    every layout, each entry measured (us): the predicted choice takes 1.2%
+    (per-channel), 0.6% (subchannel) and 0.8, 0.4% (SwiGLU) more than the best
+    of the entries, and of 5200 calls 23 take 3% more than on the entry that
     the figures alone, without predictions, rank first.  Groups of 64, 1536 x
     704 x 768 NT: 64 x 64 tile 12.4, edge 18.1, skinny 24.6; groups of 128, 320
     x 16384 x 4096 skinny 221, edge 56.5; per-channel 8176 x 16384 x 4096
